@@ -938,6 +938,245 @@ __global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) 
     }
 }
 
+// Closest hit with G lanes per ray, for launches with too few rays to fill the
+// chip: as with occlusion, the per-ray kernel then lasts as long as its
+// slowest ray's chain of dependent record loads.  A group of G lanes takes one
+// ray and one stack in LDS, kept in the reference's visiting order (the next
+// entry on top).  Each step up to G entries come off the top, lane 0's the
+// next in order; every lane tests its record's slots, or its leaf, at the
+// ray's tmax so far, and the passing slots go back in order.
+// The result is the reference's.  Its walk is a fold over the leaves in
+// visiting order: a leaf whose exact box passes at the current tmax offers
+// its nearest prim, which replaces the hit unless its t is past tmax (boxes
+// above the leaf pass whenever the leaf's does).  A leaf tested here at a
+// larger tmax than the walk would have there offers the same prim (the
+// nearest of its prims, the last of equal ones) or one the fold then refuses:
+// its entry distance and its t are compared with tmax again when it is
+// folded, and only in order -- when no entry before it may still hold a
+// leaf.  A leaf that offers a prim but has a record before it goes back on
+// the stack at its place; a leaf that offers none at the larger tmax offers
+// none later.  NaN needs no case of its own in the box test (the comparisons
+// are negated as in slab), but a hit at t = NaN takes the limit off tmax:
+// such a ray starts over, one entry a step and no slot left out by tmax
+// before it is popped, which is the reference's walk.
+// Stack bound: as in k_occlude_group, a leaf put back being one of the k
+// entries its step took.
+// What bounds it: latency, like the kernel it replaces.  GSTK_CL entries of
+// (ref, entry distance), 24 KB a block, leave six blocks a CU.
+// SEG: the rays come from a segment table (served launch) instead of one array.
+constexpr int GSTK_CL = 96;
+template <int G, bool SEG>
+__global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(6))) void k_closest_group(
+    SceneView sv, Ray* rays, uint32_t n_host, const uint32_t* n_dev, Hit* hits, uint32_t lim, uint32_t* err,
+    const TraceSeg* segs, uint32_t nseg) {
+    static_assert(G >= 2 && G <= 64 && (64 % G) == 0, "a group lies within one wave");
+    // (the grid covers n_host rays: a count on the device never exceeds it)
+    const uint32_t n = n_dev ? min(*n_dev, n_host) : n_host;
+    const uint32_t gpb = blockDim.x / G;  // groups per block
+    if ((uint64_t)blockIdx.x * gpb >= (uint64_t)n) return;
+    __shared__ int2 s_stk[MAX_BLOCK / G][GSTK_CL];  // ref, entry distance
+    const uint32_t tid = threadIdx.x, lane = __lane_id();
+    const uint32_t g = tid / G, gl = tid % G;
+    const uint32_t id = blockIdx.x * gpb + g;
+    uint32_t rid = id, rseg = 0;  // SEG: rid is the ray's index in segment rseg
+    const uint32_t gbase = lane & ~(uint32_t)(G - 1);
+    const unsigned long long gm = (G == 64 ? ~0ull : ((1ull << G) - 1ull)) << gbase;  // the group's lanes
+    const unsigned long long lowg = gm & (lane == 0 ? 0ull : (~0ull >> (64 - lane)));  // ... below this one
+    const unsigned long long highg = gm & ~lowg & ~(1ull << lane);                      // ... above it
+    int2* stk = s_stk[g];
+    RayState r{};
+    bool done = id >= n;
+    uint32_t top = 0;
+    if (!done) {
+        if (SEG) {
+            rseg = find_seg(segs, nseg, id);
+            rid = id - segs[rseg].start;
+            load_ray(segs[rseg].rays, rid, r);
+        } else {
+            load_ray(rays, rid, r);
+        }
+        float tn;
+        // the root's own box (popped first by the reference)
+        if (slab(sv.root_lo[0], sv.root_hi[0], sv.root_lo[1], sv.root_hi[1], sv.root_lo[2], sv.root_hi[2], r.ox,
+                 r.oy, r.oz, r.ix, r.iy, r.iz, r.tmin, r.tmax, &tn)) {
+            top = 1;
+            if (gl == 0) stk[0] = make_int2(sv.qroot, (int)0xFF800000u);
+        }
+        done = top == 0;
+    }
+    const float tmax0 = r.tmax;
+    const bool neg0 = r.ix < 0.0f, neg1 = r.iy < 0.0f, neg2 = r.iz < 0.0f;
+    const uint32_t negm = (neg0 ? 1u : 0u) | (neg1 ? 2u : 0u) | (neg2 ? 4u : 0u);
+    // every ray of the wave may take the ray-space record test (cq_fast_ray)
+    const bool wfast = cq_fast_scene(sv) && __ballot(id < n && !cq_fast_ray(r)) == 0ull;
+    uint32_t hpos = NO_HIT;
+    float hb1 = 0.0f, hb2 = 0.0f;
+    bool one = false;  // one entry a step
+    while (__any(!done)) {
+        // entries for this step: up to G, fewer near the stack's bound
+        uint32_t k = 0;
+        if (!done) {
+            k = top < (uint32_t)G ? top : (uint32_t)G;
+            const uint32_t room = top + 6u <= lim && !one ? (lim - top) / 3u : 1u;
+            k = k < room ? k : room;
+        }
+        int2 ent = make_int2(0, 0);
+        bool mine = gl < k;
+        if (mine) ent = stk[top - 1u - gl];
+        top -= k;
+        // the entry's box lies past the hit so far
+        mine = mine && !(as_f((uint32_t)ent.y) > r.tmax);
+        const int32_t ref = ent.x;
+        // what this lane puts back, in visiting order
+        int32_t r0 = 0, r1 = 0, r2 = 0, r3 = 0;
+        float t0 = 0.0f, t1 = 0.0f, t2 = 0.0f, t3 = 0.0f;
+        bool p0 = false, p1 = false, p2 = false, p3 = false;
+        // a leaf's offer
+        bool cand = false;
+        uint32_t cpos = NO_HIT;
+        float ct = 0.0f, cb1 = 0.0f, cb2 = 0.0f;
+        if (mine && ref >= 0) {
+            const float4* q = reinterpret_cast<const float4*>(sv.cnodes + ref);
+            const float4 W0 = q[0], W1 = q[1], W2 = q[2], W3 = q[3];
+            const uint32_t em = as_u(W0.w);
+            const uint32_t nqx = neg0 ? as_u(W1.y) : as_u(W1.x), fqx = neg0 ? as_u(W1.x) : as_u(W1.y);
+            const uint32_t nqy = neg1 ? as_u(W1.w) : as_u(W1.z), fqy = neg1 ? as_u(W1.z) : as_u(W1.w);
+            const uint32_t nqz = neg2 ? as_u(W2.y) : as_u(W2.x), fqz = neg2 ? as_u(W2.x) : as_u(W2.y);
+            r0 = (int)as_u(W2.z); r1 = (int)as_u(W2.w); r2 = (int)as_u(W3.x); r3 = (int)as_u(W3.y);
+            const uint32_t meta = em >> 24;
+            const float rtmax = one ? tmax0 : r.tmax;  // (one: tmax may rise again before the slot is popped)
+            if (wfast) {
+                const CqAxis X = cq_axis_ray(W0.x, em & 0xFFu, r.ox, r.ix);
+                const CqAxis Y = cq_axis_ray(W0.y, (em >> 8) & 0xFFu, r.oy, r.iy);
+                const CqAxis Z = cq_axis_ray(W0.z, (em >> 16) & 0xFFu, r.oz, r.iz);
+#define PX_CQ_SLOT(I) \
+    p##I = (r##I != QEMPTY) & slab_ray(nqx, fqx, nqy, fqy, nqz, fqz, I, X, Y, Z, r.tmin, rtmax, &t##I);
+                PX_CQ_SLOT(0)
+                PX_CQ_SLOT(1)
+                PX_CQ_SLOT(2)
+                PX_CQ_SLOT(3)
+#undef PX_CQ_SLOT
+            } else {
+                const float sx = cq_scale(em & 0xFFu), sy = cq_scale((em >> 8) & 0xFFu),
+                            sz = cq_scale((em >> 16) & 0xFFu);
+#define PX_CQ_SLOT(I)                                                                                         \
+    p##I = r##I != QEMPTY &&                                                                                  \
+           slab_signed(cq_bound(nqx, I, W0.x, sx), cq_bound(fqx, I, W0.x, sx), cq_bound(nqy, I, W0.y, sy),    \
+                       cq_bound(fqy, I, W0.y, sy), cq_bound(nqz, I, W0.z, sz), cq_bound(fqz, I, W0.z, sz),    \
+                       r.ox, r.oy, r.oz, r.ix, r.iy, r.iz, r.tmin, rtmax, &t##I);
+                PX_CQ_SLOT(0)
+                PX_CQ_SLOT(1)
+                PX_CQ_SLOT(2)
+                PX_CQ_SLOT(3)
+#undef PX_CQ_SLOT
+            }
+            // the reference's visiting order of the four slots (bvh.rs:409-415)
+            const bool nA = (negm >> (meta & 3u)) & 1u;
+            const bool nB = (negm >> ((meta >> 2) & 3u)) & 1u;
+            const bool nC = (negm >> ((meta >> 4) & 3u)) & 1u;
+#define PX_SWAP(C, I, J)                                                                 \
+    {                                                                                     \
+        const bool pa = C ? p##J : p##I, pb = C ? p##I : p##J;                            \
+        const int32_t ra = C ? r##J : r##I, rb = C ? r##I : r##J;                         \
+        const float ta = C ? t##J : t##I, tb = C ? t##I : t##J;                           \
+        p##I = pa; p##J = pb; r##I = ra; r##J = rb; t##I = ta; t##J = tb;                 \
+    }
+            PX_SWAP(nB, 0, 1)
+            PX_SWAP(nC, 2, 3)
+            PX_SWAP(nA, 0, 2)
+            PX_SWAP(nA, 1, 3)
+#undef PX_SWAP
+        } else if (mine) {
+            // leaf: its exact box, then prims in order until the record flagged last
+            uint32_t pos = (uint32_t)(~ref);
+            const float4* p = reinterpret_cast<const float4*>(sv.prims64 + pos);
+            float4 P2 = p[2], P3 = p[3];
+            if (slab(P2.y, P3.x, P2.z, P3.y, P2.w, P3.z, r.ox, r.oy, r.oz, r.ix, r.iy, r.iz, r.tmin, r.tmax, &t0)) {
+                const float tmax = r.tmax;  // the offer leaves the ray as it is
+                bool nan = false;
+                while (true) {
+                    const float4 P0 = p[0], P1 = p[1];
+                    const uint32_t kind = as_u(P3.w);
+                    if (prim_test64(sv, pos, P0, P1, P2, kind, r, &cpos, &cb1, &cb2)) {
+                        cand = true;
+                        nan = nan || r.tmax != r.tmax;
+                    }
+                    if (kind & 0x100u) break;
+                    ++pos;
+                    p += 4;
+                    P2 = p[2];
+                    P3 = p[3];
+                }
+                ct = nan && !one ? __builtin_nanf("") : r.tmax;
+                r.tmax = tmax;
+            }
+        }
+        // offers with no record before them are folded now, in order; the
+        // others go back as the leaves they came from
+        const unsigned long long rec = __ballot(p0 | p1 | p2 | p3);
+        const bool now = cand && (rec & lowg) == 0ull;
+        if (cand && !now) {
+            p0 = true;
+            r0 = ref;
+        }
+        unsigned long long fold = __ballot(now) & gm;
+        bool again = false;
+        while (__any(fold != 0ull)) {
+            const int src = fold ? __builtin_ctzll(fold) : (int)lane;
+            const float ft = __shfl(ct, src), fn = __shfl(t0, src);
+            const float fb1 = __shfl(cb1, src), fb2 = __shfl(cb2, src);
+            const uint32_t fp = (uint32_t)__shfl((int)cpos, src);
+            if (fold && (one || (!(fn > r.tmax) && !(ft > r.tmax)))) {
+                r.tmax = ft;
+                hpos = fp;
+                hb1 = fb1;
+                hb2 = fb2;
+                again = again || (ft != ft && !one);
+            }
+            fold &= fold - 1ull;
+        }
+        // the entries go on the stack, lane 0's on top: each lane's lie above
+        // those of its group's higher lanes (three ballots of the bits of each
+        // lane's count)
+        const uint32_t c = (p0 ? 1u : 0u) + (p1 ? 1u : 0u) + (p2 ? 1u : 0u) + (p3 ? 1u : 0u);
+        const unsigned long long c0 = __ballot(c & 1u), c1 = __ballot(c & 2u), c2 = __ballot(c & 4u);
+        const uint32_t pre = (uint32_t)__popcll(c0 & highg) + 2u * (uint32_t)__popcll(c1 & highg) +
+                             4u * (uint32_t)__popcll(c2 & highg);
+        const uint32_t tot = (uint32_t)__popcll(c0 & gm) + 2u * (uint32_t)__popcll(c1 & gm) +
+                             4u * (uint32_t)__popcll(c2 & gm);
+        if (!done) {
+            if (top + tot > (uint32_t)GSTK_CL) {
+                if (gl == 0) atomicOr(err, 1u);  // outside the bound above: never expected
+                done = true;
+            } else {
+                uint32_t w = top + pre;
+                if (p3) stk[w++] = make_int2(r3, (int)as_u(t3));
+                if (p2) stk[w++] = make_int2(r2, (int)as_u(t2));
+                if (p1) stk[w++] = make_int2(r1, (int)as_u(t1));
+                if (p0) stk[w] = make_int2(r0, (int)as_u(t0));
+                top += tot;
+            }
+            if (again) {
+                // a hit at t = NaN: from the root again, one entry a step
+                one = true;
+                r.tmax = tmax0;
+                hpos = NO_HIT;
+                hb1 = hb2 = 0.0f;
+                top = 1;
+                if (gl == 0) stk[0] = make_int2(sv.qroot, (int)0xFF800000u);
+            }
+            done = done || top == 0u;
+        }
+    }
+    if (id < n && gl == 0) {
+        Hit* hp = SEG ? segs[rseg].hits : hits;
+        Ray* rp = SEG ? segs[rseg].rays : rays;
+        const bool hit = hpos != NO_HIT;
+        hp[rid] = Hit{hit ? sv.order[hpos] : NO_HIT, hit ? r.tmax : 0.0f, hb1, hb2};
+        if (hit) rp[rid].tmax = r.tmax;
+    }
+}
+
 constexpr int PSTK = 96;  // stack entries per wave of the packet closest-hit kernel below
 constexpr int PWAVES = MAX_BLOCK / 64;
 
@@ -1417,6 +1656,7 @@ static bool use_compressed(const SceneView& s, const TraceTuning& tun) {
 // Four lanes a ray hold more registers and LDS per lane and lose to eight
 // wherever either wins.
 constexpr uint32_t GROUP_MAX = 1u << 20;
+constexpr uint32_t CLOSEST_GROUP_MAX = 1u << 20;
 static int group_lanes(const SceneView& s, uint32_t n, const TraceTuning& tun) {
     if (tun.lanes == 1 || !s.cnodes || !s.prims64) return 1;
     if (3u * (uint64_t)s.odepth + 8u > (uint64_t)GSTK) return 1;
@@ -1427,6 +1667,33 @@ static int group_lanes(const SceneView& s, uint32_t n, const TraceTuning& tun) {
 template <bool SEG>
 static auto group_kernel(int G) -> decltype(&k_occlude_group<8, SEG>) {
     return G == 4 ? &k_occlude_group<4, SEG> : G == 8 ? &k_occlude_group<8, SEG> : &k_occlude_group<16, SEG>;
+}
+template <bool SEG>
+static auto closest_group_kernel(int G) -> decltype(&k_closest_group<8, SEG>) {
+    return G == 4 ? &k_closest_group<4, SEG> : G == 8 ? &k_closest_group<8, SEG> : &k_closest_group<16, SEG>;
+}
+// Lanes per ray of a batched closest-hit launch of up to n rays, as
+// group_lanes.  From launches of random rays (origins in the box, uniform
+// directions, no limit) in random-triangle soups (us at 1 / 4 / 8 lanes per ray):
+//   16K triangles, 1,021 rays:         161 /   45 /   30
+//   16K triangles, 150,001 rays:       240 /  144 /  109
+//   16K triangles, 1,000,000 rays:     611 /  782 /  594
+//   200K triangles, 1,021 rays:        259 /   64 /   39
+//   200K triangles, 65,536 rays:       359 /  151 /   94
+//   200K triangles, 150,001 rays:      430 /  231 /  162
+//   200K triangles, 600,000 rays:      745 /  797 /  554
+//   200K triangles, 1,000,000 rays:    944 / 1285 /  883
+//   200K triangles, 2,000,000 rays:   1318 / 2495 / 1713
+//   500K triangles, 1,000,000 rays:   1022 / 1300 /  955
+//   500K triangles, 4,000,000 rays:   2498 / 5073 / 3689
+// The per-ray kernel's time starts at the slowest ray's chain (160-350 us)
+// and grows by about 0.4 ms a million rays; the group's starts at a
+// fraction of it and grows by about 0.9 ms, so the line is near 2^20 rays.
+static int closest_lanes(const SceneView& s, uint32_t n, const TraceTuning& tun) {
+    if (tun.lanes == 1 || !s.cnodes || !s.prims64) return 1;
+    if (3u * (uint64_t)s.qdepth + 8u > (uint64_t)GSTK_CL) return 1;
+    if (tun.lanes >= 2) return tun.lanes;
+    return n <= CLOSEST_GROUP_MAX ? 8 : 1;
 }
 
 size_t trace_any_block_spill(const SceneView& s, const TraceTuning& tun) {
@@ -1492,6 +1759,17 @@ static hipError_t launch(const SceneView& s, Ray* rays, uint32_t n, Hit* hits, u
             const auto kern = group_kernel<false>(G);
             hipLaunchKernelGGL(kern, dim3(grid), dim3(block), 0, st, s, rays, n, n_dev, occ, occ8, lim, err,
                                (const TraceSeg*)nullptr, 0u);
+            return hipGetLastError();
+        }
+    }
+    if constexpr (!ANY) {
+        const int G = cq ? closest_lanes(s, n, tun) : 1;
+        if (G > 1) {
+            const uint32_t lim = (uint32_t)GSTK_CL - 3u * s.qdepth;
+            const uint32_t gpb = (uint32_t)block / (uint32_t)G;
+            const unsigned grid = (unsigned)(((size_t)n + gpb - 1) / gpb);
+            hipLaunchKernelGGL(closest_group_kernel<false>(G), dim3(grid), dim3(block), 0, st, s, rays, n, n_dev, hits,
+                               lim, err, (const TraceSeg*)nullptr, 0u);
             return hipGetLastError();
         }
     }
@@ -1614,6 +1892,17 @@ hipError_t trace_segments(const SceneView& s, bool any, const TraceSeg* d_segs, 
             hipLaunchKernelGGL(group_kernel<true>(G), dim3(grid), dim3(block), 0, st, s, (const Ray*)nullptr, total,
                                (const uint32_t*)nullptr, (uint32_t*)nullptr, (uint8_t*)nullptr, lim, err, d_segs,
                                nseg);
+            return hipGetLastError();
+        }
+    }
+    if (!any && cq) {
+        const int G = closest_lanes(s, total, tun);
+        if (G > 1) {
+            const uint32_t lim = (uint32_t)GSTK_CL - 3u * s.qdepth;
+            const uint32_t gpb = (uint32_t)block / (uint32_t)G;
+            const unsigned grid = (unsigned)(((size_t)total + gpb - 1) / gpb);
+            hipLaunchKernelGGL(closest_group_kernel<true>(G), dim3(grid), dim3(block), 0, st, s, (Ray*)nullptr, total,
+                               (const uint32_t*)nullptr, (Hit*)nullptr, lim, err, d_segs, nseg);
             return hipGetLastError();
         }
     }

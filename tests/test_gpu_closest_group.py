@@ -1,0 +1,141 @@
+"""Closest hit with several lanes per ray (k_closest_group): batched launches
+of up to 2^20 rays against the oracle, bit for bit, at the sizes, trees and
+rays where its ordered commit could go wrong, and a host model of its stack."""
+import random
+
+import numpy as np
+import pytest
+
+import oracle_lib as ol
+import pbrt_rust_amd as px
+import test_group_stack_model as model
+from pbrt_rust_amd import scenes
+from gpu_util import F32, check_closest, mesh_pair, random_rays
+
+GSTK_CL = 96  # stack entries of a closest-hit group
+
+
+@pytest.fixture(params=[0, 1, 4, 8, 16])
+def lanes(request):
+    # 0: the rule by launch size; 1: the per-ray kernel
+    px.lib().pbrtx_set_ray_lanes(request.param)
+    yield request.param
+    px.reset_tuning()
+
+
+def tied_rays(v, idx, n, seed):
+    """Rays at an icosphere's vertices and edge midpoints: several faces share the closest t."""
+    rng = np.random.default_rng(seed)
+    f = idx[rng.integers(0, len(idx), n)]
+    tgt = np.where((rng.random(n) < 0.5)[:, None], v[f[:, 0]], 0.5 * (v[f[:, 0]] + v[f[:, 1]]))
+    o = (rng.normal(size=(n, 3)) * 1.2).astype(F32)
+    return o, (tgt - o).astype(F32)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("max_prims,split", [(1, "sah"), (4, "middle"), (8, "equal")])
+def test_ties_and_leaves_of_several_prims(lanes, max_prims, split):
+    v, idx = scenes.icosphere(4)
+    v, idx = v.astype(F32), idx.astype(np.uint32)
+    bvh, orc = mesh_pair(v, idx, split, max_prims)
+    o, d = tied_rays(v, idx, 20000, 3)
+    check_closest(bvh, orc, o, d)
+    check_closest(bvh, orc, o, d, mint=1e-3, maxt=0.9999)
+    # duplicated faces: every hit is tied
+    idx2 = np.concatenate([idx, idx[::-1]])
+    bvh, orc = mesh_pair(v, idx2, split, max_prims)
+    check_closest(bvh, orc, o, d)
+    px.synchronize()
+
+
+@pytest.mark.gpu
+def test_ragged_counts(lanes):
+    v, idx = scenes.random_triangles(5000, 21, 0.05, 0.3)
+    bvh, orc = mesh_pair(v, idx, "sah", 2)
+    for n in (1, 3, 4, 7, 8, 9, 15, 17, 31, 63, 65, 255, 257, 4099):
+        o, d = random_rays(n, 100 + n)
+        check_closest(bvh, orc, o, d)
+    px.synchronize()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,split", [(100, "middle"), (50, "middle"), (2000, "sah")])
+def test_deep_and_wide_frontiers(lanes, n, split):
+    # a chain too deep for the group stack (61 levels: the per-ray kernel), one
+    # that just fits, and thin triangles whose boxes all overlap (the stack
+    # fills to its bound and continues depth first)
+    if split == "middle":
+        xs = 2.0 ** np.arange(n)
+        v = np.concatenate([np.array([[x, 0, 0], [x, 1, 0], [x, 0, 1]]) for x in xs]).astype(F32)
+        o = np.concatenate([np.full((3000, 1), -1.0), np.random.default_rng(n).uniform(0.05, 0.7, (3000, 2))], 1)
+        d = np.tile(np.array([[1, 0, 0]], F32), (3000, 1))
+    else:
+        rng = np.random.default_rng(9)
+        z = np.sort(rng.uniform(-1, 1, n))
+        v = np.concatenate([np.array([[-1, -1, q], [1, 1, q], [-0.95, -1, q]]) for q in z]).astype(F32)
+        o = np.concatenate([rng.uniform(-1, 1, (4000, 2)), np.full((4000, 1), -2.0)], 1)
+        o[::3, 0] = rng.uniform(-0.99, -0.97, len(o[::3]))
+        o[::3, 1] = o[::3, 0] - 0.005
+        d = np.concatenate([rng.normal(0, 1e-3, (4000, 2)), np.ones((4000, 1))], 1)
+    idx = np.arange(3 * n, dtype=np.uint32).reshape(-1, 3)
+    bvh, orc = mesh_pair(v, idx, split)
+    check_closest(bvh, orc, o.astype(F32), d.astype(F32))
+    px.synchronize()  # raises if a traversal stack overflowed
+
+
+@pytest.mark.gpu
+def test_hits_at_nan_distance(lanes):
+    # triangles of size 1e-20 with a corner at the rays' origin: 1/div is
+    # infinite and t = 0 * inf = NaN, after which nothing limits tmax; the
+    # last prim that the reference meets wins
+    if lanes == 1:
+        pytest.skip("the per-ray kernel leaves out slots by the tmax of the time their record was read")
+    v, idx = scenes.random_triangles(400, 5, 0.1, 0.6)
+    e = 1e-20
+    tiny = np.array([[e, 0, 0], [0, e, 0], [0, 0, 0], [0, e, 0], [0, 0, e], [0, 0, 0]], F32)
+    idx = np.concatenate([idx, np.arange(6, dtype=np.uint32).reshape(2, 3) + len(v)])
+    v = np.concatenate([v, tiny])
+    bvh, orc = mesh_pair(v, idx, "sah")
+    _, d = random_rays(3000, 6)
+    o = np.zeros_like(d)
+    ref = orc.intersect(o, d, 0.0, float(np.finfo(np.float32).max), nthreads=4)
+    for path in ("plain", "batched"):
+        hits = bvh.intersect(px.RayBatch(o, d), path)
+        assert np.array_equal(hits["prim"], ref["prim"]), path
+        fin = np.isfinite(ref["t"]) & (ref["prim"] != px.NO_HIT)
+        assert np.array_equal(hits["t"][fin].view(np.uint32), ref["t"][fin].view(np.uint32))
+        assert np.isnan(hits["t"][np.isnan(ref["t"])]).all()
+    assert np.isnan(ref["t"]).any() and fin.any()
+    px.synchronize()
+
+
+def walk_put_back(tree, depth, G, rng):
+    """model.walk with leaves that go back on the stack while a record of the same step lies before them."""
+    lim = GSTK_CL - 3 * depth
+    assert 3 * depth + 8 <= GSTK_CL
+    stack, steps = [0], 0
+    while stack:
+        top = len(stack)
+        k = min(G, top, (lim - top) // 3 if top + 6 <= lim else 1)
+        taken = [stack.pop() for _ in range(k)]
+        pushes, record = [], False
+        for e in taken:  # in visiting order
+            if e is not None:
+                pushes.append(list(tree[e]))
+                record = record or bool(tree[e])
+            elif record and rng.random() < 0.7:
+                pushes.append([None])
+        for p in reversed(pushes):
+            stack.extend(reversed(p))
+        assert len(stack) <= GSTK_CL, len(stack)
+        steps += 1
+        assert steps < 200000
+    return steps
+
+
+@pytest.mark.parametrize("G", [4, 8, 16])
+@pytest.mark.parametrize("depth,fan", [(1, 0), (6, 4), (9, 3), (14, 2), (29, 1), (29, 2)])
+def test_model_of_the_stack_bound(G, depth, fan):
+    rng = random.Random(depth * 7 + fan + G)
+    tree = model.chain(depth) if fan == 0 else model.bushy(depth, fan, rng, 4000)
+    walk_put_back(tree, depth, G, rng)
