@@ -797,7 +797,8 @@ __global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) 
     // (the grid covers n_host rays: a count on the device never exceeds it)
     const uint32_t n = n_dev ? min(*n_dev, n_host) : n_host;
     const uint32_t gpb = blockDim.x / G;  // groups per block
-    if ((uint64_t)blockIdx.x * gpb >= (uint64_t)n) return;
+    // (bits: the grid covers n_host's words, and the blocks past n write zeros)
+    if ((occ8 || SEG) && (uint64_t)blockIdx.x * gpb >= (uint64_t)n) return;
     __shared__ int32_t s_stk[MAX_BLOCK / G][GSTK];
     const uint32_t tid = threadIdx.x, lane = __lane_id();
     const uint32_t g = tid / G, gl = tid % G;
@@ -928,13 +929,26 @@ __global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) 
         hit = hit || ghit;
         done = done || ghit || top == 0u;
     }
-    if (id < n && gl == 0) {
-        if (occ8) {
-            occ8[rid] = hit ? 1u : 0u;
-        } else if (hit) {
-            uint32_t* ow = SEG ? segs[rseg].occ : occ;
-            atomicOr(ow + (rid >> 5), 1u << (rid & 31u));
+    if (occ8 || SEG) {
+        if (id < n && gl == 0) {
+            if (occ8) occ8[rid] = hit ? 1u : 0u;
+            else if (hit) atomicOr(segs[rseg].occ + (rid >> 5), 1u << (rid & 31u));
         }
+        return;
+    }
+    // bits: the block's rays are gpb consecutive bits (8, 16, 32 or 64), so it
+    // writes them whole -- words that nobody has to clear first
+    __shared__ uint32_t s_bits[2];
+    if (tid < 2) s_bits[tid] = 0u;
+    __syncthreads();
+    if (gl == 0 && hit) atomicOr(&s_bits[g >> 5], 1u << (g & 31u));
+    __syncthreads();
+    const uint32_t base = blockIdx.x * gpb;
+    if (gpb >= 32u) {
+        if (tid < gpb / 32u && base + 32u * tid < n_host) occ[base / 32u + tid] = s_bits[tid];
+    } else if (tid == 0) {
+        if (gpb == 16u) reinterpret_cast<uint16_t*>(occ)[base / 16u] = (uint16_t)s_bits[0];
+        else reinterpret_cast<uint8_t*>(occ)[base / 8u] = (uint8_t)s_bits[0];
     }
 }
 
@@ -1655,13 +1669,17 @@ static bool use_compressed(const SceneView& s, const TraceTuning& tun) {
 // loads; with many, the group's idle lanes (a narrow frontier) cost more.
 // Four lanes a ray hold more registers and LDS per lane and lose to eight
 // wherever either wins.
+// Sixteen lanes a ray (us at 8 / 16 lanes, as above): 16K triangles, 1,021 rays 20.6 / 15.8,
+// 8,000 rays 19.9 / 16.8, 20,011 rays 23.3 / 23.8, 40,000 rays 29.5 / 36.0;
+// 500K triangles 32.0 / 23.0, 35.5 / 31.1, 48.3 / 44.0, 51.8 / 64.9: ahead
+// while the launch leaves half the chip's wave slots empty.
 constexpr uint32_t GROUP_MAX = 1u << 20;
-constexpr uint32_t CLOSEST_GROUP_MAX = 1u << 20;
+constexpr uint32_t GROUP16_MAX = 1u << 14;
 static int group_lanes(const SceneView& s, uint32_t n, const TraceTuning& tun) {
     if (tun.lanes == 1 || !s.cnodes || !s.prims64) return 1;
     if (3u * (uint64_t)s.odepth + 8u > (uint64_t)GSTK) return 1;
     if (tun.lanes >= 2) return tun.lanes;
-    return n <= GROUP_MAX ? 8 : 1;
+    return n <= GROUP16_MAX ? 16 : n <= GROUP_MAX ? 8 : 1;
 }
 
 template <bool SEG>
@@ -1689,11 +1707,17 @@ static auto closest_group_kernel(int G) -> decltype(&k_closest_group<8, SEG>) {
 // The per-ray kernel's time starts at the slowest ray's chain (160-350 us)
 // and grows by about 0.4 ms a million rays; the group's starts at a
 // fraction of it and grows by about 0.9 ms, so the line is near 2^20 rays.
+// Sixteen lanes (us at 8 / 16): 16K triangles, 1,021 rays 31.7 / 22.2, 16,000
+// rays 34.2 / 29.3, 24,000 rays 38.5 / 37.3; 200K triangles 42.2 / 33.7, 65.4
+// / 57.0, 66.9 / 73.6; but 500K triangles 45.7 / 54.9, 61.1 / 67.6, 66.1 /
+// 79.8: entries further down the ordered stack are more often past the hit,
+// and their reads miss the L2 there.
+constexpr uint32_t CLOSEST16_PRIMS = 1u << 18;
 static int closest_lanes(const SceneView& s, uint32_t n, const TraceTuning& tun) {
     if (tun.lanes == 1 || !s.cnodes || !s.prims64) return 1;
     if (3u * (uint64_t)s.qdepth + 8u > (uint64_t)GSTK_CL) return 1;
     if (tun.lanes >= 2) return tun.lanes;
-    return n <= CLOSEST_GROUP_MAX ? 8 : 1;
+    return n <= GROUP16_MAX && s.n_prims <= CLOSEST16_PRIMS ? 16 : n <= GROUP_MAX ? 8 : 1;
 }
 
 size_t trace_any_block_spill(const SceneView& s, const TraceTuning& tun) {
@@ -1725,16 +1749,18 @@ static hipError_t launch(const SceneView& s, Ray* rays, uint32_t n, Hit* hits, u
     if (n == 0) return hipSuccess;
     const int block = tun.block;
     if (block != 64 && block != 128 && block != 256) return hipErrorInvalidValue;
-    if (ANY && !occ8) {
-        hipError_t e = fill_u32(occ, 0u, ((size_t)n + 31) / 32, st);
-        if (e != hipSuccess) return e;
-    }
     uint32_t* err = scr->counter + 1;
+    // the plain and the per-ray kernel set the bits of the rays that hit
+    auto clear_bits = [&]() -> hipError_t {
+        return ANY && !occ8 ? fill_u32(occ, 0u, ((size_t)n + 31) / 32, st) : hipSuccess;
+    };
     if (path == PATH_PLAIN) {
         if (n_dev) return hipErrorInvalidValue;
         const int grid = plain_grid(n, block);
         const uint32_t lv = plain_levels(s);
         if ((size_t)lv * grid * block * sizeof(uint32_t) > scr->spill_bytes) return hipErrorInvalidValue;
+        const hipError_t e = clear_bits();
+        if (e != hipSuccess) return e;
         hipLaunchKernelGGL(k_trace_plain<ANY>, dim3(grid), dim3(block), 0, st, s, rays, n, hits, occ, occ8,
                            (uint32_t*)scr->spill, lv, err);
         return hipGetLastError();
@@ -1751,11 +1777,13 @@ static hipError_t launch(const SceneView& s, Ray* rays, uint32_t n, Hit* hits, u
     if (!stack_supported(tun.stack)) return hipErrorInvalidValue;
     const bool cq = use_compressed(s, tun);
     if (ANY && cq && s.prims64) {
-        const int G = group_lanes(s, n, tun);
+        int G = group_lanes(s, n, tun);
+        if (!occ8 && block / G < 8) G = 8;  // bits: at least a byte of them a block
         if (G > 1) {
             const uint32_t lim = (uint32_t)GSTK - 3u * s.odepth;
             const uint32_t gpb = (uint32_t)block / (uint32_t)G;
-            const unsigned grid = (unsigned)(((size_t)n + gpb - 1) / gpb);
+            const size_t cover = occ8 ? (size_t)n : ((size_t)n + 31) / 32 * 32;
+            const unsigned grid = (unsigned)((cover + gpb - 1) / gpb);
             const auto kern = group_kernel<false>(G);
             hipLaunchKernelGGL(kern, dim3(grid), dim3(block), 0, st, s, rays, n, n_dev, occ, occ8, lim, err,
                                (const TraceSeg*)nullptr, 0u);
@@ -1783,7 +1811,9 @@ static hipError_t launch(const SceneView& s, Ray* rays, uint32_t n, Hit* hits, u
         grid = (int)(scr->spill_bytes / per_block);
     }
     uint32_t* parts = scr->counter + WIDE_PARTS_AT;
-    hipError_t e = fill_u32(parts, 0u, (size_t)WIDE_PARTS * WIDE_PART_STRIDE, st);
+    hipError_t e = ANY && !occ8 ? zero3_u32(parts, (size_t)WIDE_PARTS * WIDE_PART_STRIDE, occ, ((size_t)n + 31) / 32,
+                                            nullptr, 0, st)
+                                : fill_u32(parts, 0u, (size_t)WIDE_PARTS * WIDE_PART_STRIDE, st);
     if (e != hipSuccess) return e;
     const uint32_t refill = (uint32_t)(tun.refill_pct < 0 ? 0 : (tun.refill_pct > 100 ? 100 : tun.refill_pct));
     hipLaunchKernelGGL(kern, dim3(grid), dim3(block), 0, st, s, rays, n, n_dev, hits, occ, occ8, parts,

@@ -1,6 +1,7 @@
-"""Closest hit with several lanes per ray (k_closest_group): batched launches
-of up to 2^20 rays against the oracle, bit for bit, at the sizes, trees and
-rays where its ordered commit could go wrong, and a host model of its stack."""
+"""Queries with several lanes per ray, batched launches of up to 2^20 rays.
+Closest hit (k_closest_group) against the oracle, bit for bit, at the sizes,
+trees and rays where its ordered commit could go wrong, and a host model of
+its stack; occlusion's bit words (k_occlude_group), which its blocks write whole."""
 import random
 
 import numpy as np
@@ -107,6 +108,33 @@ def test_hits_at_nan_distance(lanes):
         assert np.isnan(hits["t"][np.isnan(ref["t"])]).all()
     assert np.isnan(ref["t"]).any() and fin.any()
     px.synchronize()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("block", [64, 128, 256])
+@pytest.mark.parametrize("g", [0, 1, 4, 8, 16])
+def test_occlusion_words_are_written_whole(block, g):
+    # occlusion bits into words that hold ones before the call: every word of
+    # the rays is written, the bits past the last ray are zero, and the word
+    # after them is left alone
+    v, idx = scenes.random_triangles(4000, 31, 0.05, 0.2)
+    bvh, orc = mesh_pair(v, idx)
+    try:
+        px.set_tuning("batched", "any", block, 0, 60, "ray", lanes=g)
+        for n in (1, 7, 8, 9, 16, 31, 32, 33, 63, 64, 65, 129, 1000, 20011):
+            o, d = random_rays(n, 200 + n)
+            rays = px.DeviceBuffer.from_array(px.RayBatch(o, d, 0.0, 0.7).a)
+            nw = (n + 31) // 32
+            bits = px.DeviceBuffer.from_array(np.full(nw + 1, 0xFFFFFFFF, np.uint32))
+            bvh.intersect_p_device(rays.ptr, n, bits.ptr)
+            px.synchronize()
+            got = bits.download(np.uint32, nw + 1)
+            assert got[nw] == 0xFFFFFFFF
+            got = np.unpackbits(got[:nw].view(np.uint8), bitorder="little")
+            ref, _ = orc.intersect_p(o, d, 0.0, 0.7, nthreads=4)
+            assert np.array_equal(got[:n], ref.astype(np.uint8)) and not got[n:].any(), n
+    finally:
+        px.reset_tuning()
 
 
 def walk_put_back(tree, depth, G, rng):
