@@ -153,7 +153,7 @@ int pbrtx_set_tuning(int32_t path, int32_t kind, int32_t block, int32_t blocks_p
    that kind.  Process-wide setting, kept by pbrtx_set_tuning. */
 int pbrtx_set_stack_depth(int32_t path, int32_t kind, int32_t entries);
 /* Lanes per ray of the batched path's closest-hit and occlusion queries (the
-   per-ray scheme): 0 (the default) chooses by launch size, several lanes per
+   per-ray scheme): 0 (the default) chooses by launch size, up to 32 lanes per
    ray for launches too small to fill the GPU; 1 always one; 4, 8 or 16 always
    that many (when the scene has the compressed records and its record depth
    fits the group stack, else one).  No reference counterpart: a launch

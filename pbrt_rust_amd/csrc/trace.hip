@@ -787,19 +787,25 @@ __global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) 
 // odepth = GSTK (three pending slots per record level below the entry it
 // started from, the fourth child taken), and every run starts from a top of
 // at most lim (the first step, or one after a step of k >= 2).
+// Blocks are as small as whole bytes of result bits allow, so that a finished
+// wave's LDS goes to the next one: 2^20 rays in 200K triangles 572 us with
+// 256 threads a block, 557 with 64.
 // SEG: the rays come from a segment table (served launch) instead of one array.
-constexpr int GSTK = 128;
+// More lanes take more entries a step and need the room for them.
+constexpr int gstk_occlude(int G) { return G <= 8 ? 128 : (G == 16 ? 192 : 256); }
+constexpr int oc_block(int G) { return G <= 8 ? 64 : 8 * G; }
 template <int G, bool SEG>
-__global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) void k_occlude_group(
+__global__ __launch_bounds__(oc_block(G)) __attribute__((amdgpu_waves_per_eu(8))) void k_occlude_group(
     SceneView sv, const Ray* rays, uint32_t n_host, const uint32_t* n_dev, uint32_t* occ, uint8_t* occ8,
     uint32_t lim, uint32_t* err, const TraceSeg* segs, uint32_t nseg) {
     static_assert(G >= 2 && G <= 64 && (64 % G) == 0, "a group lies within one wave");
     // (the grid covers n_host rays: a count on the device never exceeds it)
     const uint32_t n = n_dev ? min(*n_dev, n_host) : n_host;
-    const uint32_t gpb = blockDim.x / G;  // groups per block
+    const uint32_t gpb = oc_block(G) / G;  // groups per block
     // (bits: the grid covers n_host's words, and the blocks past n write zeros)
     if ((occ8 || SEG) && (uint64_t)blockIdx.x * gpb >= (uint64_t)n) return;
-    __shared__ int32_t s_stk[MAX_BLOCK / G][GSTK];
+    constexpr int GSTK = gstk_occlude(G);
+    __shared__ int32_t s_stk[oc_block(G) / G][GSTK];
     const uint32_t tid = threadIdx.x, lane = __lane_id();
     const uint32_t g = tid / G, gl = tid % G;
     const uint32_t id = blockIdx.x * gpb + g;
@@ -975,20 +981,28 @@ __global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) 
 // before it is popped, which is the reference's walk.
 // Stack bound: as in k_occlude_group, a leaf put back being one of the k
 // entries its step took.
-// What bounds it: latency, like the kernel it replaces.  GSTK_CL entries of
-// (ref, entry distance), 24 KB a block, leave six blocks a CU.
+// What bounds it: the latency of its chain of dependent record reads, like
+// the kernel it replaces, with about a quarter of the steps.  One wave a
+// block, so that a finished wave's LDS goes to the next one (2^20 rays in
+// 200K triangles 943 us with 256 threads a block, 906 with 64), and stacks of
+// (ref, entry distance) as deep as six waves a SIMD leave room for: the room
+// decides how many entries a step may take in a deep tree (2^20 rays in 500K
+// triangles, 8 lanes: 984 us with 96 entries, 1436 with 72 though eight waves
+// fit then, 1105 with 128; 1,021 rays, 16 lanes: 52 us with 96, 29 with 160).
 // SEG: the rays come from a segment table (served launch) instead of one array.
-constexpr int GSTK_CL = 96;
+constexpr int CL_BLOCK = 64;
+constexpr int gstk_closest(int G) { return G <= 8 ? 96 : (G == 16 ? 160 : 192); }
 template <int G, bool SEG>
-__global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(6))) void k_closest_group(
+__global__ __launch_bounds__(CL_BLOCK) __attribute__((amdgpu_waves_per_eu(6))) void k_closest_group(
     SceneView sv, Ray* rays, uint32_t n_host, const uint32_t* n_dev, Hit* hits, uint32_t lim, uint32_t* err,
     const TraceSeg* segs, uint32_t nseg) {
     static_assert(G >= 2 && G <= 64 && (64 % G) == 0, "a group lies within one wave");
     // (the grid covers n_host rays: a count on the device never exceeds it)
     const uint32_t n = n_dev ? min(*n_dev, n_host) : n_host;
-    const uint32_t gpb = blockDim.x / G;  // groups per block
+    const uint32_t gpb = CL_BLOCK / G;  // groups per block
     if ((uint64_t)blockIdx.x * gpb >= (uint64_t)n) return;
-    __shared__ int2 s_stk[MAX_BLOCK / G][GSTK_CL];  // ref, entry distance
+    constexpr int GSTK_CL = gstk_closest(G);
+    __shared__ int2 s_stk[CL_BLOCK / G][GSTK_CL];  // ref, entry distance
     const uint32_t tid = threadIdx.x, lane = __lane_id();
     const uint32_t g = tid / G, gl = tid % G;
     const uint32_t id = blockIdx.x * gpb + g;
@@ -1669,26 +1683,37 @@ static bool use_compressed(const SceneView& s, const TraceTuning& tun) {
 // loads; with many, the group's idle lanes (a narrow frontier) cost more.
 // Four lanes a ray hold more registers and LDS per lane and lose to eight
 // wherever either wins.
-// Sixteen lanes a ray (us at 8 / 16 lanes, as above): 16K triangles, 1,021 rays 20.6 / 15.8,
-// 8,000 rays 19.9 / 16.8, 20,011 rays 23.3 / 23.8, 40,000 rays 29.5 / 36.0;
-// 500K triangles 32.0 / 23.0, 35.5 / 31.1, 48.3 / 44.0, 51.8 / 64.9: ahead
-// while the launch leaves half the chip's wave slots empty.
+// While the launch leaves most of the chip's wave slots empty, more lanes a ray
+// still gain (us at 8 / 16 / 32 lanes):
+//   16K triangles:   1,021 rays 17.2 / 13.2 / 13.0;   8,000 rays 18.0 / 14.2 / 17.9;
+//                   20,011 rays 20.7 / 22.9 / 31.9;  32,768 rays 24.1 / 28.6 / 45.9
+//   200K triangles:  4,000 rays 32.7 / 23.7 / 17.6;  20,011 rays 40.9 / 33.5 / 41.6;
+//                   32,768 rays 48.1 / 45.0 / 60.3;  50,000 rays 55.2 / 56.9 / 84.2
+//   500K triangles:  4,000 rays 28.5 / 21.3 / 20.0;  32,768 rays 47.6 / 43.0 / 61.9
+// Sixteen lanes end sooner in a small scene, whose records the caches hold.
 constexpr uint32_t GROUP_MAX = 1u << 20;
-constexpr uint32_t GROUP16_MAX = 1u << 14;
+constexpr uint32_t GROUP32_MAX = 1u << 12;
+static uint32_t group16_max(const SceneView& s) { return s.n_prims >= (1u << 16) ? 1u << 15 : 1u << 14; }
 static int group_lanes(const SceneView& s, uint32_t n, const TraceTuning& tun) {
     if (tun.lanes == 1 || !s.cnodes || !s.prims64) return 1;
-    if (3u * (uint64_t)s.odepth + 8u > (uint64_t)GSTK) return 1;
+    if (3u * (uint64_t)s.odepth + 8u > (uint64_t)gstk_occlude(8)) return 1;
     if (tun.lanes >= 2) return tun.lanes;
-    return n <= GROUP16_MAX ? 16 : n <= GROUP_MAX ? 8 : 1;
+    return n <= GROUP32_MAX ? 32 : n <= group16_max(s) ? 16 : n <= GROUP_MAX ? 8 : 1;
 }
 
 template <bool SEG>
 static auto group_kernel(int G) -> decltype(&k_occlude_group<8, SEG>) {
-    return G == 4 ? &k_occlude_group<4, SEG> : G == 8 ? &k_occlude_group<8, SEG> : &k_occlude_group<16, SEG>;
+    return G == 4    ? &k_occlude_group<4, SEG>
+           : G == 8  ? &k_occlude_group<8, SEG>
+           : G == 16 ? &k_occlude_group<16, SEG>
+                     : &k_occlude_group<32, SEG>;
 }
 template <bool SEG>
 static auto closest_group_kernel(int G) -> decltype(&k_closest_group<8, SEG>) {
-    return G == 4 ? &k_closest_group<4, SEG> : G == 8 ? &k_closest_group<8, SEG> : &k_closest_group<16, SEG>;
+    return G == 4    ? &k_closest_group<4, SEG>
+           : G == 8  ? &k_closest_group<8, SEG>
+           : G == 16 ? &k_closest_group<16, SEG>
+                     : &k_closest_group<32, SEG>;
 }
 // Lanes per ray of a batched closest-hit launch of up to n rays, as
 // group_lanes.  From launches of random rays (origins in the box, uniform
@@ -1707,17 +1732,18 @@ static auto closest_group_kernel(int G) -> decltype(&k_closest_group<8, SEG>) {
 // The per-ray kernel's time starts at the slowest ray's chain (160-350 us)
 // and grows by about 0.4 ms a million rays; the group's starts at a
 // fraction of it and grows by about 0.9 ms, so the line is near 2^20 rays.
-// Sixteen lanes (us at 8 / 16): 16K triangles, 1,021 rays 31.7 / 22.2, 16,000
-// rays 34.2 / 29.3, 24,000 rays 38.5 / 37.3; 200K triangles 42.2 / 33.7, 65.4
-// / 57.0, 66.9 / 73.6; but 500K triangles 45.7 / 54.9, 61.1 / 67.6, 66.1 /
-// 79.8: entries further down the ordered stack are more often past the hit,
-// and their reads miss the L2 there.
-constexpr uint32_t CLOSEST16_PRIMS = 1u << 18;
+// More lanes (us at 8 / 16 / 32):
+//   16K triangles:   1,021 rays 28.1 / 20.5 / 19.5;   8,000 rays 29.7 / 22.7 / 25.7;
+//                   20,000 rays 39.0 / 35.1 / 46.7;  32,768 rays 44.8 / 46.2 / 67.9
+//   200K triangles:  1,021 rays 38.6 / 28.7 / 23.9;  20,000 rays 67.4 / 50.1 / 67.8;
+//                   32,768 rays 68.7 / 72.2 / 96.0
+//   500K triangles:  4,000 rays 45.6 / 37.2 / 33.7;  20,000 rays 64.8 / 55.0 / 73.4
+constexpr uint32_t CLOSEST16_MAX = 3u << 13;
 static int closest_lanes(const SceneView& s, uint32_t n, const TraceTuning& tun) {
     if (tun.lanes == 1 || !s.cnodes || !s.prims64) return 1;
-    if (3u * (uint64_t)s.qdepth + 8u > (uint64_t)GSTK_CL) return 1;
+    if (3u * (uint64_t)s.qdepth + 8u > (uint64_t)gstk_closest(8)) return 1;
     if (tun.lanes >= 2) return tun.lanes;
-    return n <= GROUP16_MAX && s.n_prims <= CLOSEST16_PRIMS ? 16 : n <= GROUP_MAX ? 8 : 1;
+    return n <= GROUP32_MAX ? 32 : n <= CLOSEST16_MAX ? 16 : n <= GROUP_MAX ? 8 : 1;
 }
 
 size_t trace_any_block_spill(const SceneView& s, const TraceTuning& tun) {
@@ -1778,14 +1804,13 @@ static hipError_t launch(const SceneView& s, Ray* rays, uint32_t n, Hit* hits, u
     const bool cq = use_compressed(s, tun);
     if (ANY && cq && s.prims64) {
         int G = group_lanes(s, n, tun);
-        if (!occ8 && block / G < 8) G = 8;  // bits: at least a byte of them a block
         if (G > 1) {
-            const uint32_t lim = (uint32_t)GSTK - 3u * s.odepth;
-            const uint32_t gpb = (uint32_t)block / (uint32_t)G;
+            const uint32_t lim = (uint32_t)gstk_occlude(G) - 3u * s.odepth;
+            const uint32_t gpb = (uint32_t)oc_block(G) / (uint32_t)G;
             const size_t cover = occ8 ? (size_t)n : ((size_t)n + 31) / 32 * 32;
             const unsigned grid = (unsigned)((cover + gpb - 1) / gpb);
             const auto kern = group_kernel<false>(G);
-            hipLaunchKernelGGL(kern, dim3(grid), dim3(block), 0, st, s, rays, n, n_dev, occ, occ8, lim, err,
+            hipLaunchKernelGGL(kern, dim3(grid), dim3(oc_block(G)), 0, st, s, rays, n, n_dev, occ, occ8, lim, err,
                                (const TraceSeg*)nullptr, 0u);
             return hipGetLastError();
         }
@@ -1793,10 +1818,10 @@ static hipError_t launch(const SceneView& s, Ray* rays, uint32_t n, Hit* hits, u
     if constexpr (!ANY) {
         const int G = cq ? closest_lanes(s, n, tun) : 1;
         if (G > 1) {
-            const uint32_t lim = (uint32_t)GSTK_CL - 3u * s.qdepth;
-            const uint32_t gpb = (uint32_t)block / (uint32_t)G;
+            const uint32_t lim = (uint32_t)gstk_closest(G) - 3u * s.qdepth;
+            const uint32_t gpb = (uint32_t)CL_BLOCK / (uint32_t)G;
             const unsigned grid = (unsigned)(((size_t)n + gpb - 1) / gpb);
-            hipLaunchKernelGGL(closest_group_kernel<false>(G), dim3(grid), dim3(block), 0, st, s, rays, n, n_dev, hits,
+            hipLaunchKernelGGL(closest_group_kernel<false>(G), dim3(grid), dim3(CL_BLOCK), 0, st, s, rays, n, n_dev, hits,
                                lim, err, (const TraceSeg*)nullptr, 0u);
             return hipGetLastError();
         }
@@ -1916,10 +1941,10 @@ hipError_t trace_segments(const SceneView& s, bool any, const TraceSeg* d_segs, 
     if (any && cq && s.prims64) {
         const int G = group_lanes(s, total, tun);
         if (G > 1) {
-            const uint32_t lim = (uint32_t)GSTK - 3u * s.odepth;
-            const uint32_t gpb = (uint32_t)block / (uint32_t)G;
+            const uint32_t lim = (uint32_t)gstk_occlude(G) - 3u * s.odepth;
+            const uint32_t gpb = (uint32_t)oc_block(G) / (uint32_t)G;
             const unsigned grid = (unsigned)(((size_t)total + gpb - 1) / gpb);
-            hipLaunchKernelGGL(group_kernel<true>(G), dim3(grid), dim3(block), 0, st, s, (const Ray*)nullptr, total,
+            hipLaunchKernelGGL(group_kernel<true>(G), dim3(grid), dim3(oc_block(G)), 0, st, s, (const Ray*)nullptr, total,
                                (const uint32_t*)nullptr, (uint32_t*)nullptr, (uint8_t*)nullptr, lim, err, d_segs,
                                nseg);
             return hipGetLastError();
@@ -1928,10 +1953,10 @@ hipError_t trace_segments(const SceneView& s, bool any, const TraceSeg* d_segs, 
     if (!any && cq) {
         const int G = closest_lanes(s, total, tun);
         if (G > 1) {
-            const uint32_t lim = (uint32_t)GSTK_CL - 3u * s.qdepth;
-            const uint32_t gpb = (uint32_t)block / (uint32_t)G;
+            const uint32_t lim = (uint32_t)gstk_closest(G) - 3u * s.qdepth;
+            const uint32_t gpb = (uint32_t)CL_BLOCK / (uint32_t)G;
             const unsigned grid = (unsigned)(((size_t)total + gpb - 1) / gpb);
-            hipLaunchKernelGGL(closest_group_kernel<true>(G), dim3(grid), dim3(block), 0, st, s, (Ray*)nullptr, total,
+            hipLaunchKernelGGL(closest_group_kernel<true>(G), dim3(grid), dim3(CL_BLOCK), 0, st, s, (Ray*)nullptr, total,
                                (const uint32_t*)nullptr, (Hit*)nullptr, lim, err, d_segs, nseg);
             return hipGetLastError();
         }

@@ -13,7 +13,7 @@ import test_group_stack_model as model
 from pbrt_rust_amd import scenes
 from gpu_util import F32, check_closest, mesh_pair, random_rays
 
-GSTK_CL = 96  # stack entries of a closest-hit group
+GSTK_CL = {4: 96, 8: 96, 16: 160, 32: 192}  # stack entries of a closest-hit group, by its lanes
 
 
 @pytest.fixture(params=[0, 1, 4, 8, 16])
@@ -53,7 +53,7 @@ def test_ties_and_leaves_of_several_prims(lanes, max_prims, split):
 def test_ragged_counts(lanes):
     v, idx = scenes.random_triangles(5000, 21, 0.05, 0.3)
     bvh, orc = mesh_pair(v, idx, "sah", 2)
-    for n in (1, 3, 4, 7, 8, 9, 15, 17, 31, 63, 65, 255, 257, 4099):
+    for n in (1, 3, 4, 7, 8, 9, 15, 17, 31, 63, 65, 255, 257, 4096, 4097, 24577):
         o, d = random_rays(n, 100 + n)
         check_closest(bvh, orc, o, d)
     px.synchronize()
@@ -121,7 +121,7 @@ def test_occlusion_words_are_written_whole(block, g):
     bvh, orc = mesh_pair(v, idx)
     try:
         px.set_tuning("batched", "any", block, 0, 60, "ray", lanes=g)
-        for n in (1, 7, 8, 9, 16, 31, 32, 33, 63, 64, 65, 129, 1000, 20011):
+        for n in (1, 7, 8, 9, 16, 31, 32, 33, 63, 64, 65, 129, 1000, 4096, 4097, 16385, 33001):
             o, d = random_rays(n, 200 + n)
             rays = px.DeviceBuffer.from_array(px.RayBatch(o, d, 0.0, 0.7).a)
             nw = (n + 31) // 32
@@ -139,8 +139,8 @@ def test_occlusion_words_are_written_whole(block, g):
 
 def walk_put_back(tree, depth, G, rng):
     """model.walk with leaves that go back on the stack while a record of the same step lies before them."""
-    lim = GSTK_CL - 3 * depth
-    assert 3 * depth + 8 <= GSTK_CL
+    lim = GSTK_CL[G] - 3 * depth
+    assert 3 * depth + 8 <= GSTK_CL[G]
     stack, steps = [0], 0
     while stack:
         top = len(stack)
@@ -155,13 +155,13 @@ def walk_put_back(tree, depth, G, rng):
                 pushes.append([None])
         for p in reversed(pushes):
             stack.extend(reversed(p))
-        assert len(stack) <= GSTK_CL, len(stack)
+        assert len(stack) <= GSTK_CL[G], len(stack)
         steps += 1
         assert steps < 200000
     return steps
 
 
-@pytest.mark.parametrize("G", [4, 8, 16])
+@pytest.mark.parametrize("G", [4, 8, 16, 32])
 @pytest.mark.parametrize("depth,fan", [(1, 0), (6, 4), (9, 3), (14, 2), (29, 1), (29, 2)])
 def test_model_of_the_stack_bound(G, depth, fan):
     rng = random.Random(depth * 7 + fan + G)
