@@ -171,7 +171,7 @@ int run_closest(const SceneView& v, Ray* rays, uint32_t n, Hit* hits, int path, 
     if (path != PATH_PLAIN && path != PATH_BATCHED) return fail(PBRTX_ERR_ARG, "unknown path");
     const TraceTuning& tun = g_tuning[path][0];
     TraceScratch* scr;
-    int rc = stream_scratch(st, trace_spill_bytes(v, path, tun), &scr);
+    int rc = stream_scratch(st, trace_spill_bytes(v, path, tun, n), &scr);
     if (rc) return rc;
     hipError_t e = trace_closest(v, rays, n, hits, path, tun, scr, st);
     if (e != hipSuccess) return hip_fail(e, "trace_closest");
@@ -182,7 +182,7 @@ int run_any(const SceneView& v, const Ray* rays, uint32_t n, uint32_t* occ, int 
     if (path != PATH_PLAIN && path != PATH_BATCHED) return fail(PBRTX_ERR_ARG, "unknown path");
     const TraceTuning& tun = g_tuning[path][1];
     TraceScratch* scr;
-    int rc = stream_scratch(st, trace_spill_bytes(v, path, tun), &scr);
+    int rc = stream_scratch(st, trace_spill_bytes(v, path, tun, n), &scr);
     if (rc) return rc;
     hipError_t e = trace_any(v, rays, n, occ, path, tun, scr, st);
     if (e != hipSuccess) return hip_fail(e, "trace_any");

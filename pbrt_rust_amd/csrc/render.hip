@@ -1556,12 +1556,12 @@ CamParams cam_params(const RenderParams& P, uint64_t g0) {
     return cp;
 }
 
-size_t render_spill_bytes(const SceneView& sv, int path) {
-    const size_t a = trace_spill_bytes(sv, path, g_tuning[path][0]);
-    const size_t b = trace_spill_bytes(sv, path, g_tuning[path][1]);
+size_t render_spill_bytes(const SceneView& sv, int path, uint64_t rays) {
+    const size_t a = trace_spill_bytes(sv, path, g_tuning[path][0], rays);
+    const size_t b = trace_spill_bytes(sv, path, g_tuning[path][1], rays);
     // camera rays: either scheme the frame's samples per pixel may pick
-    const size_t c = trace_spill_bytes(sv, path, camera_tuning(path, 1));
-    const size_t d = trace_spill_bytes(sv, path, camera_tuning(path, 1u << 20));
+    const size_t c = trace_spill_bytes(sv, path, camera_tuning(path, 1), rays);
+    const size_t d = trace_spill_bytes(sv, path, camera_tuning(path, 1u << 20), rays);
     return std::max(std::max(a, b), std::max(c, d));
 }
 
@@ -1985,9 +1985,13 @@ static int enqueue_frame(Renderer* R, int path, TraceScratch* scr, Stager& sg, u
 static int render_frame(Renderer* R, int path, pbrtx_render_stats* stats) {
     hipStream_t st = R->stream;
     TraceScratch* scr;
-    ICHK(stream_scratch(st, render_spill_bytes(R->sc.scene.view, path), &scr));
+    // a chunk's largest launch: its paths, or its samples' shadow slots
+    const uint64_t most = std::min<uint64_t>(std::max(R->chunk, R->P.spp), R->n_samples) *
+                          (R->sc.integrator == 0 ? std::max(R->P.S, 1u) : 1u);
+    const size_t need = render_spill_bytes(R->sc.scene.view, path, most);
+    ICHK(stream_scratch(st, need, &scr));
     TraceScratch* scr2 = nullptr;
-    if (R->stream2) ICHK(stream_scratch(R->stream2, render_spill_bytes(R->sc.scene.view, path), &scr2));
+    if (R->stream2) ICHK(stream_scratch(R->stream2, need, &scr2));
     R->events.used = 0;
     Timing T;
     uint64_t total_camera = 0;

@@ -533,7 +533,8 @@ int pbrtx_render_server_add_scene(pbrtx_render_server* p, const pbrtx_render_des
     RenderServer& s = p->s;
     std::lock_guard<std::mutex> lk(s.mu);
     const SceneView& v = sc->scene.view;
-    s.spill_need = std::max(s.spill_need, std::max(render_spill_bytes(v, PATH_BATCHED), render_spill_bytes(v, PATH_PLAIN)));
+    s.spill_need = std::max(s.spill_need, std::max(render_spill_bytes(v, PATH_BATCHED, s.cfg.batch_samples),
+                                                   render_spill_bytes(v, PATH_PLAIN, s.cfg.batch_samples)));
     s.scene_bytes += sc->scene.bytes;
     s.scenes.push_back(std::move(sc));
     *scene_id = (uint32_t)(s.scenes.size() - 1);

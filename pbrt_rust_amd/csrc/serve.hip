@@ -498,10 +498,10 @@ int pbrtx_server_add_scene(pbrtx_server* p, const pbrtx_scene* scene, uint32_t* 
         return fail(PBRTX_ERR_OOM, "scene exceeds the server's resident-scene budget");
     const TraceTuning& a = g_tuning[PATH_BATCHED][0];
     const TraceTuning& b = g_tuning[PATH_BATCHED][1];
-    const size_t need = std::max(std::max(trace_spill_bytes(scene->s.view, PATH_BATCHED, a),
-                                          trace_spill_bytes(scene->s.view, PATH_BATCHED, b)),
-                                 std::max(trace_spill_bytes(scene->s.view, PATH_PLAIN, g_tuning[PATH_PLAIN][0]),
-                                          trace_spill_bytes(scene->s.view, PATH_PLAIN, g_tuning[PATH_PLAIN][1])));
+    const size_t need = std::max(std::max(trace_spill_bytes(scene->s.view, PATH_BATCHED, a, s.cfg.batch_rays),
+                                          trace_spill_bytes(scene->s.view, PATH_BATCHED, b, s.cfg.batch_rays)),
+                                 std::max(trace_spill_bytes(scene->s.view, PATH_PLAIN, g_tuning[PATH_PLAIN][0], 0),
+                                          trace_spill_bytes(scene->s.view, PATH_PLAIN, g_tuning[PATH_PLAIN][1], 0)));
     s.spill_need = std::max(s.spill_need, need);
     s.scenes.push_back(&scene->s);
     s.scene_bytes += scene->s.bytes;

@@ -422,7 +422,32 @@ constexpr uint32_t WIDE_PART_STRIDE = 32;
 // where the part counters sit in a stream's scratch counter block (words;
 // word 0 is the packet kernels' counter, word 1 the stack-overflow flag)
 constexpr uint32_t WIDE_PARTS_AT = 32;
-static_assert(WIDE_PARTS_AT + WIDE_PARTS * WIDE_PART_STRIDE <= TRACE_COUNTER_WORDS, "scratch counter block");
+// the part counters, then the count of rays handed over (TailRec): cleared together
+constexpr uint32_t WIDE_COUNTERS = WIDE_PARTS * WIDE_PART_STRIDE + 1;
+static_assert(WIDE_PARTS_AT + WIDE_COUNTERS <= TRACE_COUNTER_WORDS, "scratch counter block");
+
+// The rays a large launch of the per-ray kernel does not finish itself.  Once
+// its rays are all claimed, a wave's lanes fall idle one by one and the last
+// rays run alone: the launch's time fits c + m * rays with c = 0.35-0.55 ms
+// (2^20 to 2^22 rays).  A wave with at most tail.lanes rays left hands them
+// over instead -- ray, hit so far and stack, in visiting order -- and a
+// launch of the several-lane kernel takes each up where it stopped.  A
+// launch of at most tail.cap rays (a queue that turns out short) hands all of
+// them over at once.
+constexpr int TAIL_STK = 20;  // entries a record holds; a ray with more stays
+struct TailRec {
+    uint32_t id, sp;      // ray of the launch, entries
+    uint32_t hpos;        // hit so far (closest hit): position, t, b1, b2
+    float tmax, b1, b2;
+    uint32_t pad[2];
+};
+static_assert(sizeof(TailRec) == 32, "two 16-byte words");
+struct TailView {
+    TailRec* recs = nullptr;  // null: rays are finished where they run
+    int2* stk = nullptr;      // TAIL_STK entries (ref, entry distance) a record
+    uint32_t* count = nullptr;
+    uint32_t cap = 0, lanes = 0;
+};
 
 template <bool ANY, bool SEG, bool CQ, int STK_WIDE>
 __global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) void k_trace_wide(SceneView sv, Ray* rays, uint32_t n_host,
@@ -430,7 +455,8 @@ __global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) 
                                                           uint32_t* occ, uint8_t* occ8, uint32_t* counter,
                                                           uint2* spill, uint32_t spill_levels,
                                                           uint32_t refill, uint32_t* err,
-                                                          const TraceSeg* segs, uint32_t nseg) {
+                                                          const TraceSeg* segs, uint32_t nseg,
+                                                          TailView tail) {
     const uint32_t n = n_dev ? *n_dev : n_host;
     // A launch sized for a queue's capacity: blocks beyond what the queue's
     // count can occupy (64 rays a wave) leave before touching the work
@@ -549,6 +575,35 @@ __global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) 
             }
         }
         if (!__any(has)) break;
+        if constexpr (CQ) {
+            // hand the last rays over (see TailRec)
+            if (tail.recs && (n <= tail.cap || (res_b == res_e && tries >= nparts &&
+                                                (uint32_t)__popcll(__ballot(has)) <= tail.lanes))) {
+                const int cnt = sp + (have_cur ? 1 : 0);
+                const unsigned long long give = __ballot(has && cnt <= TAIL_STK);
+                if (give) {
+                    uint32_t b = 0;
+                    if (lane == 0) b = atomicAdd(tail.count, (uint32_t)__popcll(give));
+                    b = __builtin_amdgcn_readfirstlane(__shfl(b, 0)) + (uint32_t)__popcll(give & lt_mask);
+                    if (((give >> lane) & 1ull) && b < tail.cap) {
+                        tail.recs[b] = TailRec{SEG ? segs[rseg].start + rid : rid, (uint32_t)cnt, hprim, r.tmax,
+                                               hb1, hb2, {0u, 0u}};
+                        int2* to = tail.stk + (size_t)b * TAIL_STK;
+                        for (int k = 0; k < sp; ++k) {
+                            if (k < STK_WIDE) {
+                                to[k] = make_int2(s_ref[k][tid], ANY ? 0 : (int)as_u(s_tn[ANY ? 0 : k][tid]));
+                            } else {
+                                const uint2 e = spill[(size_t)(k - STK_WIDE) * total + gtid];
+                                to[k] = make_int2((int)e.x, (int)e.y);
+                            }
+                        }
+                        if (have_cur) to[sp] = make_int2(cur, (int)0xFF800000u);
+                        has = false;
+                    }
+                }
+                if (!__any(has)) continue;
+            }
+        }
         if (CQ) wfast = fast_scene && __ballot(has && !fastr) == 0ull;
         // ---- traverse until too few lanes are busy
         while (has) {
@@ -791,19 +846,22 @@ __global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) 
 // wave's LDS goes to the next one: 2^20 rays in 200K triangles 572 us with
 // 256 threads a block, 557 with 64.
 // SEG: the rays come from a segment table (served launch) instead of one array.
+// TAIL: they are those that the per-ray kernel handed over, with their stacks
+// (at most TAIL_STK entries of its walk: a step takes one entry of them until
+// the rest are within lim).
 // More lanes take more entries a step and need the room for them.
 constexpr int gstk_occlude(int G) { return G <= 8 ? 128 : (G == 16 ? 192 : 256); }
 constexpr int oc_block(int G) { return G <= 8 ? 64 : 8 * G; }
-template <int G, bool SEG>
+template <int G, bool SEG, bool TAIL>
 __global__ __launch_bounds__(oc_block(G)) __attribute__((amdgpu_waves_per_eu(8))) void k_occlude_group(
     SceneView sv, const Ray* rays, uint32_t n_host, const uint32_t* n_dev, uint32_t* occ, uint8_t* occ8,
-    uint32_t lim, uint32_t* err, const TraceSeg* segs, uint32_t nseg) {
+    uint32_t lim, uint32_t* err, const TraceSeg* segs, uint32_t nseg, TailView tail) {
     static_assert(G >= 2 && G <= 64 && (64 % G) == 0, "a group lies within one wave");
     // (the grid covers n_host rays: a count on the device never exceeds it)
-    const uint32_t n = n_dev ? min(*n_dev, n_host) : n_host;
+    const uint32_t n = TAIL ? min(*tail.count, tail.cap) : n_dev ? min(*n_dev, n_host) : n_host;
     const uint32_t gpb = oc_block(G) / G;  // groups per block
     // (bits: the grid covers n_host's words, and the blocks past n write zeros)
-    if ((occ8 || SEG) && (uint64_t)blockIdx.x * gpb >= (uint64_t)n) return;
+    if ((occ8 || SEG || TAIL) && (uint64_t)blockIdx.x * gpb >= (uint64_t)n) return;
     constexpr int GSTK = gstk_occlude(G);
     __shared__ int32_t s_stk[oc_block(G) / G][GSTK];
     const uint32_t tid = threadIdx.x, lane = __lane_id();
@@ -818,17 +876,22 @@ __global__ __launch_bounds__(oc_block(G)) __attribute__((amdgpu_waves_per_eu(8))
     bool done = id >= n;
     uint32_t top = 0;
     if (!done) {
+        if (TAIL) rid = tail.recs[id].id;
         if (SEG) {
-            rseg = find_seg(segs, nseg, id);
-            rid = id - segs[rseg].start;
+            rseg = find_seg(segs, nseg, rid);
+            rid -= segs[rseg].start;
             load_ray(segs[rseg].rays, rid, r);
         } else {
             load_ray(rays, rid, r);
         }
         float tn;
-        // the root's own box (popped first by the reference)
-        if (slab(sv.root_lo[0], sv.root_hi[0], sv.root_lo[1], sv.root_hi[1], sv.root_lo[2], sv.root_hi[2], r.ox,
-                 r.oy, r.oz, r.ix, r.iy, r.iz, r.tmin, r.tmax, &tn)) {
+        if (TAIL) {
+            // the walk goes on from the entries its wave handed over
+            top = tail.recs[id].sp;
+            for (uint32_t e = gl; e < top; e += G) stk[e] = tail.stk[(size_t)id * TAIL_STK + e].x;
+        } else if (slab(sv.root_lo[0], sv.root_hi[0], sv.root_lo[1], sv.root_hi[1], sv.root_lo[2], sv.root_hi[2], r.ox,
+                        r.oy, r.oz, r.ix, r.iy, r.iz, r.tmin, r.tmax, &tn)) {
+            // the root's own box (popped first by the reference)
             top = 1;
             if (gl == 0) stk[0] = sv.ocroot;
         }
@@ -935,10 +998,10 @@ __global__ __launch_bounds__(oc_block(G)) __attribute__((amdgpu_waves_per_eu(8))
         hit = hit || ghit;
         done = done || ghit || top == 0u;
     }
-    if (occ8 || SEG) {
+    if (occ8 || SEG || TAIL) {
         if (id < n && gl == 0) {
             if (occ8) occ8[rid] = hit ? 1u : 0u;
-            else if (hit) atomicOr(segs[rseg].occ + (rid >> 5), 1u << (rid & 31u));
+            else if (hit) atomicOr((SEG ? segs[rseg].occ : occ) + (rid >> 5), 1u << (rid & 31u));
         }
         return;
     }
@@ -990,15 +1053,17 @@ __global__ __launch_bounds__(oc_block(G)) __attribute__((amdgpu_waves_per_eu(8))
 // triangles, 8 lanes: 984 us with 96 entries, 1436 with 72 though eight waves
 // fit then, 1105 with 128; 1,021 rays, 16 lanes: 52 us with 96, 29 with 160).
 // SEG: the rays come from a segment table (served launch) instead of one array.
+// TAIL: they are those that the per-ray kernel handed over, with their hits
+// and stacks (as in k_occlude_group).
 constexpr int CL_BLOCK = 64;
 constexpr int gstk_closest(int G) { return G <= 8 ? 96 : (G == 16 ? 160 : 192); }
-template <int G, bool SEG>
+template <int G, bool SEG, bool TAIL>
 __global__ __launch_bounds__(CL_BLOCK) __attribute__((amdgpu_waves_per_eu(6))) void k_closest_group(
     SceneView sv, Ray* rays, uint32_t n_host, const uint32_t* n_dev, Hit* hits, uint32_t lim, uint32_t* err,
-    const TraceSeg* segs, uint32_t nseg) {
+    const TraceSeg* segs, uint32_t nseg, TailView tail) {
     static_assert(G >= 2 && G <= 64 && (64 % G) == 0, "a group lies within one wave");
     // (the grid covers n_host rays: a count on the device never exceeds it)
-    const uint32_t n = n_dev ? min(*n_dev, n_host) : n_host;
+    const uint32_t n = TAIL ? min(*tail.count, tail.cap) : n_dev ? min(*n_dev, n_host) : n_host;
     const uint32_t gpb = CL_BLOCK / G;  // groups per block
     if ((uint64_t)blockIdx.x * gpb >= (uint64_t)n) return;
     constexpr int GSTK_CL = gstk_closest(G);
@@ -1015,30 +1080,41 @@ __global__ __launch_bounds__(CL_BLOCK) __attribute__((amdgpu_waves_per_eu(6))) v
     RayState r{};
     bool done = id >= n;
     uint32_t top = 0;
+    float tmax0 = 0.0f;
+    uint32_t hpos = NO_HIT;
+    float hb1 = 0.0f, hb2 = 0.0f;
     if (!done) {
+        if (TAIL) rid = tail.recs[id].id;
         if (SEG) {
-            rseg = find_seg(segs, nseg, id);
-            rid = id - segs[rseg].start;
+            rseg = find_seg(segs, nseg, rid);
+            rid -= segs[rseg].start;
             load_ray(segs[rseg].rays, rid, r);
         } else {
             load_ray(rays, rid, r);
         }
+        tmax0 = r.tmax;
         float tn;
-        // the root's own box (popped first by the reference)
-        if (slab(sv.root_lo[0], sv.root_hi[0], sv.root_lo[1], sv.root_hi[1], sv.root_lo[2], sv.root_hi[2], r.ox,
-                 r.oy, r.oz, r.ix, r.iy, r.iz, r.tmin, r.tmax, &tn)) {
+        if (TAIL) {
+            // the walk goes on from the hit and the entries its wave handed over
+            const TailRec t = tail.recs[id];
+            hpos = t.hpos;
+            r.tmax = t.tmax;
+            hb1 = t.b1;
+            hb2 = t.b2;
+            top = t.sp;
+            for (uint32_t e = gl; e < top; e += G) stk[e] = tail.stk[(size_t)id * TAIL_STK + e];
+        } else if (slab(sv.root_lo[0], sv.root_hi[0], sv.root_lo[1], sv.root_hi[1], sv.root_lo[2], sv.root_hi[2], r.ox,
+                        r.oy, r.oz, r.ix, r.iy, r.iz, r.tmin, r.tmax, &tn)) {
+            // the root's own box (popped first by the reference)
             top = 1;
             if (gl == 0) stk[0] = make_int2(sv.qroot, (int)0xFF800000u);
         }
         done = top == 0;
     }
-    const float tmax0 = r.tmax;
     const bool neg0 = r.ix < 0.0f, neg1 = r.iy < 0.0f, neg2 = r.iz < 0.0f;
     const uint32_t negm = (neg0 ? 1u : 0u) | (neg1 ? 2u : 0u) | (neg2 ? 4u : 0u);
     // every ray of the wave may take the ray-space record test (cq_fast_ray)
     const bool wfast = cq_fast_scene(sv) && __ballot(id < n && !cq_fast_ray(r)) == 0ull;
-    uint32_t hpos = NO_HIT;
-    float hb1 = 0.0f, hb2 = 0.0f;
     bool one = false;  // one entry a step
     while (__any(!done)) {
         // entries for this step: up to G, fewer near the stack's bound
@@ -1702,18 +1778,18 @@ static int group_lanes(const SceneView& s, uint32_t n, const TraceTuning& tun) {
 }
 
 template <bool SEG>
-static auto group_kernel(int G) -> decltype(&k_occlude_group<8, SEG>) {
-    return G == 4    ? &k_occlude_group<4, SEG>
-           : G == 8  ? &k_occlude_group<8, SEG>
-           : G == 16 ? &k_occlude_group<16, SEG>
-                     : &k_occlude_group<32, SEG>;
+static auto group_kernel(int G) -> decltype(&k_occlude_group<8, SEG, false>) {
+    return G == 4    ? &k_occlude_group<4, SEG, false>
+           : G == 8  ? &k_occlude_group<8, SEG, false>
+           : G == 16 ? &k_occlude_group<16, SEG, false>
+                     : &k_occlude_group<32, SEG, false>;
 }
 template <bool SEG>
-static auto closest_group_kernel(int G) -> decltype(&k_closest_group<8, SEG>) {
-    return G == 4    ? &k_closest_group<4, SEG>
-           : G == 8  ? &k_closest_group<8, SEG>
-           : G == 16 ? &k_closest_group<16, SEG>
-                     : &k_closest_group<32, SEG>;
+static auto closest_group_kernel(int G) -> decltype(&k_closest_group<8, SEG, false>) {
+    return G == 4    ? &k_closest_group<4, SEG, false>
+           : G == 8  ? &k_closest_group<8, SEG, false>
+           : G == 16 ? &k_closest_group<16, SEG, false>
+                     : &k_closest_group<32, SEG, false>;
 }
 // Lanes per ray of a batched closest-hit launch of up to n rays, as
 // group_lanes.  From launches of random rays (origins in the box, uniform
@@ -1746,11 +1822,45 @@ static int closest_lanes(const SceneView& s, uint32_t n, const TraceTuning& tun)
     return n <= GROUP32_MAX ? 32 : n <= CLOSEST16_MAX ? 16 : n <= GROUP_MAX ? 8 : 1;
 }
 
+// Rays that a wave of the per-ray kernel hands over when its launch's rays are
+// all claimed, and the most a launch hands over.  Random rays in random-triangle
+// soups, us with no hand-over / at 8 / 16 / 32 rays a wave:
+//   closest hit, 200K triangles, 1.2M rays:  998 /  867 /  824 /  829
+//                                  4M rays: 2123 / 1988 / 1915 / 1921
+//                500K triangles,   4M rays: 2478 / 2381 / 2338 / 2345
+//   occlusion,   200K triangles, 1.2M rays:  718 /  610 /  597 /  606
+//                                  4M rays: 1445 / 1318 / 1303 / 1313
+// The 1920x1080 64-spp path-tracing frame 15.3 -> 14.8 ms; a frame of 12
+// spheres, whose rays are short, 2.39 -> 2.45: not worth its launch there.
+constexpr uint32_t TAIL_LANES = 16;
+constexpr size_t TAIL_CAP = 1u << 18;
+constexpr uint32_t TAIL_PRIMS = 1u << 12;
+static size_t tail_cap(size_t threads) { return std::min<size_t>(threads / 64 * TAIL_LANES, TAIL_CAP); }
+static size_t tail_bytes(size_t cap) { return cap * (sizeof(TailRec) + TAIL_STK * sizeof(int2)); }
+// The tail of a launch of `grid` blocks whose spill stacks take `used` bytes of
+// the scratch; none if the rest does not hold it (a fixed scratch), or if the
+// several-lane kernel cannot take the rays up.
+static TailView make_tail(bool any, const SceneView& s, TraceScratch* scr, size_t used, int grid, int block) {
+    TailView t;
+    const uint32_t depth = any ? s.odepth : s.qdepth;
+    if (!s.cnodes || !s.prims64 || s.n_prims < TAIL_PRIMS || 3u * (uint64_t)depth + 8u > (uint64_t)(any ? gstk_occlude(8) : gstk_closest(8)))
+        return t;
+    const size_t waves = (size_t)grid * block / 64, cap = tail_cap((size_t)grid * block);
+    const size_t at = (used + 255) / 256 * 256;
+    if (cap < waves || at + tail_bytes(cap) > scr->spill_bytes) return t;
+    t.recs = reinterpret_cast<TailRec*>((uint8_t*)scr->spill + at);
+    t.stk = reinterpret_cast<int2*>(t.recs + cap);
+    t.count = scr->counter + WIDE_PARTS_AT + WIDE_PARTS * WIDE_PART_STRIDE;
+    t.cap = (uint32_t)cap;
+    t.lanes = (uint32_t)(cap / waves);
+    return t;
+}
+
 size_t trace_any_block_spill(const SceneView& s, const TraceTuning& tun) {
     return (size_t)wide_levels(s, tun.stack) * tun.block * sizeof(uint2);
 }
 
-size_t trace_spill_bytes(const SceneView& s, int path, const TraceTuning& tun) {
+size_t trace_spill_bytes(const SceneView& s, int path, const TraceTuning& tun, uint64_t rays) {
     const int block = tun.block;
     if (path == PATH_PLAIN) {
         size_t threads = (size_t)device_cu_count() * PLAIN_BLOCKS_PER_CU * block;
@@ -1765,7 +1875,8 @@ size_t trace_spill_bytes(const SceneView& s, int path, const TraceTuning& tun) {
                      wide_grid(wide_kernel<false, false, true>(k), t), wide_grid(wide_kernel<true, false, true>(k), t),
                      wide_grid(wide_kernel<false, true, true>(k), t), wide_grid(wide_kernel<true, true, true>(k), t)})
         threads = std::max(threads, g * (size_t)block);
-    return (size_t)wide_levels(s, k) * threads * sizeof(uint2);
+    const size_t spill = (size_t)wide_levels(s, k) * threads * sizeof(uint2);
+    return rays > GROUP_MAX ? spill + 256 + tail_bytes(tail_cap(threads)) : spill;
 }
 
 template <bool ANY>
@@ -1811,7 +1922,7 @@ static hipError_t launch(const SceneView& s, Ray* rays, uint32_t n, Hit* hits, u
             const unsigned grid = (unsigned)((cover + gpb - 1) / gpb);
             const auto kern = group_kernel<false>(G);
             hipLaunchKernelGGL(kern, dim3(grid), dim3(oc_block(G)), 0, st, s, rays, n, n_dev, occ, occ8, lim, err,
-                               (const TraceSeg*)nullptr, 0u);
+                               (const TraceSeg*)nullptr, 0u, TailView{});
             return hipGetLastError();
         }
     }
@@ -1822,7 +1933,7 @@ static hipError_t launch(const SceneView& s, Ray* rays, uint32_t n, Hit* hits, u
             const uint32_t gpb = (uint32_t)CL_BLOCK / (uint32_t)G;
             const unsigned grid = (unsigned)(((size_t)n + gpb - 1) / gpb);
             hipLaunchKernelGGL(closest_group_kernel<false>(G), dim3(grid), dim3(CL_BLOCK), 0, st, s, rays, n, n_dev, hits,
-                               lim, err, (const TraceSeg*)nullptr, 0u);
+                               lim, err, (const TraceSeg*)nullptr, 0u, TailView{});
             return hipGetLastError();
         }
     }
@@ -1836,13 +1947,24 @@ static hipError_t launch(const SceneView& s, Ray* rays, uint32_t n, Hit* hits, u
         grid = (int)(scr->spill_bytes / per_block);
     }
     uint32_t* parts = scr->counter + WIDE_PARTS_AT;
-    hipError_t e = ANY && !occ8 ? zero3_u32(parts, (size_t)WIDE_PARTS * WIDE_PART_STRIDE, occ, ((size_t)n + 31) / 32,
+    hipError_t e = ANY && !occ8 ? zero3_u32(parts, (size_t)WIDE_COUNTERS, occ, ((size_t)n + 31) / 32,
                                             nullptr, 0, st)
-                                : fill_u32(parts, 0u, (size_t)WIDE_PARTS * WIDE_PART_STRIDE, st);
+                                : fill_u32(parts, 0u, (size_t)WIDE_COUNTERS, st);
     if (e != hipSuccess) return e;
     const uint32_t refill = (uint32_t)(tun.refill_pct < 0 ? 0 : (tun.refill_pct > 100 ? 100 : tun.refill_pct));
+    const TailView tail = cq && tun.lanes != 1 ? make_tail(ANY, s, scr, per_block * grid, grid, block) : TailView{};
     hipLaunchKernelGGL(kern, dim3(grid), dim3(block), 0, st, s, rays, n, n_dev, hits, occ, occ8, parts,
-                       (uint2*)scr->spill, lv, refill, err, (const TraceSeg*)nullptr, 0u);
+                       (uint2*)scr->spill, lv, refill, err, (const TraceSeg*)nullptr, 0u, tail);
+    e = hipGetLastError();
+    if (e != hipSuccess || !tail.recs) return e;
+    if constexpr (ANY)
+        hipLaunchKernelGGL((k_occlude_group<8, false, true>), dim3((tail.cap + 7) / 8), dim3(oc_block(8)), 0, st, s, rays,
+                           n, n_dev, occ, occ8, (uint32_t)gstk_occlude(8) - 3u * s.odepth, err,
+                           (const TraceSeg*)nullptr, 0u, tail);
+    else
+        hipLaunchKernelGGL((k_closest_group<8, false, true>), dim3((tail.cap + 7) / 8), dim3(CL_BLOCK), 0, st, s, rays,
+                           n, n_dev, hits, (uint32_t)gstk_closest(8) - 3u * s.qdepth, err, (const TraceSeg*)nullptr, 0u,
+                           tail);
     return hipGetLastError();
 }
 
@@ -1946,7 +2068,7 @@ hipError_t trace_segments(const SceneView& s, bool any, const TraceSeg* d_segs, 
             const unsigned grid = (unsigned)(((size_t)total + gpb - 1) / gpb);
             hipLaunchKernelGGL(group_kernel<true>(G), dim3(grid), dim3(oc_block(G)), 0, st, s, (const Ray*)nullptr, total,
                                (const uint32_t*)nullptr, (uint32_t*)nullptr, (uint8_t*)nullptr, lim, err, d_segs,
-                               nseg);
+                               nseg, TailView{});
             return hipGetLastError();
         }
     }
@@ -1957,7 +2079,7 @@ hipError_t trace_segments(const SceneView& s, bool any, const TraceSeg* d_segs, 
             const uint32_t gpb = (uint32_t)CL_BLOCK / (uint32_t)G;
             const unsigned grid = (unsigned)(((size_t)total + gpb - 1) / gpb);
             hipLaunchKernelGGL(closest_group_kernel<true>(G), dim3(grid), dim3(CL_BLOCK), 0, st, s, (Ray*)nullptr, total,
-                               (const uint32_t*)nullptr, (Hit*)nullptr, lim, err, d_segs, nseg);
+                               (const uint32_t*)nullptr, (Hit*)nullptr, lim, err, d_segs, nseg, TailView{});
             return hipGetLastError();
         }
     }
@@ -1966,12 +2088,24 @@ hipError_t trace_segments(const SceneView& s, bool any, const TraceSeg* d_segs, 
     const int grid = wide_grid(kern, tun);
     if ((size_t)lv * grid * block * sizeof(uint2) > scr->spill_bytes) return hipErrorInvalidValue;
     uint32_t* parts = scr->counter + WIDE_PARTS_AT;
-    hipError_t e = fill_u32(parts, 0u, (size_t)WIDE_PARTS * WIDE_PART_STRIDE, st);
+    hipError_t e = fill_u32(parts, 0u, (size_t)WIDE_COUNTERS, st);
     if (e != hipSuccess) return e;
     const uint32_t refill = (uint32_t)(tun.refill_pct < 0 ? 0 : (tun.refill_pct > 100 ? 100 : tun.refill_pct));
+    const TailView tail =
+        cq && tun.lanes != 1 ? make_tail(any, s, scr, (size_t)lv * grid * block * sizeof(uint2), grid, block) : TailView{};
     hipLaunchKernelGGL(kern, dim3(grid), dim3(block), 0, st, s, (Ray*)nullptr, total, (const uint32_t*)nullptr,
                        (Hit*)nullptr, (uint32_t*)nullptr, (uint8_t*)nullptr, parts, (uint2*)scr->spill, lv, refill,
-                       err, d_segs, nseg);
+                       err, d_segs, nseg, tail);
+    e = hipGetLastError();
+    if (e != hipSuccess || !tail.recs) return e;
+    if (any)
+        hipLaunchKernelGGL((k_occlude_group<8, true, true>), dim3((tail.cap + 7) / 8), dim3(oc_block(8)), 0, st, s,
+                           (const Ray*)nullptr, total, (const uint32_t*)nullptr, (uint32_t*)nullptr,
+                           (uint8_t*)nullptr, (uint32_t)gstk_occlude(8) - 3u * s.odepth, err, d_segs, nseg, tail);
+    else
+        hipLaunchKernelGGL((k_closest_group<8, true, true>), dim3((tail.cap + 7) / 8), dim3(CL_BLOCK), 0, st, s,
+                           (Ray*)nullptr, total, (const uint32_t*)nullptr, (Hit*)nullptr,
+                           (uint32_t)gstk_closest(8) - 3u * s.qdepth, err, d_segs, nseg, tail);
     return hipGetLastError();
 }
 

@@ -118,8 +118,10 @@ struct TraceSeg {
 // (d_segs in device memory); closest hit (any = false) or occlusion.
 hipError_t trace_segments(const SceneView& s, bool any, const TraceSeg* d_segs, uint32_t nseg, uint32_t total,
                           const TraceTuning& tun, TraceScratch* scr, hipStream_t st);
-// Number of spill bytes a launch needs for this scene and tuning.
-size_t trace_spill_bytes(const SceneView& s, int path, const TraceTuning& tun);
+// Scratch bytes a launch of up to `rays` rays wants for this scene and tuning:
+// its spill stacks and, where one lane traces a ray, the rays its waves hand
+// over.
+size_t trace_spill_bytes(const SceneView& s, int path, const TraceTuning& tun, uint64_t rays);
 hipError_t fill_u32(uint32_t* p, uint32_t value, size_t n, hipStream_t st);
 // zeroes a[0..na), b[0..nb) and c[0..nc) with one launch (null ranges of length 0)
 hipError_t zero3_u32(uint32_t* a, size_t na, uint32_t* b, size_t nb, uint32_t* c, size_t nc, hipStream_t st);

@@ -137,6 +137,46 @@ def test_occlusion_words_are_written_whole(block, g):
         px.reset_tuning()
 
 
+def query_all(bvh, rec, path):
+    n = len(rec)
+    rays, hits = px.DeviceBuffer.from_array(rec), px.DeviceBuffer(16 * n)
+    bits = px.DeviceBuffer(4 * ((n + 31) // 32))
+    bvh.intersect_p_device(rays.ptr, n, bits.ptr, path)
+    bvh.intersect_device(rays.ptr, n, hits.ptr, path)
+    px.synchronize()  # raises if a traversal stack overflowed
+    return hits.download(np.uint32, 4 * n), rays.download(np.uint32, 8 * n), bits.download(np.uint32, (n + 31) // 32)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [(1 << 20) + 1, 1500000])
+@pytest.mark.parametrize("scene", ["soup", "ties", "overlap"])
+def test_launches_that_hand_their_last_rays_over(scene, n):
+    # past 2^20 rays one lane takes a ray and each wave hands its last rays to
+    # the several-lane kernels: the same bits as the plain path, in a soup, at
+    # tied hits, and among boxes that all overlap (stacks too long for a record)
+    rng = np.random.default_rng(77)
+    if scene == "ties":
+        v, idx = scenes.icosphere(5)
+        v, idx = v.astype(F32), idx.astype(np.uint32)
+        o, d = tied_rays(v, idx, n, 78)
+    elif scene == "soup":
+        v, idx = scenes.random_triangles(30000, 79)
+        o, d = random_rays(n, 80)
+    else:
+        k = 5000
+        z = np.sort(rng.uniform(-1, 1, k))
+        v = np.stack([np.stack([np.full(k, -1), np.full(k, -1), z], 1), np.stack([np.ones(k), np.ones(k), z], 1),
+                      np.stack([np.full(k, -0.95), np.full(k, -1), z], 1)], 1).reshape(-1, 3).astype(F32)
+        idx = np.arange(3 * k, dtype=np.uint32).reshape(-1, 3)
+        o, d = random_rays(n, 81)
+        o[::4096] = (0.7, -0.7, -2.0)  # a few rays along z, through every box
+        d[::4096] = (1e-4, 1e-4, 1.0)
+    bvh = px.BVHAccelerator([px.Primitive.simple(px.TriangleMesh(None, None, False, idx, v))], 2, "sah")
+    rec = px.RayBatch(o, d, 0.0, np.where(rng.random(n) < 0.5, F32(1.1), F32(np.finfo(np.float32).max))).a
+    for a, b in zip(query_all(bvh, rec, "plain"), query_all(bvh, rec, "batched")):
+        assert np.array_equal(a, b)
+
+
 def walk_put_back(tree, depth, G, rng):
     """model.walk with leaves that go back on the stack while a record of the same step lies before them."""
     lim = GSTK_CL[G] - 3 * depth
