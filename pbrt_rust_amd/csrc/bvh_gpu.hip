@@ -13,20 +13,26 @@
 // Pipeline, all on the device:
 //   1. each primitive's box (the refined triple [c,b,a], mesh.rs:196-205;
 //      spheres' boxes come from the host as build_bvh computes them) and
-//      centroid (bvh.rs:77);
-//   2. the centroids' bounds; 63-bit Morton codes (21 bits an axis);
+//      centroid (bvh.rs:77), the centroids' bounds, and the check that every
+//      vertex index is in range;
+//   2. 63-bit Morton codes (21 bits an axis);
 //   3. radix sort of (code, prim) pairs (rocPRIM);
 //   4. the binary radix tree over the sorted codes (T. Karras, "Maximizing
 //      Parallelism in the Construction of BVHs, Octrees, and k-d Trees",
 //      HPG 2012), duplicate codes split by their sorted position;
-//   5. boxes and leaf counts bottom up (the second child to arrive at a node
-//      finishes it);
-//   6. depth-first positions top down, one level a launch (the reference
-//      layout: first child at i + 1, second child at `off`);
+//   5. the sorted leaves' boxes and the boxes of aligned runs of 8, 64, 512 ..
+//      of them; an interior node covers a run of leaves, so its box is the
+//      union of a few of those;
+//   6. depth-first positions in closed form (the reference layout: first child
+//      at i + 1, second child at `off`);
 //   7. the layouts the traversal kernels read: reference nodes, prim records
 //      in leaf order, four-wide records (interior nodes at even depth, their
 //      grandchildren as slots) and their compressed form.  Any-hit queries
 //      walk the compressed records (there are no separate occlusion records).
+// Nothing in it waits on another thread's result: steps 5 and 6 had been a
+// climb with one atomic and two device-wide fences a node (1.84 ms of a
+// 300,000-triangle build) and a launch a level (32 launches, 0.5 ms); they
+// take 0.07 ms.  16.8M triangles, uploads included: 170 -> 36.5 ms.
 #include <hip/hip_runtime.h>
 #include <string.h>
 
@@ -47,16 +53,55 @@ namespace {
 
 constexpr int GB = 256;
 constexpr uint32_t LEAF_BIT = 0x80000000u;  // child reference: a leaf (sorted position)
+constexpr uint32_t LEFT_BIT = 0x80000000u;  // parent reference: from the first child
 constexpr int MAX_LEVELS = 100;              // tree depth <= 63 code bits + 32 position bits + 1
 
 struct DBox {
     float lo[3], hi[3];
 };
 
-// 1. primitive boxes and centroids
-__global__ __launch_bounds__(GB) void k_prim_boxes(const float* verts, const uint32_t* idx, uint32_t nfaces,
-                                                   const DBox* sph_box, uint32_t nsph, DBox* box, float* cen) {
+// What the host reads back, written on the device.
+struct Header {
+    uint32_t nq;        // four-wide records
+    uint32_t maxdepth;  // of the deepest leaf
+    uint32_t bad_index; // a vertex index was out of range
+    uint32_t bad_cq;    // a record that the compressed form cannot hold
+    RNode root;
+};
+
+__device__ __forceinline__ float wave_min(float v) {
+    for (int o = 32; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o));
+    return v;
+}
+__device__ __forceinline__ float wave_max(float v) {
+    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
+    return v;
+}
+// the block's bounds (lo, hi of thread 0 .. GB-1) to out[6], by its first wave
+__device__ __forceinline__ void block_bounds(const float* lo, const float* hi, float* out) {
+    __shared__ float s[6][GB / 64];
+    const uint32_t lane = threadIdx.x & 63u, wid = threadIdx.x >> 6;
+    for (int a = 0; a < 3; ++a) {
+        const float l = wave_min(lo[a]), h = wave_max(hi[a]);
+        if (lane == 0) { s[a][wid] = l; s[3 + a][wid] = h; }
+    }
+    __syncthreads();
+    if (threadIdx.x < 6) {
+        float v = s[threadIdx.x][0];
+        for (uint32_t w = 1; w < GB / 64; ++w)
+            v = threadIdx.x < 3 ? fminf(v, s[threadIdx.x][w]) : fmaxf(v, s[threadIdx.x][w]);
+        out[threadIdx.x] = v;
+    }
+}
+
+// 1. primitive boxes and centroids, and the bounds of each block's centroids.
+// An index out of range is noted and read as the last vertex (the build then
+// ends with an error).
+__global__ __launch_bounds__(GB) void k_prim_boxes(const float* verts, uint32_t nverts, const uint32_t* idx,
+                                                   uint32_t nfaces, const DBox* sph_box, uint32_t nsph, DBox* box,
+                                                   float* cen, float* part, Header* hdr) {
     const uint32_t n = nfaces + nsph;
+    float lo[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, hi[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
     for (uint32_t i = blockIdx.x * GB + threadIdx.x; i < n; i += gridDim.x * GB) {
         DBox b;
         if (i < nfaces) {
@@ -64,7 +109,12 @@ __global__ __launch_bounds__(GB) void k_prim_boxes(const float* verts, const uin
             // then unions (fmin / fmax, bbox.rs:155-168)
             b = DBox{{FLT_MAX, FLT_MAX, FLT_MAX}, {-FLT_MAX, -FLT_MAX, -FLT_MAX}};
             for (int k = 2; k >= 0; --k) {
-                const float* p = verts + 3 * (size_t)idx[3 * (size_t)i + k];
+                uint32_t vi = idx[3 * (size_t)i + k];
+                if (vi >= nverts) {
+                    hdr->bad_index = 1u;
+                    vi = nverts - 1u;
+                }
+                const float* p = verts + 3 * (size_t)vi;
                 for (int a = 0; a < 3; ++a) {
                     b.lo[a] = fminf(b.lo[a], p[a]);
                     b.hi[a] = fmaxf(b.hi[a], p[a]);
@@ -74,41 +124,23 @@ __global__ __launch_bounds__(GB) void k_prim_boxes(const float* verts, const uin
             b = sph_box[i - nfaces];
         }
         box[i] = b;
-        for (int a = 0; a < 3; ++a) cen[3 * (size_t)i + a] = (b.lo[a] + b.hi[a]) * 0.5f;  // bvh.rs:77
-    }
-}
-
-// 2. centroid bounds: per-block partial min / max, then one block over them
-__global__ __launch_bounds__(GB) void k_cen_bounds(const float* cen, uint32_t n, float* part) {
-    __shared__ float s[6][GB];
-    float lo[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, hi[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
-    for (uint32_t i = blockIdx.x * GB + threadIdx.x; i < n; i += gridDim.x * GB)
         for (int a = 0; a < 3; ++a) {
-            const float c = cen[3 * (size_t)i + a];
+            const float c = (b.lo[a] + b.hi[a]) * 0.5f;  // bvh.rs:77
+            cen[3 * (size_t)i + a] = c;
             lo[a] = fminf(lo[a], c);
             hi[a] = fmaxf(hi[a], c);
         }
-    for (int a = 0; a < 3; ++a) { s[a][threadIdx.x] = lo[a]; s[3 + a][threadIdx.x] = hi[a]; }
-    __syncthreads();
-    for (int w = GB / 2; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w)
-            for (int a = 0; a < 3; ++a) {
-                s[a][threadIdx.x] = fminf(s[a][threadIdx.x], s[a][threadIdx.x + w]);
-                s[3 + a][threadIdx.x] = fmaxf(s[3 + a][threadIdx.x], s[3 + a][threadIdx.x + w]);
-            }
-        __syncthreads();
     }
-    if (threadIdx.x < 6) part[6 * blockIdx.x + threadIdx.x] = s[threadIdx.x][0];
+    block_bounds(lo, hi, part + 6 * (size_t)blockIdx.x);
 }
-__global__ __launch_bounds__(GB) void k_cen_bounds_final(const float* part, uint32_t nb, float* out) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    float r[6] = {FLT_MAX, FLT_MAX, FLT_MAX, -FLT_MAX, -FLT_MAX, -FLT_MAX};
-    for (uint32_t b = 0; b < nb; ++b)
+__global__ __launch_bounds__(GB) void k_cen_bounds(const float* part, uint32_t nb, float* out) {
+    float lo[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, hi[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
+    for (uint32_t b = threadIdx.x; b < nb; b += GB)
         for (int a = 0; a < 3; ++a) {
-            r[a] = fminf(r[a], part[6 * b + a]);
-            r[3 + a] = fmaxf(r[3 + a], part[6 * b + 3 + a]);
+            lo[a] = fminf(lo[a], part[6 * (size_t)b + a]);
+            hi[a] = fmaxf(hi[a], part[6 * (size_t)b + 3 + a]);
         }
-    for (int k = 0; k < 6; ++k) out[k] = r[k];
+    block_bounds(lo, hi, out);
 }
 
 __device__ __forceinline__ uint64_t spread21(uint64_t v) {
@@ -144,8 +176,9 @@ __device__ __forceinline__ int delta(const uint64_t* k, uint32_t n, int64_t i, i
     if (x) return __clzll((long long)x);
     return 64 + __clz((int)((uint32_t)i ^ (uint32_t)j));  // equal codes: by position
 }
-__global__ __launch_bounds__(GB) void k_karras(const uint64_t* k, uint32_t n, uint32_t* child, uint32_t* parent_i,
-                                               uint32_t* parent_l, uint2* range) {
+// parent[x] of an interior node: its parent, LEFT_BIT when it is the first child.
+__global__ __launch_bounds__(GB) void k_karras(const uint64_t* k, uint32_t n, uint32_t* child, uint32_t* parent,
+                                               uint2* range) {
     for (uint32_t ii = blockIdx.x * GB + threadIdx.x; ii + 1 < n; ii += gridDim.x * GB) {
         const int64_t i = ii;
         const int d = (delta(k, n, i, i + 1) - delta(k, n, i, i - 1)) >= 0 ? 1 : -1;
@@ -169,92 +202,146 @@ __global__ __launch_bounds__(GB) void k_karras(const uint64_t* k, uint32_t n, ui
         child[2 * ii] = left;
         child[2 * ii + 1] = right;
         range[ii] = make_uint2((uint32_t)lo, (uint32_t)hi);
-        if (left & LEAF_BIT) parent_l[left & ~LEAF_BIT] = ii;
-        else parent_i[left] = ii;
-        if (right & LEAF_BIT) parent_l[right & ~LEAF_BIT] = ii;
-        else parent_i[right] = ii;
+        if (!(left & LEAF_BIT)) parent[left] = (uint32_t)ii | LEFT_BIT;
+        if (!(right & LEAF_BIT)) parent[right] = (uint32_t)ii;
     }
 }
 
-// 5. boxes and leaf counts bottom up: a leaf's thread climbs while it is the
-// second child to arrive
-__global__ __launch_bounds__(GB) void k_bottom_up(const uint32_t* val, const DBox* pbox, uint32_t n,
-                                                  const uint32_t* child, const uint32_t* parent_i,
-                                                  const uint32_t* parent_l, uint32_t* arrive, DBox* ibox,
-                                                  uint32_t* nleaf) {
-    for (uint32_t j = blockIdx.x * GB + threadIdx.x; j < n; j += gridDim.x * GB) {
-        if (n == 1) break;
-        uint32_t node = parent_l[j];
-        while (true) {
-            __threadfence();
-            if (atomicAdd(arrive + node, 1u) == 0u) break;  // the sibling finishes this node
-            __threadfence();
-            DBox b{{FLT_MAX, FLT_MAX, FLT_MAX}, {-FLT_MAX, -FLT_MAX, -FLT_MAX}};
-            uint32_t cnt = 0;
-            for (int c = 0; c < 2; ++c) {
-                const uint32_t ch = child[2 * node + c];
-                DBox cb;
-                if (ch & LEAF_BIT) {
-                    cb = pbox[val[ch & ~LEAF_BIT]];
-                    cnt += 1;
-                } else {
-                    // written by the other climber before its atomic
-                    const volatile DBox* vb = ibox + ch;
-                    for (int a = 0; a < 3; ++a) { cb.lo[a] = vb->lo[a]; cb.hi[a] = vb->hi[a]; }
-                    cnt += ((volatile uint32_t*)nleaf)[ch];
-                }
-                // Union<BBox> (bbox.rs:170-183): left first, then right
-                for (int a = 0; a < 3; ++a) {
-                    b.lo[a] = fminf(b.lo[a], cb.lo[a]);
-                    b.hi[a] = fmaxf(b.hi[a], cb.hi[a]);
-                }
-            }
-            ibox[node] = b;
-            nleaf[node] = cnt;
-            if (node == 0) break;
-            node = parent_i[node];
+__device__ __forceinline__ void grow(DBox& b, const DBox& c) {
+    // Union<BBox> (bbox.rs:170-183); min and max give the same bits in any order
+    for (int a = 0; a < 3; ++a) {
+        b.lo[a] = fminf(b.lo[a], c.lo[a]);
+        b.hi[a] = fmaxf(b.hi[a], c.hi[a]);
+    }
+}
+__device__ __forceinline__ DBox empty_box() {
+    return DBox{{FLT_MAX, FLT_MAX, FLT_MAX}, {-FLT_MAX, -FLT_MAX, -FLT_MAX}};
+}
+
+// 5a. Runs of boxes: level 0 holds the sorted leaves' boxes, level k the boxes
+// of aligned runs of 8^k of them (the last run may be short).  One launch
+// makes three levels from one: a block takes 512 boxes of level `base`, its
+// 64 runs of 8, 8 runs of 64 and the run of 512.  val (level 0 only): where
+// the sorted leaves' boxes are.  Streaming: 24 B in and 27 out a leaf.
+constexpr int RUN_LEVELS = 11;  // 8^10 = 2^30 leaves
+struct Runs {
+    DBox* box;
+    uint32_t first[RUN_LEVELS], count[RUN_LEVELS];  // a level's boxes: box[first ..]
+    uint32_t levels;
+};
+constexpr int RUN_B = 512;
+__global__ __launch_bounds__(RUN_B) void k_runs(Runs r, uint32_t base, const uint32_t* val, const DBox* pbox) {
+    __shared__ DBox s0[RUN_B], s1[RUN_B / 8], s2[RUN_B / 64];
+    const uint32_t t = threadIdx.x, i = blockIdx.x * RUN_B + t;
+    DBox b = empty_box();
+    if (i < r.count[base]) {
+        if (val) {
+            b = pbox[val[i]];
+            r.box[r.first[base] + i] = b;
+        } else {
+            b = r.box[r.first[base] + i];
         }
     }
+    s0[t] = b;
+    __syncthreads();
+    if (t < RUN_B / 8 && base + 1 < r.levels) {
+        DBox c = empty_box();
+        for (int k = 0; k < 8; ++k) grow(c, s0[8 * t + k]);
+        s1[t] = c;
+        const uint32_t j = blockIdx.x * (RUN_B / 8) + t;
+        if (j < r.count[base + 1]) r.box[r.first[base + 1] + j] = c;
+    }
+    __syncthreads();
+    if (t < RUN_B / 64 && base + 2 < r.levels) {
+        DBox c = empty_box();
+        for (int k = 0; k < 8; ++k) grow(c, s1[8 * t + k]);
+        s2[t] = c;
+        const uint32_t j = blockIdx.x * (RUN_B / 64) + t;
+        if (j < r.count[base + 2]) r.box[r.first[base + 2] + j] = c;
+    }
+    __syncthreads();
+    if (t == 0 && base + 3 < r.levels) {
+        DBox c = empty_box();
+        for (int k = 0; k < 8; ++k) grow(c, s2[k]);
+        r.box[r.first[base + 3] + blockIdx.x] = c;
+    }
 }
 
-// 6. depth-first positions, one tree level a launch: internal node x at
-// position p has its first child at p + 1 and its second at p + 2 * (leaves
-// under the first child); depth d for both.  Lists double-buffered, counts in
-// three rotating words (level L reads count L % 3, adds to (L + 1) % 3 and
-// clears (L + 2) % 3, which level L - 1 read).
-__global__ __launch_bounds__(GB) void k_preorder_level(int level, const uint32_t* child, const uint32_t* nleaf,
-                                                       const uint32_t* list_in, uint32_t* list_out, uint32_t* counts,
-                                                       uint32_t* pos_i, uint32_t* pos_l, uint32_t* depth_i,
-                                                       uint32_t* maxdepth) {
-    const uint32_t cnt = counts[level % 3];
-    if (blockIdx.x == 0 && threadIdx.x == 0) counts[(level + 2) % 3] = 0u;
-    for (uint32_t t = blockIdx.x * GB + threadIdx.x; t < cnt; t += gridDim.x * GB) {
-        const uint32_t x = list_in[t];
-        const uint32_t p = pos_i[x];
+// 5b, 6. An interior node's box from its leaves lo .. hi: level by level the
+// boxes up to the next aligned run from either end, then whole runs (half the
+// nodes hold two leaves; a node of m leaves reads at most 14 log8 m boxes).
+// Its depth-first position: before it come its ancestors and, for each of
+// them that it lies in the second child of, the whole first child, 2m - 1
+// nodes for m leaves; those leaves are the lo before its own, so the position
+// is 2 lo + the ancestors that it lies in the first child of.  A leaf's is the
+// same.
+__global__ __launch_bounds__(GB) void k_nodes(uint32_t n, const uint32_t* child, const uint32_t* parent,
+                                              const uint2* range, Runs r, DBox* ibox, uint32_t* pos_i,
+                                              uint32_t* pos_l, uint32_t* depth_i, Header* hdr) {
+    uint32_t deepest = 0, recs = 0;
+    for (uint32_t x = blockIdx.x * GB + threadIdx.x; x + 1 < n; x += gridDim.x * GB) {
+        const uint2 rg = range[x];
+        uint32_t lo = rg.x, hi = rg.y;
+        const uint32_t first = lo;
+        DBox b = empty_box();
+        // a run's box may be joined twice, so the ends take seven boxes each,
+        // whatever lies before the next aligned run: independent loads
+        for (uint32_t lv = 0;; ++lv) {
+            const DBox* box = r.box + r.first[lv];
+            if (hi - lo < 16u) {
+                for (uint32_t k = 0; k <= hi - lo; k += 4)
+#pragma unroll
+                    for (uint32_t u = 0; u < 4; ++u) grow(b, box[min(lo + k + u, hi)]);
+                break;
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < 7; ++k) {
+                grow(b, box[lo + k]);
+                grow(b, box[hi - k]);
+            }
+            lo = (lo + 7u) >> 3;
+            hi = ((hi + 1u) >> 3) - 1u;
+        }
+        ibox[x] = b;
+        uint32_t depth = 0, lefts = 0;
+        for (uint32_t y = x; y != 0u;) {
+            const uint32_t p = parent[y];
+            ++depth;
+            lefts += p >> 31;
+            y = p & ~LEFT_BIT;
+        }
+        pos_i[x] = 2u * first + lefts;
+        depth_i[x] = depth;
+        deepest = max(deepest, depth + 1u);
+        recs += (depth & 1u) ^ 1u;  // a record starts at every even depth
         const uint32_t L = child[2 * x], R = child[2 * x + 1];
-        const uint32_t nl = (L & LEAF_BIT) ? 1u : nleaf[L];
-        const uint32_t pl = p + 1, pr = p + 2 * nl;
-        const uint32_t d = (uint32_t)level + 1;
-        atomicMax(maxdepth, d);
-        if (L & LEAF_BIT) pos_l[L & ~LEAF_BIT] = pl;
-        else { pos_i[L] = pl; depth_i[L] = d; list_out[atomicAdd(counts + (level + 1) % 3, 1u)] = L; }
-        if (R & LEAF_BIT) pos_l[R & ~LEAF_BIT] = pr;
-        else { pos_i[R] = pr; depth_i[R] = d; list_out[atomicAdd(counts + (level + 1) % 3, 1u)] = R; }
+        if (L & LEAF_BIT) pos_l[L & ~LEAF_BIT] = 2u * (L & ~LEAF_BIT) + lefts + 1u;
+        if (R & LEAF_BIT) pos_l[R & ~LEAF_BIT] = 2u * (R & ~LEAF_BIT) + lefts;
+    }
+    __shared__ uint32_t s_deep, s_recs;
+    if (threadIdx.x == 0) s_deep = s_recs = 0u;
+    __syncthreads();
+    atomicMax(&s_deep, deepest);
+    atomicAdd(&s_recs, recs);
+    __syncthreads();
+    if (threadIdx.x == 0 && s_deep) {
+        atomicMax(&hdr->maxdepth, s_deep);
+        atomicAdd(&hdr->nq, s_recs);
     }
 }
 
 // 7a. reference nodes in depth-first order, record flags, prim records
-__global__ __launch_bounds__(GB) void k_rnodes(uint32_t n, const uint32_t* child, const DBox* ibox, const DBox* pbox,
-                                               const uint32_t* val, const uint32_t* pos_i, const uint32_t* pos_l,
-                                               const uint32_t* depth_i, RNode* rn, uint32_t* is_rec) {
+__global__ __launch_bounds__(GB) void k_rnodes(uint32_t n, const uint32_t* child, const DBox* ibox, const DBox* leaf,
+                                               const uint32_t* pos_i, const uint32_t* pos_l, const uint32_t* depth_i,
+                                               RNode* rn, uint32_t* is_rec) {
     const uint32_t total = 2 * n - 1;
     for (uint32_t t = blockIdx.x * GB + threadIdx.x; t < total; t += gridDim.x * GB) {
         if (t < n - 1) {
             // interior node t: the children's axis of greatest centre separation
             // picks the near child (bvh.rs:409-415 reads the node's axis)
             const uint32_t L = child[2 * t], R = child[2 * t + 1];
-            const DBox bl = (L & LEAF_BIT) ? pbox[val[L & ~LEAF_BIT]] : ibox[L];
-            const DBox br = (R & LEAF_BIT) ? pbox[val[R & ~LEAF_BIT]] : ibox[R];
+            const DBox bl = (L & LEAF_BIT) ? leaf[L & ~LEAF_BIT] : ibox[L];
+            const DBox br = (R & LEAF_BIT) ? leaf[R & ~LEAF_BIT] : ibox[R];
             int axis = 0;
             float best = -1.0f;
             for (int a = 0; a < 3; ++a) {
@@ -271,7 +358,7 @@ __global__ __launch_bounds__(GB) void k_rnodes(uint32_t n, const uint32_t* child
         } else {
             const uint32_t j = t - (n - 1);  // leaf at sorted position j
             RNode r;
-            const DBox& b = pbox[val[j]];
+            const DBox& b = leaf[j];
             for (int a = 0; a < 3; ++a) { r.lo[a] = b.lo[a]; r.hi[a] = b.hi[a]; }
             r.off = j;
             r.meta = 3u | (1u << 2);
@@ -285,18 +372,20 @@ __global__ __launch_bounds__(GB) void k_rnodes(uint32_t n, const uint32_t* child
 __device__ __forceinline__ float as_f(uint32_t u) { return __uint_as_float(u); }
 
 __global__ __launch_bounds__(GB) void k_prim_recs(uint32_t n, uint32_t nfaces, const uint32_t* val,
-                                                  const float* verts, const uint32_t* idx, const RNode* rn,
-                                                  const uint32_t* pos_l, PrimRec* pr, PrimRec64* pr64) {
+                                                  const float* verts, uint32_t nverts, const uint32_t* idx,
+                                                  const DBox* leaf, PrimRec* pr, PrimRec64* pr64, uint32_t* order) {
     for (uint32_t j = blockIdx.x * GB + threadIdx.x; j < n; j += gridDim.x * GB) {
         const uint32_t id = val[j];
+        order[j] = id;
         PrimRec r;
         for (int k = 0; k < 12; ++k) r.w[k] = 0.0f;
         r.w[10] = as_f(id);
         uint32_t kind;
         if (id < nfaces) {
-            const float* p1 = verts + 3 * (size_t)idx[3 * (size_t)id + 2];
-            const float* p2 = verts + 3 * (size_t)idx[3 * (size_t)id + 1];
-            const float* p3 = verts + 3 * (size_t)idx[3 * (size_t)id + 0];
+            // (an index out of range is the last vertex, as in k_prim_boxes)
+            const float* p1 = verts + 3 * (size_t)min(idx[3 * (size_t)id + 2], nverts - 1u);
+            const float* p2 = verts + 3 * (size_t)min(idx[3 * (size_t)id + 1], nverts - 1u);
+            const float* p3 = verts + 3 * (size_t)min(idx[3 * (size_t)id + 0], nverts - 1u);
             for (int a = 0; a < 3; ++a) {
                 r.w[a] = p1[a];
                 r.w[3 + a] = p2[a] - p1[a];
@@ -314,8 +403,8 @@ __global__ __launch_bounds__(GB) void k_prim_recs(uint32_t n, uint32_t nfaces, c
         PrimRec64 q;
         for (int k = 0; k < 9; ++k) q.w[k] = r.w[k];
         if ((kind & 0xFFu) != 0u) q.w[0] = r.w[9];
-        const RNode& leaf = rn[n == 1 ? 0u : pos_l[j]];
-        for (int a = 0; a < 3; ++a) { q.w[9 + a] = leaf.lo[a]; q.w[12 + a] = leaf.hi[a]; }
+        const DBox b = leaf[j];
+        for (int a = 0; a < 3; ++a) { q.w[9 + a] = b.lo[a]; q.w[12 + a] = b.hi[a]; }
         q.w[15] = r.w[11];
         pr64[j] = q;
     }
@@ -326,36 +415,14 @@ __global__ __launch_bounds__(GB) void k_prim_recs(uint32_t n, uint32_t nfaces, c
 // child is a slot itself); refs: ~(prim position) for a leaf, else the
 // record index of the node (qidx = exclusive scan of is_rec)
 __device__ __forceinline__ bool is_leaf_node(const RNode& r) { return (r.meta & 3u) == 3u; }
-__global__ __launch_bounds__(GB) void k_qnodes(uint32_t nnodes, const RNode* rn, const uint32_t* is_rec,
-                                               const uint32_t* qidx, QNode* qn) {
+// rec[q] = the position of record q; and the root for the host
+__global__ __launch_bounds__(GB) void k_rec_list(uint32_t nnodes, const uint32_t* is_rec, const uint32_t* qidx,
+                                                 const RNode* rn, uint32_t* rec, Header* hdr) {
     for (uint32_t a = blockIdx.x * GB + threadIdx.x; a < nnodes; a += gridDim.x * GB) {
-        if (!is_rec[a]) continue;
-        QNode q;
-        const uint32_t b = a + 1, c = rn[a].off;
-        uint32_t s[4];
-        const uint32_t none = 0xFFFFFFFFu;
-        if (is_leaf_node(rn[b])) { s[0] = b; s[1] = none; } else { s[0] = b + 1; s[1] = rn[b].off; }
-        if (is_leaf_node(rn[c])) { s[2] = c; s[3] = none; } else { s[2] = c + 1; s[3] = rn[c].off; }
-        const uint32_t ab = is_leaf_node(rn[b]) ? 0u : (rn[b].meta & 3u);
-        const uint32_t ac = is_leaf_node(rn[c]) ? 0u : (rn[c].meta & 3u);
-        q.meta = (rn[a].meta & 3u) | (ab << 2) | (ac << 4);
-        q.pad[0] = q.pad[1] = q.pad[2] = 0u;
-        for (int k = 0; k < 4; ++k) {
-            if (s[k] == none) {
-                q.ref[k] = QEMPTY;
-                q.lx[k] = q.ly[k] = q.lz[k] = FLT_MAX;
-                q.hx[k] = q.hy[k] = q.hz[k] = -FLT_MAX;
-                continue;
-            }
-            const RNode& r = rn[s[k]];
-            q.ref[k] = is_leaf_node(r) ? ~(int32_t)r.off : (int32_t)qidx[s[k]];
-            q.lx[k] = r.lo[0]; q.ly[k] = r.lo[1]; q.lz[k] = r.lo[2];
-            q.hx[k] = r.hi[0]; q.hy[k] = r.hi[1]; q.hz[k] = r.hi[2];
-        }
-        qn[qidx[a]] = q;
+        if (is_rec[a]) rec[qidx[a]] = a;
+        if (a == 0) hdr->root = rn[0];
     }
 }
-
 // 7c. the compressed records (as compress_records on the host: per axis the
 // smallest power-of-two scale that spans the union box in 255 steps, bytes
 // rounded outward and checked against the float the traversal decodes)
@@ -392,30 +459,54 @@ __device__ bool cq_axis_d(float ulo, float uhi, const float* lo, const float* hi
     *ebyte = (uint32_t)(e + 127);
     return true;
 }
-__global__ __launch_bounds__(GB) void k_cnodes(uint32_t nq, const QNode* qn, CNode* cn, uint32_t* bad) {
+__global__ __launch_bounds__(GB) void k_records(uint32_t nq, const uint32_t* rec, const RNode* rn,
+                                                const uint32_t* qidx, QNode* qn, CNode* cn, Header* hdr) {
     for (uint32_t i = blockIdx.x * GB + threadIdx.x; i < nq; i += gridDim.x * GB) {
-        const QNode& q = qn[i];
-        CNode c;
+        const uint32_t a = rec[i];
+        QNode q;
+        const uint32_t b = a + 1, c = rn[a].off;
+        uint32_t s[4];
+        const uint32_t none = 0xFFFFFFFFu;
+        if (is_leaf_node(rn[b])) { s[0] = b; s[1] = none; } else { s[0] = b + 1; s[1] = rn[b].off; }
+        if (is_leaf_node(rn[c])) { s[2] = c; s[3] = none; } else { s[2] = c + 1; s[3] = rn[c].off; }
+        const uint32_t ab = is_leaf_node(rn[b]) ? 0u : (rn[b].meta & 3u);
+        const uint32_t ac = is_leaf_node(rn[c]) ? 0u : (rn[c].meta & 3u);
+        q.meta = (rn[a].meta & 3u) | (ab << 2) | (ac << 4);
+        q.pad[0] = q.pad[1] = q.pad[2] = 0u;
+        for (int k = 0; k < 4; ++k) {
+            if (s[k] == none) {
+                q.ref[k] = QEMPTY;
+                q.lx[k] = q.ly[k] = q.lz[k] = FLT_MAX;
+                q.hx[k] = q.hy[k] = q.hz[k] = -FLT_MAX;
+                continue;
+            }
+            const RNode& r = rn[s[k]];
+            q.ref[k] = is_leaf_node(r) ? ~(int32_t)r.off : (int32_t)qidx[s[k]];
+            q.lx[k] = r.lo[0]; q.ly[k] = r.lo[1]; q.lz[k] = r.lo[2];
+            q.hx[k] = r.hi[0]; q.hy[k] = r.hi[1]; q.hz[k] = r.hi[2];
+        }
+        qn[i] = q;
+        CNode cr;
         bool used[4];
         float u[6] = {FLT_MAX, FLT_MAX, FLT_MAX, -FLT_MAX, -FLT_MAX, -FLT_MAX};
         for (int k = 0; k < 4; ++k) {
             used[k] = q.ref[k] != QEMPTY;
-            c.ref[k] = q.ref[k];
+            cr.ref[k] = q.ref[k];
             if (!used[k]) continue;
             u[0] = fminf(u[0], q.lx[k]); u[1] = fminf(u[1], q.ly[k]); u[2] = fminf(u[2], q.lz[k]);
             u[3] = fmaxf(u[3], q.hx[k]); u[4] = fmaxf(u[4], q.hy[k]); u[5] = fmaxf(u[5], q.hz[k]);
         }
         uint32_t ex = 0, ey = 0, ez = 0;
-        if (!cq_axis_d(u[0], u[3], q.lx, q.hx, used, c.q + 0, c.q + 4, &ex) ||
-            !cq_axis_d(u[1], u[4], q.ly, q.hy, used, c.q + 8, c.q + 12, &ey) ||
-            !cq_axis_d(u[2], u[5], q.lz, q.hz, used, c.q + 16, c.q + 20, &ez)) {
-            atomicOr(bad, 1u);
+        if (!cq_axis_d(u[0], u[3], q.lx, q.hx, used, cr.q + 0, cr.q + 4, &ex) ||
+            !cq_axis_d(u[1], u[4], q.ly, q.hy, used, cr.q + 8, cr.q + 12, &ey) ||
+            !cq_axis_d(u[2], u[5], q.lz, q.hz, used, cr.q + 16, cr.q + 20, &ez)) {
+            hdr->bad_cq = 1u;
             continue;
         }
-        c.ox = u[0]; c.oy = u[1]; c.oz = u[2];
-        c.emeta = ex | (ey << 8) | (ez << 16) | ((q.meta & 63u) << 24);
-        c.pad[0] = c.pad[1] = 0u;
-        cn[i] = c;
+        cr.ox = u[0]; cr.oy = u[1]; cr.oz = u[2];
+        cr.emeta = ex | (ey << 8) | (ez << 16) | ((q.meta & 63u) << 24);
+        cr.pad[0] = cr.pad[1] = 0u;
+        cn[i] = cr;
     }
 }
 
@@ -424,21 +515,28 @@ uint32_t grid_for(uint64_t n) {
     return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(b, (uint64_t)device_cu_count() * 16));
 }
 
-template <typename T>
-hipError_t dalloc(T** p, size_t count) {
-    return hipMalloc((void**)p, std::max<size_t>(count, 1) * sizeof(T));
-}
-
-struct Scratch {
-    std::vector<void*> ptrs;
-    ~Scratch() {
-        for (void* p : ptrs) (void)hipFree(p);
+// One device allocation for several arrays: take() them all twice, before
+// alloc() to add up their bytes and after it to have their places.
+struct Slab {
+    uint8_t* p = nullptr;
+    size_t at = 0;
+    ~Slab() {
+        if (p) (void)hipFree(p);
     }
-    template <typename T>
-    hipError_t get(T** p, size_t count) {
-        hipError_t e = dalloc(p, count);
-        if (e == hipSuccess) ptrs.push_back(*p);
+    template <typename U>
+    void take(U** out, size_t count) {
+        *out = reinterpret_cast<U*>(p + at);
+        at += (std::max<size_t>(count, 1) * sizeof(U) + 255) / 256 * 256;
+    }
+    hipError_t alloc() {
+        const hipError_t e = hipMalloc((void**)&p, at);
+        at = 0;
         return e;
+    }
+    void* release() {
+        void* q = p;
+        p = nullptr;
+        return q;
     }
 };
 
@@ -476,8 +574,7 @@ int gpu_build_scene(const float* verts, uint32_t nverts, const uint32_t* idx, ui
     if (N64 >= (1ull << 30)) return fail(PBRTX_ERR_BUILD, "too many primitives");
     if (nfaces && (!verts || !idx)) return fail(PBRTX_ERR_ARG, "null mesh arrays");
     if (nsph && !sph) return fail(PBRTX_ERR_ARG, "null sphere array");
-    for (uint64_t i = 0; i < 3ull * nfaces; ++i)
-        if (idx[i] >= nverts) return fail(PBRTX_ERR_BUILD, "vertex index out of range");
+    if (nfaces && nverts == 0) return fail(PBRTX_ERR_BUILD, "vertex index out of range");
     std::string err;
     std::vector<DBox> sbox;
     std::vector<SphereRec> srec;
@@ -485,154 +582,133 @@ int gpu_build_scene(const float* verts, uint32_t nverts, const uint32_t* idx, ui
     const uint32_t n = (uint32_t)N64;
     const uint32_t nnodes = 2 * n - 1;
     hipStream_t st = nullptr;
-    Scratch T;
+    // the boxes' runs: level k holds ceil(n / 8^k)
+    Runs runs{};
+    uint32_t nruns = 0;
+    for (uint64_t c = n;; c = (c + 7) / 8) {
+        runs.first[runs.levels] = nruns;
+        runs.count[runs.levels++] = (uint32_t)c;
+        nruns += (uint32_t)c;
+        if (c == 1) break;
+    }
+    const uint32_t nb = grid_for(n);
+    size_t sort_bytes = 0, scan_bytes = 0;
+    GCHK(rocprim::radix_sort_pairs((void*)nullptr, sort_bytes, (uint64_t*)nullptr, (uint64_t*)nullptr,
+                                   (uint32_t*)nullptr, (uint32_t*)nullptr, n, 0, 63, st));
+    GCHK(rocprim::exclusive_scan((void*)nullptr, scan_bytes, (uint32_t*)nullptr, (uint32_t*)nullptr, 0u, nnodes,
+                                 rocprim::plus<uint32_t>(), st));
+    // One allocation holds everything that the build itself needs and one the
+    // scene: an allocation costs some 0.1 ms, a release 0.1-0.2 and a wait for
+    // the device (40 of each: 4 of the 7.5 ms of a 300,000-triangle build).
     float *d_verts, *d_cen, *d_part, *d_cb;
-    uint32_t *d_idx, *d_val, *d_val2, *d_child, *d_pi, *d_pl, *d_arrive, *d_nleaf, *d_posi, *d_posl, *d_depth,
-        *d_list0, *d_list1, *d_counts, *d_maxd, *d_isrec, *d_qidx, *d_bad;
+    uint32_t *d_idx, *d_val, *d_val2, *d_child, *d_parent, *d_posi, *d_posl, *d_depth, *d_isrec, *d_qidx;
     uint64_t *d_key, *d_key2;
     uint2* d_range;
     DBox *d_pbox, *d_sbox, *d_ibox;
-    GCHK(T.get(&d_verts, 3 * (size_t)nverts));
-    GCHK(T.get(&d_idx, 3 * (size_t)nfaces));
-    GCHK(T.get(&d_sbox, nsph));
-    GCHK(T.get(&d_pbox, n));
-    GCHK(T.get(&d_cen, 3 * (size_t)n));
+    Header* d_hdr;
+    uint8_t *sort_tmp, *scan_tmp;
+    Slab T;
+    for (int pass = 0; pass < 2; ++pass) {
+        T.take(&d_verts, 3 * (size_t)nverts);
+        T.take(&d_idx, 3 * (size_t)nfaces);
+        T.take(&d_sbox, nsph);
+        T.take(&d_pbox, n);
+        T.take(&d_cen, 3 * (size_t)n);
+        T.take(&d_part, 6 * (size_t)nb);
+        T.take(&d_cb, 6);
+        T.take(&d_key, n);
+        T.take(&d_key2, n);
+        T.take(&d_val, n);
+        T.take(&d_val2, n);
+        T.take(&sort_tmp, sort_bytes);
+        T.take(&scan_tmp, scan_bytes);
+        T.take(&d_child, 2 * (size_t)n);
+        T.take(&d_parent, n);
+        T.take(&d_range, n);
+        T.take(&runs.box, nruns);
+        T.take(&d_ibox, n);
+        T.take(&d_posi, n);
+        T.take(&d_posl, n);
+        T.take(&d_depth, n);
+        T.take(&d_isrec, nnodes);
+        T.take(&d_qidx, nnodes);
+        T.take(&d_hdr, 1);
+        if (pass == 0) GCHK(T.alloc());
+    }
+    GCHK(fill_u32((uint32_t*)d_hdr, 0u, sizeof(Header) / 4, st));
     if (nverts) GCHK(hipMemcpyAsync(d_verts, verts, 12 * (size_t)nverts, hipMemcpyHostToDevice, st));
     if (nfaces) GCHK(hipMemcpyAsync(d_idx, idx, 12 * (size_t)nfaces, hipMemcpyHostToDevice, st));
     if (nsph) GCHK(hipMemcpyAsync(d_sbox, sbox.data(), sizeof(DBox) * nsph, hipMemcpyHostToDevice, st));
-    hipLaunchKernelGGL(k_prim_boxes, dim3(grid_for(n)), dim3(GB), 0, st, d_verts, d_idx, nfaces, d_sbox, nsph, d_pbox,
-                       d_cen);
-    GCHK(hipGetLastError());
-    const uint32_t nb = std::min<uint32_t>(grid_for(n), 1024u);
-    GCHK(T.get(&d_part, 6 * (size_t)nb));
-    GCHK(T.get(&d_cb, 6));
-    hipLaunchKernelGGL(k_cen_bounds, dim3(nb), dim3(GB), 0, st, d_cen, n, d_part);
-    hipLaunchKernelGGL(k_cen_bounds_final, dim3(1), dim3(GB), 0, st, d_part, nb, d_cb);
-    GCHK(hipGetLastError());
-    GCHK(T.get(&d_key, n));
-    GCHK(T.get(&d_key2, n));
-    GCHK(T.get(&d_val, n));
-    GCHK(T.get(&d_val2, n));
+    hipLaunchKernelGGL(k_prim_boxes, dim3(nb), dim3(GB), 0, st, d_verts, nverts, d_idx, nfaces, d_sbox, nsph, d_pbox,
+                       d_cen, d_part, d_hdr);
+    hipLaunchKernelGGL(k_cen_bounds, dim3(1), dim3(GB), 0, st, d_part, nb, d_cb);
     hipLaunchKernelGGL(k_morton, dim3(grid_for(n)), dim3(GB), 0, st, d_cen, n, d_cb, d_key, d_val);
     GCHK(hipGetLastError());
-    {
-        size_t tb = 0;
-        GCHK(rocprim::radix_sort_pairs(nullptr, tb, d_key, d_key2, d_val, d_val2, n, 0, 63, st));
-        void* tmp;
-        GCHK(T.get((uint8_t**)&tmp, tb));
-        GCHK(rocprim::radix_sort_pairs(tmp, tb, d_key, d_key2, d_val, d_val2, n, 0, 63, st));
-    }
+    GCHK(rocprim::radix_sort_pairs((void*)sort_tmp, sort_bytes, d_key, d_key2, d_val, d_val2, n, 0, 63, st));
     std::swap(d_key, d_key2);
     std::swap(d_val, d_val2);
-    GCHK(T.get(&d_child, 2 * (size_t)n));
-    GCHK(T.get(&d_pi, n));
-    GCHK(T.get(&d_pl, n));
-    GCHK(T.get(&d_range, n));
-    GCHK(T.get(&d_arrive, n));
-    GCHK(T.get(&d_nleaf, n));
-    GCHK(T.get(&d_ibox, n));
-    GCHK(fill_u32(d_arrive, 0u, n, st));
     if (n > 1) {
-        hipLaunchKernelGGL(k_karras, dim3(grid_for(n)), dim3(GB), 0, st, d_key, n, d_child, d_pi, d_pl, d_range);
-        hipLaunchKernelGGL(k_bottom_up, dim3(grid_for(n)), dim3(GB), 0, st, d_val, d_pbox, n, d_child, d_pi, d_pl,
-                           d_arrive, d_ibox, d_nleaf);
+        hipLaunchKernelGGL(k_karras, dim3(grid_for(n)), dim3(GB), 0, st, d_key, n, d_child, d_parent, d_range);
         GCHK(hipGetLastError());
     }
-    GCHK(T.get(&d_posi, n));
-    GCHK(T.get(&d_posl, n));
-    GCHK(T.get(&d_depth, n));
-    GCHK(T.get(&d_list0, n));
-    GCHK(T.get(&d_list1, n));
-    GCHK(T.get(&d_counts, 4));
-    GCHK(T.get(&d_maxd, 1));
-    {
-        // level 0: the root (internal node 0) at position 0, depth 0
-        const uint32_t init_counts[4] = {n > 1 ? 1u : 0u, 0u, 0u, 0u};
-        const uint32_t zero = 0;
-        GCHK(hipMemcpyAsync(d_counts, init_counts, sizeof(init_counts), hipMemcpyHostToDevice, st));
-        GCHK(hipMemcpyAsync(d_list0, &zero, 4, hipMemcpyHostToDevice, st));
-        GCHK(hipMemcpyAsync(d_posi, &zero, 4, hipMemcpyHostToDevice, st));
-        GCHK(hipMemcpyAsync(d_depth, &zero, 4, hipMemcpyHostToDevice, st));
-        GCHK(hipMemcpyAsync(d_maxd, &zero, 4, hipMemcpyHostToDevice, st));
-        GCHK(hipStreamSynchronize(st));  // the host values above stay valid until here
-        for (int level = 0; level < MAX_LEVELS && n > 1; ++level) {
-            hipLaunchKernelGGL(k_preorder_level, dim3(grid_for(n / 2 + 1)), dim3(GB), 0, st, level, d_child, d_nleaf,
-                               (level & 1) ? d_list1 : d_list0, (level & 1) ? d_list0 : d_list1, d_counts, d_posi,
-                               d_posl, d_depth, d_maxd);
-            GCHK(hipGetLastError());
-            if ((level & 15) == 15) {
-                uint32_t c[3];
-                GCHK(hipMemcpy(c, d_counts, sizeof(c), hipMemcpyDeviceToHost));
-                if (c[(level + 1) % 3] == 0) break;
-            }
-        }
+    for (uint32_t lv = 0; lv == 0 || lv + 1 < runs.levels; lv += 3)
+        hipLaunchKernelGGL(k_runs, dim3((runs.count[lv] + RUN_B - 1) / RUN_B), dim3(RUN_B), 0, st, runs, lv,
+                           lv == 0 ? d_val : (const uint32_t*)nullptr, d_pbox);
+    GCHK(hipGetLastError());
+    if (n > 1) {
+        hipLaunchKernelGGL(k_nodes, dim3(grid_for(n)), dim3(GB), 0, st, n, d_child, d_parent, d_range, runs, d_ibox,
+                           d_posi, d_posl, d_depth, d_hdr);
+        GCHK(hipGetLastError());
     }
+    Header hdr;
+    GCHK(hipMemcpyAsync(&hdr, d_hdr, sizeof(hdr), hipMemcpyDeviceToHost, st));
+    GCHK(hipStreamSynchronize(st));
+    if (hdr.bad_index) return fail(PBRTX_ERR_BUILD, "vertex index out of range");
+    const uint32_t nq = hdr.nq, maxd = hdr.maxdepth;
+    if (n > 1 && maxd + 1 >= (uint32_t)MAX_LEVELS) return fail(PBRTX_ERR_BUILD, "linear BVH deeper than expected");
     // layouts
     RNode* d_rn;
-    GCHK(dalloc(&d_rn, nnodes));
-    S->d_rnodes = d_rn;
-    GCHK(T.get(&d_isrec, nnodes));
-    GCHK(T.get(&d_qidx, nnodes));
-    hipLaunchKernelGGL(k_rnodes, dim3(grid_for(nnodes)), dim3(GB), 0, st, n, d_child, d_ibox, d_pbox, d_val, d_posi,
-                       d_posl, d_depth, d_rn, d_isrec);
-    GCHK(hipGetLastError());
     PrimRec* d_pr;
     PrimRec64* d_pr64;
-    GCHK(dalloc(&d_pr, n));
-    S->d_prims = d_pr;
-    GCHK(dalloc(&d_pr64, n));
-    S->d_prims64 = d_pr64;
-    hipLaunchKernelGGL(k_prim_recs, dim3(grid_for(n)), dim3(GB), 0, st, n, nfaces, d_val, d_verts, d_idx, d_rn, d_posl,
-                       d_pr, d_pr64);
-    GCHK(hipGetLastError());
-    {
-        size_t tb = 0;
-        GCHK(rocprim::exclusive_scan(nullptr, tb, d_isrec, d_qidx, 0u, nnodes, rocprim::plus<uint32_t>(), st));
-        void* tmp;
-        GCHK(T.get((uint8_t**)&tmp, tb));
-        GCHK(rocprim::exclusive_scan(tmp, tb, d_isrec, d_qidx, 0u, nnodes, rocprim::plus<uint32_t>(), st));
-    }
-    uint32_t nq = 0, maxd = 0, last_flag = 0;
-    GCHK(hipMemcpyAsync(&nq, d_qidx + (nnodes - 1), 4, hipMemcpyDeviceToHost, st));
-    GCHK(hipMemcpyAsync(&last_flag, d_isrec + (nnodes - 1), 4, hipMemcpyDeviceToHost, st));
-    GCHK(hipMemcpyAsync(&maxd, d_maxd, 4, hipMemcpyDeviceToHost, st));
-    GCHK(hipStreamSynchronize(st));
-    nq += last_flag;
-    if (n > 1 && maxd + 1 >= (uint32_t)MAX_LEVELS) return fail(PBRTX_ERR_BUILD, "linear BVH deeper than expected");
+    uint32_t* d_order;
+    SphereRec* d_s;
     QNode* d_qn;
     CNode* d_cn;
-    GCHK(dalloc(&d_qn, nq));
-    S->d_qnodes = d_qn;
-    GCHK(dalloc(&d_cn, nq));
-    S->d_cnodes = d_cn;
-    GCHK(T.get(&d_bad, 1));
-    GCHK(fill_u32(d_bad, 0u, 1, st));
-    if (nq) {
-        hipLaunchKernelGGL(k_qnodes, dim3(grid_for(nnodes)), dim3(GB), 0, st, nnodes, d_rn, d_isrec, d_qidx, d_qn);
-        hipLaunchKernelGGL(k_cnodes, dim3(grid_for(nq)), dim3(GB), 0, st, nq, d_qn, d_cn, d_bad);
-        GCHK(hipGetLastError());
+    Slab A;
+    for (int pass = 0; pass < 2; ++pass) {
+        A.take(&d_rn, nnodes);
+        A.take(&d_pr, n);
+        A.take(&d_pr64, n);
+        A.take(&d_order, n);
+        A.take(&d_s, nsph);
+        A.take(&d_qn, nq);
+        A.take(&d_cn, nq);
+        if (pass == 0) GCHK(A.alloc());
     }
-    // ordered prim ids, spheres, root box
-    uint32_t* d_order;
-    GCHK(dalloc(&d_order, n));
-    S->d_order = d_order;
-    GCHK(hipMemcpyAsync(d_order, d_val, 4 * (size_t)n, hipMemcpyDeviceToDevice, st));
-    if (nsph) {
-        SphereRec* d_s;
-        GCHK(dalloc(&d_s, nsph));
-        S->d_spheres = d_s;
-        GCHK(hipMemcpyAsync(d_s, srec.data(), sizeof(SphereRec) * nsph, hipMemcpyHostToDevice, st));
-    }
-    RNode root;
-    uint32_t bad = 0;
-    GCHK(hipMemcpyAsync(&root, d_rn, sizeof(RNode), hipMemcpyDeviceToHost, st));
-    GCHK(hipMemcpyAsync(&bad, d_bad, 4, hipMemcpyDeviceToHost, st));
+    S->d_rnodes = A.release();  // holds the other arrays as well
+    hipLaunchKernelGGL(k_rnodes, dim3(grid_for(nnodes)), dim3(GB), 0, st, n, d_child, d_ibox, runs.box, d_posi, d_posl,
+                       d_depth, d_rn, d_isrec);
+    hipLaunchKernelGGL(k_prim_recs, dim3(grid_for(n)), dim3(GB), 0, st, n, nfaces, d_val, d_verts, nverts, d_idx,
+                       runs.box, d_pr, d_pr64, d_order);
+    GCHK(hipGetLastError());
+    GCHK(rocprim::exclusive_scan((void*)scan_tmp, scan_bytes, d_isrec, d_qidx, 0u, nnodes, rocprim::plus<uint32_t>(),
+                                 st));
+    // (the list takes the place of the interior nodes' positions, no longer needed)
+    uint32_t* d_rec = d_posi;
+    hipLaunchKernelGGL(k_rec_list, dim3(grid_for(nnodes)), dim3(GB), 0, st, nnodes, d_isrec, d_qidx, d_rn, d_rec, d_hdr);
+    if (nq)
+        hipLaunchKernelGGL(k_records, dim3(grid_for(nq)), dim3(GB), 0, st, nq, d_rec, d_rn, d_qidx, d_qn, d_cn, d_hdr);
+    GCHK(hipGetLastError());
+    if (nsph) GCHK(hipMemcpyAsync(d_s, srec.data(), sizeof(SphereRec) * nsph, hipMemcpyHostToDevice, st));
+    GCHK(hipMemcpyAsync(&hdr, d_hdr, sizeof(hdr), hipMemcpyDeviceToHost, st));
     GCHK(hipStreamSynchronize(st));
+    const RNode root = hdr.root;
+    const uint32_t bad = hdr.bad_cq;
     SceneView& v = S->view;
     v.rnodes = d_rn;
     v.qnodes = d_qn;
     v.prims = d_pr;
-    v.spheres = nsph ? (const SphereRec*)S->d_spheres : nullptr;
+    v.spheres = nsph ? d_s : nullptr;
     const bool cq = nq > 0 && !bad;
     v.cnodes = cq ? d_cn : nullptr;
     v.prims64 = cq ? d_pr64 : nullptr;
