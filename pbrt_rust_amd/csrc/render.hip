@@ -1676,7 +1676,10 @@ int enqueue_path_batch(const RenderParams& P, const SceneView& sv, WorkBufs& W, 
         }
         // the previous bounce's shadow work has read the shadow queue and
         // added its results to the path states the vertex kernel reads
-        if (joined) RCHK(hipStreamWaitEvent(st, joined, 0));
+        if (joined) {
+            RCHK(hipStreamWaitEvent(st, joined, 0));
+            sg.restart();  // the wait is no stage's
+        }
         a = sg.begin();
         {
             const uint32_t nb = (n + VERTEX_B - 1) / VERTEX_B;
@@ -1700,10 +1703,14 @@ int enqueue_path_batch(const RenderParams& P, const SceneView& sv, WorkBufs& W, 
         TraceScratch* sscr = split ? ss->scr : scr;
         Stager& ssg = split ? *ss->sg : sg;
         if (split) {
-            hipEvent_t fork = ss->ev->next();
-            if (!fork) return fail(PBRTX_ERR_OOM, "events");
-            RCHK(hipEventRecord(fork, st));
+            hipEvent_t fork = sg.last;  // the vertex stage's end, where it is timed
+            if (!fork) {
+                fork = ss->ev->next();
+                if (!fork) return fail(PBRTX_ERR_OOM, "events");
+                RCHK(hipEventRecord(fork, st));
+            }
             RCHK(hipStreamWaitEvent(sst, fork, 0));
+            ssg.restart();
         }
         a = ssg.begin();
         if (batched)
@@ -1720,9 +1727,12 @@ int enqueue_path_batch(const RenderParams& P, const SceneView& sv, WorkBufs& W, 
         RCHK(hipGetLastError());
         if (split) {
             RCHK(ssg.end(a, &Timing::other));
-            joined = ss->ev->next();
-            if (!joined) return fail(PBRTX_ERR_OOM, "events");
-            RCHK(hipEventRecord(joined, sst));
+            joined = ssg.last;
+            if (!joined) {
+                joined = ss->ev->next();
+                if (!joined) return fail(PBRTX_ERR_OOM, "events");
+                RCHK(hipEventRecord(joined, sst));
+            }
             a = sg.begin();
         }
         if (bounce < P.max_depth)
@@ -1743,7 +1753,10 @@ int enqueue_path_batch(const RenderParams& P, const SceneView& sv, WorkBufs& W, 
         std::swap(cin, cout);
     }
     // the batch ends when its last shadow work has
-    if (joined) RCHK(hipStreamWaitEvent(st, joined, 0));
+    if (joined) {
+        RCHK(hipStreamWaitEvent(st, joined, 0));
+        sg.restart();
+    }
     return PBRTX_OK;
 }
 
@@ -1979,10 +1992,10 @@ static int enqueue_frame(Renderer* R, int path, TraceScratch* scr, Stager& sg, u
     return PBRTX_OK;
 }
 
-// One frame: eagerly with per-stage timing, or -- graph mode, after one eager
+// One frame (its image to rgb_out, host memory, when given): eagerly with per-stage timing, or -- graph mode, after one eager
 // frame of that path has sized every buffer -- as a captured graph replayed
 // (captured again when the launch tuning changed since).
-static int render_frame(Renderer* R, int path, pbrtx_render_stats* stats) {
+static int render_frame(Renderer* R, int path, float* rgb_out, pbrtx_render_stats* stats) {
     hipStream_t st = R->stream;
     TraceScratch* scr;
     // a chunk's largest launch: its paths, or its samples' shadow slots
@@ -2027,8 +2040,14 @@ static int render_frame(Renderer* R, int path, pbrtx_render_stats* stats) {
         R->warm[path] = true;
     }
     RCHK(hipEventRecord(e_end, st));
-    RCHK(hipEventSynchronize(e_end));
-    uint32_t* cnt = R->counters.p;
+    // the image and the counters leave behind the frame's kernels, with no
+    // wait of the host between
+    if (rgb_out)
+        RCHK(hipMemcpyAsync(rgb_out, R->rgb.p, (size_t)R->P.xres * R->P.yres * 3 * sizeof(float),
+                            hipMemcpyDeviceToHost, st));
+    uint32_t c[10];
+    if (stats) RCHK(hipMemcpyAsync(c, R->counters.p, sizeof(c), hipMemcpyDeviceToHost, st));
+    RCHK(hipStreamSynchronize(st));
     if (stats) {
         float ms = 0.0f;
         RCHK(hipEventElapsedTime(&ms, e_start, e_end));
@@ -2048,8 +2067,6 @@ static int render_frame(Renderer* R, int path, pbrtx_render_stats* stats) {
         ICHK(sum(T.other, &stats->ms_other));
         stats->launches_closest = (uint32_t)T.closest.size();
         stats->launches_any = (uint32_t)T.any.size();
-        uint32_t c[10];
-        RCHK(hipMemcpy(c, cnt, sizeof(c), hipMemcpyDeviceToHost));
         stats->camera_rays = total_camera;
         stats->shadow_rays = (uint64_t)c[6] | ((uint64_t)c[7] << 32);
         stats->extension_rays = (uint64_t)c[8] | ((uint64_t)c[9] << 32);
@@ -2162,14 +2179,7 @@ int pbrtx_renderer_render(pbrtx_renderer* h, int32_t path, float* rgb_out, pbrtx
     if (!h) return fail(PBRTX_ERR_ARG, "renderer is null");
     if (path != PATH_PLAIN && path != PATH_BATCHED) return fail(PBRTX_ERR_ARG, "unknown path");
     if (stats) memset(stats, 0, sizeof(*stats));
-    int rc = render_frame(&h->r, path, stats);
-    if (rc) return rc;
-    if (rgb_out) {
-        const size_t bytes = (size_t)h->r.P.xres * h->r.P.yres * 3 * sizeof(float);
-        hipError_t e = hipMemcpy(rgb_out, h->r.rgb.p, bytes, hipMemcpyDeviceToHost);
-        if (e != hipSuccess) return hip_fail(e, "hipMemcpy(rgb)");
-    }
-    return PBRTX_OK;
+    return render_frame(&h->r, path, rgb_out, stats);
 }
 
 int pbrtx_renderer_sample_slots(pbrtx_renderer* h, uint32_t* slots_per_pixel) {

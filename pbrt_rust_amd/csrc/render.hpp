@@ -197,22 +197,28 @@ using EventPairs = std::vector<std::pair<hipEvent_t, hipEvent_t>>;
 struct Timing {
     EventPairs closest, any, other;
 };
-// Per-stage event pairs on a stream; a null pool records nothing.
+// Per-stage event pairs on a stream; a null pool records nothing.  A stage
+// that follows another begins at its end event: an event holds the stream
+// for some 5 us, as long as the smallest stages take.
 struct Stager {
     EventPool* pool = nullptr;
     Timing* T = nullptr;
     hipStream_t st = nullptr;
+    hipEvent_t last = nullptr;  // the end of the stage before, if nothing came between
     hipEvent_t begin() {
         if (!pool) return nullptr;
+        if (last) return last;
         hipEvent_t e = pool->next();
         return (e && hipEventRecord(e, st) == hipSuccess) ? e : nullptr;
     }
+    void restart() { last = nullptr; }
     hipError_t end(hipEvent_t a, EventPairs Timing::*which) {
         if (!pool || !a) return hipSuccess;
         hipEvent_t b = pool->next();
         if (!b) return hipErrorOutOfMemory;
         hipError_t e = hipEventRecord(b, st);
         if (e == hipSuccess) (T->*which).push_back({a, b});
+        last = e == hipSuccess ? b : nullptr;
         return e;
     }
 };
