@@ -437,15 +437,48 @@ __global__ __launch_bounds__(RB) void k_accum_direct(RenderParams P, uint64_t g0
     }
 }
 
-// hi:lo += *add (a 64-bit running total in two words); then (when given) *add and *clr are cleared for the next
-// chunk, which saves that chunk a clearing launch.
-__global__ void k_add_counter(uint32_t* lo, uint32_t* add, uint32_t* hi, bool clear_add, uint32_t* clr) {
-    uint64_t v = ((uint64_t)*hi << 32) | (uint64_t)*lo;
-    v += *add;
-    *lo = (uint32_t)v;
-    *hi = (uint32_t)(v >> 32);
-    if (clear_add) *add = 0u;
-    if (clr) *clr = 0u;
+// Ends a direct-lighting chunk: the running total of shadow rays hi:lo += *add,
+// then *add, the list's count *clr and the occlusion launch's work counters
+// are cleared for the next chunk (one wave).
+__global__ void k_chunk_end(uint32_t* lo, uint32_t* hi, uint32_t* add, uint32_t* clr, uint32_t* parts) {
+    if (threadIdx.x == 0) {
+        const uint64_t v = (((uint64_t)*hi << 32) | (uint64_t)*lo) + *add;
+        *lo = (uint32_t)v;
+        *hi = (uint32_t)(v >> 32);
+        *add = 0u;
+        *clr = 0u;
+    }
+    parts[threadIdx.x] = 0u;
+}
+static_assert(TRACE_PART_WORDS == 64, "one wave clears them");
+
+// Adds nb bounces' shadow and extension rays to the running totals (two words
+// each) and clears the bounces' counters (render.hpp: BOUNCE_WORDS); more: the
+// batch goes on, its next bounce taking the first place with the paths that
+// the last one left.  One block.
+__global__ __launch_bounds__(RB) void k_bounce_totals(uint32_t* cnt, uint32_t nb, bool more) {
+    uint32_t* bc = cnt + BOUNCES_AT;
+    __shared__ uint32_t s_carry;
+    if (threadIdx.x < 64) {
+        static_assert(BOUNCE_RING <= 64, "a lane a bounce");
+        uint64_t sh = 0, ext = 0;
+        if (threadIdx.x < nb) {
+            sh = bc[threadIdx.x * BOUNCE_WORDS + BOUNCE_SHADOW];
+            ext = bc[(threadIdx.x + 1) * BOUNCE_WORDS + BOUNCE_PATHS];
+        }
+        for (int o = 32; o > 0; o >>= 1) {
+            sh += __shfl_xor((unsigned long long)sh, o);
+            ext += __shfl_xor((unsigned long long)ext, o);
+        }
+        if (threadIdx.x == 0) {
+            const uint64_t a = (((uint64_t)cnt[7] << 32) | cnt[6]) + sh, b = (((uint64_t)cnt[9] << 32) | cnt[8]) + ext;
+            cnt[6] = (uint32_t)a; cnt[7] = (uint32_t)(a >> 32);
+            cnt[8] = (uint32_t)b; cnt[9] = (uint32_t)(b >> 32);
+            s_carry = more ? bc[nb * BOUNCE_WORDS + BOUNCE_PATHS] : 0u;
+        }
+    }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < (nb + 1) * BOUNCE_WORDS; i += RB) bc[i] = i == BOUNCE_PATHS ? s_carry : 0u;
 }
 
 // ---- path tracing ------------------------------------------------------------
@@ -750,6 +783,7 @@ __global__ __launch_bounds__(VERTEX_B) void k_path_shade(RenderParams P, uint64_
     __shared__ uint32_t s_bid, s_es, s_en;
     constexpr uint32_t TILE = VERTEX_B * PATH_PER;
     const uint32_t ntiles = (n + TILE - 1) / TILE;
+    if (blockIdx.x >= ntiles) return;  // a short queue: no ticket drawn in vain
     while (true) {
         if (threadIdx.x == 0) s_bid = atomicAdd(ticket, 1u);
         __syncthreads();
@@ -1364,7 +1398,7 @@ void RenderScene::release() {
 void WorkBufs::release() {
     rays.release(); rays2.release(); rays3.release(); sh.release(); hits.release(); hits2.release(); contrib.release();
     lbase.release(); qidx.release(); occ.release(); pid.release(); pid2.release(); pid3.release();
-    shpid.release(); bcounts.release(); st.release();
+    shpid.release(); st.release();
 }
 
 // Triangle::intersect's dg with the default uvs (mesh.rs:212-254) for the
@@ -1590,7 +1624,6 @@ int reserve_path_work(WorkBufs& W, uint32_t cap, bool osort) {
     ICHK(W.pid.ensure(cap));
     ICHK(W.pid2.ensure(cap));
     ICHK(W.shpid.ensure(cap));
-    ICHK(W.bcounts.ensure(2));
     if (osort) {
         ICHK(W.rays3.ensure(cap));
         ICHK(W.pid3.ensure(cap));
@@ -1631,25 +1664,30 @@ int enqueue_path_batch(const RenderParams& P, const SceneView& sv, WorkBufs& W, 
         ICHK(W.hits2.ensure(n));
     }
     hipEvent_t a = sg.begin();
-    if (fused || fused_seg) {
-        // fused: the camera kernel lists the hits and counts them here
-        RCHK(fill_u32(cnt + 1, fused ? 0u : n, 1, st));
-    } else {
+    // the bounces' counters, cleared with the frame's and by the batch before
+    // (fused: the camera kernel lists the hits and counts them in the first)
+    uint32_t* bc = cnt + BOUNCES_AT;
+    if (!fused && !fused_seg) {
         hipLaunchKernelGGL(k_path_init, dim3(grid_for(n)), dim3(RB), 0, st, P, g0, n, W.rays.p, W.st.p,
-                           batched ? W.pid.p : nullptr, batched ? cnt + 1 : nullptr);
+                           batched ? W.pid.p : nullptr, batched ? bc + BOUNCE_PATHS : nullptr);
         RCHK(hipGetLastError());
+        RCHK(sg.end(a, &Timing::other));
+        a = sg.begin();
     }
-    RCHK(sg.end(a, &Timing::other));
     Ray* rin = W.rays.p;
     Ray* rout = W.rays2.p;
     Ray* rspare = W.rays3.p;
     uint32_t* pin = W.pid.p;
     uint32_t* pout = W.pid2.p;
     uint32_t* pspare = W.pid3.p;
-    uint32_t* cin = cnt + 1;
-    uint32_t* cout = cnt + 2;
+    TraceScratch cscr = *scr, ascr = split ? *ss->scr : *scr;  // with a bounce's work counters
     for (uint32_t bounce = 0; bounce <= P.max_depth; ++bounce) {
-        a = sg.begin();
+        if (bounce > 0) a = sg.begin();
+        uint32_t* cin = bc + BOUNCE_PATHS;                  // paths of this bounce
+        uint32_t* cout = bc + BOUNCE_WORDS + BOUNCE_PATHS;  // and of the next
+        uint32_t* csh = bc + BOUNCE_SHADOW;                 // its shadow rays
+        cscr.parts = batched ? bc + BOUNCE_CLOSEST : nullptr;
+        ascr.parts = batched ? bc + BOUNCE_ANY : nullptr;
         const TraceTuning& tb = (bounce == 0 && !P.segs) ? tunCam : tunC;  // frames' bounce 0: camera rays
         if (fused && bounce == 0) {
             // a missed camera ray's path ends in the traversal (zero
@@ -1659,7 +1697,7 @@ int enqueue_path_batch(const RenderParams& P, const SceneView& sv, WorkBufs& W, 
         } else if (fused_seg && bounce == 0) {
             RCHK(trace_camera(sv, CamParams{}, n, W.hits.p, tunCam, scr, st, &ct));
         } else if (batched) {
-            RCHK(trace_closest(sv, rin, n, W.hits.p, path, tb, scr, st, cin));
+            RCHK(trace_closest(sv, rin, n, W.hits.p, path, tb, &cscr, st, cin));
         } else {
             RCHK(trace_closest(sv, rin, n, W.hits.p, path, tb, scr, st));
         }
@@ -1668,7 +1706,6 @@ int enqueue_path_batch(const RenderParams& P, const SceneView& sv, WorkBufs& W, 
             // the misses end here; the hits' path ids become the queue
             a = sg.begin();
             const uint32_t mb = (uint32_t)(((uint64_t)n + MISS_B * MISS_PER - 1) / (MISS_B * MISS_PER));
-            RCHK(fill_u32(cin, 0u, 1, st));  // the list's count
             hipLaunchKernelGGL(k_path_miss0<true>, dim3(mb), dim3(MISS_B), 0, st, P, g0, n, W.hits.p, sample_l,
                                pin, cin, rin, W.hits2.p, W.st.p);
             RCHK(hipGetLastError());
@@ -1683,9 +1720,6 @@ int enqueue_path_batch(const RenderParams& P, const SceneView& sv, WorkBufs& W, 
         a = sg.begin();
         {
             const uint32_t nb = (n + VERTEX_B - 1) / VERTEX_B;
-            // the two queues' counts and (queue form) the tile ticket
-            ICHK(W.bcounts.ensure(2));
-            RCHK(zero3_u32(cout, 1, cnt + 5, 1, W.bcounts.p, batched ? 1 : 0, st));
             // queue form: persistent blocks over the live paths' tiles
             const uint32_t grid = batched ? std::min<uint32_t>(nb, (uint32_t)device_cu_count() * 8u) : nb;
             hipLaunchKernelGGL(k_path_shade, dim3(grid), dim3(VERTEX_B), 0, st, P, g0, bounce, n,
@@ -1694,13 +1728,12 @@ int enqueue_path_batch(const RenderParams& P, const SceneView& sv, WorkBufs& W, 
                                (fused && bounce == 0) ? (const Ray*)nullptr : rin,
                                (fused_seg && bounce == 0) ? W.hits2.p : W.hits.p, W.st.p, rout,
                                batched ? pout : nullptr, cout, W.sh.p, batched ? W.shpid.p : nullptr, W.contrib.p,
-                               cnt + 5, sample_l, W.bcounts.p, (int)(batched ? PSHADE_QUEUE : PSHADE_PLAIN));
+                               csh, sample_l, bc + BOUNCE_TICKET, (int)(batched ? PSHADE_QUEUE : PSHADE_PLAIN));
             RCHK(hipGetLastError());
         }
         RCHK(sg.end(a, &Timing::other));
         // shadow rays: occlusion, then the unoccluded samples added
         hipStream_t sst = split ? ss->st : st;
-        TraceScratch* sscr = split ? ss->scr : scr;
         Stager& ssg = split ? *ss->sg : sg;
         if (split) {
             hipEvent_t fork = sg.last;  // the vertex stage's end, where it is timed
@@ -1714,16 +1747,14 @@ int enqueue_path_batch(const RenderParams& P, const SceneView& sv, WorkBufs& W, 
         }
         a = ssg.begin();
         if (batched)
-            RCHK(trace_any_bytes(sv, W.sh.p, n, W.occ.p, path, tunA, sscr, sst, cnt + 5));
+            RCHK(trace_any_bytes(sv, W.sh.p, n, W.occ.p, path, tunA, &ascr, sst, csh));
         else
-            RCHK(trace_any_bytes(sv, W.sh.p, n, W.occ.p, path, tunA, sscr, sst));
+            RCHK(trace_any_bytes(sv, W.sh.p, n, W.occ.p, path, tunA, &ascr, sst));
         RCHK(ssg.end(a, &Timing::any));
         a = ssg.begin();
         hipLaunchKernelGGL(k_path_shadow, dim3(grid_for(n)), dim3(RB), 0, sst, P, g0, n,
-                           batched ? cnt + 5 : (const uint32_t*)nullptr,
+                           batched ? csh : (const uint32_t*)nullptr,
                            batched ? W.shpid.p : (const uint32_t*)nullptr, W.contrib.p, W.occ.p, W.st.p, sample_l);
-        RCHK(hipGetLastError());
-        hipLaunchKernelGGL(k_add_counter, dim3(1), dim3(1), 0, sst, cnt + 6, cnt + 5, cnt + 7, false, (uint32_t*)nullptr);
         RCHK(hipGetLastError());
         if (split) {
             RCHK(ssg.end(a, &Timing::other));
@@ -1735,9 +1766,6 @@ int enqueue_path_batch(const RenderParams& P, const SceneView& sv, WorkBufs& W, 
             }
             a = sg.begin();
         }
-        if (bounce < P.max_depth)
-            hipLaunchKernelGGL(k_add_counter, dim3(1), dim3(1), 0, st, cnt + 8, cout, cnt + 9, false, (uint32_t*)nullptr);
-        RCHK(hipGetLastError());
         if (osort && bounce < P.max_depth) {
             const uint32_t tiles = (n + OS_TILE - 1) / OS_TILE;
             const uint32_t grid = std::min<uint32_t>(tiles, (uint32_t)device_cu_count() * 2u);
@@ -1747,15 +1775,24 @@ int enqueue_path_batch(const RenderParams& P, const SceneView& sv, WorkBufs& W, 
             std::swap(rout, rspare);
             std::swap(pout, pspare);
         }
-        RCHK(sg.end(a, &Timing::other));
+        if (!split || osort) RCHK(sg.end(a, &Timing::other));
         std::swap(rin, rout);
         std::swap(pin, pout);
-        std::swap(cin, cout);
-    }
-    // the batch ends when its last shadow work has
-    if (joined) {
-        RCHK(hipStreamWaitEvent(st, joined, 0));
-        sg.restart();
+        bc += BOUNCE_WORDS;
+        // the counters' places used up, or the batch's last bounce: into the
+        // totals, once the shadow work has read its count as well (the batch
+        // ends when that has)
+        const uint32_t used = (uint32_t)((bc - cnt - BOUNCES_AT) / BOUNCE_WORDS);
+        if (used == BOUNCE_RING || bounce == P.max_depth) {
+            if (joined) {
+                RCHK(hipStreamWaitEvent(st, joined, 0));
+                joined = nullptr;
+                sg.restart();
+            }
+            hipLaunchKernelGGL(k_bounce_totals, dim3(1), dim3(RB), 0, st, cnt, used, bounce < P.max_depth);
+            RCHK(hipGetLastError());
+            bc = cnt + BOUNCES_AT;
+        }
     }
     return PBRTX_OK;
 }
@@ -1903,6 +1940,8 @@ static int enqueue_frame(Renderer* R, int path, TraceScratch* scr, Stager& sg, u
     uint32_t* cnt = R->counters.p;
     RCHK(fill_u32(cnt, 0u, N_COUNTERS, st));
     const SceneView& sv = R->sc.scene.view;
+    TraceScratch ascr = *scr;  // with work counters cleared by the chunk before
+    ascr.parts = cnt + BOUNCES_AT + BOUNCE_ANY;
     uint64_t total_camera = 0;
     for (uint64_t g0 = 0; g0 < R->n_samples; g0 += per) {
         const uint32_t n = (uint32_t)((R->n_samples - g0) < per ? (R->n_samples - g0) : per);
@@ -1967,7 +2006,7 @@ static int enqueue_frame(Renderer* R, int path, TraceScratch* scr, Stager& sg, u
         if (slots) {
             a = sg.begin();
             if (batched)
-                RCHK(trace_any_bytes(sv, W.sh.p, (uint32_t)slots, W.occ.p, path, tunA, scr, st, cnt + 5));
+                RCHK(trace_any_bytes(sv, W.sh.p, (uint32_t)slots, W.occ.p, path, tunA, &ascr, st, cnt + 5));
             else
                 RCHK(trace_any_bytes(sv, W.sh.p, (uint32_t)slots, W.occ.p, path, tunA, scr, st));
             RCHK(sg.end(a, &Timing::any));
@@ -1976,9 +2015,7 @@ static int enqueue_frame(Renderer* R, int path, TraceScratch* scr, Stager& sg, u
         hipLaunchKernelGGL(k_accum_direct, dim3(grid_for(n)), dim3(RB), 0, st, P, g0, n, W.lbase.p, W.contrib.p,
                            W.qidx.p, W.occ.p, R->sample_l.p, list, nlist);
         RCHK(hipGetLastError());
-        // running total of shadow rays; the shadow-ray and list counts
-        // cleared for the next chunk
-        hipLaunchKernelGGL(k_add_counter, dim3(1), dim3(1), 0, st, cnt + 6, cnt + 5, cnt + 7, true, cnt + 1);
+        hipLaunchKernelGGL(k_chunk_end, dim3(1), dim3(64), 0, st, cnt + 6, cnt + 7, cnt + 5, cnt + 1, ascr.parts);
         RCHK(hipGetLastError());
         RCHK(sg.end(a, &Timing::other));
     }

@@ -171,7 +171,7 @@ struct WorkBufs {
     DevArr<Hit> hits;
     DevArr<Hit> hits2;  // served batches: bounce 0's hits at their queue positions
     DevArr<float4> contrib, lbase;
-    DevArr<uint32_t> qidx, pid, pid2, pid3, shpid, bcounts;
+    DevArr<uint32_t> qidx, pid, pid2, pid3, shpid;
     DevArr<uint8_t> occ;  // occlusion of each queued shadow ray: a byte per ray
     DevArr<PathState> st;
     void release();
@@ -237,17 +237,30 @@ struct ShadowStream {
 // Sizes W for batches of up to cap paths (no allocation afterwards).
 int reserve_path_work(WorkBufs& W, uint32_t cap, bool osort);
 
-// Renderer counters (u32 words): [1], [2] the two extension queues' counts,
-// [5] this bounce's shadow rays, [6,7] running total of shadow rays (lo, hi),
-// [8,9] running total of extension rays.
-constexpr uint32_t N_COUNTERS = 16;
+// Renderer counters (u32 words): direct lighting's [1] list of hits and [5]
+// shadow rays of a chunk; [6,7] running total of shadow rays (lo, hi), [8,9]
+// running total of extension rays; and the path tracer's per bounce, so that
+// nothing has to be cleared or added up between two bounces (with a kernel for
+// each of these, five of 2-5 us a bounce, a bounce of few paths took 88 us).
+// The words that waves of one launch count in lie a cache line apart.
+constexpr uint32_t N_TOTALS = 16;
+constexpr uint32_t BOUNCES_AT = N_TOTALS;
+constexpr uint32_t BOUNCE_PATHS = 0;     // paths (queue entries) of the bounce
+constexpr uint32_t BOUNCE_SHADOW = 16;   // its shadow rays
+constexpr uint32_t BOUNCE_TICKET = 32;   // tiles of its vertex kernel
+constexpr uint32_t BOUNCE_CLOSEST = 64;  // work counters of its two traversal launches
+constexpr uint32_t BOUNCE_ANY = BOUNCE_CLOSEST + TRACE_PART_WORDS;
+constexpr uint32_t BOUNCE_WORDS = BOUNCE_ANY + TRACE_PART_WORDS;
+constexpr uint32_t BOUNCE_RING = 32;     // bounces before the totals are taken
+constexpr uint32_t N_COUNTERS = N_TOTALS + (BOUNCE_RING + 1) * BOUNCE_WORDS;
 
 // The path tracer over one batch of n paths on stream st: samples g0 + i of
 // the frame (P.segs null), or the samples P's segment table maps the batch
 // to.  path: PATH_PLAIN (every slot traced each bounce) or PATH_BATCHED
 // (compacted queues, persistent traversal); osort: octant-sort the extension
 // queues (batched); sample_l: the frame's sample radiance (frames only).
-// Adds the batch's rays to cnt[6..9]; enqueues device work only.
+// Adds the batch's rays to cnt[6..9] (cnt: N_COUNTERS words, cleared before the
+// first batch; a batch leaves the bounces' clear); enqueues device work only.
 int enqueue_path_batch(const RenderParams& P, const SceneView& sv, WorkBufs& W, uint32_t* cnt, uint64_t g0,
                        uint32_t n, int path, bool osort, float4* sample_l, TraceScratch* scr, hipStream_t st,
                        Stager& sg, const ShadowStream* ss = nullptr);

@@ -306,7 +306,7 @@ int RenderServer::launch_batches() {
                                     nullptr, scr, S.st, none);
         }
         if (rc) return rc;
-        e = hipMemcpyAsync(S.h_cnt, S.cnt.p, N_COUNTERS * sizeof(uint32_t), hipMemcpyDeviceToHost, S.st);
+        e = hipMemcpyAsync(S.h_cnt, S.cnt.p, N_TOTALS * sizeof(uint32_t), hipMemcpyDeviceToHost, S.st);
         if (e == hipSuccess) e = hipEventRecord(S.end, S.st);
         if (e != hipSuccess) return hip_fail(e, "batch end");
         S.total = (uint32_t)total;
@@ -377,7 +377,7 @@ int RenderServer::serve_plain(RRequest* r) {
         r->batches++;
         ++batches;
     }
-    e = hipMemcpyAsync(S.h_cnt, S.cnt.p, N_COUNTERS * sizeof(uint32_t), hipMemcpyDeviceToHost, S.st);
+    e = hipMemcpyAsync(S.h_cnt, S.cnt.p, N_TOTALS * sizeof(uint32_t), hipMemcpyDeviceToHost, S.st);
     if (e == hipSuccess) e = hipEventRecord(S.end, S.st);
     if (e != hipSuccess) return hip_fail(e, "plain render");
     rc = start_film(r, S.st);
@@ -492,7 +492,7 @@ int pbrtx_render_server_create(const pbrtx_render_server_config* cfg, pbrtx_rend
         if (e == hipSuccess) e = hipEventCreate(&S.end);
         if (e == hipSuccess) e = hipHostMalloc((void**)&S.h_segs, MAX_RENDER_SEGS * sizeof(RenderSeg), hipHostMallocDefault);
         if (e == hipSuccess) e = hipHostMalloc((void**)&S.h_reqs, MAX_RENDER_SEGS * sizeof(ReqView), hipHostMallocDefault);
-        if (e == hipSuccess) e = hipHostMalloc((void**)&S.h_cnt, N_COUNTERS * sizeof(uint32_t), hipHostMallocDefault);
+        if (e == hipSuccess) e = hipHostMalloc((void**)&S.h_cnt, N_TOTALS * sizeof(uint32_t), hipHostMallocDefault);
         if (e == hipSuccess) e = hipMalloc((void**)&S.d_segs, MAX_RENDER_SEGS * sizeof(RenderSeg));
         if (e == hipSuccess) e = hipMalloc((void**)&S.d_reqs, MAX_RENDER_SEGS * sizeof(ReqView));
         if (e == hipSuccess) rc = S.cnt.ensure(N_COUNTERS);

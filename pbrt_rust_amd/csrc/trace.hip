@@ -425,6 +425,7 @@ constexpr uint32_t WIDE_PARTS_AT = 32;
 // the part counters, then the count of rays handed over (TailRec): cleared together
 constexpr uint32_t WIDE_COUNTERS = WIDE_PARTS * WIDE_PART_STRIDE + 1;
 static_assert(WIDE_PARTS_AT + WIDE_COUNTERS <= TRACE_COUNTER_WORDS, "scratch counter block");
+static_assert(WIDE_COUNTERS <= TRACE_PART_WORDS, "a caller's own counters");
 
 // The rays a large launch of the per-ray kernel does not finish itself.  Once
 // its rays are all claimed, a wave's lanes fall idle one by one and the last
@@ -857,154 +858,157 @@ __global__ __launch_bounds__(oc_block(G)) __attribute__((amdgpu_waves_per_eu(8))
     SceneView sv, const Ray* rays, uint32_t n_host, const uint32_t* n_dev, uint32_t* occ, uint8_t* occ8,
     uint32_t lim, uint32_t* err, const TraceSeg* segs, uint32_t nseg, TailView tail) {
     static_assert(G >= 2 && G <= 64 && (64 % G) == 0, "a group lies within one wave");
-    // (the grid covers n_host rays: a count on the device never exceeds it)
+    // (a count on the device never exceeds n_host)
     const uint32_t n = TAIL ? min(*tail.count, tail.cap) : n_dev ? min(*n_dev, n_host) : n_host;
     const uint32_t gpb = oc_block(G) / G;  // groups per block
-    // (bits: the grid covers n_host's words, and the blocks past n write zeros)
-    if ((occ8 || SEG || TAIL) && (uint64_t)blockIdx.x * gpb >= (uint64_t)n) return;
+    const bool whole = !(occ8 || SEG || TAIL);  // the block writes its rays' bits whole
     constexpr int GSTK = gstk_occlude(G);
     __shared__ int32_t s_stk[oc_block(G) / G][GSTK];
     const uint32_t tid = threadIdx.x, lane = __lane_id();
     const uint32_t g = tid / G, gl = tid % G;
-    const uint32_t id = blockIdx.x * gpb + g;
-    uint32_t rid = id, rseg = 0;  // SEG: rid is the ray's index in segment rseg
     const uint32_t gbase = lane & ~(uint32_t)(G - 1);
     const unsigned long long gm = (G == 64 ? ~0ull : ((1ull << G) - 1ull)) << gbase;  // the group's lanes
     const unsigned long long lowg = gm & (lane == 0 ? 0ull : (~0ull >> (64 - lane)));  // ... below this one
     int32_t* stk = s_stk[g];
-    RayState r{};
-    bool done = id >= n;
-    uint32_t top = 0;
-    if (!done) {
-        if (TAIL) rid = tail.recs[id].id;
-        if (SEG) {
-            rseg = find_seg(segs, nseg, rid);
-            rid -= segs[rseg].start;
-            load_ray(segs[rseg].rays, rid, r);
-        } else {
-            load_ray(rays, rid, r);
-        }
-        float tn;
-        if (TAIL) {
-            // the walk goes on from the entries its wave handed over
-            top = tail.recs[id].sp;
-            for (uint32_t e = gl; e < top; e += G) stk[e] = tail.stk[(size_t)id * TAIL_STK + e].x;
-        } else if (slab(sv.root_lo[0], sv.root_hi[0], sv.root_lo[1], sv.root_hi[1], sv.root_lo[2], sv.root_hi[2], r.ox,
-                        r.oy, r.oz, r.ix, r.iy, r.iz, r.tmin, r.tmax, &tn)) {
-            // the root's own box (popped first by the reference)
-            top = 1;
-            if (gl == 0) stk[0] = sv.ocroot;
-        }
-        done = top == 0;
-    }
-    const bool neg0 = r.ix < 0.0f, neg1 = r.iy < 0.0f, neg2 = r.iz < 0.0f;
-    // every ray of the wave may take the ray-space record test (cq_fast_ray)
-    const bool wfast = cq_fast_scene(sv) && __ballot(id < n && !cq_fast_ray(r)) == 0ull;
     bool hit = false;
-    while (__any(!done)) {
-        // entries for this step: up to G, fewer near the stack's bound
-        uint32_t k = 0;
+    // one ray a group (bits: the grid covers n_host's words, and the blocks
+    // past n write zeros), or more where the count is on the device
+    for (uint64_t blk = blockIdx.x; whole || blk * gpb < (uint64_t)n; blk += gridDim.x) {
+        const uint32_t id = (uint32_t)(blk * gpb) + g;
+        uint32_t rid = id, rseg = 0;  // SEG: rid is the ray's index in segment rseg
+        RayState r{};
+        hit = false;
+        bool done = id >= n;
+        uint32_t top = 0;
         if (!done) {
-            k = top < (uint32_t)G ? top : (uint32_t)G;
-            const uint32_t room = top + 6u <= lim ? (lim - top) / 3u : 1u;
-            k = k < room ? k : room;
-        }
-        const bool mine = gl < k;
-        const int32_t ref = mine ? stk[top - 1u - gl] : 0;
-        top -= k;
-        bool p0 = false, p1 = false, p2 = false, p3 = false, hitnow = false;
-        int4 RF = make_int4(0, 0, 0, 0);
-        if (mine && ref >= 0) {
-            const float4* q = reinterpret_cast<const float4*>(sv.ocnodes + ref);
-            const float4 W0 = q[0], W1 = q[1], W2 = q[2], W3 = q[3];
-            const uint32_t em = as_u(W0.w);
-            const uint32_t nqx = neg0 ? as_u(W1.y) : as_u(W1.x), fqx = neg0 ? as_u(W1.x) : as_u(W1.y);
-            const uint32_t nqy = neg1 ? as_u(W1.w) : as_u(W1.z), fqy = neg1 ? as_u(W1.z) : as_u(W1.w);
-            const uint32_t nqz = neg2 ? as_u(W2.y) : as_u(W2.x), fqz = neg2 ? as_u(W2.x) : as_u(W2.y);
-            RF = make_int4((int)as_u(W2.z), (int)as_u(W2.w), (int)as_u(W3.x), (int)as_u(W3.y));
-            float t0, t1, t2, t3;
-            if (wfast) {
-                const CqAxis X = cq_axis_ray(W0.x, em & 0xFFu, r.ox, r.ix);
-                const CqAxis Y = cq_axis_ray(W0.y, (em >> 8) & 0xFFu, r.oy, r.iy);
-                const CqAxis Z = cq_axis_ray(W0.z, (em >> 16) & 0xFFu, r.oz, r.iz);
-#define PX_CQ_SLOT(K, I, P, T) \
-    P = RF.K != QEMPTY && slab_ray(nqx, fqx, nqy, fqy, nqz, fqz, I, X, Y, Z, r.tmin, r.tmax, &T);
-                PX_CQ_SLOT(x, 0, p0, t0)
-                PX_CQ_SLOT(y, 1, p1, t1)
-                PX_CQ_SLOT(z, 2, p2, t2)
-                PX_CQ_SLOT(w, 3, p3, t3)
-#undef PX_CQ_SLOT
+            if (TAIL) rid = tail.recs[id].id;
+            if (SEG) {
+                rseg = find_seg(segs, nseg, rid);
+                rid -= segs[rseg].start;
+                load_ray(segs[rseg].rays, rid, r);
             } else {
-                const float sx = cq_scale(em & 0xFFu), sy = cq_scale((em >> 8) & 0xFFu),
-                            sz = cq_scale((em >> 16) & 0xFFu);
-#define PX_CQ_SLOT(K, I, P, T)                                                                                \
-    P = RF.K != QEMPTY &&                                                                                     \
-        slab_signed(cq_bound(nqx, I, W0.x, sx), cq_bound(fqx, I, W0.x, sx), cq_bound(nqy, I, W0.y, sy),       \
-                    cq_bound(fqy, I, W0.y, sy), cq_bound(nqz, I, W0.z, sz), cq_bound(fqz, I, W0.z, sz), r.ox,  \
-                    r.oy, r.oz, r.ix, r.iy, r.iz, r.tmin, r.tmax, &T);
-                PX_CQ_SLOT(x, 0, p0, t0)
-                PX_CQ_SLOT(y, 1, p1, t1)
-                PX_CQ_SLOT(z, 2, p2, t2)
-                PX_CQ_SLOT(w, 3, p3, t3)
-#undef PX_CQ_SLOT
+                load_ray(rays, rid, r);
             }
-        } else if (mine) {
-            // leaf: its exact box, then prims in order until the record flagged last
-            uint32_t pos = (uint32_t)(~ref);
-            const float4* p = reinterpret_cast<const float4*>(sv.prims64 + pos);
-            float4 P2 = p[2], P3 = p[3];
             float tn;
-            if (slab(P2.y, P3.x, P2.z, P3.y, P2.w, P3.z, r.ox, r.oy, r.oz, r.ix, r.iy, r.iz, r.tmin, r.tmax, &tn)) {
-                while (true) {
-                    const float4 P0 = p[0], P1 = p[1];
-                    const uint32_t kind = as_u(P3.w);
-                    uint32_t hp;
-                    float hb1, hb2;
-                    if (prim_test64(sv, pos, P0, P1, P2, kind, r, &hp, &hb1, &hb2)) {
-                        hitnow = true;
-                        break;
+            if (TAIL) {
+                // the walk goes on from the entries its wave handed over
+                top = tail.recs[id].sp;
+                for (uint32_t e = gl; e < top; e += G) stk[e] = tail.stk[(size_t)id * TAIL_STK + e].x;
+            } else if (slab(sv.root_lo[0], sv.root_hi[0], sv.root_lo[1], sv.root_hi[1], sv.root_lo[2], sv.root_hi[2], r.ox,
+                            r.oy, r.oz, r.ix, r.iy, r.iz, r.tmin, r.tmax, &tn)) {
+                // the root's own box (popped first by the reference)
+                top = 1;
+                if (gl == 0) stk[0] = sv.ocroot;
+            }
+            done = top == 0;
+        }
+        const bool neg0 = r.ix < 0.0f, neg1 = r.iy < 0.0f, neg2 = r.iz < 0.0f;
+        // every ray of the wave may take the ray-space record test (cq_fast_ray)
+        const bool wfast = cq_fast_scene(sv) && __ballot(id < n && !cq_fast_ray(r)) == 0ull;
+        while (__any(!done)) {
+            // entries for this step: up to G, fewer near the stack's bound
+            uint32_t k = 0;
+            if (!done) {
+                k = top < (uint32_t)G ? top : (uint32_t)G;
+                const uint32_t room = top + 6u <= lim ? (lim - top) / 3u : 1u;
+                k = k < room ? k : room;
+            }
+            const bool mine = gl < k;
+            const int32_t ref = mine ? stk[top - 1u - gl] : 0;
+            top -= k;
+            bool p0 = false, p1 = false, p2 = false, p3 = false, hitnow = false;
+            int4 RF = make_int4(0, 0, 0, 0);
+            if (mine && ref >= 0) {
+                const float4* q = reinterpret_cast<const float4*>(sv.ocnodes + ref);
+                const float4 W0 = q[0], W1 = q[1], W2 = q[2], W3 = q[3];
+                const uint32_t em = as_u(W0.w);
+                const uint32_t nqx = neg0 ? as_u(W1.y) : as_u(W1.x), fqx = neg0 ? as_u(W1.x) : as_u(W1.y);
+                const uint32_t nqy = neg1 ? as_u(W1.w) : as_u(W1.z), fqy = neg1 ? as_u(W1.z) : as_u(W1.w);
+                const uint32_t nqz = neg2 ? as_u(W2.y) : as_u(W2.x), fqz = neg2 ? as_u(W2.x) : as_u(W2.y);
+                RF = make_int4((int)as_u(W2.z), (int)as_u(W2.w), (int)as_u(W3.x), (int)as_u(W3.y));
+                float t0, t1, t2, t3;
+                if (wfast) {
+                    const CqAxis X = cq_axis_ray(W0.x, em & 0xFFu, r.ox, r.ix);
+                    const CqAxis Y = cq_axis_ray(W0.y, (em >> 8) & 0xFFu, r.oy, r.iy);
+                    const CqAxis Z = cq_axis_ray(W0.z, (em >> 16) & 0xFFu, r.oz, r.iz);
+#define PX_CQ_SLOT(K, I, P, T) \
+        P = RF.K != QEMPTY && slab_ray(nqx, fqx, nqy, fqy, nqz, fqz, I, X, Y, Z, r.tmin, r.tmax, &T);
+                    PX_CQ_SLOT(x, 0, p0, t0)
+                    PX_CQ_SLOT(y, 1, p1, t1)
+                    PX_CQ_SLOT(z, 2, p2, t2)
+                    PX_CQ_SLOT(w, 3, p3, t3)
+#undef PX_CQ_SLOT
+                } else {
+                    const float sx = cq_scale(em & 0xFFu), sy = cq_scale((em >> 8) & 0xFFu),
+                                sz = cq_scale((em >> 16) & 0xFFu);
+#define PX_CQ_SLOT(K, I, P, T)                                                                                \
+        P = RF.K != QEMPTY &&                                                                                     \
+            slab_signed(cq_bound(nqx, I, W0.x, sx), cq_bound(fqx, I, W0.x, sx), cq_bound(nqy, I, W0.y, sy),       \
+                        cq_bound(fqy, I, W0.y, sy), cq_bound(nqz, I, W0.z, sz), cq_bound(fqz, I, W0.z, sz), r.ox,  \
+                        r.oy, r.oz, r.ix, r.iy, r.iz, r.tmin, r.tmax, &T);
+                    PX_CQ_SLOT(x, 0, p0, t0)
+                    PX_CQ_SLOT(y, 1, p1, t1)
+                    PX_CQ_SLOT(z, 2, p2, t2)
+                    PX_CQ_SLOT(w, 3, p3, t3)
+#undef PX_CQ_SLOT
+                }
+            } else if (mine) {
+                // leaf: its exact box, then prims in order until the record flagged last
+                uint32_t pos = (uint32_t)(~ref);
+                const float4* p = reinterpret_cast<const float4*>(sv.prims64 + pos);
+                float4 P2 = p[2], P3 = p[3];
+                float tn;
+                if (slab(P2.y, P3.x, P2.z, P3.y, P2.w, P3.z, r.ox, r.oy, r.oz, r.ix, r.iy, r.iz, r.tmin, r.tmax, &tn)) {
+                    while (true) {
+                        const float4 P0 = p[0], P1 = p[1];
+                        const uint32_t kind = as_u(P3.w);
+                        uint32_t hp;
+                        float hb1, hb2;
+                        if (prim_test64(sv, pos, P0, P1, P2, kind, r, &hp, &hb1, &hb2)) {
+                            hitnow = true;
+                            break;
+                        }
+                        if (kind & 0x100u) break;
+                        ++pos;
+                        p += 4;
+                        P2 = p[2];
+                        P3 = p[3];
                     }
-                    if (kind & 0x100u) break;
-                    ++pos;
-                    p += 4;
-                    P2 = p[2];
-                    P3 = p[3];
                 }
             }
-        }
-        // passing slots onto the group's stack: each lane's offset is the
-        // count of its group's lower lanes' passing slots (three ballots of
-        // the bits of each lane's count)
-        const uint32_t c = (p0 ? 1u : 0u) + (p1 ? 1u : 0u) + (p2 ? 1u : 0u) + (p3 ? 1u : 0u);
-        const unsigned long long c0 = __ballot(c & 1u), c1 = __ballot(c & 2u), c2 = __ballot(c & 4u);
-        const uint32_t pre = (uint32_t)__popcll(c0 & lowg) + 2u * (uint32_t)__popcll(c1 & lowg) +
-                             4u * (uint32_t)__popcll(c2 & lowg);
-        const uint32_t tot = (uint32_t)__popcll(c0 & gm) + 2u * (uint32_t)__popcll(c1 & gm) +
-                             4u * (uint32_t)__popcll(c2 & gm);
-        const bool ghit = (__ballot(hitnow) & gm) != 0ull;
-        if (!done && !ghit) {
-            if (top + tot > (uint32_t)GSTK) {
-                if (gl == 0) atomicOr(err, 1u);  // outside the bound above: never expected
-                done = true;
-            } else {
-                uint32_t w = top + pre;
-                if (p0) stk[w++] = RF.x;
-                if (p1) stk[w++] = RF.y;
-                if (p2) stk[w++] = RF.z;
-                if (p3) stk[w] = RF.w;
-                top += tot;
+            // passing slots onto the group's stack: each lane's offset is the
+            // count of its group's lower lanes' passing slots (three ballots of
+            // the bits of each lane's count)
+            const uint32_t c = (p0 ? 1u : 0u) + (p1 ? 1u : 0u) + (p2 ? 1u : 0u) + (p3 ? 1u : 0u);
+            const unsigned long long c0 = __ballot(c & 1u), c1 = __ballot(c & 2u), c2 = __ballot(c & 4u);
+            const uint32_t pre = (uint32_t)__popcll(c0 & lowg) + 2u * (uint32_t)__popcll(c1 & lowg) +
+                                 4u * (uint32_t)__popcll(c2 & lowg);
+            const uint32_t tot = (uint32_t)__popcll(c0 & gm) + 2u * (uint32_t)__popcll(c1 & gm) +
+                                 4u * (uint32_t)__popcll(c2 & gm);
+            const bool ghit = (__ballot(hitnow) & gm) != 0ull;
+            if (!done && !ghit) {
+                if (top + tot > (uint32_t)GSTK) {
+                    if (gl == 0) atomicOr(err, 1u);  // outside the bound above: never expected
+                    done = true;
+                } else {
+                    uint32_t w = top + pre;
+                    if (p0) stk[w++] = RF.x;
+                    if (p1) stk[w++] = RF.y;
+                    if (p2) stk[w++] = RF.z;
+                    if (p3) stk[w] = RF.w;
+                    top += tot;
+                }
             }
+            hit = hit || ghit;
+            done = done || ghit || top == 0u;
         }
-        hit = hit || ghit;
-        done = done || ghit || top == 0u;
-    }
-    if (occ8 || SEG || TAIL) {
+        if (whole) break;
         if (id < n && gl == 0) {
             if (occ8) occ8[rid] = hit ? 1u : 0u;
             else if (hit) atomicOr((SEG ? segs[rseg].occ : occ) + (rid >> 5), 1u << (rid & 31u));
         }
-        return;
     }
+    if (!whole) return;
     // bits: the block's rays are gpb consecutive bits (8, 16, 32 or 64), so it
     // writes them whole -- words that nobody has to clear first
     __shared__ uint32_t s_bits[2];
@@ -1062,222 +1066,224 @@ __global__ __launch_bounds__(CL_BLOCK) __attribute__((amdgpu_waves_per_eu(6))) v
     SceneView sv, Ray* rays, uint32_t n_host, const uint32_t* n_dev, Hit* hits, uint32_t lim, uint32_t* err,
     const TraceSeg* segs, uint32_t nseg, TailView tail) {
     static_assert(G >= 2 && G <= 64 && (64 % G) == 0, "a group lies within one wave");
-    // (the grid covers n_host rays: a count on the device never exceeds it)
+    // (a count on the device never exceeds n_host)
     const uint32_t n = TAIL ? min(*tail.count, tail.cap) : n_dev ? min(*n_dev, n_host) : n_host;
     const uint32_t gpb = CL_BLOCK / G;  // groups per block
-    if ((uint64_t)blockIdx.x * gpb >= (uint64_t)n) return;
     constexpr int GSTK_CL = gstk_closest(G);
     __shared__ int2 s_stk[CL_BLOCK / G][GSTK_CL];  // ref, entry distance
     const uint32_t tid = threadIdx.x, lane = __lane_id();
     const uint32_t g = tid / G, gl = tid % G;
-    const uint32_t id = blockIdx.x * gpb + g;
-    uint32_t rid = id, rseg = 0;  // SEG: rid is the ray's index in segment rseg
     const uint32_t gbase = lane & ~(uint32_t)(G - 1);
     const unsigned long long gm = (G == 64 ? ~0ull : ((1ull << G) - 1ull)) << gbase;  // the group's lanes
     const unsigned long long lowg = gm & (lane == 0 ? 0ull : (~0ull >> (64 - lane)));  // ... below this one
     const unsigned long long highg = gm & ~lowg & ~(1ull << lane);                      // ... above it
     int2* stk = s_stk[g];
-    RayState r{};
-    bool done = id >= n;
-    uint32_t top = 0;
-    float tmax0 = 0.0f;
-    uint32_t hpos = NO_HIT;
-    float hb1 = 0.0f, hb2 = 0.0f;
-    if (!done) {
-        if (TAIL) rid = tail.recs[id].id;
-        if (SEG) {
-            rseg = find_seg(segs, nseg, rid);
-            rid -= segs[rseg].start;
-            load_ray(segs[rseg].rays, rid, r);
-        } else {
-            load_ray(rays, rid, r);
-        }
-        tmax0 = r.tmax;
-        float tn;
-        if (TAIL) {
-            // the walk goes on from the hit and the entries its wave handed over
-            const TailRec t = tail.recs[id];
-            hpos = t.hpos;
-            r.tmax = t.tmax;
-            hb1 = t.b1;
-            hb2 = t.b2;
-            top = t.sp;
-            for (uint32_t e = gl; e < top; e += G) stk[e] = tail.stk[(size_t)id * TAIL_STK + e];
-        } else if (slab(sv.root_lo[0], sv.root_hi[0], sv.root_lo[1], sv.root_hi[1], sv.root_lo[2], sv.root_hi[2], r.ox,
-                        r.oy, r.oz, r.ix, r.iy, r.iz, r.tmin, r.tmax, &tn)) {
-            // the root's own box (popped first by the reference)
-            top = 1;
-            if (gl == 0) stk[0] = make_int2(sv.qroot, (int)0xFF800000u);
-        }
-        done = top == 0;
-    }
-    const bool neg0 = r.ix < 0.0f, neg1 = r.iy < 0.0f, neg2 = r.iz < 0.0f;
-    const uint32_t negm = (neg0 ? 1u : 0u) | (neg1 ? 2u : 0u) | (neg2 ? 4u : 0u);
-    // every ray of the wave may take the ray-space record test (cq_fast_ray)
-    const bool wfast = cq_fast_scene(sv) && __ballot(id < n && !cq_fast_ray(r)) == 0ull;
-    bool one = false;  // one entry a step
-    while (__any(!done)) {
-        // entries for this step: up to G, fewer near the stack's bound
-        uint32_t k = 0;
+    // one ray a group, or more where the count is on the device
+    for (uint64_t blk = blockIdx.x; blk * gpb < (uint64_t)n; blk += gridDim.x) {
+        const uint32_t id = (uint32_t)(blk * gpb) + g;
+        uint32_t rid = id, rseg = 0;  // SEG: rid is the ray's index in segment rseg
+        RayState r{};
+        bool done = id >= n;
+        uint32_t top = 0;
+        float tmax0 = 0.0f;
+        uint32_t hpos = NO_HIT;
+        float hb1 = 0.0f, hb2 = 0.0f;
         if (!done) {
-            k = top < (uint32_t)G ? top : (uint32_t)G;
-            const uint32_t room = top + 6u <= lim && !one ? (lim - top) / 3u : 1u;
-            k = k < room ? k : room;
-        }
-        int2 ent = make_int2(0, 0);
-        bool mine = gl < k;
-        if (mine) ent = stk[top - 1u - gl];
-        top -= k;
-        // the entry's box lies past the hit so far
-        mine = mine && !(as_f((uint32_t)ent.y) > r.tmax);
-        const int32_t ref = ent.x;
-        // what this lane puts back, in visiting order
-        int32_t r0 = 0, r1 = 0, r2 = 0, r3 = 0;
-        float t0 = 0.0f, t1 = 0.0f, t2 = 0.0f, t3 = 0.0f;
-        bool p0 = false, p1 = false, p2 = false, p3 = false;
-        // a leaf's offer
-        bool cand = false;
-        uint32_t cpos = NO_HIT;
-        float ct = 0.0f, cb1 = 0.0f, cb2 = 0.0f;
-        if (mine && ref >= 0) {
-            const float4* q = reinterpret_cast<const float4*>(sv.cnodes + ref);
-            const float4 W0 = q[0], W1 = q[1], W2 = q[2], W3 = q[3];
-            const uint32_t em = as_u(W0.w);
-            const uint32_t nqx = neg0 ? as_u(W1.y) : as_u(W1.x), fqx = neg0 ? as_u(W1.x) : as_u(W1.y);
-            const uint32_t nqy = neg1 ? as_u(W1.w) : as_u(W1.z), fqy = neg1 ? as_u(W1.z) : as_u(W1.w);
-            const uint32_t nqz = neg2 ? as_u(W2.y) : as_u(W2.x), fqz = neg2 ? as_u(W2.x) : as_u(W2.y);
-            r0 = (int)as_u(W2.z); r1 = (int)as_u(W2.w); r2 = (int)as_u(W3.x); r3 = (int)as_u(W3.y);
-            const uint32_t meta = em >> 24;
-            const float rtmax = one ? tmax0 : r.tmax;  // (one: tmax may rise again before the slot is popped)
-            if (wfast) {
-                const CqAxis X = cq_axis_ray(W0.x, em & 0xFFu, r.ox, r.ix);
-                const CqAxis Y = cq_axis_ray(W0.y, (em >> 8) & 0xFFu, r.oy, r.iy);
-                const CqAxis Z = cq_axis_ray(W0.z, (em >> 16) & 0xFFu, r.oz, r.iz);
-#define PX_CQ_SLOT(I) \
-    p##I = (r##I != QEMPTY) & slab_ray(nqx, fqx, nqy, fqy, nqz, fqz, I, X, Y, Z, r.tmin, rtmax, &t##I);
-                PX_CQ_SLOT(0)
-                PX_CQ_SLOT(1)
-                PX_CQ_SLOT(2)
-                PX_CQ_SLOT(3)
-#undef PX_CQ_SLOT
+            if (TAIL) rid = tail.recs[id].id;
+            if (SEG) {
+                rseg = find_seg(segs, nseg, rid);
+                rid -= segs[rseg].start;
+                load_ray(segs[rseg].rays, rid, r);
             } else {
-                const float sx = cq_scale(em & 0xFFu), sy = cq_scale((em >> 8) & 0xFFu),
-                            sz = cq_scale((em >> 16) & 0xFFu);
-#define PX_CQ_SLOT(I)                                                                                         \
-    p##I = r##I != QEMPTY &&                                                                                  \
-           slab_signed(cq_bound(nqx, I, W0.x, sx), cq_bound(fqx, I, W0.x, sx), cq_bound(nqy, I, W0.y, sy),    \
-                       cq_bound(fqy, I, W0.y, sy), cq_bound(nqz, I, W0.z, sz), cq_bound(fqz, I, W0.z, sz),    \
-                       r.ox, r.oy, r.oz, r.ix, r.iy, r.iz, r.tmin, rtmax, &t##I);
-                PX_CQ_SLOT(0)
-                PX_CQ_SLOT(1)
-                PX_CQ_SLOT(2)
-                PX_CQ_SLOT(3)
-#undef PX_CQ_SLOT
+                load_ray(rays, rid, r);
             }
-            // the reference's visiting order of the four slots (bvh.rs:409-415)
-            const bool nA = (negm >> (meta & 3u)) & 1u;
-            const bool nB = (negm >> ((meta >> 2) & 3u)) & 1u;
-            const bool nC = (negm >> ((meta >> 4) & 3u)) & 1u;
-#define PX_SWAP(C, I, J)                                                                 \
-    {                                                                                     \
-        const bool pa = C ? p##J : p##I, pb = C ? p##I : p##J;                            \
-        const int32_t ra = C ? r##J : r##I, rb = C ? r##I : r##J;                         \
-        const float ta = C ? t##J : t##I, tb = C ? t##I : t##J;                           \
-        p##I = pa; p##J = pb; r##I = ra; r##J = rb; t##I = ta; t##J = tb;                 \
-    }
-            PX_SWAP(nB, 0, 1)
-            PX_SWAP(nC, 2, 3)
-            PX_SWAP(nA, 0, 2)
-            PX_SWAP(nA, 1, 3)
-#undef PX_SWAP
-        } else if (mine) {
-            // leaf: its exact box, then prims in order until the record flagged last
-            uint32_t pos = (uint32_t)(~ref);
-            const float4* p = reinterpret_cast<const float4*>(sv.prims64 + pos);
-            float4 P2 = p[2], P3 = p[3];
-            if (slab(P2.y, P3.x, P2.z, P3.y, P2.w, P3.z, r.ox, r.oy, r.oz, r.ix, r.iy, r.iz, r.tmin, r.tmax, &t0)) {
-                const float tmax = r.tmax;  // the offer leaves the ray as it is
-                bool nan = false;
-                while (true) {
-                    const float4 P0 = p[0], P1 = p[1];
-                    const uint32_t kind = as_u(P3.w);
-                    if (prim_test64(sv, pos, P0, P1, P2, kind, r, &cpos, &cb1, &cb2)) {
-                        cand = true;
-                        nan = nan || r.tmax != r.tmax;
-                    }
-                    if (kind & 0x100u) break;
-                    ++pos;
-                    p += 4;
-                    P2 = p[2];
-                    P3 = p[3];
-                }
-                ct = nan && !one ? __builtin_nanf("") : r.tmax;
-                r.tmax = tmax;
-            }
-        }
-        // offers with no record before them are folded now, in order; the
-        // others go back as the leaves they came from
-        const unsigned long long rec = __ballot(p0 | p1 | p2 | p3);
-        const bool now = cand && (rec & lowg) == 0ull;
-        if (cand && !now) {
-            p0 = true;
-            r0 = ref;
-        }
-        unsigned long long fold = __ballot(now) & gm;
-        bool again = false;
-        while (__any(fold != 0ull)) {
-            const int src = fold ? __builtin_ctzll(fold) : (int)lane;
-            const float ft = __shfl(ct, src), fn = __shfl(t0, src);
-            const float fb1 = __shfl(cb1, src), fb2 = __shfl(cb2, src);
-            const uint32_t fp = (uint32_t)__shfl((int)cpos, src);
-            if (fold && (one || (!(fn > r.tmax) && !(ft > r.tmax)))) {
-                r.tmax = ft;
-                hpos = fp;
-                hb1 = fb1;
-                hb2 = fb2;
-                again = again || (ft != ft && !one);
-            }
-            fold &= fold - 1ull;
-        }
-        // the entries go on the stack, lane 0's on top: each lane's lie above
-        // those of its group's higher lanes (three ballots of the bits of each
-        // lane's count)
-        const uint32_t c = (p0 ? 1u : 0u) + (p1 ? 1u : 0u) + (p2 ? 1u : 0u) + (p3 ? 1u : 0u);
-        const unsigned long long c0 = __ballot(c & 1u), c1 = __ballot(c & 2u), c2 = __ballot(c & 4u);
-        const uint32_t pre = (uint32_t)__popcll(c0 & highg) + 2u * (uint32_t)__popcll(c1 & highg) +
-                             4u * (uint32_t)__popcll(c2 & highg);
-        const uint32_t tot = (uint32_t)__popcll(c0 & gm) + 2u * (uint32_t)__popcll(c1 & gm) +
-                             4u * (uint32_t)__popcll(c2 & gm);
-        if (!done) {
-            if (top + tot > (uint32_t)GSTK_CL) {
-                if (gl == 0) atomicOr(err, 1u);  // outside the bound above: never expected
-                done = true;
-            } else {
-                uint32_t w = top + pre;
-                if (p3) stk[w++] = make_int2(r3, (int)as_u(t3));
-                if (p2) stk[w++] = make_int2(r2, (int)as_u(t2));
-                if (p1) stk[w++] = make_int2(r1, (int)as_u(t1));
-                if (p0) stk[w] = make_int2(r0, (int)as_u(t0));
-                top += tot;
-            }
-            if (again) {
-                // a hit at t = NaN: from the root again, one entry a step
-                one = true;
-                r.tmax = tmax0;
-                hpos = NO_HIT;
-                hb1 = hb2 = 0.0f;
+            tmax0 = r.tmax;
+            float tn;
+            if (TAIL) {
+                // the walk goes on from the hit and the entries its wave handed over
+                const TailRec t = tail.recs[id];
+                hpos = t.hpos;
+                r.tmax = t.tmax;
+                hb1 = t.b1;
+                hb2 = t.b2;
+                top = t.sp;
+                for (uint32_t e = gl; e < top; e += G) stk[e] = tail.stk[(size_t)id * TAIL_STK + e];
+            } else if (slab(sv.root_lo[0], sv.root_hi[0], sv.root_lo[1], sv.root_hi[1], sv.root_lo[2], sv.root_hi[2], r.ox,
+                            r.oy, r.oz, r.ix, r.iy, r.iz, r.tmin, r.tmax, &tn)) {
+                // the root's own box (popped first by the reference)
                 top = 1;
                 if (gl == 0) stk[0] = make_int2(sv.qroot, (int)0xFF800000u);
             }
-            done = done || top == 0u;
+            done = top == 0;
         }
-    }
-    if (id < n && gl == 0) {
-        Hit* hp = SEG ? segs[rseg].hits : hits;
-        Ray* rp = SEG ? segs[rseg].rays : rays;
-        const bool hit = hpos != NO_HIT;
-        hp[rid] = Hit{hit ? sv.order[hpos] : NO_HIT, hit ? r.tmax : 0.0f, hb1, hb2};
-        if (hit) rp[rid].tmax = r.tmax;
+        const bool neg0 = r.ix < 0.0f, neg1 = r.iy < 0.0f, neg2 = r.iz < 0.0f;
+        const uint32_t negm = (neg0 ? 1u : 0u) | (neg1 ? 2u : 0u) | (neg2 ? 4u : 0u);
+        // every ray of the wave may take the ray-space record test (cq_fast_ray)
+        const bool wfast = cq_fast_scene(sv) && __ballot(id < n && !cq_fast_ray(r)) == 0ull;
+        bool one = false;  // one entry a step
+        while (__any(!done)) {
+            // entries for this step: up to G, fewer near the stack's bound
+            uint32_t k = 0;
+            if (!done) {
+                k = top < (uint32_t)G ? top : (uint32_t)G;
+                const uint32_t room = top + 6u <= lim && !one ? (lim - top) / 3u : 1u;
+                k = k < room ? k : room;
+            }
+            int2 ent = make_int2(0, 0);
+            bool mine = gl < k;
+            if (mine) ent = stk[top - 1u - gl];
+            top -= k;
+            // the entry's box lies past the hit so far
+            mine = mine && !(as_f((uint32_t)ent.y) > r.tmax);
+            const int32_t ref = ent.x;
+            // what this lane puts back, in visiting order
+            int32_t r0 = 0, r1 = 0, r2 = 0, r3 = 0;
+            float t0 = 0.0f, t1 = 0.0f, t2 = 0.0f, t3 = 0.0f;
+            bool p0 = false, p1 = false, p2 = false, p3 = false;
+            // a leaf's offer
+            bool cand = false;
+            uint32_t cpos = NO_HIT;
+            float ct = 0.0f, cb1 = 0.0f, cb2 = 0.0f;
+            if (mine && ref >= 0) {
+                const float4* q = reinterpret_cast<const float4*>(sv.cnodes + ref);
+                const float4 W0 = q[0], W1 = q[1], W2 = q[2], W3 = q[3];
+                const uint32_t em = as_u(W0.w);
+                const uint32_t nqx = neg0 ? as_u(W1.y) : as_u(W1.x), fqx = neg0 ? as_u(W1.x) : as_u(W1.y);
+                const uint32_t nqy = neg1 ? as_u(W1.w) : as_u(W1.z), fqy = neg1 ? as_u(W1.z) : as_u(W1.w);
+                const uint32_t nqz = neg2 ? as_u(W2.y) : as_u(W2.x), fqz = neg2 ? as_u(W2.x) : as_u(W2.y);
+                r0 = (int)as_u(W2.z); r1 = (int)as_u(W2.w); r2 = (int)as_u(W3.x); r3 = (int)as_u(W3.y);
+                const uint32_t meta = em >> 24;
+                const float rtmax = one ? tmax0 : r.tmax;  // (one: tmax may rise again before the slot is popped)
+                if (wfast) {
+                    const CqAxis X = cq_axis_ray(W0.x, em & 0xFFu, r.ox, r.ix);
+                    const CqAxis Y = cq_axis_ray(W0.y, (em >> 8) & 0xFFu, r.oy, r.iy);
+                    const CqAxis Z = cq_axis_ray(W0.z, (em >> 16) & 0xFFu, r.oz, r.iz);
+#define PX_CQ_SLOT(I) \
+        p##I = (r##I != QEMPTY) & slab_ray(nqx, fqx, nqy, fqy, nqz, fqz, I, X, Y, Z, r.tmin, rtmax, &t##I);
+                    PX_CQ_SLOT(0)
+                    PX_CQ_SLOT(1)
+                    PX_CQ_SLOT(2)
+                    PX_CQ_SLOT(3)
+#undef PX_CQ_SLOT
+                } else {
+                    const float sx = cq_scale(em & 0xFFu), sy = cq_scale((em >> 8) & 0xFFu),
+                                sz = cq_scale((em >> 16) & 0xFFu);
+#define PX_CQ_SLOT(I)                                                                                         \
+        p##I = r##I != QEMPTY &&                                                                                  \
+               slab_signed(cq_bound(nqx, I, W0.x, sx), cq_bound(fqx, I, W0.x, sx), cq_bound(nqy, I, W0.y, sy),    \
+                           cq_bound(fqy, I, W0.y, sy), cq_bound(nqz, I, W0.z, sz), cq_bound(fqz, I, W0.z, sz),    \
+                           r.ox, r.oy, r.oz, r.ix, r.iy, r.iz, r.tmin, rtmax, &t##I);
+                    PX_CQ_SLOT(0)
+                    PX_CQ_SLOT(1)
+                    PX_CQ_SLOT(2)
+                    PX_CQ_SLOT(3)
+#undef PX_CQ_SLOT
+                }
+                // the reference's visiting order of the four slots (bvh.rs:409-415)
+                const bool nA = (negm >> (meta & 3u)) & 1u;
+                const bool nB = (negm >> ((meta >> 2) & 3u)) & 1u;
+                const bool nC = (negm >> ((meta >> 4) & 3u)) & 1u;
+#define PX_SWAP(C, I, J)                                                                 \
+        {                                                                                     \
+            const bool pa = C ? p##J : p##I, pb = C ? p##I : p##J;                            \
+            const int32_t ra = C ? r##J : r##I, rb = C ? r##I : r##J;                         \
+            const float ta = C ? t##J : t##I, tb = C ? t##I : t##J;                           \
+            p##I = pa; p##J = pb; r##I = ra; r##J = rb; t##I = ta; t##J = tb;                 \
+        }
+                PX_SWAP(nB, 0, 1)
+                PX_SWAP(nC, 2, 3)
+                PX_SWAP(nA, 0, 2)
+                PX_SWAP(nA, 1, 3)
+#undef PX_SWAP
+            } else if (mine) {
+                // leaf: its exact box, then prims in order until the record flagged last
+                uint32_t pos = (uint32_t)(~ref);
+                const float4* p = reinterpret_cast<const float4*>(sv.prims64 + pos);
+                float4 P2 = p[2], P3 = p[3];
+                if (slab(P2.y, P3.x, P2.z, P3.y, P2.w, P3.z, r.ox, r.oy, r.oz, r.ix, r.iy, r.iz, r.tmin, r.tmax, &t0)) {
+                    const float tmax = r.tmax;  // the offer leaves the ray as it is
+                    bool nan = false;
+                    while (true) {
+                        const float4 P0 = p[0], P1 = p[1];
+                        const uint32_t kind = as_u(P3.w);
+                        if (prim_test64(sv, pos, P0, P1, P2, kind, r, &cpos, &cb1, &cb2)) {
+                            cand = true;
+                            nan = nan || r.tmax != r.tmax;
+                        }
+                        if (kind & 0x100u) break;
+                        ++pos;
+                        p += 4;
+                        P2 = p[2];
+                        P3 = p[3];
+                    }
+                    ct = nan && !one ? __builtin_nanf("") : r.tmax;
+                    r.tmax = tmax;
+                }
+            }
+            // offers with no record before them are folded now, in order; the
+            // others go back as the leaves they came from
+            const unsigned long long rec = __ballot(p0 | p1 | p2 | p3);
+            const bool now = cand && (rec & lowg) == 0ull;
+            if (cand && !now) {
+                p0 = true;
+                r0 = ref;
+            }
+            unsigned long long fold = __ballot(now) & gm;
+            bool again = false;
+            while (__any(fold != 0ull)) {
+                const int src = fold ? __builtin_ctzll(fold) : (int)lane;
+                const float ft = __shfl(ct, src), fn = __shfl(t0, src);
+                const float fb1 = __shfl(cb1, src), fb2 = __shfl(cb2, src);
+                const uint32_t fp = (uint32_t)__shfl((int)cpos, src);
+                if (fold && (one || (!(fn > r.tmax) && !(ft > r.tmax)))) {
+                    r.tmax = ft;
+                    hpos = fp;
+                    hb1 = fb1;
+                    hb2 = fb2;
+                    again = again || (ft != ft && !one);
+                }
+                fold &= fold - 1ull;
+            }
+            // the entries go on the stack, lane 0's on top: each lane's lie above
+            // those of its group's higher lanes (three ballots of the bits of each
+            // lane's count)
+            const uint32_t c = (p0 ? 1u : 0u) + (p1 ? 1u : 0u) + (p2 ? 1u : 0u) + (p3 ? 1u : 0u);
+            const unsigned long long c0 = __ballot(c & 1u), c1 = __ballot(c & 2u), c2 = __ballot(c & 4u);
+            const uint32_t pre = (uint32_t)__popcll(c0 & highg) + 2u * (uint32_t)__popcll(c1 & highg) +
+                                 4u * (uint32_t)__popcll(c2 & highg);
+            const uint32_t tot = (uint32_t)__popcll(c0 & gm) + 2u * (uint32_t)__popcll(c1 & gm) +
+                                 4u * (uint32_t)__popcll(c2 & gm);
+            if (!done) {
+                if (top + tot > (uint32_t)GSTK_CL) {
+                    if (gl == 0) atomicOr(err, 1u);  // outside the bound above: never expected
+                    done = true;
+                } else {
+                    uint32_t w = top + pre;
+                    if (p3) stk[w++] = make_int2(r3, (int)as_u(t3));
+                    if (p2) stk[w++] = make_int2(r2, (int)as_u(t2));
+                    if (p1) stk[w++] = make_int2(r1, (int)as_u(t1));
+                    if (p0) stk[w] = make_int2(r0, (int)as_u(t0));
+                    top += tot;
+                }
+                if (again) {
+                    // a hit at t = NaN: from the root again, one entry a step
+                    one = true;
+                    r.tmax = tmax0;
+                    hpos = NO_HIT;
+                    hb1 = hb2 = 0.0f;
+                    top = 1;
+                    if (gl == 0) stk[0] = make_int2(sv.qroot, (int)0xFF800000u);
+                }
+                done = done || top == 0u;
+            }
+        }
+        if (id < n && gl == 0) {
+            Hit* hp = SEG ? segs[rseg].hits : hits;
+            Ray* rp = SEG ? segs[rseg].rays : rays;
+            const bool hit = hpos != NO_HIT;
+            hp[rid] = Hit{hit ? sv.order[hpos] : NO_HIT, hit ? r.tmax : 0.0f, hb1, hb2};
+            if (hit) rp[rid].tmax = r.tmax;
+        }
     }
 }
 
@@ -1554,17 +1560,12 @@ __global__ void k_fill_u32(uint32_t* p, uint32_t v, size_t n) {
     size_t stride = (size_t)gridDim.x * blockDim.x;
     for (; i < n; i += stride) p[i] = v;
 }
-// Three word ranges zeroed by one launch (the counters a stage needs
-// cleared, one launch instead of one each).
-__global__ void k_zero3_u32(uint32_t* a, size_t na, uint32_t* b, size_t nb, uint32_t* c, size_t nc) {
-    const size_t n = na + nb + nc;
+// Two word ranges zeroed by one launch.
+__global__ void k_zero2_u32(uint32_t* a, size_t na, uint32_t* b, size_t nb) {
+    const size_t n = na + nb;
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     const size_t stride = (size_t)gridDim.x * blockDim.x;
-    for (; i < n; i += stride) {
-        if (i < na) a[i] = 0u;
-        else if (i < na + nb) b[i - na] = 0u;
-        else c[i - na - nb] = 0u;
-    }
+    for (; i < n; i += stride) (i < na ? a[i] : b[i - na]) = 0u;
 }
 
 // Streaming copy, four 16-byte loads in flight a thread before their
@@ -1695,12 +1696,12 @@ hipError_t fill_u32(uint32_t* p, uint32_t value, size_t n, hipStream_t st) {
     hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)blocks), dim3(256), 0, st, p, value, n);
     return hipGetLastError();
 }
-hipError_t zero3_u32(uint32_t* a, size_t na, uint32_t* b, size_t nb, uint32_t* c, size_t nc, hipStream_t st) {
-    const size_t n = na + nb + nc;
+hipError_t zero2_u32(uint32_t* a, size_t na, uint32_t* b, size_t nb, hipStream_t st) {
+    const size_t n = na + nb;
     if (n == 0) return hipSuccess;
     size_t blocks = (n + 255) / 256;
     if (blocks > 4096) blocks = 4096;
-    hipLaunchKernelGGL(k_zero3_u32, dim3((unsigned)blocks), dim3(256), 0, st, a, na, b, nb, c, nc);
+    hipLaunchKernelGGL(k_zero2_u32, dim3((unsigned)blocks), dim3(256), 0, st, a, na, b, nb);
     return hipGetLastError();
 }
 
@@ -1777,6 +1778,15 @@ static int group_lanes(const SceneView& s, uint32_t n, const TraceTuning& tun) {
     return n <= GROUP32_MAX ? 32 : n <= group16_max(s) ? 16 : n <= GROUP_MAX ? 8 : 1;
 }
 
+// Blocks of a several-lane launch.  Of a queue whose count is on the device at
+// most GROUP_QUEUE_BLOCKS a CU, each then taking rays in turn: a block for
+// every ray that the queue could hold costs 19 us at 2^20 though the queue be
+// empty.
+constexpr size_t GROUP_QUEUE_BLOCKS = 64;
+static unsigned group_grid(size_t blocks, bool queue) {
+    return (unsigned)(queue ? std::min(blocks, GROUP_QUEUE_BLOCKS * (size_t)device_cu_count()) : blocks);
+}
+
 template <bool SEG>
 static auto group_kernel(int G) -> decltype(&k_occlude_group<8, SEG, false>) {
     return G == 4    ? &k_occlude_group<4, SEG, false>
@@ -1850,7 +1860,7 @@ static TailView make_tail(bool any, const SceneView& s, TraceScratch* scr, size_
     if (cap < waves || at + tail_bytes(cap) > scr->spill_bytes) return t;
     t.recs = reinterpret_cast<TailRec*>((uint8_t*)scr->spill + at);
     t.stk = reinterpret_cast<int2*>(t.recs + cap);
-    t.count = scr->counter + WIDE_PARTS_AT + WIDE_PARTS * WIDE_PART_STRIDE;
+    t.count = (scr->parts ? scr->parts : scr->counter + WIDE_PARTS_AT) + WIDE_PARTS * WIDE_PART_STRIDE;
     t.cap = (uint32_t)cap;
     t.lanes = (uint32_t)(cap / waves);
     return t;
@@ -1919,7 +1929,7 @@ static hipError_t launch(const SceneView& s, Ray* rays, uint32_t n, Hit* hits, u
             const uint32_t lim = (uint32_t)gstk_occlude(G) - 3u * s.odepth;
             const uint32_t gpb = (uint32_t)oc_block(G) / (uint32_t)G;
             const size_t cover = occ8 ? (size_t)n : ((size_t)n + 31) / 32 * 32;
-            const unsigned grid = (unsigned)((cover + gpb - 1) / gpb);
+            const unsigned grid = group_grid((cover + gpb - 1) / gpb, n_dev && occ8);
             const auto kern = group_kernel<false>(G);
             hipLaunchKernelGGL(kern, dim3(grid), dim3(oc_block(G)), 0, st, s, rays, n, n_dev, occ, occ8, lim, err,
                                (const TraceSeg*)nullptr, 0u, TailView{});
@@ -1931,7 +1941,7 @@ static hipError_t launch(const SceneView& s, Ray* rays, uint32_t n, Hit* hits, u
         if (G > 1) {
             const uint32_t lim = (uint32_t)gstk_closest(G) - 3u * s.qdepth;
             const uint32_t gpb = (uint32_t)CL_BLOCK / (uint32_t)G;
-            const unsigned grid = (unsigned)(((size_t)n + gpb - 1) / gpb);
+            const unsigned grid = group_grid(((size_t)n + gpb - 1) / gpb, n_dev != nullptr);
             hipLaunchKernelGGL(closest_group_kernel<false>(G), dim3(grid), dim3(CL_BLOCK), 0, st, s, rays, n, n_dev, hits,
                                lim, err, (const TraceSeg*)nullptr, 0u, TailView{});
             return hipGetLastError();
@@ -1946,10 +1956,10 @@ static hipError_t launch(const SceneView& s, Ray* rays, uint32_t n, Hit* hits, u
         if (!scr->cap_grid || per_block > scr->spill_bytes) return hipErrorInvalidValue;
         grid = (int)(scr->spill_bytes / per_block);
     }
-    uint32_t* parts = scr->counter + WIDE_PARTS_AT;
-    hipError_t e = ANY && !occ8 ? zero3_u32(parts, (size_t)WIDE_COUNTERS, occ, ((size_t)n + 31) / 32,
-                                            nullptr, 0, st)
-                                : fill_u32(parts, 0u, (size_t)WIDE_COUNTERS, st);
+    uint32_t* parts = scr->parts ? scr->parts : scr->counter + WIDE_PARTS_AT;
+    hipError_t e = hipSuccess;
+    if (ANY && !occ8) e = zero2_u32(parts, (size_t)WIDE_COUNTERS, occ, ((size_t)n + 31) / 32, st);
+    else if (!scr->parts) e = fill_u32(parts, 0u, (size_t)WIDE_COUNTERS, st);
     if (e != hipSuccess) return e;
     const uint32_t refill = (uint32_t)(tun.refill_pct < 0 ? 0 : (tun.refill_pct > 100 ? 100 : tun.refill_pct));
     const TailView tail = cq && tun.lanes != 1 ? make_tail(ANY, s, scr, per_block * grid, grid, block) : TailView{};
@@ -1958,11 +1968,11 @@ static hipError_t launch(const SceneView& s, Ray* rays, uint32_t n, Hit* hits, u
     e = hipGetLastError();
     if (e != hipSuccess || !tail.recs) return e;
     if constexpr (ANY)
-        hipLaunchKernelGGL((k_occlude_group<8, false, true>), dim3((tail.cap + 7) / 8), dim3(oc_block(8)), 0, st, s, rays,
+        hipLaunchKernelGGL((k_occlude_group<8, false, true>), dim3(group_grid((tail.cap + 7) / 8, true)), dim3(oc_block(8)), 0, st, s, rays,
                            n, n_dev, occ, occ8, (uint32_t)gstk_occlude(8) - 3u * s.odepth, err,
                            (const TraceSeg*)nullptr, 0u, tail);
     else
-        hipLaunchKernelGGL((k_closest_group<8, false, true>), dim3((tail.cap + 7) / 8), dim3(CL_BLOCK), 0, st, s, rays,
+        hipLaunchKernelGGL((k_closest_group<8, false, true>), dim3(group_grid((tail.cap + 7) / 8, true)), dim3(CL_BLOCK), 0, st, s, rays,
                            n, n_dev, hits, (uint32_t)gstk_closest(8) - 3u * s.qdepth, err, (const TraceSeg*)nullptr, 0u,
                            tail);
     return hipGetLastError();
@@ -2099,11 +2109,11 @@ hipError_t trace_segments(const SceneView& s, bool any, const TraceSeg* d_segs, 
     e = hipGetLastError();
     if (e != hipSuccess || !tail.recs) return e;
     if (any)
-        hipLaunchKernelGGL((k_occlude_group<8, true, true>), dim3((tail.cap + 7) / 8), dim3(oc_block(8)), 0, st, s,
+        hipLaunchKernelGGL((k_occlude_group<8, true, true>), dim3(group_grid((tail.cap + 7) / 8, true)), dim3(oc_block(8)), 0, st, s,
                            (const Ray*)nullptr, total, (const uint32_t*)nullptr, (uint32_t*)nullptr,
                            (uint8_t*)nullptr, (uint32_t)gstk_occlude(8) - 3u * s.odepth, err, d_segs, nseg, tail);
     else
-        hipLaunchKernelGGL((k_closest_group<8, true, true>), dim3((tail.cap + 7) / 8), dim3(CL_BLOCK), 0, st, s,
+        hipLaunchKernelGGL((k_closest_group<8, true, true>), dim3(group_grid((tail.cap + 7) / 8, true)), dim3(CL_BLOCK), 0, st, s,
                            (Ray*)nullptr, total, (const uint32_t*)nullptr, (Hit*)nullptr,
                            (uint32_t)gstk_closest(8) - 3u * s.qdepth, err, d_segs, nseg, tail);
     return hipGetLastError();

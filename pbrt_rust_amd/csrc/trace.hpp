@@ -47,6 +47,7 @@ struct TraceTuning {
 // Scratch owned by the caller (per stream): spill stacks and a block of
 // TRACE_COUNTER_WORDS device words for work counters and the overflow flag.
 constexpr uint32_t TRACE_COUNTER_WORDS = 512;
+constexpr uint32_t TRACE_PART_WORDS = 64;
 struct TraceScratch {
     void* spill = nullptr;       // spill stack entries
     size_t spill_bytes = 0;
@@ -54,6 +55,9 @@ struct TraceScratch {
     // a fixed-size scratch: the batched path's persistent grid is cut to the
     // blocks whose spill stacks fit spill_bytes (instead of failing)
     bool cap_grid = false;
+    // one launch's work counters, TRACE_PART_WORDS words that the caller has
+    // cleared; null: the launch clears its own, in the block above, first
+    uint32_t* parts = nullptr;
 };
 
 // The fixed scratch of the entry point that allocates nothing: one device
@@ -123,8 +127,8 @@ hipError_t trace_segments(const SceneView& s, bool any, const TraceSeg* d_segs, 
 // over.
 size_t trace_spill_bytes(const SceneView& s, int path, const TraceTuning& tun, uint64_t rays);
 hipError_t fill_u32(uint32_t* p, uint32_t value, size_t n, hipStream_t st);
-// zeroes a[0..na), b[0..nb) and c[0..nc) with one launch (null ranges of length 0)
-hipError_t zero3_u32(uint32_t* a, size_t na, uint32_t* b, size_t nb, uint32_t* c, size_t nc, hipStream_t st);
+// zeroes a[0..na) and b[0..nb) with one launch
+hipError_t zero2_u32(uint32_t* a, size_t na, uint32_t* b, size_t nb, hipStream_t st);
 // streaming 16-byte-vector copy (bytes a multiple of 16)
 hipError_t copy_bytes(void* dst, const void* src, size_t bytes, hipStream_t st);
 // 64-byte gather probe over a buffer of `records` (a power of two, at most
