@@ -1138,6 +1138,20 @@ __global__ __launch_bounds__(RB) void k_halton_pos(uint32_t npix, uint32_t xres,
     }
 }
 
+// A sample's place in the weight table along one axis, for the pixel at p: bit
+// 4 set when the sample's extent covers the pixel, the table index below it.
+__device__ __forceinline__ uint32_t film_code(int32_t p, float v, float w, float inv_w, int32_t n) {
+    int32_t lo, hi;
+    film_extent(v, w, n, &lo, &hi);
+    return p < lo || p > hi ? 0u : 16u | (uint32_t)film_offset(p, v, inv_w);
+}
+
+// Staging.  CODES (reach at most FILM_CODE_R either way: the usual half-widths,
+// up to 2): a sample's position becomes its codes (film_code) for the pixels
+// from FILM_CODE_R before its own to as many after, five bits each, x and y a
+// word each -- 10 evaluations a sample instead of 25 in the gather.
+constexpr int FILM_CODE_R = 2;
+template <bool CODES>
 __global__ __launch_bounds__(RB) void k_film_stage(RenderParams P, const float4* sample_l, uint64_t n) {
     const uint64_t npix = (uint64_t)P.xres * P.yres;
     for (uint64_t g = (uint64_t)blockIdx.x * RB + threadIdx.x; g < n; g += (uint64_t)gridDim.x * RB) {
@@ -1157,10 +1171,100 @@ __global__ __launch_bounds__(RB) void k_film_stage(RenderParams P, const float4*
         const float c1 = 0.212671f * v.x + 0.715160f * v.y + 0.072169f * v.z;
         const float c2 = 0.019334f * v.x + 0.119193f * v.y + 0.950227f * v.z;
         const uint64_t t = (uint64_t)s * npix + pixel;
+        if (CODES) {
+            // sample_pos: the position within the pixel plus the pixel's coordinates
+            const int32_t qx = (int32_t)(pixel % P.xres), qy = (int32_t)(pixel / P.xres);
+            const float ix = f.x + (float)qx, iy = f.y + (float)qy;
+            uint32_t cx = 0, cy = 0;
+#pragma unroll
+            for (int k = 0; k <= 2 * FILM_CODE_R; ++k) {
+                cx |= film_code(qx + k - FILM_CODE_R, ix, P.fxw, P.fixw, (int32_t)P.xres) << (5 * k);
+                cy |= film_code(qy + k - FILM_CODE_R, iy, P.fyw, P.fiyw, (int32_t)P.yres) << (5 * k);
+            }
+            if (P.scount && s >= P.scount[pixel]) cx = cy = 0u;  // an empty slot reaches nothing
+            f = make_float2(__uint_as_float(cx), __uint_as_float(cy));
+        }
         P.fpos[t] = f;
         P.fxyz[t] = make_float4(c0, c1, c2, 0.0f);
     }
 }
+
+// xyz_to_rgb: spectrum.rs:31-35, and the division by the weights' sum
+__device__ __forceinline__ void film_write(const float* xyz, float wsum, float* rgb, size_t pix) {
+    float o0 = 3.240479f * xyz[0] - 1.37150f * xyz[1] - 0.498535f * xyz[2];
+    float o1 = -0.969256f * xyz[0] + 1.875991f * xyz[1] + 0.041556f * xyz[2];
+    float o2 = 0.055648f * xyz[0] - 0.204043f * xyz[1] + 1.057311f * xyz[2];
+    if (wsum != 0.0f) {
+        const float inv = 1.0f / wsum;
+        o0 = fmaxf(o0 * inv, 0.0f); o1 = fmaxf(o1 * inv, 0.0f); o2 = fmaxf(o2 * inv, 0.0f);
+    }
+    rgb[3 * pix] = o0; rgb[3 * pix + 1] = o1; rgb[3 * pix + 2] = o2;
+}
+
+// The gather by rows, for staged codes and at most FILM_ROW_SPP samples a
+// pixel.  Every sample is read by up to 25 pixels; from global memory those
+// reads were L2-bound (1.2 GB in 313 us for a 480x270 film of 16 samples a
+// pixel and a Gaussian of half-width 2: a wave's samples of one neighbour fill
+// the L1 before the next neighbour reads most of them again).  A wave takes 64
+// - 2 frx pixels of a row and copies, row by row of its reach, the 64
+// neighbouring pixels' samples to LDS -- xyz and, in one word, the five x codes
+// and the y code of this row -- from where each pixel adds them in the same
+// order (pixels row-major, then samples).  89 us.  More samples leave too few
+// waves' LDS on a CU: 1024x1024, global / rows, Gaussian of half-width 2 and
+// triangle of 1: 25 samples a pixel 3.0 / 1.7 and 1.1 / 1.0 ms, 36 samples 4.4 /
+// 3.5 and 1.7 / 1.9 ms, 64 samples 8.9 / 11.7 and 3.9 / 6.5 ms.
+constexpr uint32_t FILM_ROW_SPP = 32;
+__global__ __launch_bounds__(64) void k_film_rows(RenderParams P, float* rgb) {
+    extern __shared__ float s_film[];
+    float* tab = s_film;
+    float4* smp = reinterpret_cast<float4*>(s_film + FILTER_TABLE_DIM * FILTER_TABLE_DIM);  // [sample][pixel]
+    const uint32_t lane = threadIdx.x;
+    for (uint32_t k = lane; k < FILTER_TABLE_DIM * FILTER_TABLE_DIM; k += 64) tab[k] = P.ftab[k];
+    const int32_t xres = (int32_t)P.xres, yres = (int32_t)P.yres, W = 64 - 2 * P.frx;
+    const int32_t x0 = (int32_t)blockIdx.x * W, x = x0 + (int32_t)lane, y = (int32_t)blockIdx.y;
+    const bool mine = (int32_t)lane < W && x < xres;
+    const int32_t sx = x0 - P.frx + (int32_t)lane;  // the pixel this lane copies
+    const bool copies = sx >= 0 && sx < xres;
+    const size_t npix = (size_t)P.xres * P.yres;
+    float xyz[3] = {0.0f, 0.0f, 0.0f};
+    float wsum = 0.0f;
+    for (int32_t qy = max(0, y - P.fry); qy <= min(yres - 1, y + P.fry); ++qy) {
+        const uint32_t ys = 5u * (uint32_t)(y - qy + FILM_CODE_R);
+        const size_t q = (size_t)qy * P.xres + (size_t)(copies ? sx : 0);
+        __syncthreads();  // the row before has been added
+#pragma unroll 8
+        for (uint32_t s = 0; s < P.spp; ++s) {
+            float4 c = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (copies) {
+                const float2 f = P.fpos[(size_t)s * npix + q];
+                c = P.fxyz[(size_t)s * npix + q];
+                c.w = __uint_as_float(__float_as_uint(f.x) | (((__float_as_uint(f.y) >> ys) & 31u) << 25));
+            }
+            smp[s * 64 + lane] = c;
+        }
+        __syncthreads();
+        if (!mine) continue;
+        for (int32_t k = 0; k <= 2 * P.frx; ++k) {  // pixel x - frx + k
+            const uint32_t xs = 5u * (uint32_t)(P.frx - k + FILM_CODE_R);
+            const float4* row = smp + lane + (uint32_t)k;
+#pragma unroll 4
+            for (uint32_t s = 0; s < P.spp; ++s) {
+                const float4 c = row[s * 64];
+                const uint32_t cx = __float_as_uint(c.w) >> xs, cy = __float_as_uint(c.w) >> 25;
+                const float wt = tab[(cy & 15u) * FILTER_TABLE_DIM + (cx & 15u)];
+                if (cx & cy & 16u) {
+                    xyz[0] = xyz[0] + wt * c.x;
+                    xyz[1] = xyz[1] + wt * c.y;
+                    xyz[2] = xyz[2] + wt * c.z;
+                    wsum = wsum + wt;
+                }
+            }
+        }
+    }
+    if (mine) film_write(xyz, wsum, rgb, (size_t)y * P.xres + (size_t)x);
+}
+
+// The gather from global memory: wider filters and more samples a pixel.
 __global__ __launch_bounds__(RB) void k_film_filter(RenderParams P, float* rgb) {
     __shared__ float s_tab[FILTER_TABLE_DIM * FILTER_TABLE_DIM];
     for (uint32_t k = threadIdx.x; k < FILTER_TABLE_DIM * FILTER_TABLE_DIM; k += RB) s_tab[k] = P.ftab[k];
@@ -1191,16 +1295,7 @@ __global__ __launch_bounds__(RB) void k_film_filter(RenderParams P, float* rgb) 
             }
         }
     }
-    // xyz_to_rgb: spectrum.rs:31-35
-    float o0 = 3.240479f * xyz[0] - 1.37150f * xyz[1] - 0.498535f * xyz[2];
-    float o1 = -0.969256f * xyz[0] + 1.875991f * xyz[1] + 0.041556f * xyz[2];
-    float o2 = 0.055648f * xyz[0] - 0.204043f * xyz[1] + 1.057311f * xyz[2];
-    if (wsum != 0.0f) {
-        const float inv = 1.0f / wsum;
-        o0 = fmaxf(o0 * inv, 0.0f); o1 = fmaxf(o1 * inv, 0.0f); o2 = fmaxf(o2 * inv, 0.0f);
-    }
-    const size_t pix = (size_t)y * P.xres + (size_t)x;
-    rgb[3 * pix] = o0; rgb[3 * pix + 1] = o1; rgb[3 * pix + 2] = o2;
+    film_write(xyz, wsum, rgb, (size_t)y * P.xres + (size_t)x);
 }
 
 // ---------------------------------------------------------------------------
@@ -1604,8 +1699,16 @@ hipError_t enqueue_film(const RenderParams& P, const float4* sample_l, float* rg
     if (P.ftab) {
         const uint64_t n = (uint64_t)P.xres * P.yres * P.spp;
         const uint64_t blocks = std::min<uint64_t>((n + RB - 1) / RB, 65536);
-        hipLaunchKernelGGL(k_film_stage, dim3((unsigned)blocks), dim3(RB), 0, st, P, sample_l, n);
-        hipLaunchKernelGGL(k_film_filter, grid, dim3(RB), 0, st, P, rgb);
+        const bool rows = P.frx <= FILM_CODE_R && P.fry <= FILM_CODE_R && P.spp <= FILM_ROW_SPP;
+        hipLaunchKernelGGL(rows ? &k_film_stage<true> : &k_film_stage<false>, dim3((unsigned)blocks), dim3(RB), 0, st,
+                           P, sample_l, n);
+        if (rows) {
+            const uint32_t W = 64u - 2u * (uint32_t)P.frx;
+            const size_t lds = (FILTER_TABLE_DIM * FILTER_TABLE_DIM + 4 * 64 * (size_t)P.spp) * sizeof(float);
+            hipLaunchKernelGGL(k_film_rows, dim3((P.xres + W - 1) / W, P.yres), dim3(64), lds, st, P, rgb);
+        } else {
+            hipLaunchKernelGGL(k_film_filter, grid, dim3(RB), 0, st, P, rgb);
+        }
     } else {
         hipLaunchKernelGGL(k_film, grid, dim3(RB), 0, st, P, sample_l, rgb);
     }
