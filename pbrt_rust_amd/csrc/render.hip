@@ -262,8 +262,7 @@ __global__ __launch_bounds__(SHADE_B) void k_shade_direct(RenderParams P, uint64
         f3 le = mk3(0, 0, 0);
         if (hs.light >= 0 && dot3(nn, wo) > 0.0f) le = ld3(P.a_le + 3 * hs.light);
         lbase[ent] = make_float4(le.x, le.y, le.z, 0.0f);
-        uint64_t g = g0 + i;
-        pixel = (uint32_t)(g / P.spp); s = (uint32_t)(g % P.spp);
+        sample_split(P, g0 + i, &pixel, &s);
     } else if (live) {
         lbase[ent] = make_float4(0, 0, 0, 0);
     }
@@ -488,7 +487,7 @@ __global__ __launch_bounds__(RB) void k_bounce_totals(uint32_t* cnt, uint32_t nb
 // batch index gid to.
 struct SampleRef {
     uint64_t g;
-    uint32_t spp, seed;
+    uint32_t spp, spp_l, seed;
     float4* out;
 };
 __device__ __forceinline__ SampleRef sample_ref(const RenderParams& P, uint64_t g0, const PathState& ps,
@@ -497,10 +496,10 @@ __device__ __forceinline__ SampleRef sample_ref(const RenderParams& P, uint64_t 
         const RenderSeg sg = P.segs[ps.flags >> 8];
         const ReqView* rq = P.reqs + sg.req;
         const uint64_t g = sg.g0 + (ps.gid - sg.start);
-        return SampleRef{g, rq->cam.spp, rq->cam.seed, rq->sample_l + g};
+        return SampleRef{g, rq->cam.spp, rq->cam.div.spp_l, rq->cam.seed, rq->sample_l + g};
     }
     const uint64_t g = g0 + ps.gid;
-    return SampleRef{g, P.spp, P.seed, sample_l + g};
+    return SampleRef{g, P.spp, P.div.spp_l, P.seed, sample_l + g};
 }
 
 // Camera rays and initial path state of the batch's paths.
@@ -580,7 +579,8 @@ __device__ __forceinline__ void path_vertex(const RenderParams& P, uint64_t g0, 
         }
         const MatRec mat = P.mats[hs.mat];
         const SampleRef sr = sample_ref(P, g0, ps, sample_l);
-        const uint32_t pixel = (uint32_t)(sr.g / sr.spp), s = (uint32_t)(sr.g % sr.spp);
+        uint32_t pixel, s;
+        sample_split(sr.spp, sr.spp_l, sr.g, &pixel, &s);
         float ua[4], ub[4];
         rng4(sr.seed, pixel, s, 1 + 2 * bounce, ua);
         rng4(sr.seed, pixel, s, 2 + 2 * bounce, ub);
@@ -1155,14 +1155,16 @@ template <bool CODES>
 __global__ __launch_bounds__(RB) void k_film_stage(RenderParams P, const float4* sample_l, uint64_t n) {
     const uint64_t npix = (uint64_t)P.xres * P.yres;
     for (uint64_t g = (uint64_t)blockIdx.x * RB + threadIdx.x; g < n; g += (uint64_t)gridDim.x * RB) {
-        const uint32_t pixel = (uint32_t)(g / P.spp), s = (uint32_t)(g % P.spp);
+        uint32_t pixel, s;
+        sample_split(P, g, &pixel, &s);
         float2 f;
         if (P.spos) {
             f = P.spos[g];
         } else {
             float u[4];
             rng4(P.seed, pixel, s, 0, u);  // sample_pos's jitter
-            const uint32_t sx = s % P.nx, sy = s / P.nx;
+            uint32_t sx, sy;
+            stratum_split(P, s, &sx, &sy);
             f = make_float2(((float)sx + u[0]) * P.dx, ((float)sy + u[1]) * P.dy);
         }
         const float4 v = sample_l[g];
@@ -1173,7 +1175,9 @@ __global__ __launch_bounds__(RB) void k_film_stage(RenderParams P, const float4*
         const uint64_t t = (uint64_t)s * npix + pixel;
         if (CODES) {
             // sample_pos: the position within the pixel plus the pixel's coordinates
-            const int32_t qx = (int32_t)(pixel % P.xres), qy = (int32_t)(pixel / P.xres);
+            uint32_t ux, uy;
+            pixel_split(P, pixel, &ux, &uy);
+            const int32_t qx = (int32_t)ux, qy = (int32_t)uy;
             const float ix = f.x + (float)qx, iy = f.y + (float)qy;
             uint32_t cx = 0, cy = 0;
 #pragma unroll
@@ -1671,6 +1675,7 @@ int camera_setup(RenderParams* P, const float* cam_to_world, float fov_deg, cons
     memcpy(P->c2w, cam_to_world, sizeof(P->c2w));
     P->xres = xres; P->yres = yres; P->nx = nx; P->ny = ny; P->spp = nx * ny; P->seed = seed;
     P->dx = 1.0f / (float)nx; P->dy = 1.0f / (float)ny;
+    P->div = cam_div(*P);
     return PBRTX_OK;
 }
 
@@ -1679,7 +1684,7 @@ CamParams cam_params(const RenderParams& P, uint64_t g0) {
     memcpy(cp.r2c, P.r2c, sizeof(cp.r2c));
     memcpy(cp.c2w, P.c2w, sizeof(cp.c2w));
     cp.xres = P.xres; cp.nx = P.nx; cp.spp = P.spp; cp.seed = P.seed;
-    cp.dx = P.dx; cp.dy = P.dy; cp.g0 = g0;
+    cp.dx = P.dx; cp.dy = P.dy; cp.div = P.div; cp.g0 = g0;
     cp.spos = P.spos;
     cp.scount = P.scount;
     return cp;
@@ -1976,6 +1981,7 @@ static int halton_setup(Renderer* R, const pbrtx_render_desc* d) {
     RCHK(hipStreamSynchronize(st));
     slots.release();
     R->P.nx = K; R->P.ny = 1; R->P.spp = K;
+    R->P.div = cam_div(R->P);
     R->P.dx = 1.0f / (float)K; R->P.dy = 1.0f;
     R->P.spos = R->spos.p;
     R->P.scount = R->scount.p;
@@ -2001,6 +2007,7 @@ static int renderer_setup(Renderer* R, const pbrtx_render_desc* d) {
         const uint32_t spp = next_pow2(d->nx * d->ny);
         if ((uint64_t)d->xres * d->yres * spp >= (1ull << 40)) return fail(PBRTX_ERR_ARG, "image too large");
         R->P.nx = spp; R->P.ny = 1; R->P.spp = spp;
+        R->P.div = cam_div(R->P);
         R->P.dx = 1.0f / (float)spp; R->P.dy = 1.0f;
         const uint32_t npix = d->xres * d->yres;
         ICHK(R->spos.ensure((size_t)npix * spp));

@@ -57,6 +57,7 @@ struct RenderParams {
     uint32_t xres, yres, nx, ny, spp, seed;
     uint32_t n_point, n_area, nlights, light_samples, max_depth, rr_start, S;
     float dx, dy;
+    CamDiv div;
     const FaceShade* faces;
     const MatRec* mats;
     const AreaTriRec* atris;

@@ -354,7 +354,7 @@ __device__ __forceinline__ bool cq_fast_ray(const RayState& r) {
     return m <= CQ_FAST_LIM && fmaxf(fabsf(r.oy), fabsf(r.oz)) <= CQ_FAST_LIM && r.tmin == r.tmin &&
            r.tmax == r.tmax;
 }
-__device__ __forceinline__ bool cq_fast_scene(const SceneView& sv) {
+__host__ __device__ __forceinline__ bool cq_fast_scene(const SceneView& sv) {
     float m = 0.0f;
     for (int a = 0; a < 3; ++a) m = fmaxf(m, fmaxf(fabsf(sv.root_lo[a]), fabsf(sv.root_hi[a])));
     return m <= CQ_FAST_LIM;  // false for a NaN bound as well
@@ -1289,6 +1289,7 @@ __global__ __launch_bounds__(CL_BLOCK) __attribute__((amdgpu_waves_per_eu(6))) v
 
 constexpr int PSTK = 96;  // stack entries per wave of the packet closest-hit kernel below
 constexpr int PWAVES = MAX_BLOCK / 64;
+constexpr int PHITS = 256;  // hits a wave of it collects before it claims a run of the hit list
 
 // Read-only scene data seen through the constant address space: a load from
 // a wave-uniform address then goes through the scalar cache (s_load) rather
@@ -1319,54 +1320,110 @@ __device__ __forceinline__ float4 cload4(const void* p, uint32_t k) {
 // here instead of read (no ray array; only the hits are written).
 // co.list (GEN, a frame's bounce 0 of path tracing): a camera ray that
 // misses ends its path here -- zero radiance written to co.miss[i], no hit
-// record -- and each packet's hits take a run of co.list (their sample
-// indices) with one atomic on co.count.
+// record -- and the wave collects the sample indices of its hits in LDS and
+// moves them to a run of co.list, with one atomic on co.count per PHITS - 64
+// or more of them (and one at its end): an atomic per packet, all on one
+// address, cost 0.7 ms of 3.9 on the 1920x1080x64 path-tracing frame.
+//
+// What bounds it: VALU issue.  A packet of that frame visits 5.9 records and
+// 1.3 leaves; it took 1440 VALU instructions at first, 860 now, and the kernel
+// 4.19 ms, 3.13 now (1024x1024x16 direct lighting: 2870 -> 1770 and 1.38 ->
+// 1.24 ms; 512x512x1: 120 -> 98 us).  What went: plane selects (the loads'
+// addresses carry the signs instead), a branch and a ballot of a branch's
+// result per slot (all lanes test all slots, masked after), the divisions of
+// CamDiv, and arguments moved between SGPRs and VGPR lanes (PacketArgs).
+// Tried and no faster: the stack in the lanes of three VGPRs (v_writelane /
+// v_readlane) instead of LDS: 1.22 -> 1.40 ms on direct lighting; the waves'
+// columns shifted from turn to turn for balance: 3.91 -> 3.85 ms on path
+// tracing but 1.24 -> 1.30 on direct lighting.
+struct PacketArgs {
+    SceneView sv;
+    Ray* rays;
+    const uint32_t* n_dev;
+    Hit* hits;
+    uint32_t* counter;
+    uint32_t* err;
+    uint32_t n_host;
+    CamParams cam;
+    CamTable ct;
+    CamOut co;
+    double rntx;        // tiles: 1 / tiles per row
+    uint32_t fast_scene;  // cq_fast_scene(sv)
+};
+typedef __attribute__((address_space(4))) const PacketArgs PacketArgsK;
+
 template <bool GEN, bool SEGS = false>
-__global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) void k_closest_packet(SceneView sv, Ray* rays, uint32_t n_host,
-                                                              const uint32_t* n_dev, Hit* hits, uint32_t* counter,
-                                                              uint32_t* err, CamParams cam, CamTable ct, CamOut co) {
-    const uint32_t n = n_dev ? *n_dev : n_host;
+__global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) void k_closest_packet(PacketArgs) {
+    // The arguments, read where they are used: as ordinary parameters they
+    // are loaded once, outlast the SGPRs and are moved to and from VGPR lanes
+    // around every use.  The empty asm keeps a load from being hoisted.
+    auto args = []() {
+        PacketArgsK* a = (PacketArgsK*)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(a));
+        return a;
+    };
     __shared__ int32_t s_ref[PWAVES][PSTK];
     __shared__ unsigned long long s_msk[PWAVES][PSTK];
-    const bool fast_scene = cq_fast_scene(sv);  // planes within 2^40: slab_ord may apply
+    __shared__ uint32_t s_hit[GEN && !SEGS ? PWAVES : 1][GEN && !SEGS ? PHITS : 1];
+    uint32_t nhit = 0;  // of them in s_hit
     const uint32_t lane = __lane_id();
-    const uint32_t w = threadIdx.x >> 6;
+    const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // GEN (camera rays, their count known at launch): a fixed schedule with
     // no shared counter.  Packets go in runs of CAM_RUN to the 8 XCDs in turn
     // (blocks are dealt to the XCDs in turn), and an XCD's waves take its
     // packets in turn: neighbouring pixels share an L2, and every XCD gets
     // a share of every part of the image.  Otherwise waves claim packets
     // from the launch's counter.
+    // the wave's hits so far to a run of co.list
+    auto flush = [&]() {
+        PacketArgsK* A = args();
+        uint32_t b = 0;
+        if (lane == 0) b = atomicAdd(A->co.count, nhit);
+        b = __builtin_amdgcn_readfirstlane(b);
+        uint32_t* to = A->co.list + b;
+        for (uint32_t j = lane; j < nhit; j += 64u) to[j] = s_hit[w][j];
+        nhit = 0;
+    };
     const uint32_t wpb = blockDim.x >> 6;
     const uint32_t nxcd = (gridDim.x % 8u == 0u) ? 8u : 1u;
-    const uint64_t npk = ((uint64_t)n + 63u) / 64u;
     const uint32_t xcd = blockIdx.x % nxcd;
     const uint32_t wstride = (gridDim.x / nxcd) * wpb;
-    uint64_t k = (uint64_t)(blockIdx.x / nxcd) * wpb + w;  // this wave's next packet among its XCD's
+    uint32_t k = (blockIdx.x / nxcd) * wpb + w;  // this wave's next packet among its XCD's
+    uint32_t n;
+    {
+        PacketArgsK* A = args();
+        n = __builtin_amdgcn_readfirstlane(A->n_dev ? *A->n_dev : A->n_host);
+    }
     while (true) {
+        PacketArgsK* A = args();
         uint32_t base = 0;
         if constexpr (GEN) {
-            const uint64_t pk = (k / CAM_RUN * nxcd + xcd) * CAM_RUN + k % CAM_RUN;
-            if (pk >= npk) break;
-            base = (uint32_t)(pk * 64u);
+            const uint32_t pk = (k / CAM_RUN * nxcd + xcd) * CAM_RUN + k % CAM_RUN;
+            if (pk >= (uint32_t)(((uint64_t)n + 63u) / 64u)) break;
+            base = pk * 64u;
             k += wstride;
         } else {
-            if (lane == 0) base = atomicAdd(counter, 64u);
+            if (lane == 0) base = atomicAdd(A->counter, 64u);
             base = __builtin_amdgcn_readfirstlane(__shfl(base, 0));
             if (base >= n) break;
         }
+        const CamParams& cam = *(const CamParams*)&A->cam;
         uint32_t i = base + lane;
-        if (GEN && cam.tile_lw != 0xFFu) {
+        const bool tiles = GEN && !SEGS && cam.tile_lw != 0xFFu;
+        uint32_t px = 0, py = 0, ps = 0;  // tiles: the pixel (in the launch's rows) and its sample
+        if (tiles) {
             // the packet is a tile of 64 / spp pixels, tile_w wide, all their
             // samples (whole rows of tiles: the launch covers whole rows)
             const uint32_t tw = 1u << cam.tile_lw;
-            const uint32_t th_l = 6u - cam.spp_l - cam.tile_lw;
-            const uint32_t ntx = cam.xres >> cam.tile_lw;
+            const uint32_t th_l = 6u - cam.div.spp_l - cam.tile_lw;
             const uint32_t tile = base >> 6;
-            const uint32_t tx = tile % ntx, ty = tile / ntx;
-            const uint32_t q = lane >> cam.spp_l, sidx = lane & ((1u << cam.spp_l) - 1u);
-            const uint32_t x = (tx << cam.tile_lw) + (q & (tw - 1u)), y = (ty << th_l) + (q >> cam.tile_lw);
-            i = ((y * cam.xres + x) << cam.spp_l) + sidx;
+            const uint32_t ty = __builtin_amdgcn_readfirstlane((uint32_t)(((double)tile + 0.5) * A->rntx));
+            const uint32_t tx = tile - ty * (cam.xres >> cam.tile_lw);
+            const uint32_t q = lane >> cam.div.spp_l;
+            ps = lane & (cam.spp - 1u);
+            px = (tx << cam.tile_lw) + (q & (tw - 1u));
+            py = (ty << th_l) + (q >> cam.tile_lw);
+            i = ((py * cam.xres + px) << cam.div.spp_l) + ps;
         }
         const bool valid = i < n;
         RayState r{};
@@ -1375,6 +1432,7 @@ __global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) 
         if (GEN && SEGS) {
             // several cameras: each distinct segment of the packet in turn,
             // its camera read with scalar loads
+            const CamTable ct = *(const CamTable*)&A->ct;
             const uint32_t sidx = valid ? cam_seg_of(ct.segs, ct.nsegs, i) : 0u;
             unsigned long long pend = __ballot(valid);
             while (pend) {
@@ -1394,78 +1452,99 @@ __global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) 
             if constexpr (GEN) {
                 if (!SEGS) {
                     Ray g;
-                    camera_ray_of(cam, cam.g0 + i, &g);
+                    if (tiles) camera_ray_at(cam, px, cam.row0 + py, ps, &g);
+                    else camera_ray_of(cam, cam.g0 + i, &g);
                     set_ray(g, r);
                 }
             } else {
-                load_ray(rays, i, r);
+                load_ray(A->rays, i, r);
             }
             negm = (r.ix < 0.0f ? 1u : 0u) | (r.iy < 0.0f ? 2u : 0u) | (r.iz < 0.0f ? 4u : 0u);
+        }
+        const SceneView& sv = *(const SceneView*)&A->sv;
+        if (valid) {
             float tn;
             alive = slab(sv.root_lo[0], sv.root_hi[0], sv.root_lo[1], sv.root_hi[1], sv.root_lo[2],
                          sv.root_hi[2], r.ox, r.oy, r.oz, r.ix, r.iy, r.iz, r.tmin, r.tmax, &tn);
         }
+        const QNode* const qnodes = sv.qnodes;
+        const PrimRec64* const prims64 = sv.prims64;
+        const int32_t qroot = sv.qroot;
         uint32_t hprim = NO_HIT;
         float hb1 = 0.0f, hb2 = 0.0f;
+        const bool fast_scene = A->fast_scene != 0u;  // planes within 2^40: slab_ord may apply
         const unsigned long long alive_m = __ballot(alive);
-        // lanes that may not take the sign-ordered box test (slab_ord)
-        const unsigned long long slow_m = __ballot(alive && !cq_fast_ray(r));
-        unsigned long long todo = __ballot(valid);
+        // Lanes that may not take the sign-ordered box test (slab_ord).  With
+        // some |1/d| > 0 that test also fails on an empty slot's planes
+        // (FLT_MAX, -FLT_MAX: the near one lies past the far one), so the fast
+        // path needs no check of the refs.
+        const unsigned long long slow_m =
+            __ballot(alive && !(cq_fast_ray(r) && fmaxf(fmaxf(fabsf(r.ix), fabsf(r.iy)), fabsf(r.iz)) > 0.0f));
+        unsigned long long todo = alive_m;
         while (todo) {
-            // the next group: lanes with the signs of the first remaining lane
+            // the next group: the live lanes with the signs of the first of them
             const uint32_t lead = (uint32_t)__builtin_ctzll(todo);
-            const uint32_t g = __builtin_amdgcn_readfirstlane(__shfl(negm, (int)lead));
-            const unsigned long long grp = __ballot(valid && negm == g) & todo;
-            todo &= ~grp;
-            const unsigned long long live = grp & alive_m;
-            if (!live) continue;
+            const uint32_t g = (uint32_t)__builtin_amdgcn_readlane((int)negm, (int)lead);
+            const unsigned long long live = __ballot(negm == g) & todo;
+            todo &= ~live;
             const bool gfast = fast_scene && (live & slow_m) == 0ull;
+            const uint32_t gx = g & 1u, gy = (g >> 1) & 1u, gz = (g >> 2) & 1u;
             int sp = 0;
-            int32_t cur = sv.qroot;
+            int32_t cur = qroot;
             unsigned long long cm = live;  // lanes that reached the current entry
             while (true) {
-                const bool act = (cm >> lane) & 1ull;
                 if (cur >= 0) {
-                    const QNode* q = sv.qnodes + cur;
-                    const float4 LX = cload4(q, 0), HX = cload4(q, 1), LY = cload4(q, 2), HY = cload4(q, 3),
-                                 LZ = cload4(q, 4), HZ = cload4(q, 5), R6 = cload4(q, 6);
+                    const QNode* q = qnodes + cur;
+                    const float4 R6 = cload4(q, 6);
                     const uint32_t meta = as_u(cload4(q, 7).x);
                     int32_t r0 = (int32_t)as_u(R6.x), r1 = (int32_t)as_u(R6.y), r2 = (int32_t)as_u(R6.z),
                             r3 = (int32_t)as_u(R6.w);
-                    bool p0, p1, p2, p3;
+                    // Every lane tests every slot, without branches, and the
+                    // lanes and slots that do not count are masked out of the
+                    // ballots.
+                    unsigned long long m0, m1, m2, m3;
                     if (gfast) {
-                        // planes ordered by the group's signs (wave-uniform selects)
-                        const float4 NX = (g & 1u) ? HX : LX, FX = (g & 1u) ? LX : HX;
-                        const float4 NY = (g & 2u) ? HY : LY, FY = (g & 2u) ? LY : HY;
-                        const float4 NZ = (g & 4u) ? HZ : LZ, FZ = (g & 4u) ? LZ : HZ;
-                        p0 = act && r0 != QEMPTY && slab_ord(NX.x, FX.x, NY.x, FY.x, NZ.x, FZ.x, r.ox, r.oy, r.oz,
-                                                             r.ix, r.iy, r.iz, r.tmin, r.tmax);
-                        p1 = act && r1 != QEMPTY && slab_ord(NX.y, FX.y, NY.y, FY.y, NZ.y, FZ.y, r.ox, r.oy, r.oz,
-                                                             r.ix, r.iy, r.iz, r.tmin, r.tmax);
-                        p2 = act && r2 != QEMPTY && slab_ord(NX.z, FX.z, NY.z, FY.z, NZ.z, FZ.z, r.ox, r.oy, r.oz,
-                                                             r.ix, r.iy, r.iz, r.tmin, r.tmax);
-                        p3 = act && r3 != QEMPTY && slab_ord(NX.w, FX.w, NY.w, FY.w, NZ.w, FZ.w, r.ox, r.oy, r.oz,
-                                                             r.ix, r.iy, r.iz, r.tmin, r.tmax);
+                        // planes ordered by the group's signs: the loads' addresses
+                        const float4 NX = cload4(q, gx), FX = cload4(q, 1u - gx), NY = cload4(q, 2u + gy),
+                                     FY = cload4(q, 3u - gy), NZ = cload4(q, 4u + gz), FZ = cload4(q, 5u - gz);
+                        m0 = __builtin_amdgcn_ballot_w64(slab_ord(NX.x, FX.x, NY.x, FY.x, NZ.x, FZ.x, r.ox, r.oy, r.oz,
+                                                                  r.ix, r.iy, r.iz, r.tmin, r.tmax));
+                        m1 = __builtin_amdgcn_ballot_w64(slab_ord(NX.y, FX.y, NY.y, FY.y, NZ.y, FZ.y, r.ox, r.oy, r.oz,
+                                                                  r.ix, r.iy, r.iz, r.tmin, r.tmax));
+                        m2 = __builtin_amdgcn_ballot_w64(slab_ord(NX.z, FX.z, NY.z, FY.z, NZ.z, FZ.z, r.ox, r.oy, r.oz,
+                                                                  r.ix, r.iy, r.iz, r.tmin, r.tmax));
+                        m3 = __builtin_amdgcn_ballot_w64(slab_ord(NX.w, FX.w, NY.w, FY.w, NZ.w, FZ.w, r.ox, r.oy, r.oz,
+                                                                  r.ix, r.iy, r.iz, r.tmin, r.tmax));
                     } else {
+                        const float4 LX = cload4(q, 0), HX = cload4(q, 1), LY = cload4(q, 2), HY = cload4(q, 3),
+                                     LZ = cload4(q, 4), HZ = cload4(q, 5);
                         float t;
-                        p0 = act && r0 != QEMPTY && slab(LX.x, HX.x, LY.x, HY.x, LZ.x, HZ.x, r.ox, r.oy, r.oz,
-                                                         r.ix, r.iy, r.iz, r.tmin, r.tmax, &t);
-                        p1 = act && r1 != QEMPTY && slab(LX.y, HX.y, LY.y, HY.y, LZ.y, HZ.y, r.ox, r.oy, r.oz,
-                                                         r.ix, r.iy, r.iz, r.tmin, r.tmax, &t);
-                        p2 = act && r2 != QEMPTY && slab(LX.z, HX.z, LY.z, HY.z, LZ.z, HZ.z, r.ox, r.oy, r.oz,
-                                                         r.ix, r.iy, r.iz, r.tmin, r.tmax, &t);
-                        p3 = act && r3 != QEMPTY && slab(LX.w, HX.w, LY.w, HY.w, LZ.w, HZ.w, r.ox, r.oy, r.oz,
-                                                         r.ix, r.iy, r.iz, r.tmin, r.tmax, &t);
+                        m0 = __builtin_amdgcn_ballot_w64(slab(LX.x, HX.x, LY.x, HY.x, LZ.x, HZ.x, r.ox, r.oy, r.oz,
+                                                              r.ix, r.iy, r.iz, r.tmin, r.tmax, &t));
+                        m1 = __builtin_amdgcn_ballot_w64(slab(LX.y, HX.y, LY.y, HY.y, LZ.y, HZ.y, r.ox, r.oy, r.oz,
+                                                              r.ix, r.iy, r.iz, r.tmin, r.tmax, &t));
+                        m2 = __builtin_amdgcn_ballot_w64(slab(LX.z, HX.z, LY.z, HY.z, LZ.z, HZ.z, r.ox, r.oy, r.oz,
+                                                              r.ix, r.iy, r.iz, r.tmin, r.tmax, &t));
+                        m3 = __builtin_amdgcn_ballot_w64(slab(LX.w, HX.w, LY.w, HY.w, LZ.w, HZ.w, r.ox, r.oy, r.oz,
+                                                              r.ix, r.iy, r.iz, r.tmin, r.tmax, &t));
+                        m0 = r0 != QEMPTY ? m0 : 0ull;
+                        m1 = r1 != QEMPTY ? m1 : 0ull;
+                        m2 = r2 != QEMPTY ? m2 : 0ull;
+                        m3 = r3 != QEMPTY ? m3 : 0ull;
                     }
-                    unsigned long long m0 = __ballot(p0), m1 = __ballot(p1), m2 = __ballot(p2), m3 = __ballot(p3);
+                    m0 &= cm;
+                    m1 &= cm;
+                    m2 &= cm;
+                    m3 &= cm;
                     // the group's visiting order: near half first, near child first
                     const bool nA = (g >> (meta & 3u)) & 1u;
                     const bool nB = (g >> ((meta >> 2) & 3u)) & 1u;
                     const bool nC = (g >> ((meta >> 4) & 3u)) & 1u;
 #define PX_SWAP2(C, I, J)                                                                \
-    if (C) {                                                                              \
-        const unsigned long long mb = m##I; m##I = m##J; m##J = mb;                       \
-        const int32_t rb = r##I; r##I = r##J; r##J = rb;                                  \
+    {                                                                                     \
+        const unsigned long long ma = C ? m##J : m##I, mb = C ? m##I : m##J;              \
+        const int32_t ra = C ? r##J : r##I, rb = C ? r##I : r##J;                         \
+        m##I = ma; m##J = mb; r##I = ra; r##J = rb;                                       \
     }
                     PX_SWAP2(nB, 0, 1)
                     PX_SWAP2(nC, 2, 3)
@@ -1480,7 +1559,7 @@ __global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) 
     if (m##K) {                                                                           \
         if (pend) {                                                                       \
             if (sp < PSTK) { s_ref[w][sp] = pref; s_msk[w][sp] = pm; ++sp; }              \
-            else atomicOr(err, 1u);                                                       \
+            else atomicOr(args()->err, 1u);                                                       \
         }                                                                                 \
         pend = true; pref = r##K; pm = m##K;                                              \
     }
@@ -1498,19 +1577,24 @@ __global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) 
                     // leaf: the reference's pop-time box test at each lane's
                     // tmax, then its prims in order until the record flagged last
                     uint32_t pos = (uint32_t)(~cur);
-                    const PrimRec64* pr = sv.prims64 + pos;
+                    const PrimRec64* pr = prims64 + pos;
                     float4 c = cload4(pr, 2), d = cload4(pr, 3);
-                    bool go;
+                    unsigned long long gm;
                     if (gfast) {
-                        go = act && slab_ord((g & 1u) ? d.x : c.y, (g & 1u) ? c.y : d.x, (g & 2u) ? d.y : c.z,
-                                             (g & 2u) ? c.z : d.y, (g & 4u) ? d.z : c.w, (g & 4u) ? c.w : d.z,
-                                             r.ox, r.oy, r.oz, r.ix, r.iy, r.iz, r.tmin, r.tmax);
+                        // w[9..14]: lo xyz, hi xyz
+                        cfloat* bx = (cfloat*)pr + 9;
+                        gm = __builtin_amdgcn_ballot_w64(
+                            slab_ord(bx[3u * gx], bx[3u - 3u * gx], bx[1u + 3u * gy], bx[4u - 3u * gy],
+                                     bx[2u + 3u * gz], bx[5u - 3u * gz], r.ox, r.oy, r.oz, r.ix, r.iy, r.iz, r.tmin,
+                                     r.tmax));
                     } else {
                         float tn;
-                        go = act && slab(c.y, d.x, c.z, d.y, c.w, d.z, r.ox, r.oy, r.oz, r.ix, r.iy, r.iz, r.tmin,
-                                         r.tmax, &tn);
+                        gm = __builtin_amdgcn_ballot_w64(slab(c.y, d.x, c.z, d.y, c.w, d.z, r.ox, r.oy, r.oz, r.ix,
+                                                              r.iy, r.iz, r.tmin, r.tmax, &tn));
                     }
-                    if (__ballot(go)) {
+                    gm &= cm;
+                    if (gm) {
+                        const bool go = (gm >> lane) & 1ull;
                         while (true) {
                             const float4 a = cload4(pr, 0), b = cload4(pr, 1);
                             const uint32_t kind = as_u(d.w);
@@ -1518,7 +1602,7 @@ __global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) 
                                 float tt, u = 0.0f, v = 0.0f;
                                 bool h;
                                 if ((kind & 0xFFu) == 0u) h = tri_test(a, b, c, r, &tt, &u, &v);
-                                else h = sphere_test(sv.spheres[as_u(a.x)], r, &tt);
+                                else h = sphere_test(((const SphereRec*)args()->sv.spheres)[as_u(a.x)], r, &tt);
                                 if (h) { r.tmax = tt; hprim = pos; hb1 = u; hb2 = v; }
                             }
                             if (kind & 0x100u) break;
@@ -1532,27 +1616,29 @@ __global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) 
                 if (sp == 0) break;
                 --sp;
                 cur = __builtin_amdgcn_readfirstlane(s_ref[w][sp]);
-                cm = s_msk[w][sp];
+                const unsigned long long pm = s_msk[w][sp];
+                cm = (unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)pm) |
+                     (unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(pm >> 32)) << 32;
             }
         }
+        A = args();
+        const CamOut co = *(const CamOut*)&A->co;
         if (valid) {
-            if (hprim != NO_HIT) hprim = sv.order[hprim];  // position -> prim id
+            if (hprim != NO_HIT) hprim = A->sv.order[hprim];  // position -> prim id
             if (GEN && co.list && hprim == NO_HIT) co.miss[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            else hits[i] = Hit{hprim, hprim != NO_HIT ? r.tmax : 0.0f, hb1, hb2};
-            if (!GEN && hprim != NO_HIT) rays[i].tmax = r.tmax;
+            else A->hits[i] = Hit{hprim, hprim != NO_HIT ? r.tmax : 0.0f, hb1, hb2};
+            if (!GEN && hprim != NO_HIT) A->rays[i].tmax = r.tmax;
         }
-        if (GEN && co.list) {
+        if (GEN && !SEGS && co.list) {
             const bool h = valid && hprim != NO_HIT;
             const unsigned long long hm = __ballot(h);
-            if (hm) {
-                uint32_t b = 0;
-                if (lane == 0) b = atomicAdd(co.count, (uint32_t)__popcll(hm));
-                b = __builtin_amdgcn_readfirstlane(__shfl(b, 0));
-                const unsigned long long lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-                if (h) co.list[b + (uint32_t)__popcll(hm & lt)] = i;
-            }
+            const unsigned long long lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+            if (h) s_hit[w][nhit + (uint32_t)__popcll(hm & lt)] = i;
+            nhit += (uint32_t)__popcll(hm);
+            if (nhit > (uint32_t)(PHITS - 64)) flush();
         }
     }
+    if (GEN && !SEGS && nhit) flush();
 }
 
 __global__ void k_fill_u32(uint32_t* p, uint32_t v, size_t n) {
@@ -1918,7 +2004,8 @@ static hipError_t launch(const SceneView& s, Ray* rays, uint32_t n, Hit* hits, u
         hipError_t e = fill_u32(scr->counter, 0u, 1, st);
         if (e != hipSuccess) return e;
         hipLaunchKernelGGL(k_closest_packet<false>, dim3(wide_grid(k_closest_packet<false>, tun)), dim3(block), 0,
-                           st, s, rays, n, n_dev, hits, scr->counter, err, CamParams{}, CamTable{}, CamOut{});
+                           st, PacketArgs{s, rays, n_dev, hits, scr->counter, err, n, CamParams{}, CamTable{}, CamOut{}, 0.0,
+                                      cq_fast_scene(s) ? 1u : 0u});
         return hipGetLastError();
     }
     if (!stack_supported(tun.stack)) return hipErrorInvalidValue;
@@ -2045,19 +2132,20 @@ hipError_t trace_camera(const SceneView& s, const CamParams& cam, uint32_t n, Hi
         if (cam.g0 % row == 0 && n % row == 0 && (cam.xres & ((1u << wl) - 1u)) == 0 &&
             ((n / row) & ((1u << hl) - 1u)) == 0) {
             c.tile_lw = wl;
-            c.spp_l = sl;
+            c.row0 = (uint32_t)(cam.g0 / row);
         }
     }
+    const PacketArgs args{s,       nullptr, nullptr, hits, scr->counter, scr->counter + 1, n, c, ct ? *ct : CamTable{},
+                          co ? *co : CamOut{}, c.tile_lw != 0xFFu ? 1.0 / (double)(c.xres >> c.tile_lw) : 0.0,
+                          cq_fast_scene(s) ? 1u : 0u};
     // several cameras: their own instance, so that the single-camera kernel
     // keeps its registers
     if (ct)
         hipLaunchKernelGGL((k_closest_packet<true, true>), dim3(wide_grid(k_closest_packet<true, true>, tun)),
-                           dim3(block), 0, st, s, (Ray*)nullptr, n, (const uint32_t*)nullptr, hits, scr->counter,
-                           scr->counter + 1, c, *ct, CamOut{});
+                           dim3(block), 0, st, args);
     else
         hipLaunchKernelGGL((k_closest_packet<true, false>), dim3(wide_grid(k_closest_packet<true, false>, tun)),
-                           dim3(block), 0, st, s, (Ray*)nullptr, n, (const uint32_t*)nullptr, hits, scr->counter,
-                           scr->counter + 1, c, CamTable{}, co ? *co : CamOut{});
+                           dim3(block), 0, st, args);
     return hipGetLastError();
 }
 
