@@ -402,7 +402,28 @@ __device__ __forceinline__ bool prim_test64(const SceneView& sv, uint32_t pos, c
     return hit;
 }
 
-constexpr uint32_t LEAF_WAIT_PCT = 25;
+// The per-ray kernel's leaves.  A step that some lane spends on a leaf costs
+// the whole wave the leaf code, so a lane that reaches a leaf puts it aside
+// and walks on; it waits only at a second one, and the wave takes all the
+// leaves put aside when LEAF_WAIT_PCT % of its tracing lanes wait.  Occlusion
+// does not depend on the order.  For the closest hit the leaves still come in
+// visiting order, and the records visited meanwhile are tested against a tmax
+// no smaller than the reference's, so that they can only lead to more leaves,
+// whose exact boxes are tested at the tmax of their turn.  (After a hit at t =
+// NaN that would not hold: tmax may rise again.  Such a ray starts over and
+// tests nothing early.)
+// Lanes busy per VALU instruction: 49 -> 57 % (occlusion of the 1024x1024x16
+// direct-lighting frame, 3.05 -> 2.82 ms; 4M random rays in 1M triangles: 2.62
+// -> 2.53 ms closest hit), against leaves taken at 25 % of lanes waiting at
+// their first one (no waiting: 3.87 ms; 15 %: 3.52, 35 %: 3.52, 50 %: 3.62,
+// when 25 % took 3.45).  With a leaf put aside: 1 % 3.06 ms, 5 % 2.91, 10 %
+// 2.82, 25 % 2.87, 40 % 3.01, 60 % 3.26; also as soon as half or 70 % of the
+// lanes hold a leaf: 2.83.  Tried and slower: each leaf reached put in a
+// per-wave queue in LDS and the whole wave taking 64 queued leaves at a time,
+// one per lane, on rays read across lanes (exact, but 3.19 -> 3.58-3.78 ms: a
+// round lasts as long as its largest leaf, and lanes whose rays wait on
+// queued leaves idle).
+constexpr uint32_t LEAF_WAIT_PCT = 10;
 
 // SEG: the rays come from a segment table (served launch) instead of one array.
 // CQ: the compressed records (CNode, PrimRec64) instead of QNode / PrimRec.
@@ -488,8 +509,9 @@ __global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) 
     uint32_t rid = 0, hprim = NO_HIT;
     uint32_t rseg = 0;  // SEG: segment of the ray; rid is then its index in the segment
     float hb1 = 0.0f, hb2 = 0.0f;
-    int32_t cur = 0;
-    bool have_cur = false;  // false: take the next stack entry
+    int32_t cur = QEMPTY;  // the entry to visit; QEMPTY: take the next from the stack
+    int32_t lf = 0;        // < 0: a leaf put aside (see below)
+    bool one = false;      // closest hit: after a hit at t = NaN, nothing is tested early
     int sp = 0;
     bool has = false, drained = false;
     // CQ: this ray, and every busy ray of the wave, may take the ray-space
@@ -563,12 +585,13 @@ __global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) 
                     negm = (neg0 ? 1u : 0u) | (neg1 ? 2u : 0u) | (neg2 ? 4u : 0u);
                     hprim = NO_HIT; hb1 = 0.0f; hb2 = 0.0f;
                     sp = 0;
+                    if (!ANY && CQ) one = r.tmax != r.tmax;
                     float tn;
                     // the root's own box (popped first by the reference)
-                    have_cur = slab(sv.root_lo[0], sv.root_hi[0], sv.root_lo[1], sv.root_hi[1],
-                                    sv.root_lo[2], sv.root_hi[2], r.ox, r.oy, r.oz, r.ix, r.iy, r.iz,
-                                    r.tmin, r.tmax, &tn);
-                    cur = (ANY && CQ) ? sv.ocroot : sv.qroot;
+                    const bool in = slab(sv.root_lo[0], sv.root_hi[0], sv.root_lo[1], sv.root_hi[1],
+                                         sv.root_lo[2], sv.root_hi[2], r.ox, r.oy, r.oz, r.ix, r.iy, r.iz,
+                                         r.tmin, r.tmax, &tn);
+                    cur = in ? ((ANY && CQ) ? sv.ocroot : sv.qroot) : QEMPTY;
                     has = true;
                 } else {
                     drained = true;
@@ -580,8 +603,8 @@ __global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) 
             // hand the last rays over (see TailRec)
             if (tail.recs && (n <= tail.cap || (res_b == res_e && tries >= nparts &&
                                                 (uint32_t)__popcll(__ballot(has)) <= tail.lanes))) {
-                const int cnt = sp + (have_cur ? 1 : 0);
-                const unsigned long long give = __ballot(has && cnt <= TAIL_STK);
+                const int cnt = sp + (cur != QEMPTY ? 1 : 0) + (lf < 0 ? 1 : 0);
+                const unsigned long long give = __ballot(has && cnt <= TAIL_STK && !one);
                 if (give) {
                     uint32_t b = 0;
                     if (lane == 0) b = atomicAdd(tail.count, (uint32_t)__popcll(give));
@@ -598,8 +621,11 @@ __global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) 
                                 to[k] = make_int2((int)e.x, (int)e.y);
                             }
                         }
-                        if (have_cur) to[sp] = make_int2(cur, (int)0xFF800000u);
+                        if (cur != QEMPTY) to[sp] = make_int2(cur, (int)0xFF800000u);
+                        if (lf < 0) to[cnt - 1] = make_int2(lf, (int)0xFF800000u);
                         has = false;
+                        cur = QEMPTY;
+                        lf = 0;
                     }
                 }
                 if (!__any(has)) continue;
@@ -607,22 +633,34 @@ __global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) 
         }
         if (CQ) wfast = fast_scene && __ballot(has && !fastr) == 0ull;
         // ---- traverse until too few lanes are busy
-        while (has) {
-            if (!have_cur) {
-                while (sp > 0) {
-                    --sp;
-                    int32_t ref;
-                    float tn = 0.0f;
-                    if (sp < STK_WIDE) {
-                        ref = s_ref[sp][tid];
-                        if (!ANY) tn = s_tn[sp][tid];
-                    } else {
-                        const uint2 e = spill[(size_t)(sp - STK_WIDE) * total + gtid];
-                        ref = (int32_t)e.x; tn = as_f(e.y);
+        while (true) {
+            if (has) {
+                // The next entry, a leaf reached put aside (LEAF_WAIT_PCT);
+                // without leaf boxes (CQ false), and after a hit at t = NaN,
+                // that leaf is taken first.
+                while (true) {
+                    if (cur == QEMPTY) {
+                        if (lf < 0 && (!CQ || one)) break;
+                        while (sp > 0) {
+                            --sp;
+                            int32_t ref;
+                            float tn = 0.0f;
+                            if (sp < STK_WIDE) {
+                                ref = s_ref[sp][tid];
+                                if (!ANY) tn = s_tn[sp][tid];
+                            } else {
+                                const uint2 e = spill[(size_t)(sp - STK_WIDE) * total + gtid];
+                                ref = (int32_t)e.x; tn = as_f(e.y);
+                            }
+                            if (ANY || one || tn <= r.tmax) { cur = ref; break; }
+                        }
+                        if (cur == QEMPTY) break;
                     }
-                    if (ANY || tn <= r.tmax) { cur = ref; have_cur = true; break; }
+                    if (cur >= 0 || lf < 0) break;
+                    lf = cur;
+                    cur = QEMPTY;
                 }
-                if (!have_cur) {
+                if (cur == QEMPTY && lf >= 0) {
                     // ray finished
                     if (ANY && occ8) occ8[rid] = 0u;  // no hit
                     if (!ANY) {
@@ -635,27 +673,79 @@ __global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) 
                     has = false;
                 }
             }
-            // A lane at a leaf waits while fewer than LEAF_WAIT_PCT % of the
-            // wave's tracing lanes are at one (and some are at records): every
-            // step that some lane spends on a leaf costs the whole wave the
-            // leaf code, so leaves are taken in bunches.  On the 1024x1024
-            // direct-lighting frame, occlusion 3.87 -> 3.45 ms at 25 % (15 %:
-            // 3.52, 35 %: 3.52, 50 %: 3.62); the path-tracing frame gains too.
-            // Tried and slower there: no waiting, with each leaf reached put
-            // in a per-wave queue in LDS and the whole wave taking 64 queued
-            // leaves at a time, one per lane, on rays read across lanes
-            // (exact, but 3.19 -> 3.58-3.78 ms: a round lasts as long as its
-            // largest leaf, and lanes whose rays wait on queued leaves idle).
-            const unsigned long long at_rec = __ballot(has && cur >= 0);
-            const unsigned long long at_leaf = __ballot(has && cur < 0);
-            const bool leaf_now = at_rec == 0ull || (uint32_t)__popcll(at_leaf) * 100u >=
+            const unsigned long long at_rec = __builtin_amdgcn_ballot_w64(cur >= 0);
+            const unsigned long long at_leaf = __builtin_amdgcn_ballot_w64(lf < 0);
+            const bool leaf_now = at_rec == 0ull || (uint32_t)__popcll(at_leaf & ~at_rec) * 100u >=
                                                         LEAF_WAIT_PCT * (uint32_t)__popcll(at_leaf | at_rec);
-            if (has && cur >= 0) {
+            if (leaf_now && lf < 0) {
+                // leaf: prims in order until the record flagged last
+                uint32_t pos = (uint32_t)(~lf);
+                lf = 0;
+                bool hitnow = false;
+                if constexpr (CQ) {
+                    // the leaf's exact box at the current tmax: the reference's
+                    // pop-time test (the record boxes above it are wider)
+                    const float4* p = reinterpret_cast<const float4*>(sv.prims64 + pos);
+                    float4 P2 = p[2], P3 = p[3];
+                    float tn;
+                    if (slab(P2.y, P3.x, P2.z, P3.y, P2.w, P3.z, r.ox, r.oy, r.oz, r.ix, r.iy, r.iz, r.tmin, r.tmax,
+                             &tn)) {
+                        while (true) {
+                            const float4 P0 = p[0], P1 = p[1];
+                            const uint32_t kind = as_u(P3.w);
+                            if (prim_test64(sv, pos, P0, P1, P2, kind, r, &hprim, &hb1, &hb2)) {
+                                hitnow = true;
+                                if (ANY) break;
+                            }
+                            if (kind & 0x100u) break;
+                            ++pos;
+                            p += 4;
+                            P2 = p[2];
+                            P3 = p[3];
+                        }
+                    }
+                    if (!ANY && hitnow && r.tmax != r.tmax && !one) {
+                        // A hit at t = NaN: every later box passes, also those
+                        // left out since the leaf was put aside and, as tmax
+                        // may be a number again and larger, before: from the
+                        // root again, nothing tested early.
+                        one = true;
+                        r.tmax = (SEG ? segs[rseg].rays : rays)[rid].tmax;
+                        hprim = NO_HIT;
+                        hb1 = hb2 = 0.0f;
+                        sp = 0;
+                        cur = sv.qroot;
+                    }
+                } else {
+                    while (true) {
+                        bool last;
+                        if (prim_test(sv, pos, r, &hprim, &hb1, &hb2, &last)) {
+                            hitnow = true;
+                            if (ANY) break;
+                        }
+                        if (last) break;
+                        ++pos;
+                    }
+                }
+                if (ANY && hitnow) {
+                    if (occ8) {
+                        occ8[rid] = 1u;  // a byte per ray: one plain store, no atomic
+                    } else {
+                        uint32_t* ow = SEG ? segs[rseg].occ : occ;
+                        atomicOr(ow + (rid >> 5), 1u << (rid & 31u));
+                    }
+                    has = false;
+                    cur = QEMPTY;
+                    sp = 0;
+                }
+            }
+            if (cur >= 0) {
                 int4 RF;
                 uint32_t meta;
                 float t0, t1, t2, t3;
                 bool p0, p1, p2, p3;
                 if constexpr (CQ) {
+                    const float rtmax = !ANY && one ? __builtin_inff() : r.tmax;
                     // occlusion reads the order-free records
                     const float4* q = reinterpret_cast<const float4*>((ANY ? sv.ocnodes : sv.cnodes) + cur);
                     const float4 W0 = q[0], W1 = q[1], W2 = q[2], W3 = q[3];
@@ -678,7 +768,7 @@ __global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) 
 // instructions per axis they save.  The same form in the camera packet
 // kernel was slower (1.355 -> 1.39 ms on that frame's camera rays).
 #define PX_CQ_SLOT(K, I, P, T) \
-    P = (RF.K != QEMPTY) & slab_ray(nqx, fqx, nqy, fqy, nqz, fqz, I, X, Y, Z, r.tmin, r.tmax, &T);
+    P = (RF.K != QEMPTY) & slab_ray(nqx, fqx, nqy, fqy, nqz, fqz, I, X, Y, Z, r.tmin, rtmax, &T);
                         PX_CQ_SLOT(x, 0, p0, t0)
                         PX_CQ_SLOT(y, 1, p1, t1)
                         PX_CQ_SLOT(z, 2, p2, t2)
@@ -691,7 +781,7 @@ __global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) 
     P = RF.K != QEMPTY &&                                                                                     \
         slab_signed(cq_bound(nqx, I, W0.x, sx), cq_bound(fqx, I, W0.x, sx), cq_bound(nqy, I, W0.y, sy),       \
                     cq_bound(fqy, I, W0.y, sy), cq_bound(nqz, I, W0.z, sz), cq_bound(fqz, I, W0.z, sz), r.ox,  \
-                    r.oy, r.oz, r.ix, r.iy, r.iz, r.tmin, r.tmax, &T);
+                    r.oy, r.oz, r.ix, r.iy, r.iz, r.tmin, rtmax, &T);
                         PX_CQ_SLOT(x, 0, p0, t0)
                         PX_CQ_SLOT(y, 1, p1, t1)
                         PX_CQ_SLOT(z, 2, p2, t2)
@@ -725,9 +815,9 @@ __global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) 
                     s_ref[k][tid] = RF.z; k += p2 ? 1 : 0;
                     s_ref[k][tid] = RF.y; k += p1 ? 1 : 0;
                     s_ref[k][tid] = RF.x; k += p0 ? 1 : 0;
-                    have_cur = k > sp;
-                    cur = p0 ? RF.x : (p1 ? RF.y : (p2 ? RF.z : RF.w));
-                    sp = have_cur ? k - 1 : sp;
+                    const bool any = k > sp;
+                    cur = p0 ? RF.x : (p1 ? RF.y : (p2 ? RF.z : (p3 ? RF.w : QEMPTY)));
+                    sp = any ? k - 1 : sp;
                 } else {
                     // visiting order of the reference (bvh.rs:409-415 applied at A,
                     // then at B and C): near half first, near child first in each.
@@ -769,60 +859,12 @@ __global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) 
                     PX_VISIT(1)
                     PX_VISIT(0)
 #undef PX_VISIT
-                    have_cur = pend;
-                    cur = pref;
-                }
-            } else if (has && leaf_now) {
-                // leaf: prims in order until the record flagged last
-                uint32_t pos = (uint32_t)(~cur);
-                bool hitnow = false;
-                if constexpr (CQ) {
-                    // the leaf's exact box at the current tmax: the reference's
-                    // pop-time test (the record boxes above it are wider)
-                    const float4* p = reinterpret_cast<const float4*>(sv.prims64 + pos);
-                    float4 P2 = p[2], P3 = p[3];
-                    float tn;
-                    if (slab(P2.y, P3.x, P2.z, P3.y, P2.w, P3.z, r.ox, r.oy, r.oz, r.ix, r.iy, r.iz, r.tmin, r.tmax,
-                             &tn)) {
-                        while (true) {
-                            const float4 P0 = p[0], P1 = p[1];
-                            const uint32_t kind = as_u(P3.w);
-                            if (prim_test64(sv, pos, P0, P1, P2, kind, r, &hprim, &hb1, &hb2)) {
-                                hitnow = true;
-                                if (ANY) break;
-                            }
-                            if (kind & 0x100u) break;
-                            ++pos;
-                            p += 4;
-                            P2 = p[2];
-                            P3 = p[3];
-                        }
-                    }
-                } else {
-                    while (true) {
-                        bool last;
-                        if (prim_test(sv, pos, r, &hprim, &hb1, &hb2, &last)) {
-                            hitnow = true;
-                            if (ANY) break;
-                        }
-                        if (last) break;
-                        ++pos;
-                    }
-                }
-                have_cur = false;
-                if (ANY && hitnow) {
-                    if (occ8) {
-                        occ8[rid] = 1u;  // a byte per ray: one plain store, no atomic
-                    } else {
-                        uint32_t* ow = SEG ? segs[rseg].occ : occ;
-                        atomicOr(ow + (rid >> 5), 1u << (rid & 31u));
-                    }
-                    has = false;
+                    cur = pend ? pref : QEMPTY;
                 }
             }
             // leave to refill when the wave has gone sparse
             const unsigned long long busy = __ballot(has);
-            if ((uint32_t)__popcll(busy) * 100u < refill * 64u) break;
+            if (busy == 0ull || (uint32_t)__popcll(busy) * 100u < refill * 64u) break;
         }
     }
 }
