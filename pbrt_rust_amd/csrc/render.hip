@@ -447,9 +447,8 @@ __global__ void k_chunk_end(uint32_t* lo, uint32_t* hi, uint32_t* add, uint32_t*
         *add = 0u;
         *clr = 0u;
     }
-    parts[threadIdx.x] = 0u;
+    for (uint32_t i = threadIdx.x; i < TRACE_PART_WORDS; i += blockDim.x) parts[i] = 0u;
 }
-static_assert(TRACE_PART_WORDS == 64, "one wave clears them");
 
 // Adds nb bounces' shadow and extension rays to the running totals (two words
 // each) and clears the bounces' counters (render.hpp: BOUNCE_WORDS); more: the

@@ -430,21 +430,32 @@ constexpr uint32_t LEAF_WAIT_PCT = 10;
 // Camera-ray packets dealt to one XCD at a time (see k_closest_packet).
 constexpr uint32_t CAM_RUN = 16;
 
-// Work claims of the persistent per-ray kernel (see k_trace_wide): rays per
-// claim and counters (parts of the ray range), WIDE_PART_STRIDE words apart.
-// On the 1024x1024 direct-lighting frame's 26.5M shadow rays the occlusion
-// kernel took 6.7 ms with one counter and claims of exactly what idle lanes
-// needed, 5.2 ms with claims of 256, and 5.5 ms with claims of 256 from
-// eight per-XCD parts (faster on the path tracer's shadow rays, 3.4 -> 3.2
-// ms, slower on its extension rays): one part.
-constexpr uint32_t WIDE_CHUNK = 256;
-constexpr uint32_t WIDE_PARTS = 1;
+// Work claims of the persistent per-ray kernel (see k_trace_wide).  An atomic
+// on one address takes about 11 ns here, whoever asks, so one counter for 8192
+// waves is a queue of 90 us at a launch's start and another at its end, and
+// with claims of 64 rays bounds any launch of cheap rays (0.17 ns a ray).
+// Hence the first chunk of each wave by its place (launches of up to 2^19
+// rays claim nothing), then WIDE_PARTS counters WIDE_PART_STRIDE words apart,
+// one per XCD, each handing out every WIDE_PARTS-th chunk: the rays in flight
+// stay neighbours, as with one counter (contiguous parts, each XCD in its own
+// eighth of the rays, were slower).  That allows chunks of 64 rays, which
+// spread a costly stretch of rays over more waves than 256 did; from 32 rays
+// a lane on, 128.
+// One counter, claims of 64 below 8 rays a lane and else 256 -> this:
+// 480x270x16 path tracing (launches of 0.05 to 2M rays) 1.80 -> 1.31 ms,
+// 1920x1080x64 11.77 -> 11.20, 1024x1024x16 direct lighting 5.43 -> 5.26; 4M
+// random rays in 1M triangles 2.61 -> 2.30 ms closest hit, 1.45 -> 1.34
+// occlusion; 2M coherent ones 1.20 -> 0.98 and 1.04 -> 0.80.  Claims of 256:
+// 2.60 ms for those 4M closest hits; always 64: direct lighting 5.30-5.37.
+constexpr uint32_t WIDE_CHUNK = 128;
+constexpr uint32_t WIDE_PARTS = 8;
 constexpr uint32_t WIDE_PART_STRIDE = 32;
-// where the part counters sit in a stream's scratch counter block (words;
-// word 0 is the packet kernels' counter, word 1 the stack-overflow flag)
-constexpr uint32_t WIDE_PARTS_AT = 32;
-// the part counters, then the count of rays handed over (TailRec): cleared together
-constexpr uint32_t WIDE_COUNTERS = WIDE_PARTS * WIDE_PART_STRIDE + 1;
+// where the counters sit in a stream's scratch counter block (words; word 0
+// is the packet kernels' counter, word 1 the stack-overflow flag)
+constexpr uint32_t WIDE_PARTS_AT = 64;
+// the work counters, then the count of rays handed over (TailRec): cleared together
+constexpr uint32_t WIDE_TAIL = WIDE_PARTS * WIDE_PART_STRIDE;
+constexpr uint32_t WIDE_COUNTERS = WIDE_TAIL + 1;
 static_assert(WIDE_PARTS_AT + WIDE_COUNTERS <= TRACE_COUNTER_WORDS, "scratch counter block");
 static_assert(WIDE_COUNTERS <= TRACE_PART_WORDS, "a caller's own counters");
 
@@ -471,6 +482,8 @@ struct TailView {
     uint32_t cap = 0, lanes = 0;
 };
 
+__device__ __forceinline__ uint32_t min64(uint64_t a, uint32_t b) { return a < b ? (uint32_t)a : b; }
+
 template <bool ANY, bool SEG, bool CQ, int STK_WIDE>
 __global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) void k_trace_wide(SceneView sv, Ray* rays, uint32_t n_host,
                                                           const uint32_t* n_dev, Hit* hits,
@@ -489,17 +502,19 @@ __global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) 
     const uint32_t tid = threadIdx.x;
     const uint32_t gtid = blockIdx.x * blockDim.x + tid;
     const uint32_t total = gridDim.x * blockDim.x;
-    // Work is claimed in chunks (WIDE_CHUNK rays with plenty of rays per
-    // lane, else 64) from WIDE_PARTS counters, one per contiguous part of
-    // the rays: a wave starts on its XCD's part (blocks are dealt to the 8
-    // XCDs in turn), so neighbouring rays share an L2 and the claims spread
-    // over eight addresses, and moves on to the next part when its part is
-    // used up.  A part's counter only grows: a part found used up stays so.
+    // The work: a first chunk of ids for each wave by its place in the launch,
+    // the rest in chunks from WIDE_PARTS counters (see there); a wave starts
+    // with its XCD's counter (blocks are dealt to the 8 XCDs in turn) and
+    // moves on to the next when that has no chunk left.
     const uint32_t nparts = (gridDim.x % WIDE_PARTS == 0u) ? WIDE_PARTS : 1u;
-    const uint32_t chunk = (uint64_t)n >= 8ull * total ? WIDE_CHUNK : 64u;
-    uint32_t cur_part = blockIdx.x % nparts, tries = 0;
-    uint32_t res_b = 0, res_e = 0;  // the wave's claimed ids not handed out yet
-    auto part_start = [&](uint32_t q) { return (uint32_t)((uint64_t)n * q / nparts); };
+    const uint32_t chunk = (uint64_t)n >= 32ull * total ? WIDE_CHUNK : 64u;
+    const uint32_t claim0 = min64((uint64_t)(total >> 6) * chunk, n);  // the counters' first id
+    const uint32_t nchunks = (uint32_t)(((uint64_t)(n - claim0) + chunk - 1) / chunk);
+    uint32_t part = blockIdx.x % nparts, tries = nchunks ? 0u : nparts;
+    uint32_t res_b = min64((uint64_t)(gtid >> 6) * chunk, n);  // the wave's ids not handed out yet
+    uint32_t res_e = min64((uint64_t)res_b + chunk, n);
+    res_b = __builtin_amdgcn_readfirstlane(res_b);
+    res_e = __builtin_amdgcn_readfirstlane(res_e);
     const uint32_t lane = __lane_id();
     const unsigned long long lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
 
@@ -547,17 +562,22 @@ __global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) 
                 const uint32_t avail = res_e - res_b;
                 if (avail == 0) {
                     if (tries >= nparts) break;
+                    uint32_t* ctr = counter + WIDE_PART_STRIDE * part;
+                    const uint32_t mine_n = nchunks > part ? (nchunks - part + nparts - 1) / nparts : 0u;
                     uint32_t b = 0;
-                    if (lane == 0) b = atomicAdd(counter + WIDE_PART_STRIDE * cur_part, chunk);
-                    b = __builtin_amdgcn_readfirstlane(__shfl(b, 0));
-                    const uint32_t p0 = part_start(cur_part), plen = part_start(cur_part + 1) - p0;
-                    if (b >= plen) {
-                        cur_part = cur_part + 1 == nparts ? 0u : cur_part + 1;
+                    // another XCD's counter: a look first, most are used up by then
+                    if (tries) b = __hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    if (__builtin_amdgcn_readfirstlane(b) < mine_n) {
+                        if (lane == 0) b = atomicAdd(ctr, 1u);
+                    }
+                    b = __builtin_amdgcn_readfirstlane(b);
+                    if (b >= mine_n) {
+                        part = part + 1 == nparts ? 0u : part + 1;
                         ++tries;
                         continue;
                     }
-                    res_b = p0 + b;
-                    res_e = p0 + (plen - b < chunk ? plen : b + chunk);
+                    res_b = claim0 + (b * nparts + part) * chunk;
+                    res_e = min64((uint64_t)res_b + chunk, n);
                     continue;
                 }
                 const uint32_t pre = (uint32_t)__popcll(pend & lt_mask);
@@ -1988,7 +2008,7 @@ static TailView make_tail(bool any, const SceneView& s, TraceScratch* scr, size_
     if (cap < waves || at + tail_bytes(cap) > scr->spill_bytes) return t;
     t.recs = reinterpret_cast<TailRec*>((uint8_t*)scr->spill + at);
     t.stk = reinterpret_cast<int2*>(t.recs + cap);
-    t.count = (scr->parts ? scr->parts : scr->counter + WIDE_PARTS_AT) + WIDE_PARTS * WIDE_PART_STRIDE;
+    t.count = (scr->parts ? scr->parts : scr->counter + WIDE_PARTS_AT) + WIDE_TAIL;
     t.cap = (uint32_t)cap;
     t.lanes = (uint32_t)(cap / waves);
     return t;

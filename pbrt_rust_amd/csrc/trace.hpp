@@ -47,7 +47,7 @@ struct TraceTuning {
 // Scratch owned by the caller (per stream): spill stacks and a block of
 // TRACE_COUNTER_WORDS device words for work counters and the overflow flag.
 constexpr uint32_t TRACE_COUNTER_WORDS = 512;
-constexpr uint32_t TRACE_PART_WORDS = 64;
+constexpr uint32_t TRACE_PART_WORDS = 320;
 struct TraceScratch {
     void* spill = nullptr;       // spill stack entries
     size_t spill_bytes = 0;

@@ -53,3 +53,25 @@ def test_hits_at_nan_distance(per_ray):
         hit = (ref["prim"] != px.NO_HIT) & ~nan
         assert np.array_equal(hits["t"][hit].view(np.uint32), ref["t"][hit].view(np.uint32))
     px.synchronize()
+
+
+@pytest.mark.parametrize("block,bpc", [(64, 1), (256, 1), (128, 3)])
+def test_claims_at_the_edges_of_a_launch(block, bpc):
+    # every ray taken once: counts around the waves' first chunks, the first
+    # claims of each counter and the change of the chunk size
+    v, idx = scenes.random_triangles(3000, 13, 0.05, 0.4)
+    bvh, orc = mesh_pair(v, idx, "sah", 1)
+    lanes = 256 * bpc * block  # of the launch: 256 CUs
+    px.set_tuning("batched", "closest", block, bpc, 60, "ray")
+    px.set_tuning("batched", "any", block, bpc, 60, "ray", lanes=1)
+    try:
+        for n in (63, 65, lanes - 1, lanes, lanes + 1, lanes + 64 * 7 + 1, lanes + 64 * 9, 3 * lanes - 5,
+                  32 * lanes - 1, 32 * lanes + 129):
+            if n > 1 << 20:
+                continue
+            o, d = random_rays(n, n)
+            check_closest(bvh, orc, o, d)
+            check_any(bvh, orc, o, d)
+    finally:
+        px.reset_tuning()
+    px.synchronize()
