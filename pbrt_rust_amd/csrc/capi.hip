@@ -35,11 +35,15 @@ uint32_t g_tuning_gen = 1;
 // the batched path walks them as packets)
 // Defaults from the autotuner (python -m pbrt_rust_amd.autotune --path) on
 // the 1024x1024 direct-lighting and 1920x1080 path-tracing frames: batched
-// closest hit 256 threads, occupancy grid, refill below 60% busy lanes, 8
-// LDS stack entries; occlusion the same with 16 entries.
+// closest hit 256 threads, 7 blocks per CU, refill below 70% busy lanes, 8
+// LDS stack entries; occlusion 256 threads, occupancy grid, refill below 60%,
+// 16 entries.  Closest hit at 5 / 6 / 7 / 8 blocks per CU: the path-tracing
+// frame 11.19 / 11.04 / 11.06 / 11.16 ms, 4M random rays in 1M triangles
+// 2.57 / 2.39 / 2.27 / 2.28; refill at 50 / 60 / 70 / 80% with 7: 11.27 /
+// 11.14 / 11.06 / 11.09 and 2.38 / 2.31 / 2.27 / 2.26.
 static const TraceTuning k_default_tuning[2][3] = {
     {TraceTuning{256, 0, 0, SCHEME_RAY}, TraceTuning{256, 0, 0, SCHEME_RAY}, TraceTuning{256, 0, 0, SCHEME_RAY}},
-    {TraceTuning{256, 0, 60, SCHEME_RAY, 8}, TraceTuning{256, 0, 60, SCHEME_RAY, 16},
+    {TraceTuning{256, 7, 70, SCHEME_RAY, 8}, TraceTuning{256, 0, 60, SCHEME_RAY, 16},
      TraceTuning{128, 8, 0, SCHEME_PACKET}}};
 TraceTuning g_tuning[2][3] = {
     {k_default_tuning[0][0], k_default_tuning[0][1], k_default_tuning[0][2]},

@@ -2037,6 +2037,16 @@ size_t trace_spill_bytes(const SceneView& s, int path, const TraceTuning& tun, u
     return rays > GROUP_MAX ? spill + 256 + tail_bytes(tail_cap(threads)) : spill;
 }
 
+// Waves per CU of an occlusion launch on rays that the caller handed in
+// (their count known at launch), where the tuning leaves it open.  Such rays
+// seldom start next to each other, and with fewer waves their records stay
+// longer in the caches: 4M random segments in 20K / 200K / 1M triangles 768 /
+// 1253 / 1575 us with 32 waves, 656 / 1090 / 1421 with 24, 676 / 1023 / 1342
+// with 20; rays of a pinhole grid 627 / 758 / 797, 652 / 795 / 824 and 691 /
+// 851 / 882.  A renderer's shadow rays (a queue on the device) gain from
+// every wave: 1024x1024x16 direct lighting 5.24, 5.40 and 5.67 ms.
+constexpr int QUERY_WAVES = 24;
+
 template <bool ANY>
 static hipError_t launch(const SceneView& s, Ray* rays, uint32_t n, Hit* hits, uint32_t* occ, uint8_t* occ8,
                          int path, const TraceTuning& tun, TraceScratch* scr, hipStream_t st,
@@ -2098,6 +2108,8 @@ static hipError_t launch(const SceneView& s, Ray* rays, uint32_t n, Hit* hits, u
     }
     const auto kern = cq ? wide_kernel<ANY, false, true>(tun.stack) : wide_kernel<ANY, false, false>(tun.stack);
     int grid = wide_grid(kern, tun);
+    if (ANY && !n_dev && tun.blocks_per_cu <= 0)
+        grid = std::min(grid, device_cu_count() * std::max(1, QUERY_WAVES * 64 / block));
     const uint32_t lv = wide_levels(s, tun.stack);
     const size_t per_block = (size_t)lv * block * sizeof(uint2);
     if (per_block * grid > scr->spill_bytes) {
