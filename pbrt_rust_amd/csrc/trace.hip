@@ -1351,7 +1351,7 @@ __global__ __launch_bounds__(CL_BLOCK) __attribute__((amdgpu_waves_per_eu(6))) v
 
 constexpr int PSTK = 96;  // stack entries per wave of the packet closest-hit kernel below
 constexpr int PWAVES = MAX_BLOCK / 64;
-constexpr int PHITS = 256;  // hits a wave of it collects before it claims a run of the hit list
+constexpr int PHITS = 512;  // hits a wave of it collects before it claims a run of the hit list
 
 // Read-only scene data seen through the constant address space: a load from
 // a wave-uniform address then goes through the scalar cache (s_load) rather
@@ -1384,8 +1384,10 @@ __device__ __forceinline__ float4 cload4(const void* p, uint32_t k) {
 // misses ends its path here -- zero radiance written to co.miss[i], no hit
 // record -- and the wave collects the sample indices of its hits in LDS and
 // moves them to a run of co.list, with one atomic on co.count per PHITS - 64
-// or more of them (and one at its end): an atomic per packet, all on one
-// address, cost 0.7 ms of 3.9 on the 1920x1080x64 path-tracing frame.
+// or more of them (and one a block at its end): an atomic per packet, all on
+// one address, cost 0.7 ms of 3.9 on the 1920x1080x64 path-tracing frame, and
+// one per wave at its end 0.19 ms of the 1.30 of a 480x270x16 one.  (Buffers
+// of 256: 1.120 ms there, of 512: 1.105.)
 //
 // What bounds it: VALU issue.  A packet of that frame visits 5.9 records and
 // 1.3 leaves; it took 1440 VALU instructions at first, 860 now, and the kernel
@@ -1436,13 +1438,9 @@ __global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) 
     // packets in turn: neighbouring pixels share an L2, and every XCD gets
     // a share of every part of the image.  Otherwise waves claim packets
     // from the launch's counter.
-    // the wave's hits so far to a run of co.list
-    auto flush = [&]() {
-        PacketArgsK* A = args();
-        uint32_t b = 0;
-        if (lane == 0) b = atomicAdd(A->co.count, nhit);
-        b = __builtin_amdgcn_readfirstlane(b);
-        uint32_t* to = A->co.list + b;
+    // the wave's hits so far to the run of co.list that starts at b
+    auto flush = [&](uint32_t b) {
+        uint32_t* to = args()->co.list + b;
         for (uint32_t j = lane; j < nhit; j += 64u) to[j] = s_hit[w][j];
         nhit = 0;
     };
@@ -1697,10 +1695,31 @@ __global__ __launch_bounds__(MAX_BLOCK) __attribute__((amdgpu_waves_per_eu(8))) 
             const unsigned long long lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
             if (h) s_hit[w][nhit + (uint32_t)__popcll(hm & lt)] = i;
             nhit += (uint32_t)__popcll(hm);
-            if (nhit > (uint32_t)(PHITS - 64)) flush();
+            if (nhit > (uint32_t)(PHITS - 64)) {
+                uint32_t b = 0;
+                if (lane == 0) b = atomicAdd(co.count, nhit);
+                flush(__builtin_amdgcn_readfirstlane(b));
+            }
         }
     }
-    if (GEN && !SEGS && nhit) flush();
+    if constexpr (GEN && !SEGS) {
+        // what is left, with one claim for the block
+        PacketArgsK* A = args();
+        if (A->co.list) {
+            __shared__ uint32_t s_left[PWAVES + 1];
+            if (lane == 0) s_left[w] = nhit;
+            __syncthreads();
+            uint32_t before = 0, sum = 0;
+            for (uint32_t j = 0; j < wpb; ++j) {
+                before += j < w ? s_left[j] : 0u;
+                sum += s_left[j];
+            }
+            if (sum == 0u) return;
+            if (threadIdx.x == 0) s_left[PWAVES] = atomicAdd(A->co.count, sum);
+            __syncthreads();
+            flush(__builtin_amdgcn_readfirstlane(s_left[PWAVES]) + before);
+        }
+    }
 }
 
 __global__ void k_fill_u32(uint32_t* p, uint32_t v, size_t n) {
