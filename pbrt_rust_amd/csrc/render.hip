@@ -223,7 +223,14 @@ constexpr uint32_t SH_CACHE = 4;
 // scans, 256 / 512 / 1024 threads: direct-lighting frame 8.63 / 8.41 / 8.32
 // ms, path-tracing frame 24.3 / 23.0 / 22.6 ms).
 constexpr int SHADE_B = 512;
-constexpr int VERTEX_B = 1024;
+// The path vertex kernel's block: each of its tiles costs three atomics on one
+// address each, so large batches take blocks of 1024 (1920x1080x64: 1.62 ms a
+// frame, 1.67 with 256 threads), while a batch of fewer paths leaves the chip
+// idle with one such block per CU (480x270x16, 2M: 226 us with 1024, 189 with
+// 512, 188 with 256; batches of up to 2^20 of a render server: 17.9, 13.8 and
+// 12.1 us a launch).
+constexpr int VERTEX_B = 1024, VERTEX_SMALL_B = 256;
+constexpr uint32_t VERTEX_LARGE = 1u << 23;  // paths in the batch
 
 // list (queue form, with its count at n_dev): the samples to shade, those
 // whose camera rays hit (the others ended in the miss pass); entry q is
@@ -740,7 +747,7 @@ __global__ __launch_bounds__(MISS_B) void k_path_miss0(RenderParams P, uint64_t 
 }
 
 // The path vertex kernel.  PSHADE_QUEUE: persistent blocks take tiles of
-// VERTEX_B * PATH_PER paths (PATH_PER consecutive paths a thread) by ticket,
+// VB * PATH_PER paths (PATH_PER consecutive paths a thread) by ticket,
 // and write the tile's shadow and next rays densely, each queue's rays in
 // path order within a run that the tile takes with one atomic on that
 // queue's count (tiles in whatever order they get there: a ray's result does
@@ -748,7 +755,8 @@ __global__ __launch_bounds__(MISS_B) void k_path_miss0(RenderParams P, uint64_t 
 // ticket is a device-scope atomic on one address, so fewer, larger tiles.
 // PSHADE_PLAIN: one path per thread, every path's slot written.
 constexpr uint32_t PATH_PER = 2;
-__global__ __launch_bounds__(VERTEX_B) void k_path_shade(RenderParams P, uint64_t g0, uint32_t bounce, uint32_t cap,
+template <int VB>
+__global__ __launch_bounds__(VB) void k_path_shade(RenderParams P, uint64_t g0, uint32_t bounce, uint32_t cap,
                                                    const uint32_t* q_count, const uint32_t* pid_q,
                                                    const Ray* rays_in, const Hit* hits, PathState* st,
                                                    Ray* rays_out, uint32_t* pid_out, uint32_t* out_count,
@@ -758,7 +766,7 @@ __global__ __launch_bounds__(VERTEX_B) void k_path_shade(RenderParams P, uint64_
     const uint32_t n = q_count ? *q_count : cap;
     const bool fresh = rays_in == nullptr;
     if (mode == PSHADE_PLAIN) {
-        const uint32_t i = blockIdx.x * VERTEX_B + threadIdx.x;
+        const uint32_t i = blockIdx.x * VB + threadIdx.x;
         VertexOut o;
         o.shadow = o.next = false;
         o.contrib = mk3(0, 0, 0);
@@ -771,8 +779,8 @@ __global__ __launch_bounds__(VERTEX_B) void k_path_shade(RenderParams P, uint64_
             rays_out[i] = o.nray;
         }
         uint32_t ts, tn;
-        block_exclusive_scan<VERTEX_B>(o.shadow ? 1u : 0u, &ts);
-        block_exclusive_scan<VERTEX_B>(o.next ? 1u : 0u, &tn);
+        block_exclusive_scan<VB>(o.shadow ? 1u : 0u, &ts);
+        block_exclusive_scan<VB>(o.next ? 1u : 0u, &tn);
         if (threadIdx.x == 0) {
             if (ts) atomicAdd(sh_count, ts);
             if (tn) atomicAdd(out_count, tn);
@@ -780,7 +788,7 @@ __global__ __launch_bounds__(VERTEX_B) void k_path_shade(RenderParams P, uint64_
         return;
     }
     __shared__ uint32_t s_bid, s_es, s_en;
-    constexpr uint32_t TILE = VERTEX_B * PATH_PER;
+    constexpr uint32_t TILE = VB * PATH_PER;
     const uint32_t ntiles = (n + TILE - 1) / TILE;
     if (blockIdx.x >= ntiles) return;  // a short queue: no ticket drawn in vain
     while (true) {
@@ -802,7 +810,7 @@ __global__ __launch_bounds__(VERTEX_B) void k_path_shade(RenderParams P, uint64_
         // one scan for both queues: shadow count in the low half, next in
         // the high half (a tile holds at most 1024 of each)
         uint32_t tot;
-        const uint32_t ex = block_exclusive_scan<VERTEX_B>(cs | (cn << 16), &tot);
+        const uint32_t ex = block_exclusive_scan<VB>(cs | (cn << 16), &tot);
         const uint32_t ts = tot & 0xFFFFu, tn = tot >> 16;
         // the tile's runs of the two queues
         if (threadIdx.x == 0) s_es = ts ? atomicAdd(sh_count, ts) : 0u;
@@ -1826,10 +1834,12 @@ int enqueue_path_batch(const RenderParams& P, const SceneView& sv, WorkBufs& W, 
         }
         a = sg.begin();
         {
-            const uint32_t nb = (n + VERTEX_B - 1) / VERTEX_B;
+            const bool large = n >= VERTEX_LARGE;
+            const uint32_t vb = large ? VERTEX_B : VERTEX_SMALL_B;
+            const uint32_t nb = (n + vb - 1) / vb;
             // queue form: persistent blocks over the live paths' tiles
-            const uint32_t grid = batched ? std::min<uint32_t>(nb, (uint32_t)device_cu_count() * 8u) : nb;
-            hipLaunchKernelGGL(k_path_shade, dim3(grid), dim3(VERTEX_B), 0, st, P, g0, bounce, n,
+            const uint32_t grid = batched ? std::min<uint32_t>(nb, (uint32_t)device_cu_count() * (large ? 8u : 4u)) : nb;
+            hipLaunchKernelGGL(large ? k_path_shade<VERTEX_B> : k_path_shade<VERTEX_SMALL_B>, dim3(grid), dim3(vb), 0, st, P, g0, bounce, n,
                                batched ? (const uint32_t*)cin : (const uint32_t*)nullptr,
                                batched ? (const uint32_t*)pin : (const uint32_t*)nullptr,
                                (fused && bounce == 0) ? (const Ray*)nullptr : rin,

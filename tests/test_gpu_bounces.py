@@ -46,3 +46,17 @@ def test_depths_around_the_counters_places(depth):
                 assert np.array_equal(img.view(np.uint32), plain.view(np.uint32))
                 assert [st[k] for k in keys] == [sp[k] for k in keys]
     r.close()
+
+
+def test_large_and_small_vertex_tiles_agree():
+    # batches of 2^23 paths and more take vertex tiles of 2048 paths, smaller
+    # ones of 512: the same radiance bit for bit
+    scene, cam = mirror_room(), scenes.pinhole(512, 257, cam_pos=(0.3, 0.2, -1.0))
+    r = px.SamplerRenderer(scene, cam, px.StratifiedSampler(8, 8, 5), px.PathIntegrator(3, 3))
+    out = []
+    for chunk in (512 * 257 * 64, (1 << 23) - 64, 1 << 20):
+        r.set_chunk(chunk)
+        img, st = r.render("batched")
+        out.append((img.view(np.uint32).copy(), [st[k] for k in ("camera_rays", "shadow_rays", "extension_rays")]))
+    assert all(np.array_equal(i, out[0][0]) and c == out[0][1] for i, c in out[1:])
+    r.close()
