@@ -38,7 +38,7 @@ uint32_t g_tuning_gen = 1;
 // closest hit 256 threads, 7 blocks per CU, refill below 70% busy lanes, 8
 // LDS stack entries; occlusion 256 threads, occupancy grid, refill below 60%,
 // 16 entries.  Closest hit at 5 / 6 / 7 / 8 blocks per CU: the path-tracing
-// frame 11.19 / 11.04 / 11.06 / 11.16 ms, 4M random rays in 1M triangles
+// frame 11.19 / 11.04 / 11.06 / 11.16 ms, 4M random rays in 500K triangles
 // 2.57 / 2.39 / 2.27 / 2.28; refill at 50 / 60 / 70 / 80% with 7: 11.27 /
 // 11.14 / 11.06 / 11.09 and 2.38 / 2.31 / 2.27 / 2.26.
 static const TraceTuning k_default_tuning[2][3] = {

@@ -1934,6 +1934,7 @@ struct Renderer {
     EventPool events;
     bool octant_sort = false;  // path tracer, batched: octant-sort the extension queue
     bool have_frame = false;   // rgb holds a finished frame
+    bool image_copied = false; // an image has left for the host
     // graph mode, per path: warm after one eager frame; the captured frame
     // and the tuning generation it was captured under
     bool use_graph = false;
@@ -2197,7 +2198,14 @@ static int render_frame(Renderer* R, int path, float* rgb_out, pbrtx_render_stat
     }
     RCHK(hipEventRecord(e_end, st));
     // the image and the counters leave behind the frame's kernels, with no
-    // wait of the host between
+    // wait of the host between; but the first image waits for them: a
+    // process's first such copy makes the runtime create a copy queue, and
+    // with kernels running their waves are saved and restored for it (a
+    // 1024x1024x16 frame's occlusion launch took 9.9 ms instead of 2.9)
+    if (rgb_out && !R->image_copied) {
+        RCHK(hipStreamSynchronize(st));
+        R->image_copied = true;
+    }
     if (rgb_out)
         RCHK(hipMemcpyAsync(rgb_out, R->rgb.p, (size_t)R->P.xres * R->P.yres * 3 * sizeof(float),
                             hipMemcpyDeviceToHost, st));

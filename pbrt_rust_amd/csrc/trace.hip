@@ -413,7 +413,7 @@ __device__ __forceinline__ bool prim_test64(const SceneView& sv, uint32_t pos, c
 // NaN that would not hold: tmax may rise again.  Such a ray starts over and
 // tests nothing early.)
 // Lanes busy per VALU instruction: 49 -> 57 % (occlusion of the 1024x1024x16
-// direct-lighting frame, 3.05 -> 2.82 ms; 4M random rays in 1M triangles: 2.62
+// direct-lighting frame, 3.05 -> 2.82 ms; 4M random rays in 500K triangles: 2.62
 // -> 2.53 ms closest hit), against leaves taken at 25 % of lanes waiting at
 // their first one (no waiting: 3.87 ms; 15 %: 3.52, 35 %: 3.52, 50 %: 3.62,
 // when 25 % took 3.45).  With a leaf put aside: 1 % 3.06 ms, 5 % 2.91, 10 %
@@ -444,8 +444,8 @@ constexpr uint32_t CAM_RUN = 16;
 // One counter, claims of 64 below 8 rays a lane and else 256 -> this:
 // 480x270x16 path tracing (launches of 0.05 to 2M rays) 1.80 -> 1.31 ms,
 // 1920x1080x64 11.77 -> 11.20, 1024x1024x16 direct lighting 5.43 -> 5.26; 4M
-// random rays in 1M triangles 2.61 -> 2.30 ms closest hit, 1.45 -> 1.34
-// occlusion; 2M coherent ones 1.20 -> 0.98 and 1.04 -> 0.80.  Claims of 256:
+// random rays in 500K triangles 2.61 -> 2.30 ms closest hit, 1.45 -> 1.34
+// occlusion; 4M of a pinhole grid in 1M 1.90 -> 1.82 and 1.04 -> 0.80.  Claims of 256:
 // 2.60 ms for those 4M closest hits; always 64: direct lighting 5.30-5.37.
 constexpr uint32_t WIDE_CHUNK = 128;
 constexpr uint32_t WIDE_PARTS = 8;
