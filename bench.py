@@ -282,7 +282,7 @@ def main():
     # VALU issue: SQ_INSTS_VALU of the kernel's dispatch (committed counter
     # pass) against the issue slots of the live launch time at the peak
     # engine clock (each of the 1024 SIMDs issues at most one wave64 VALU
-    # instruction every 4 cycles), so the fraction cannot pass 1; lanes
+    # instruction every 4 cycles; slightly more where some take less); lanes
     # active per VALU instruction from SQ_THREAD_CYCLES_VALU over
     # SQ_ACTIVE_INST_VALU x 64
     issue = None

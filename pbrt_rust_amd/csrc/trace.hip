@@ -10,7 +10,7 @@
 // PATH_PLAIN   one lane per ray, static schedule, the 32-byte reference node
 //              record, box test at pop time (exactly the reference loop), a
 //              per-lane LDS stack of node indices with a global spill.
-// PATH_BATCHED persistent waves pulling rays from a global counter and
+// PATH_BATCHED persistent waves taking rays from shared counters and
 //              refilling idle lanes (wave ballot + prefix rank), 128-byte
 //              four-wide records (two reference levels per fetch).  The four
 //              grandchild boxes are tested when their record is fetched; a
