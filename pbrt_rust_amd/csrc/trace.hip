@@ -1215,7 +1215,8 @@ __global__ __launch_bounds__(CL_BLOCK) __attribute__((amdgpu_waves_per_eu(6))) v
                 const uint32_t nqz = neg2 ? as_u(W2.y) : as_u(W2.x), fqz = neg2 ? as_u(W2.x) : as_u(W2.y);
                 r0 = (int)as_u(W2.z); r1 = (int)as_u(W2.w); r2 = (int)as_u(W3.x); r3 = (int)as_u(W3.y);
                 const uint32_t meta = em >> 24;
-                const float rtmax = one ? tmax0 : r.tmax;  // (one: tmax may rise again before the slot is popped)
+                // (one: no limit, tmax may rise past the ray's own before the slot is popped)
+                const float rtmax = one ? __builtin_inff() : r.tmax;
                 if (wfast) {
                     const CqAxis X = cq_axis_ray(W0.x, em & 0xFFu, r.ox, r.ix);
                     const CqAxis Y = cq_axis_ray(W0.y, (em >> 8) & 0xFFu, r.oy, r.iy);
