@@ -13,6 +13,7 @@ each hit ray's tmax to the hit t, the reference's maxt side effect
 """
 import collections
 import ctypes
+import mmap
 import os
 import warnings
 
@@ -729,53 +730,51 @@ def encode8(rgb):
     return out
 
 
+def _pages(nbytes):
+    """Ordinary memory as bytes, its contents undefined; from 1 MB on a mapping
+    of its own in huge pages, where the system has them (those of a 1920x1080
+    image are made in 1 ms, 4 KB pages in 2-3)."""
+    if nbytes < 1 << 20:
+        return np.empty(nbytes, np.uint8)
+    m = mmap.mmap(-1, nbytes, flags=mmap.MAP_PRIVATE | mmap.MAP_ANONYMOUS)
+    try:
+        m.madvise(mmap.MADV_HUGEPAGE)
+    except (AttributeError, OSError):
+        pass
+    return np.frombuffer(m, np.uint8)
+
+
 class _ImageBlocks:
-    """Page-locked image buffers that a renderer lends to the images it
-    returns: the film is copied straight into one (57 GB/s; 17 through HIP's
-    staging into pageable memory: 2.3 ms of a 1920x1080 frame).  At most two, a
-    buffer coming back when the image (and every view of it) is gone; with
-    both lent out, images are ordinary arrays.  Locking the pages costs 0.4 ms,
-    so an image under 1 MB gets one from the renderer's second frame on.
-    Safe with several threads: the deque hands each buffer to one taker."""
-    LARGE = 1 << 20
+    """Image buffers that a renderer lends to the images it returns, whose
+    pages exist from an earlier frame.  At most two, a buffer coming back when
+    the image (and every view of it) is gone; with both lent out, images have
+    memory of their own.  Safe with several threads: the deque hands each
+    buffer to one taker."""
 
     def __init__(self):
         self.free = collections.deque([None, None])  # None: not allocated yet
-        self.used = self.closed = False
+        self.closed = False
 
     def image(self, shape):
         nbytes = 4 * int(np.prod(shape))
-        first, self.used = not self.used, True
-        if nbytes == 0 or (first and nbytes < self.LARGE):
-            return np.empty(shape, F32)
         try:
             block = self.free.pop()
         except IndexError:
-            return np.empty(shape, F32)
+            return _pages(nbytes).view(F32).reshape(shape)
         if block is None:
-            try:
-                block = _lib.PinnedArray((nbytes,), np.uint8)
-            except _lib.PbrtxError:
-                self.free.appendleft(None)
-                return np.empty(shape, F32)
-        mem = (ctypes.c_char * nbytes).from_address(block.ptr)
+            block = _pages(nbytes)
+        mem = (ctypes.c_char * nbytes).from_address(block.ctypes.data)
         mem.lent = _Lent(self, block)  # lives as long as an array over mem does
         return np.frombuffer(mem, F32).reshape(shape)
 
     def give_back(self, block):
         self.free.append(block)
         if self.closed:
-            self.close()
+            self.free.clear()
 
     def close(self):
         self.closed = True
-        while True:
-            try:
-                block = self.free.pop()
-            except IndexError:
-                return
-            if block is not None:
-                block.free()
+        self.free.clear()
 
 
 class _Lent:
@@ -854,7 +853,7 @@ class SamplerRenderer:
             lib().pbrtx_renderer_destroy(self._h)
             self._h = None
         if hasattr(self, "_images"):
-            self._images.close()  # (a buffer still lent out is released with its image)
+            self._images.close()  # (a buffer still lent out goes with its image)
 
     def __del__(self):
         try:

@@ -17,6 +17,7 @@
 // counter-based sample values, so images match sample for sample.
 #include <hip/hip_runtime.h>
 #include <string.h>
+#include <sys/mman.h>
 
 #include <algorithm>
 #include <chrono>
@@ -1915,6 +1916,73 @@ int enqueue_path_batch(const RenderParams& P, const SceneView& sv, WorkBufs& W, 
 }
 
 // ---- the frame renderer ----------------------------------------------------------
+// An image's way to ordinary host memory: through a ring of page-locked chunks,
+// one filled by the GPU while the host copies another out.  The caller gets
+// ordinary memory, as it may fork with the image or queue copies from it that
+// outlast it; page-locked memory is not inherited by a forked child, and the
+// driver refuses to have it so.  The host's copy bounds it (30 GB/s; one to
+// seven threads more: 25 % less time at best).  A kernel fills the chunks: the
+// copy engine also clears the memory that was freed lately, and for some 15 ms
+// each of its copies then takes 0.1 ms longer; and its first use in a process
+// takes 9 ms.  Frames of 512x512 / 1024x1024 / 1920x1080 of which the GPU needs
+// 0.15 / 0.2 / 0.35 ms, in ms: the first 0.56 / 1.4 / 2.4 with the kernel, 0.99 /
+// 2.7 / 5.4 with the engine, 1.2 / 3.1 / 5.0 through the runtime's own staging;
+// later ones 0.29 / 0.80 / 1.30, 0.31 / 0.78 / 1.37 and 0.42 / 1.2 / 2.4
+// (straight into page-locked memory 0.23 / 0.54 / 1.02).  Eight chunks an image
+// within 256 KB .. 1 MB: fixed chunks of 512 KB, 1 MB, 2 MB 0.29, 0.31, 0.31 ms at
+// 512x512 and 5.2, 4.7, 4.5 at 3840x2160.
+constexpr size_t STAGE_MIN = 1u << 18, STAGE_MAX = 1u << 20;
+constexpr size_t STAGE_SLOTS = 4;
+struct ImageStage {
+    uint8_t* buf = nullptr;
+    hipEvent_t ev[STAGE_SLOTS] = {};
+    hipError_t ensure() {
+        if (buf) return hipSuccess;
+        hipError_t e = hipSuccess;
+        for (size_t k = 0; k < STAGE_SLOTS && e == hipSuccess; ++k)
+            if (!ev[k]) e = hipEventCreateWithFlags(&ev[k], hipEventDisableTiming);
+        return e != hipSuccess ? e : hipHostMalloc((void**)&buf, STAGE_SLOTS * STAGE_MAX, hipHostMallocDefault);
+    }
+    // `bytes` of the device's src (readable to the next 16) to dst, behind the
+    // stream's work; dst holds them on return
+    hipError_t copy(void* dst, const void* src, size_t bytes, hipStream_t st) {
+        const size_t chunk = std::min(STAGE_MAX, std::max(STAGE_MIN, (bytes / 8 + 4095) / 4096 * 4096));
+        const size_t nc = (bytes + chunk - 1) / chunk;
+        auto len = [&](size_t c) { return std::min(chunk, bytes - c * chunk); };
+        for (size_t done = 0, sent = 0; done < nc; ++done) {
+            for (; sent < nc && sent < done + STAGE_SLOTS; ++sent) {
+                const size_t k = sent % STAGE_SLOTS;
+                hipError_t e = copy_bytes(buf + k * STAGE_MAX, (const uint8_t*)src + sent * chunk,
+                                          (len(sent) + 15) / 16 * 16, st);
+                if (e == hipSuccess) e = hipEventRecord(ev[k], st);
+                if (e != hipSuccess) return e;
+            }
+            const size_t k = done % STAGE_SLOTS;
+            const hipError_t e = hipEventSynchronize(ev[k]);
+            if (e != hipSuccess) return e;
+            memcpy((uint8_t*)dst + done * chunk, buf + k * STAGE_MAX, len(done));
+        }
+        return hipSuccess;
+    }
+    void release() {
+        if (buf) (void)hipHostFree(buf);
+        buf = nullptr;
+        for (auto& e : ev) {
+            if (e) (void)hipEventDestroy(e);
+            e = nullptr;
+        }
+    }
+};
+// Memory that the runtime does not know: neither the device's nor page-locked.
+static bool ordinary_memory(const void* p) {
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return a.type == hipMemoryTypeUnregistered;
+}
+
 struct Renderer {
     RenderScene sc;
     RenderParams P{};
@@ -1934,7 +2002,8 @@ struct Renderer {
     EventPool events;
     bool octant_sort = false;  // path tracer, batched: octant-sort the extension queue
     bool have_frame = false;   // rgb holds a finished frame
-    bool image_copied = false; // an image has left for the host
+    bool image_sent = false;   // an image has left by the copy engine
+    ImageStage stage;
     // graph mode, per path: warm after one eager frame; the captured frame
     // and the tuning generation it was captured under
     bool use_graph = false;
@@ -2198,17 +2267,28 @@ static int render_frame(Renderer* R, int path, float* rgb_out, pbrtx_render_stat
     }
     RCHK(hipEventRecord(e_end, st));
     // the image and the counters leave behind the frame's kernels, with no
-    // wait of the host between; but the first image waits for them: a
-    // process's first such copy makes the runtime create a copy queue, and
-    // with kernels running their waves are saved and restored for it (a
-    // 1024x1024x16 frame's occlusion launch took 9.9 ms instead of 2.9)
-    if (rgb_out && !R->image_copied) {
-        RCHK(hipStreamSynchronize(st));
-        R->image_copied = true;
+    // wait of the host between
+    if (rgb_out) {
+        const size_t bytes = (size_t)R->P.xres * R->P.yres * 3 * sizeof(float);
+        if (ordinary_memory(rgb_out) && R->stage.ensure() == hipSuccess) {
+            // its pages are made while the kernels run (those of a 1920x1080
+            // image take 1-3 ms); where the system cannot, the copy does it
+            const uintptr_t page = 4095, from = ((uintptr_t)rgb_out + page) & ~page,
+                            to = ((uintptr_t)rgb_out + bytes) & ~page;
+            if (to > from) (void)madvise((void*)from, to - from, 23 /* MADV_POPULATE_WRITE */);
+            RCHK(R->stage.copy(rgb_out, R->rgb.p, bytes, st));
+        } else {
+            // page-locked memory of the caller's (or none left for the stage);
+            // the renderer's first such copy waits: it may make the runtime
+            // create a copy queue, and with kernels running their waves are
+            // saved and restored for it (a 1024x1024x16 frame's occlusion
+            // launch took 9.9 ms instead of 2.9)
+            (void)hipGetLastError();
+            if (!R->image_sent) RCHK(hipStreamSynchronize(st));
+            R->image_sent = true;
+            RCHK(hipMemcpyAsync(rgb_out, R->rgb.p, bytes, hipMemcpyDeviceToHost, st));
+        }
     }
-    if (rgb_out)
-        RCHK(hipMemcpyAsync(rgb_out, R->rgb.p, (size_t)R->P.xres * R->P.yres * 3 * sizeof(float),
-                            hipMemcpyDeviceToHost, st));
     uint32_t c[10];
     if (stats) RCHK(hipMemcpyAsync(c, R->counters.p, sizeof(c), hipMemcpyDeviceToHost, st));
     RCHK(hipStreamSynchronize(st));
@@ -2382,6 +2462,7 @@ int pbrtx_renderer_destroy(pbrtx_renderer* h) {
     R.sc.release();
     R.W.release();
     R.sample_l.release(); R.counters.release(); R.rgb.release(); R.ftab.release(); R.fpos.release(); R.fxyz.release(); R.spos.release(); R.scount.release();
+    R.stage.release();
     for (hipStream_t st : {R.stream, R.stream2})
         if (st) {
             (void)hipStreamSynchronize(st);
