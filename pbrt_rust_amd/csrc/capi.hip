@@ -72,9 +72,28 @@ std::mutex g_scr_mu;
 std::map<hipStream_t, TraceScratch> g_scratch;
 }  // namespace
 
-// Scratch of a stream, grown to at least `spill` bytes.  Calls on one stream
-// are ordered, so one scratch per stream is race free.
-int stream_scratch(hipStream_t st, size_t spill, TraceScratch** out) {
+// Memory for the rays that a stream's launches hand over (25 MB), once and for
+// the stream's life, so that a captured launch may keep it.  A launch does
+// without it, so none is made while the stream is captured, and a capture on
+// another thread goes on.
+static void ensure_tail(hipStream_t st, TraceScratch& s) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (s.tail || hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return;
+    }
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool swapped = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    if (hipMalloc(&s.tail, trace_tail_bytes()) != hipSuccess) {
+        (void)hipGetLastError();
+        s.tail = nullptr;
+    }
+    if (swapped) (void)hipThreadExchangeStreamCaptureMode(&mode);
+}
+
+// Scratch of a stream, its spill grown to at least `spill` bytes.  Calls on one
+// stream are ordered, so one scratch per stream is race free.
+int stream_scratch(hipStream_t st, size_t spill, bool tail, TraceScratch** out) {
     std::lock_guard<std::mutex> lk(g_scr_mu);
     TraceScratch& s = g_scratch[st];
     if (!s.counter) {
@@ -95,6 +114,7 @@ int stream_scratch(hipStream_t st, size_t spill, TraceScratch** out) {
         if (e != hipSuccess) return hip_fail(e, "hipMalloc(spill)");
         s.spill_bytes = spill;
     }
+    if (tail) ensure_tail(st, s);
     *out = &s;
     return PBRTX_OK;
 }
@@ -105,6 +125,7 @@ void release_stream_scratch(hipStream_t st) {
     if (it == g_scratch.end()) return;
     if (it->second.counter) (void)hipFree(it->second.counter);
     if (it->second.spill) (void)hipFree(it->second.spill);
+    if (it->second.tail) (void)hipFree(it->second.tail);
     g_scratch.erase(it);
 }
 
@@ -175,7 +196,7 @@ int run_closest(const SceneView& v, Ray* rays, uint32_t n, Hit* hits, int path, 
     if (path != PATH_PLAIN && path != PATH_BATCHED) return fail(PBRTX_ERR_ARG, "unknown path");
     const TraceTuning& tun = g_tuning[path][0];
     TraceScratch* scr;
-    int rc = stream_scratch(st, trace_spill_bytes(v, path, tun, n), &scr);
+    int rc = stream_scratch(st, trace_spill_bytes(v, path, tun), trace_wants_tail(v, path, n), &scr);
     if (rc) return rc;
     hipError_t e = trace_closest(v, rays, n, hits, path, tun, scr, st);
     if (e != hipSuccess) return hip_fail(e, "trace_closest");
@@ -186,7 +207,7 @@ int run_any(const SceneView& v, const Ray* rays, uint32_t n, uint32_t* occ, int 
     if (path != PATH_PLAIN && path != PATH_BATCHED) return fail(PBRTX_ERR_ARG, "unknown path");
     const TraceTuning& tun = g_tuning[path][1];
     TraceScratch* scr;
-    int rc = stream_scratch(st, trace_spill_bytes(v, path, tun, n), &scr);
+    int rc = stream_scratch(st, trace_spill_bytes(v, path, tun), trace_wants_tail(v, path, n), &scr);
     if (rc) return rc;
     hipError_t e = trace_any(v, rays, n, occ, path, tun, scr, st);
     if (e != hipSuccess) return hip_fail(e, "trace_any");

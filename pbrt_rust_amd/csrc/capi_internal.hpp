@@ -17,7 +17,8 @@ struct DeviceScene {
 
 int fail(int code, const std::string& msg);
 int hip_fail(hipError_t e, const char* what);
-int stream_scratch(hipStream_t st, size_t spill, TraceScratch** out);
+// tail: also memory for the rays handed over, where it can be had.
+int stream_scratch(hipStream_t st, size_t spill, bool tail, TraceScratch** out);
 // Frees the scratch of a stream about to be destroyed (its work finished).
 void release_stream_scratch(hipStream_t st);
 // the render description's split value for a tree built on the device

@@ -1698,12 +1698,12 @@ CamParams cam_params(const RenderParams& P, uint64_t g0) {
     return cp;
 }
 
-size_t render_spill_bytes(const SceneView& sv, int path, uint64_t rays) {
-    const size_t a = trace_spill_bytes(sv, path, g_tuning[path][0], rays);
-    const size_t b = trace_spill_bytes(sv, path, g_tuning[path][1], rays);
+size_t render_spill_bytes(const SceneView& sv, int path) {
+    const size_t a = trace_spill_bytes(sv, path, g_tuning[path][0]);
+    const size_t b = trace_spill_bytes(sv, path, g_tuning[path][1]);
     // camera rays: either scheme the frame's samples per pixel may pick
-    const size_t c = trace_spill_bytes(sv, path, camera_tuning(path, 1), rays);
-    const size_t d = trace_spill_bytes(sv, path, camera_tuning(path, 1u << 20), rays);
+    const size_t c = trace_spill_bytes(sv, path, camera_tuning(path, 1));
+    const size_t d = trace_spill_bytes(sv, path, camera_tuning(path, 1u << 20));
     return std::max(std::max(a, b), std::max(c, d));
 }
 
@@ -2227,10 +2227,11 @@ static int render_frame(Renderer* R, int path, float* rgb_out, pbrtx_render_stat
     // a chunk's largest launch: its paths, or its samples' shadow slots
     const uint64_t most = std::min<uint64_t>(std::max(R->chunk, R->P.spp), R->n_samples) *
                           (R->sc.integrator == 0 ? std::max(R->P.S, 1u) : 1u);
-    const size_t need = render_spill_bytes(R->sc.scene.view, path, most);
-    ICHK(stream_scratch(st, need, &scr));
+    const size_t need = render_spill_bytes(R->sc.scene.view, path);
+    const bool tail = trace_wants_tail(R->sc.scene.view, path, most);
+    ICHK(stream_scratch(st, need, tail, &scr));
     TraceScratch* scr2 = nullptr;
-    if (R->stream2) ICHK(stream_scratch(R->stream2, need, &scr2));
+    if (R->stream2) ICHK(stream_scratch(R->stream2, need, tail, &scr2));
     R->events.used = 0;
     Timing T;
     uint64_t total_camera = 0;

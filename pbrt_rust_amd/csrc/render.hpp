@@ -267,8 +267,7 @@ int enqueue_path_batch(const RenderParams& P, const SceneView& sv, WorkBufs& W, 
                        Stager& sg, const ShadowStream* ss = nullptr);
 // Film::add_sample + write_image over a frame's sample radiance.
 hipError_t enqueue_film(const RenderParams& P, const float4* sample_l, float* rgb, hipStream_t st);
-// Scratch bytes of the traversal launches of a path, of up to `rays` rays each
-// (largest over the kinds).
-size_t render_spill_bytes(const SceneView& sv, int path, uint64_t rays);
+// Spill bytes of the traversal launches of a path (largest over the kinds).
+size_t render_spill_bytes(const SceneView& sv, int path);
 
 }  // namespace px

@@ -106,6 +106,7 @@ struct RenderServer {
     std::vector<std::unique_ptr<RenderScene>> scenes;
     uint64_t scene_bytes = 0;
     size_t spill_need = 0;
+    bool tail_need = false;
     Slot slots[NSLOT];
     std::deque<int> inflight;  // busy slots in launch order
 
@@ -267,10 +268,12 @@ int RenderServer::launch_batches() {
         }
         const RenderScene* scn;
         size_t spill;
+        bool tail;
         {
             std::lock_guard<std::mutex> lk(mu);  // add_scene may grow the table
             scn = scenes[sc].get();
             spill = spill_need;
+            tail = tail_need;
         }
         RenderParams P = scn->base;
         P.segs = S.d_segs;
@@ -287,7 +290,7 @@ int RenderServer::launch_batches() {
         if (e == hipSuccess) e = fill_u32(S.cnt.p, 0u, N_COUNTERS, S.st);
         if (e != hipSuccess) return hip_fail(e, "batch set-up");
         TraceScratch* scr;
-        int rc = stream_scratch(S.st, spill, &scr);
+        int rc = stream_scratch(S.st, spill, tail, &scr);
         if (rc) return rc;
         // (the shadow rays stay on the batch's stream: with three batches
         // in flight, a second stream per batch as in the frame renderer
@@ -362,7 +365,7 @@ int RenderServer::serve_plain(RRequest* r) {
         spill = spill_need;
     }
     TraceScratch* scr;
-    int rc = stream_scratch(S.st, spill, &scr);
+    int rc = stream_scratch(S.st, spill, false, &scr);
     if (rc) return rc;
     r->t_first = now_ms();
     hipError_t e = hipEventRecord(S.start, S.st);
@@ -533,8 +536,8 @@ int pbrtx_render_server_add_scene(pbrtx_render_server* p, const pbrtx_render_des
     RenderServer& s = p->s;
     std::lock_guard<std::mutex> lk(s.mu);
     const SceneView& v = sc->scene.view;
-    s.spill_need = std::max(s.spill_need, std::max(render_spill_bytes(v, PATH_BATCHED, s.cfg.batch_samples),
-                                                   render_spill_bytes(v, PATH_PLAIN, s.cfg.batch_samples)));
+    s.spill_need = std::max(s.spill_need, std::max(render_spill_bytes(v, PATH_BATCHED), render_spill_bytes(v, PATH_PLAIN)));
+    s.tail_need = s.tail_need || trace_wants_tail(v, PATH_BATCHED, s.cfg.batch_samples);
     s.scene_bytes += sc->scene.bytes;
     s.scenes.push_back(std::move(sc));
     *scene_id = (uint32_t)(s.scenes.size() - 1);

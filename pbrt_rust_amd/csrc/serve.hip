@@ -89,6 +89,7 @@ struct Server {
     std::vector<const DeviceScene*> scenes;  // guarded by mu (add_scene runs on client threads)
     uint64_t scene_bytes = 0;
     size_t spill_need = 0;                   // guarded by mu
+    bool tail_need = false;                  // likewise
     // compute, upload and download streams (all default priority)
     hipStream_t s_comp = nullptr, s_up = nullptr, s_down = nullptr;
     // a step's launches (one per scene and kind) go to s_comp and these in
@@ -230,10 +231,12 @@ int Server::launch_step() {
     // pbrtx_server_add_scene may grow the scene table meanwhile (under mu)
     std::vector<const DeviceScene*> scn;
     size_t spill;
+    bool tail;
     {
         std::lock_guard<std::mutex> lk(mu);
         scn = scenes;
         spill = spill_need;
+        tail = tail_need;
     }
     Step st;
     if (!spare.empty()) {
@@ -290,7 +293,7 @@ int Server::launch_step() {
         const hipStream_t stg = g % (size_t)(nside + 1) == 0 ? s_comp : s_side[g % (size_t)(nside + 1) - 1];
         const TraceTuning& tun = g_tuning[PATH_BATCHED][L.any ? 1 : 0];
         TraceScratch* scr;
-        int rc = stream_scratch(stg, spill, &scr);
+        int rc = stream_scratch(stg, spill, tail, &scr);
         if (rc) return rc;
         e = trace_segments(L.sc->view, L.any, ds + L.s0, L.nseg, L.rays, tun, scr, stg);
         if (e != hipSuccess) return hip_fail(e, "trace_segments");
@@ -498,11 +501,12 @@ int pbrtx_server_add_scene(pbrtx_server* p, const pbrtx_scene* scene, uint32_t* 
         return fail(PBRTX_ERR_OOM, "scene exceeds the server's resident-scene budget");
     const TraceTuning& a = g_tuning[PATH_BATCHED][0];
     const TraceTuning& b = g_tuning[PATH_BATCHED][1];
-    const size_t need = std::max(std::max(trace_spill_bytes(scene->s.view, PATH_BATCHED, a, s.cfg.batch_rays),
-                                          trace_spill_bytes(scene->s.view, PATH_BATCHED, b, s.cfg.batch_rays)),
-                                 std::max(trace_spill_bytes(scene->s.view, PATH_PLAIN, g_tuning[PATH_PLAIN][0], 0),
-                                          trace_spill_bytes(scene->s.view, PATH_PLAIN, g_tuning[PATH_PLAIN][1], 0)));
+    const size_t need = std::max(std::max(trace_spill_bytes(scene->s.view, PATH_BATCHED, a),
+                                          trace_spill_bytes(scene->s.view, PATH_BATCHED, b)),
+                                 std::max(trace_spill_bytes(scene->s.view, PATH_PLAIN, g_tuning[PATH_PLAIN][0]),
+                                          trace_spill_bytes(scene->s.view, PATH_PLAIN, g_tuning[PATH_PLAIN][1])));
     s.spill_need = std::max(s.spill_need, need);
+    s.tail_need = s.tail_need || trace_wants_tail(scene->s.view, PATH_BATCHED, s.cfg.batch_rays);
     s.scenes.push_back(&scene->s);
     s.scene_bytes += scene->s.bytes;
     *scene_id = (uint32_t)(s.scenes.size() - 1);

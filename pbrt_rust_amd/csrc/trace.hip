@@ -2011,22 +2011,26 @@ static int closest_lanes(const SceneView& s, uint32_t n, const TraceTuning& tun)
 // The 1920x1080 64-spp path-tracing frame 15.3 -> 14.8 ms; a frame of 12
 // spheres, whose rays are short, 2.39 -> 2.45: not worth its launch there.
 constexpr uint32_t TAIL_LANES = 16;
-constexpr size_t TAIL_CAP = 1u << 18;
+constexpr size_t TAIL_CAP = 1u << 17;  // the waves of 8 blocks of 256 threads a CU
 constexpr uint32_t TAIL_PRIMS = 1u << 12;
 static size_t tail_cap(size_t threads) { return std::min<size_t>(threads / 64 * TAIL_LANES, TAIL_CAP); }
 static size_t tail_bytes(size_t cap) { return cap * (sizeof(TailRec) + TAIL_STK * sizeof(int2)); }
 // The tail of a launch of `grid` blocks whose spill stacks take `used` bytes of
-// the scratch; none if the rest does not hold it (a fixed scratch), or if the
-// several-lane kernel cannot take the rays up.
+// the scratch (a fixed scratch: the rest holds the tail); none if there is no
+// memory for it, or if the several-lane kernel cannot take the rays up.
 static TailView make_tail(bool any, const SceneView& s, TraceScratch* scr, size_t used, int grid, int block) {
     TailView t;
     const uint32_t depth = any ? s.odepth : s.qdepth;
     if (!s.cnodes || !s.prims64 || s.n_prims < TAIL_PRIMS || 3u * (uint64_t)depth + 8u > (uint64_t)(any ? gstk_occlude(8) : gstk_closest(8)))
         return t;
     const size_t waves = (size_t)grid * block / 64, cap = tail_cap((size_t)grid * block);
-    const size_t at = (used + 255) / 256 * 256;
-    if (cap < waves || at + tail_bytes(cap) > scr->spill_bytes) return t;
-    t.recs = reinterpret_cast<TailRec*>((uint8_t*)scr->spill + at);
+    uint8_t* at = (uint8_t*)scr->tail;
+    if (!at && scr->cap_grid) {
+        const size_t o = (used + 255) / 256 * 256;
+        if (o + tail_bytes(cap) <= scr->spill_bytes) at = (uint8_t*)scr->spill + o;
+    }
+    if (!at || cap < waves) return t;
+    t.recs = reinterpret_cast<TailRec*>(at);
     t.stk = reinterpret_cast<int2*>(t.recs + cap);
     t.count = (scr->parts ? scr->parts : scr->counter + WIDE_PARTS_AT) + WIDE_TAIL;
     t.cap = (uint32_t)cap;
@@ -2038,7 +2042,7 @@ size_t trace_any_block_spill(const SceneView& s, const TraceTuning& tun) {
     return (size_t)wide_levels(s, tun.stack) * tun.block * sizeof(uint2);
 }
 
-size_t trace_spill_bytes(const SceneView& s, int path, const TraceTuning& tun, uint64_t rays) {
+size_t trace_spill_bytes(const SceneView& s, int path, const TraceTuning& tun) {
     const int block = tun.block;
     if (path == PATH_PLAIN) {
         size_t threads = (size_t)device_cu_count() * PLAIN_BLOCKS_PER_CU * block;
@@ -2053,9 +2057,13 @@ size_t trace_spill_bytes(const SceneView& s, int path, const TraceTuning& tun, u
                      wide_grid(wide_kernel<false, false, true>(k), t), wide_grid(wide_kernel<true, false, true>(k), t),
                      wide_grid(wide_kernel<false, true, true>(k), t), wide_grid(wide_kernel<true, true, true>(k), t)})
         threads = std::max(threads, g * (size_t)block);
-    const size_t spill = (size_t)wide_levels(s, k) * threads * sizeof(uint2);
-    return rays > GROUP_MAX ? spill + 256 + tail_bytes(tail_cap(threads)) : spill;
+    return (size_t)wide_levels(s, k) * threads * sizeof(uint2);
 }
+
+bool trace_wants_tail(const SceneView& s, int path, uint64_t rays) {
+    return path == PATH_BATCHED && rays > GROUP_MAX && s.cnodes && s.n_prims >= TAIL_PRIMS;
+}
+size_t trace_tail_bytes() { return tail_bytes(TAIL_CAP); }
 
 // Waves per CU of an occlusion launch on rays that the caller handed in
 // (their count known at launch), where the tuning leaves it open.  Such rays

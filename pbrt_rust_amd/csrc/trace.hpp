@@ -51,6 +51,7 @@ constexpr uint32_t TRACE_PART_WORDS = 320;
 struct TraceScratch {
     void* spill = nullptr;       // spill stack entries
     size_t spill_bytes = 0;
+    void* tail = nullptr;        // trace_tail_bytes() for rays handed over, or null: they stay where they run
     uint32_t* counter = nullptr; // TRACE_COUNTER_WORDS words, device
     // a fixed-size scratch: the batched path's persistent grid is cut to the
     // blocks whose spill stacks fit spill_bytes (instead of failing)
@@ -122,10 +123,12 @@ struct TraceSeg {
 // (d_segs in device memory); closest hit (any = false) or occlusion.
 hipError_t trace_segments(const SceneView& s, bool any, const TraceSeg* d_segs, uint32_t nseg, uint32_t total,
                           const TraceTuning& tun, TraceScratch* scr, hipStream_t st);
-// Scratch bytes a launch of up to `rays` rays wants for this scene and tuning:
-// its spill stacks and, where one lane traces a ray, the rays its waves hand
-// over.
-size_t trace_spill_bytes(const SceneView& s, int path, const TraceTuning& tun, uint64_t rays);
+// Number of spill bytes a launch needs for this scene and tuning, whatever its rays.
+size_t trace_spill_bytes(const SceneView& s, int path, const TraceTuning& tun);
+// Whether launches of up to `rays` rays hand their last rays over, through
+// memory of trace_tail_bytes() where there is any.
+bool trace_wants_tail(const SceneView& s, int path, uint64_t rays);
+size_t trace_tail_bytes();
 hipError_t fill_u32(uint32_t* p, uint32_t value, size_t n, hipStream_t st);
 // zeroes a[0..na) and b[0..nb) with one launch
 hipError_t zero2_u32(uint32_t* a, size_t na, uint32_t* b, size_t nb, hipStream_t st);
