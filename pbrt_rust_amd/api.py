@@ -516,9 +516,8 @@ def set_tuning(path, kind, block=256, blocks_per_cu=0, refill_pct=0, scheme="ray
     consecutive rays in equal-sign groups; batched closest hit and camera rays
     only, refused for occlusion).  stack: LDS stack entries per lane
     of the per-ray kernel (8, 16 or 24; None keeps the current depth).
-    lanes: given with kind "any" only, lanes per ray of the batched path's
-    occlusion and closest-hit queries (0 chooses by launch size, 1, 4, 8 or
-    16; None keeps the current choice)."""
+    lanes: batched occlusion only, lanes per ray (0 chooses by launch size,
+    1, 4, 8 or 16; None keeps the current choice)."""
     k = KINDS[kind] if isinstance(kind, str) else int(kind)
     sc = SCHEMES[scheme] if isinstance(scheme, str) else int(scheme)
     check(lib().pbrtx_set_tuning(_path_code(path), k, block, blocks_per_cu, refill_pct, sc))

@@ -415,8 +415,15 @@ int pbrtx_set_stack_depth(int32_t path, int32_t kind, int32_t entries) {
 int pbrtx_set_ray_lanes(int32_t lanes) {
     if (lanes != 0 && lanes != 1 && lanes != 4 && lanes != 8 && lanes != 16)
         return fail(PBRTX_ERR_ARG, "lanes per ray must be 0 (by launch size), 1, 4, 8 or 16");
-    g_tuning[PATH_BATCHED][0].lanes = lanes;
     g_tuning[PATH_BATCHED][1].lanes = lanes;
+    ++g_tuning_gen;
+    return PBRTX_OK;
+}
+
+int pbrtx_set_closest_lanes(int32_t lanes) {
+    if (lanes != 0 && lanes != 1 && lanes != 4 && lanes != 8 && lanes != 16 && lanes != 32)
+        return fail(PBRTX_ERR_ARG, "lanes per ray must be 0 (by launch size), 1, 4, 8, 16 or 32");
+    g_tuning[PATH_BATCHED][0].lanes = lanes;
     ++g_tuning_gen;
     return PBRTX_OK;
 }

@@ -2128,7 +2128,8 @@ static hipError_t launch(const SceneView& s, Ray* rays, uint32_t n, Hit* hits, u
         if (G > 1) {
             const uint32_t lim = (uint32_t)gstk_closest(G) - 3u * s.qdepth;
             const uint32_t gpb = (uint32_t)CL_BLOCK / (uint32_t)G;
-            const unsigned grid = group_grid(((size_t)n + gpb - 1) / gpb, n_dev != nullptr);
+            // (64 n / gpb threads pass the launch limit of 2^32 from 2^27 rays on)
+            const unsigned grid = group_grid(((size_t)n + gpb - 1) / gpb, n_dev != nullptr || n > (1u << 26));
             hipLaunchKernelGGL(closest_group_kernel<false>(G), dim3(grid), dim3(CL_BLOCK), 0, st, s, rays, n, n_dev, hits,
                                lim, err, (const TraceSeg*)nullptr, 0u, TailView{});
             return hipGetLastError();

@@ -31,13 +31,13 @@ def same_hits(hits, rays, ref, ref_maxt, maxt):
 
 
 @pytest.mark.parametrize("maxt", [FMAX, 1.0, 0.2])
-@pytest.mark.parametrize("lanes", [0, 1, 4, 8, 16])
+@pytest.mark.parametrize("lanes", [0, 1, 4, 8, 16, 32])
 def test_limits_end_at_a_nan_hit(lanes, maxt):
     bvh, orc = mesh_pair(*nan_scene(400), "sah")
     _, d = random_rays(3000, 6)
     o = np.zeros_like(d)
     ref = orc.intersect(o, d, 0.0, maxt, nthreads=4)
-    px.lib().pbrtx_set_ray_lanes(lanes)
+    px.lib().pbrtx_set_closest_lanes(lanes)
     try:
         rays = px.RayBatch(o, d, 0.0, maxt)
         past = same_hits(bvh.intersect(rays, "batched"), rays, ref, ref["maxt"], maxt)

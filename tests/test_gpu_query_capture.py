@@ -117,7 +117,7 @@ def test_captured_spills_outlive_larger_calls():
     d = np.tile(np.array([[1, 0, 0]], F32), (3000, 1))
     st = Stream()
     px.set_tuning("batched", "closest", 256, 0, 60, "ray", stack=8)
-    px.lib().pbrtx_set_ray_lanes(1)
+    px.lib().pbrtx_set_closest_lanes(1)
     try:
         q = Query(bvh, o, d, "closest")
         want = q.plain()
