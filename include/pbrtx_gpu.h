@@ -165,7 +165,8 @@ int pbrtx_set_stack_depth(int32_t path, int32_t kind, int32_t entries);
    stack, else one).  No reference counterpart: a launch setting of this
    implementation.  Process-wide setting, kept by pbrtx_set_tuning. */
 int pbrtx_set_ray_lanes(int32_t lanes);
-/* The same for closest-hit queries: 0 (the default), 1, 4, 8, 16 or 32. */
+/* The same for closest-hit queries (by launch size: several lanes up to 3 *
+   2^17 rays): 0 (the default), 1, 4, 8, 16 or 32. */
 int pbrtx_set_closest_lanes(int32_t lanes);
 /* Back to the built-in launch settings (the autotuner's choices on the
    direct-lighting and path-tracing frames).  Unless set explicitly, the

@@ -1906,28 +1906,29 @@ static bool use_compressed(const SceneView& s, const TraceTuning& tun) {
 }
 
 // Lanes per ray of a batched occlusion launch of up to n rays (n: the count,
-// or the capacity when the count is on the device).  Several lanes per ray
-// (k_occlude_group) need the compressed records and a stack bound with room
-// for more than one entry a step.  By launch size, from shadow-ray launches
-// of direct-lighting frames (occlusion ms at 1 / 4 / 8 lanes per ray):
-//   512x512 1 spp, 16K-triangle soup, 62,815 of 262,144:     0.201 / 0.060 / 0.048
-//   512x512 4 spp, the same soup, 251,606 of 1,048,576:       0.266 / 0.127 / 0.106
-//   512x512 16 spp, the same soup, 1,004,569 of 4,194,304:    0.518 / 0.367 / 0.358
-//   512x512 1 spp, 82K-triangle sphere, 413,511 of 1,048,576: 0.311 / 0.173 / 0.161
-//   512x512 4 spp, that sphere, 1,654,016 of 4,194,304:       0.573 / 0.535 / 0.559
-//   1024x1024 16 spp, 1.3M-triangle sphere, 26.5M of 67.1M:   3.47 / 10.7 / 10.7
-// and from launches of random shadow segments (origins in the box, uniform
-// directions, lengths up to half its diagonal) in random-triangle soups,
-// four triangles a leaf (ms at 1 / 4 / 8 lanes per ray):
-//   200K triangles, 131,072 rays:     0.345 / 0.147 / 0.104
-//   200K triangles, 1,048,576 rays:   0.718 / 0.794 / 0.567
-//   200K triangles, 4,194,304 rays:   1.53 / 2.97 / 2.09
-//   2M triangles, 2,097,152 rays:     1.31 / 1.63 / 1.30
-//   2M triangles, 4,194,304 rays:     2.20 / 3.23 / 2.55
-// With few rays per SIMD the per-ray walk is a chain of dependent record
-// loads; with many, the group's idle lanes (a narrow frontier) cost more.
-// Four lanes a ray hold more registers and LDS per lane and lose to eight
-// wherever either wins.
+// or, queue, the capacity when the count is on the device).  Several lanes per
+// ray (k_occlude_group) need the compressed records and a stack bound with room
+// for more than one entry a step.  With few rays per SIMD the per-ray walk is a
+// chain of dependent record loads; with many, the group's idle lanes (a narrow
+// frontier) cost more.  Four lanes a ray hold more registers and LDS per lane
+// and lose to eight wherever either wins.  Launches of segments, four triangles
+// a leaf, us at eight lanes / at one with the last rays handed over.  Random
+// ones (origins in the box, uniform directions, lengths up to half its
+// diagonal):
+//   2K-triangle soup:      524,288 rays 127 / 107;  1,048,576 rays 244 / 143
+//   16K-triangle soup:     262,144 rays 104 / 126;  400,000 rays 147 / 201;  600,000 rays 211 / 205
+//   200K-triangle soup:    262,144 rays 163 / 178;  400,000 rays 229 / 274;  600,000 rays 321 / 296
+//   500K-triangle soup:    262,144 rays 174 / 193;  400,000 rays 257 / 296;  600,000 rays 356 / 323
+//   327K-triangle sphere:  262,144 rays 127 / 125;  400,000 rays 174 / 191;  600,000 rays 245 / 192
+// and of a pinhole grid's:
+//   16K-triangle soup:     400,000 rays 122 / 138;  600,000 rays 174 / 171;  1,048,576 rays 298 / 222
+//   200K-triangle soup:    400,000 rays 198 / 216;  600,000 rays 277 / 237;  1,048,576 rays 450 / 318
+//   327K-triangle sphere:  400,000 rays 133 / 185;  800,000 rays 234 / 250;  1,048,576 rays 306 / 257
+// so the line is at 2^19 rays.  A queue's count is a fraction of its capacity,
+// and its line 2^20: shadow rays of 512x512 frames, 251,137 of 1,048,576 in a
+// 16K soup 121 / 158, 252,357 of 640,000 around an 82K sphere 111 / 128, 413,578
+// of 1,048,576 around that 173 / 154; a burst of 8 served renders 1731 us with
+// 2^20 for its queues and 1851 with the lines of counted launches.
 // While the launch leaves most of the chip's wave slots empty, more lanes a ray
 // still gain (us at 8 / 16 / 32 lanes):
 //   16K triangles:   1,021 rays 17.2 / 13.2 / 13.0;   8,000 rays 18.0 / 14.2 / 17.9;
@@ -1936,14 +1937,14 @@ static bool use_compressed(const SceneView& s, const TraceTuning& tun) {
 //                   32,768 rays 48.1 / 45.0 / 60.3;  50,000 rays 55.2 / 56.9 / 84.2
 //   500K triangles:  4,000 rays 28.5 / 21.3 / 20.0;  32,768 rays 47.6 / 43.0 / 61.9
 // Sixteen lanes end sooner in a small scene, whose records the caches hold.
-constexpr uint32_t GROUP_MAX = 1u << 20;
+constexpr uint32_t QUEUE_GROUP_MAX = 1u << 20, OCCLUDE_GROUP_MAX = 1u << 19, CLOSEST_GROUP_MAX = 3u << 17;
 constexpr uint32_t GROUP32_MAX = 1u << 12;
 static uint32_t group16_max(const SceneView& s) { return s.n_prims >= (1u << 16) ? 1u << 15 : 1u << 14; }
-static int group_lanes(const SceneView& s, uint32_t n, const TraceTuning& tun) {
+static int group_lanes(const SceneView& s, uint32_t n, const TraceTuning& tun, bool queue) {
     if (tun.lanes == 1 || !s.cnodes || !s.prims64) return 1;
     if (3u * (uint64_t)s.odepth + 8u > (uint64_t)gstk_occlude(8)) return 1;
     if (tun.lanes >= 2) return tun.lanes;
-    return n <= GROUP32_MAX ? 32 : n <= group16_max(s) ? 16 : n <= GROUP_MAX ? 8 : 1;
+    return n <= GROUP32_MAX ? 32 : n <= group16_max(s) ? 16 : n <= (queue ? QUEUE_GROUP_MAX : OCCLUDE_GROUP_MAX) ? 8 : 1;
 }
 
 // Blocks of a several-lane launch.  Of a queue whose count is on the device at
@@ -1970,22 +1971,20 @@ static auto closest_group_kernel(int G) -> decltype(&k_closest_group<8, SEG, fal
                      : &k_closest_group<32, SEG, false>;
 }
 // Lanes per ray of a batched closest-hit launch of up to n rays, as
-// group_lanes.  From launches of random rays (origins in the box, uniform
-// directions, no limit) in random-triangle soups (us at 1 / 4 / 8 lanes per ray):
-//   16K triangles, 1,021 rays:         161 /   45 /   30
-//   16K triangles, 150,001 rays:       240 /  144 /  109
-//   16K triangles, 1,000,000 rays:     611 /  782 /  594
-//   200K triangles, 1,021 rays:        259 /   64 /   39
-//   200K triangles, 65,536 rays:       359 /  151 /   94
-//   200K triangles, 150,001 rays:      430 /  231 /  162
-//   200K triangles, 600,000 rays:      745 /  797 /  554
-//   200K triangles, 1,000,000 rays:    944 / 1285 /  883
-//   200K triangles, 2,000,000 rays:   1318 / 2495 / 1713
-//   500K triangles, 1,000,000 rays:   1022 / 1300 /  955
-//   500K triangles, 4,000,000 rays:   2498 / 5073 / 3689
-// The per-ray kernel's time starts at the slowest ray's chain (160-350 us)
-// and grows by about 0.4 ms a million rays; the group's starts at a
-// fraction of it and grows by about 0.9 ms, so the line is near 2^20 rays.
+// group_lanes (us at eight lanes / at one with the last rays handed over; four
+// lanes lose to eight here too).  Random rays (origins in the box, uniform
+// directions, no limit):
+//   2K-triangle soup:      393,216 rays 144 / 128;  1,048,576 rays 344 / 240
+//   16K-triangle soup:     262,144 rays 173 / 184;  400,000 rays 247 / 232;  600,000 rays 353 / 297
+//   200K-triangle soup:    262,144 rays 258 / 270;  400,000 rays 370 / 353;  600,000 rays 510 / 462
+//   500K-triangle soup:    262,144 rays 288 / 306;  400,000 rays 428 / 402;  600,000 rays 591 / 558
+//   327K-triangle sphere:  262,144 rays 179 / 162;  400,000 rays 254 / 210;  600,000 rays 360 / 259
+// and of a pinhole grid:
+//   16K-triangle soup:     262,144 rays 147 / 166;  400,000 rays 195 / 196;  600,000 rays 281 / 270
+//   200K-triangle soup:    262,144 rays 211 / 321;  400,000 rays 289 / 362;  600,000 rays 415 / 411
+//   500K-triangle soup:    262,144 rays 242 / 346;  400,000 rays 340 / 378;  600,000 rays 483 / 446
+//   327K-triangle sphere:  262,144 rays 142 / 153;  400,000 rays 183 / 225;  600,000 rays 253 / 270
+// so the line is at 3 * 2^17 rays.
 // More lanes (us at 8 / 16 / 32):
 //   16K triangles:   1,021 rays 28.1 / 20.5 / 19.5;   8,000 rays 29.7 / 22.7 / 25.7;
 //                   20,000 rays 39.0 / 35.1 / 46.7;  32,768 rays 44.8 / 46.2 / 67.9
@@ -1993,11 +1992,11 @@ static auto closest_group_kernel(int G) -> decltype(&k_closest_group<8, SEG, fal
 //                   32,768 rays 68.7 / 72.2 / 96.0
 //   500K triangles:  4,000 rays 45.6 / 37.2 / 33.7;  20,000 rays 64.8 / 55.0 / 73.4
 constexpr uint32_t CLOSEST16_MAX = 3u << 13;
-static int closest_lanes(const SceneView& s, uint32_t n, const TraceTuning& tun) {
+static int closest_lanes(const SceneView& s, uint32_t n, const TraceTuning& tun, bool queue) {
     if (tun.lanes == 1 || !s.cnodes || !s.prims64) return 1;
     if (3u * (uint64_t)s.qdepth + 8u > (uint64_t)gstk_closest(8)) return 1;
     if (tun.lanes >= 2) return tun.lanes;
-    return n <= GROUP32_MAX ? 32 : n <= CLOSEST16_MAX ? 16 : n <= GROUP_MAX ? 8 : 1;
+    return n <= GROUP32_MAX ? 32 : n <= CLOSEST16_MAX ? 16 : n <= (queue ? QUEUE_GROUP_MAX : CLOSEST_GROUP_MAX) ? 8 : 1;
 }
 
 // Rays that a wave of the per-ray kernel hands over when its launch's rays are
@@ -2061,18 +2060,20 @@ size_t trace_spill_bytes(const SceneView& s, int path, const TraceTuning& tun) {
 }
 
 bool trace_wants_tail(const SceneView& s, int path, uint64_t rays) {
-    return path == PATH_BATCHED && rays > GROUP_MAX && s.cnodes && s.n_prims >= TAIL_PRIMS;
+    return path == PATH_BATCHED && rays > CLOSEST_GROUP_MAX && s.cnodes && s.n_prims >= TAIL_PRIMS;
 }
 size_t trace_tail_bytes() { return tail_bytes(TAIL_CAP); }
 
 // Waves per CU of an occlusion launch on rays that the caller handed in
 // (their count known at launch), where the tuning leaves it open.  Such rays
 // seldom start next to each other, and with fewer waves their records stay
-// longer in the caches: 4M random segments in 20K / 200K / 1M triangles 768 /
-// 1253 / 1575 us with 32 waves, 656 / 1090 / 1421 with 24, 676 / 1023 / 1342
-// with 20; rays of a pinhole grid 627 / 758 / 797, 652 / 795 / 824 and 691 /
-// 851 / 882.  A renderer's shadow rays (a queue on the device) gain from
-// every wave: 1024x1024x16 direct lighting 5.24, 5.40 and 5.67 ms.
+// longer in the caches: 4M random segments in 16K / 200K / 500K triangles 688 /
+// 1197 / 1344 us with 32 waves, 622 / 1090 / 1230 with 24 (20K / 200K / 1M: 676 /
+// 1023 / 1342 with 20, when 24 took 656 / 1090 / 1421).  A caller's coherent
+// segments would gain from the rest of the waves: a pinhole grid's 479 / 697 /
+// 729 us with 32, 494 / 741 / 773 with 24, 6 % at most, less than the random ones
+// lose.  A renderer's shadow rays (a queue on the device) do: 1024x1024x16
+// direct lighting 5.24, 5.40 and 5.67 ms with 32, 24 and 20.
 constexpr int QUERY_WAVES = 24;
 
 template <bool ANY>
@@ -2111,7 +2112,7 @@ static hipError_t launch(const SceneView& s, Ray* rays, uint32_t n, Hit* hits, u
     if (!stack_supported(tun.stack)) return hipErrorInvalidValue;
     const bool cq = use_compressed(s, tun);
     if (ANY && cq && s.prims64) {
-        int G = group_lanes(s, n, tun);
+        const int G = group_lanes(s, n, tun, n_dev != nullptr);
         if (G > 1) {
             const uint32_t lim = (uint32_t)gstk_occlude(G) - 3u * s.odepth;
             const uint32_t gpb = (uint32_t)oc_block(G) / (uint32_t)G;
@@ -2124,7 +2125,7 @@ static hipError_t launch(const SceneView& s, Ray* rays, uint32_t n, Hit* hits, u
         }
     }
     if constexpr (!ANY) {
-        const int G = cq ? closest_lanes(s, n, tun) : 1;
+        const int G = cq ? closest_lanes(s, n, tun, n_dev != nullptr) : 1;
         if (G > 1) {
             const uint32_t lim = (uint32_t)gstk_closest(G) - 3u * s.qdepth;
             const uint32_t gpb = (uint32_t)CL_BLOCK / (uint32_t)G;
@@ -2262,7 +2263,7 @@ hipError_t trace_segments(const SceneView& s, bool any, const TraceSeg* d_segs, 
     const bool cq = use_compressed(s, tun);
     uint32_t* err = scr->counter + 1;
     if (any && cq && s.prims64) {
-        const int G = group_lanes(s, total, tun);
+        const int G = group_lanes(s, total, tun, false);
         if (G > 1) {
             const uint32_t lim = (uint32_t)gstk_occlude(G) - 3u * s.odepth;
             const uint32_t gpb = (uint32_t)oc_block(G) / (uint32_t)G;
@@ -2274,7 +2275,7 @@ hipError_t trace_segments(const SceneView& s, bool any, const TraceSeg* d_segs, 
         }
     }
     if (!any && cq) {
-        const int G = closest_lanes(s, total, tun);
+        const int G = closest_lanes(s, total, tun, false);
         if (G > 1) {
             const uint32_t lim = (uint32_t)gstk_closest(G) - 3u * s.qdepth;
             const uint32_t gpb = (uint32_t)CL_BLOCK / (uint32_t)G;
