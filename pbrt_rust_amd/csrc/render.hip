@@ -2012,6 +2012,7 @@ struct Renderer {
     hipGraphExec_t gexec[2] = {nullptr, nullptr};
     uint32_t gen[2] = {0, 0};
     uint64_t gcamera[2] = {0, 0};
+    void* graph_spill[2] = {nullptr, nullptr};  // the streams' spill stacks that captured frames name
     void drop_graphs() {
         for (int k = 0; k < 2; ++k) {
             if (gexec[k]) (void)hipGraphExecDestroy(gexec[k]);
@@ -2232,6 +2233,10 @@ static int render_frame(Renderer* R, int path, float* rgb_out, pbrtx_render_stat
     ICHK(stream_scratch(st, need, tail, &scr));
     TraceScratch* scr2 = nullptr;
     if (R->stream2) ICHK(stream_scratch(R->stream2, need, tail, &scr2));
+    // spill stacks that have grown (the other path may need more) have moved
+    void* const spill[2] = {scr->spill, scr2 ? scr2->spill : nullptr};
+    if (memcmp(spill, R->graph_spill, sizeof(spill)) != 0) R->drop_graphs();
+    memcpy(R->graph_spill, spill, sizeof(spill));
     R->events.used = 0;
     Timing T;
     uint64_t total_camera = 0;
