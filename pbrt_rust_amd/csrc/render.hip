@@ -809,7 +809,8 @@ __global__ __launch_bounds__(VB) void k_path_shade(RenderParams P, uint64_t g0, 
             cn += o[k].next ? 1u : 0u;
         }
         // one scan for both queues: shadow count in the low half, next in
-        // the high half (a tile holds at most 1024 of each)
+        // the high half
+        static_assert(TILE < 65536u, "at most a tile's paths in either half");
         uint32_t tot;
         const uint32_t ex = block_exclusive_scan<VB>(cs | (cn << 16), &tot);
         const uint32_t ts = tot & 0xFFFFu, tn = tot >> 16;

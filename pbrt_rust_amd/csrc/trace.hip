@@ -432,10 +432,12 @@ constexpr uint32_t CAM_RUN = 16;
 
 // Work claims of the persistent per-ray kernel (see k_trace_wide).  An atomic
 // on one address takes about 11 ns here, whoever asks, so one counter for 8192
-// waves is a queue of 90 us at a launch's start and another at its end, and
-// with claims of 64 rays bounds any launch of cheap rays (0.17 ns a ray).
-// Hence the first chunk of each wave by its place (launches of up to 2^19
-// rays claim nothing), then WIDE_PARTS counters WIDE_PART_STRIDE words apart,
+// waves (8 blocks of 256 threads a CU) is a queue of 90 us at a launch's start
+// and another at its end, and with claims of 64 rays bounds any launch of cheap
+// rays (0.17 ns a ray).  Hence the first chunk of each wave by its place (a
+// launch of no more rays than threads claims nothing: 458,752 closest hit,
+// 393,216 an occlusion query, 524,288 a renderer's shadow rays), then
+// WIDE_PARTS counters WIDE_PART_STRIDE words apart,
 // one per XCD, each handing out every WIDE_PARTS-th chunk: the rays in flight
 // stay neighbours, as with one counter (contiguous parts, each XCD in its own
 // eighth of the rays, were slower).  That allows chunks of 64 rays, which
@@ -922,7 +924,7 @@ __global__ __launch_bounds__(oc_block(G)) __attribute__((amdgpu_waves_per_eu(8))
     static_assert(G >= 2 && G <= 64 && (64 % G) == 0, "a group lies within one wave");
     // (a count on the device never exceeds n_host)
     const uint32_t n = TAIL ? min(*tail.count, tail.cap) : n_dev ? min(*n_dev, n_host) : n_host;
-    const uint32_t gpb = oc_block(G) / G;  // groups per block
+    constexpr uint32_t gpb = oc_block(G) / G;  // groups per block
     const bool whole = !(occ8 || SEG || TAIL);  // the block writes its rays' bits whole
     constexpr int GSTK = gstk_occlude(G);
     __shared__ int32_t s_stk[oc_block(G) / G][GSTK];
@@ -1071,19 +1073,17 @@ __global__ __launch_bounds__(oc_block(G)) __attribute__((amdgpu_waves_per_eu(8))
         }
     }
     if (!whole) return;
-    // bits: the block's rays are gpb consecutive bits (8, 16, 32 or 64), so it
-    // writes them whole -- words that nobody has to clear first
-    __shared__ uint32_t s_bits[2];
-    if (tid < 2) s_bits[tid] = 0u;
+    // bits: the block's rays are 8 or 16 consecutive bits, so it writes them
+    // whole -- words that nobody has to clear first
+    static_assert(gpb == 8u || gpb == 16u, "a block's bits are one or two bytes");
+    __shared__ uint32_t s_bits;
+    if (tid == 0) s_bits = 0u;
     __syncthreads();
-    if (gl == 0 && hit) atomicOr(&s_bits[g >> 5], 1u << (g & 31u));
+    if (gl == 0 && hit) atomicOr(&s_bits, 1u << g);
     __syncthreads();
-    const uint32_t base = blockIdx.x * gpb;
-    if (gpb >= 32u) {
-        if (tid < gpb / 32u && base + 32u * tid < n_host) occ[base / 32u + tid] = s_bits[tid];
-    } else if (tid == 0) {
-        if (gpb == 16u) reinterpret_cast<uint16_t*>(occ)[base / 16u] = (uint16_t)s_bits[0];
-        else reinterpret_cast<uint8_t*>(occ)[base / 8u] = (uint8_t)s_bits[0];
+    if (tid == 0) {
+        if (gpb == 16u) reinterpret_cast<uint16_t*>(occ)[blockIdx.x] = (uint16_t)s_bits;
+        else reinterpret_cast<uint8_t*>(occ)[blockIdx.x] = (uint8_t)s_bits;
     }
 }
 
