@@ -279,19 +279,21 @@ def main():
             calib = {k: tj[k] for k in ("fetch_factor", "write_factor", "copy_fetch_factor") if k in tj}
         except (KeyError, ValueError):
             traffic = prof_t = None
-    # VALU issue: SQ_INSTS_VALU of the kernel's dispatch (committed counter
-    # pass) against the issue slots of the live launch time at the peak
-    # engine clock (each of the 1024 SIMDs issues at most one wave64 VALU
-    # instruction every 4 cycles; slightly more where some take less); lanes
-    # active per VALU instruction from SQ_THREAD_CYCLES_VALU over
-    # SQ_ACTIVE_INST_VALU x 64
+    # VALU instruction rate: SQ_INSTS_VALU of the kernel's dispatch (committed
+    # counter pass) per SIMD and 4 cycles of the live launch time at the peak
+    # engine clock, beside the same rate of the live fma probe.  A wave64 fp32
+    # fma takes 4 cycles of its SIMD, other instructions less, so this is a
+    # ratio of rates and no share of a limit; lanes active per VALU instruction
+    # from SQ_THREAD_CYCLES_VALU over SQ_ACTIVE_INST_VALU x 64
     issue = None
     if os.path.exists(PROFILE_VALU):
         try:
             kv = json.load(open(PROFILE_VALU))["kernels"][kname]
-            slots = kernel_ms * 1e-3 * PEAK_CLOCK_HZ * SIMDS / 4.0
+            slots = PEAK_CLOCK_HZ * SIMDS / 4.0  # a second
+            fma = peaks.get("fp32_fma_tflops")
             issue = {"valu_insts_per_launch": int(kv["valu"]), "salu_insts_per_launch": int(kv["salu"]),
-                     "slots_per_launch": int(slots), "frac": round(kv["valu"] / slots, 4),
+                     "valu_per_4_cycles": round(kv["valu"] / (kernel_ms * 1e-3) / slots, 4),
+                     "fma_probe_valu_per_4_cycles": None if not fma else round(fma * 1e12 / 128.0 / slots, 4),
                      "lane_efficiency": None if kv.get("lane_efficiency") is None else round(kv["lane_efficiency"], 3),
                      "clock_ghz_in_profile": None if kv.get("clock_ghz") is None else round(kv["clock_ghz"], 3),
                      "l2_hit_rate": None if kv.get("l2_hit_rate") is None else round(kv["l2_hit_rate"], 3),
@@ -301,9 +303,6 @@ def main():
     compulsory = n_rays * (32 + out_b)
     achieved = None if traffic is None else traffic / (kernel_ms * 1e-3) / 1e9
     hbm_frac = None if achieved is None else achieved / HBM_PEAK_GBS
-    binding = None
-    if hbm_frac is not None and issue is not None:
-        binding = "valu_issue" if issue["frac"] >= hbm_frac else "hbm"
 
     out = {
         "metric": "Mrays/s batched vs plain GPU kernel; p50/p99 request latency at fixed rate",
@@ -346,7 +345,6 @@ def main():
             "calibration": calib if traffic is not None else None,
             "kernel_ms_per_launch": round(kernel_ms, 4),
             "rays_per_launch": int(n_rays),
-            "binding": binding,
             "issue": issue,
             "compulsory_bytes_per_launch": int(compulsory),
             "bytes_touched": {"per_ray": round(touched_per_ray, 2), "per_launch": int(touched),
