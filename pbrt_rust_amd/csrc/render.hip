@@ -22,6 +22,9 @@
 #include <algorithm>
 #include <chrono>
 #include <cmath>
+#include <mutex>
+#include <new>
+#include <utility>
 #include <vector>
 
 #include "render.hpp"
@@ -1935,14 +1938,17 @@ int enqueue_path_batch(const RenderParams& P, const SceneView& sv, WorkBufs& W, 
 constexpr size_t STAGE_MIN = 1u << 18, STAGE_MAX = 1u << 20;
 constexpr size_t STAGE_SLOTS = 4;
 struct ImageStage {
+    int device = 0;
     uint8_t* buf = nullptr;
     hipEvent_t ev[STAGE_SLOTS] = {};
-    hipError_t ensure() {
-        if (buf) return hipSuccess;
-        hipError_t e = hipSuccess;
+    bool make() {
+        hipError_t e = hipGetDevice(&device);
         for (size_t k = 0; k < STAGE_SLOTS && e == hipSuccess; ++k)
-            if (!ev[k]) e = hipEventCreateWithFlags(&ev[k], hipEventDisableTiming);
-        return e != hipSuccess ? e : hipHostMalloc((void**)&buf, STAGE_SLOTS * STAGE_MAX, hipHostMallocDefault);
+            e = hipEventCreateWithFlags(&ev[k], hipEventDisableTiming);
+        if (e == hipSuccess) e = hipHostMalloc((void**)&buf, STAGE_SLOTS * STAGE_MAX, hipHostMallocDefault);
+        if (e == hipSuccess) return true;
+        (void)hipGetLastError();
+        return false;
     }
     // `bytes` of the device's src (readable to the next 16) to dst, behind the
     // stream's work; dst holds them on return
@@ -1965,15 +1971,45 @@ struct ImageStage {
         }
         return hipSuccess;
     }
-    void release() {
+    ~ImageStage() {
         if (buf) (void)hipHostFree(buf);
-        buf = nullptr;
-        for (auto& e : ev) {
+        for (auto& e : ev)
             if (e) (void)hipEventDestroy(e);
-            e = nullptr;
-        }
     }
 };
+// The stages at rest.  A stage serves one image at a time and any renderer of
+// its device: making one and touching its pages for the first time takes 0.7
+// ms, twice what a new renderer's first 512x512 frame takes without.  At most
+// STAGES_KEPT rest here (32 MB); what more renderers at once have needed is freed.
+constexpr size_t STAGES_KEPT = 8;
+static std::mutex g_stage_mu;
+static ImageStage* g_stages[STAGES_KEPT];
+// null: none to be had
+static ImageStage* take_stage() {
+    int dev = 0;
+    if (hipGetDevice(&dev) == hipSuccess) {
+        std::lock_guard<std::mutex> lk(g_stage_mu);
+        for (auto& s : g_stages)
+            if (s && s->device == dev) return std::exchange(s, nullptr);
+    }
+    ImageStage* s = new (std::nothrow) ImageStage();
+    if (s && !s->make()) {
+        delete s;
+        s = nullptr;
+    }
+    return s;
+}
+static void give_stage(ImageStage* s) {
+    {
+        std::lock_guard<std::mutex> lk(g_stage_mu);
+        for (auto& g : g_stages)
+            if (!g) {
+                g = s;
+                return;
+            }
+    }
+    delete s;
+}
 // Memory that the runtime does not know: neither the device's nor page-locked.
 static bool ordinary_memory(const void* p) {
     hipPointerAttribute_t a;
@@ -2004,7 +2040,6 @@ struct Renderer {
     bool octant_sort = false;  // path tracer, batched: octant-sort the extension queue
     bool have_frame = false;   // rgb holds a finished frame
     bool image_sent = false;   // an image has left by the copy engine
-    ImageStage stage;
     // graph mode, per path: warm after one eager frame; the captured frame
     // and the tuning generation it was captured under
     bool use_graph = false;
@@ -2277,20 +2312,24 @@ static int render_frame(Renderer* R, int path, float* rgb_out, pbrtx_render_stat
     // wait of the host between
     if (rgb_out) {
         const size_t bytes = (size_t)R->P.xres * R->P.yres * 3 * sizeof(float);
-        if (ordinary_memory(rgb_out) && R->stage.ensure() == hipSuccess) {
+        ImageStage* const stage = ordinary_memory(rgb_out) ? take_stage() : nullptr;
+        if (stage) {
             // its pages are made while the kernels run (those of a 1920x1080
             // image take 1-3 ms); where the system cannot, the copy does it
             const uintptr_t page = 4095, from = ((uintptr_t)rgb_out + page) & ~page,
                             to = ((uintptr_t)rgb_out + bytes) & ~page;
             if (to > from) (void)madvise((void*)from, to - from, 23 /* MADV_POPULATE_WRITE */);
-            RCHK(R->stage.copy(rgb_out, R->rgb.p, bytes, st));
+            const hipError_t e = stage->copy(rgb_out, R->rgb.p, bytes, st);
+            // (a chunk may still be on its way after an error: the stage is then
+            // no one's)
+            if (e == hipSuccess || hipStreamSynchronize(st) == hipSuccess) give_stage(stage);
+            RCHK(e);
         } else {
-            // page-locked memory of the caller's (or none left for the stage);
+            // page-locked memory of the caller's (or none left for a stage);
             // the renderer's first such copy waits: it may make the runtime
             // create a copy queue, and with kernels running their waves are
             // saved and restored for it (a 1024x1024x16 frame's occlusion
             // launch took 9.9 ms instead of 2.9)
-            (void)hipGetLastError();
             if (!R->image_sent) RCHK(hipStreamSynchronize(st));
             R->image_sent = true;
             RCHK(hipMemcpyAsync(rgb_out, R->rgb.p, bytes, hipMemcpyDeviceToHost, st));
@@ -2469,7 +2508,6 @@ int pbrtx_renderer_destroy(pbrtx_renderer* h) {
     R.sc.release();
     R.W.release();
     R.sample_l.release(); R.counters.release(); R.rgb.release(); R.ftab.release(); R.fpos.release(); R.fxyz.release(); R.spos.release(); R.scount.release();
-    R.stage.release();
     for (hipStream_t st : {R.stream, R.stream2})
         if (st) {
             (void)hipStreamSynchronize(st);

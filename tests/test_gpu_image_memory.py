@@ -2,6 +2,7 @@
 too, filled through page-locked chunks -- images of every length around the
 chunks' against the same frame copied straight into page-locked memory."""
 import os
+import threading
 
 import numpy as np
 import pytest
@@ -69,3 +70,24 @@ def test_images_around_the_chunks_lengths(pixels):
     assert np.array_equal(room[5:-11].copy().view(np.uint32), straight.array.view(np.uint32))
     assert (room[:5] == 0xA5).all() and (room[-11:] == 0xA5).all()
     r.close()
+
+
+def test_more_renderers_at_once_than_stages_rest():
+    # each image's copy has a stage of its own, whichever renderer gives or takes it
+    want = [renderer(96 + k, 640).render()[0].copy() for k in range(2)]
+    bad = []
+
+    def work(k):
+        for _ in range(3):
+            r = renderer(96 + k % 2, 640)
+            for _ in range(4):
+                if not np.array_equal(r.render()[0], want[k % 2]):
+                    bad.append(k)
+            r.close()
+
+    ts = [threading.Thread(target=work, args=(k,)) for k in range(12)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not bad
