@@ -2007,11 +2007,21 @@ static int closest_lanes(const SceneView& s, uint32_t n, const TraceTuning& tun,
 //                500K triangles,   4M rays: 2478 / 2381 / 2338 / 2345
 //   occlusion,   200K triangles, 1.2M rays:  718 /  610 /  597 /  606
 //                                  4M rays: 1445 / 1318 / 1303 / 1313
-// The 1920x1080 64-spp path-tracing frame 15.3 -> 14.8 ms; a frame of 12
-// spheres, whose rays are short, 2.39 -> 2.45: not worth its launch there.
+// The 1920x1080 64-spp path-tracing frame 15.3 -> 14.8 ms.  In a small scene the
+// last rays end soon by themselves, and the hand-over costs its launch.  600K and
+// 4M rays, us without / with it:
+//   closest hit, random rays: 4.1K triangles 231 / 224, 699 / 684; 8K 298 / 259, 883 / 839;
+//                             16K 387 / 311, 1110 / 1022; 100K 690 / 445, 1731 / 1528
+//           a pinhole grid's: 4.1K 157 / 174, 501 / 523; 8K 197 / 202, 655 / 669;
+//                             16K 276 / 269, 857 / 851; 100K 505 / 381, 1217 / 1157
+//   occlusion, random ones:   4.1K 135 / 159, 402 / 428; 16K 205 / 203, 635 / 618;
+//                             40K 279 / 241, 848 / 798; 100K 361 / 283, 1097 / 1002
+//           a pinhole grid's: 4.1K 96 / 132, 290 / 326; 16K 144 / 171, 464 / 493;
+//                             40K 192 / 207, 608 / 626; 82K 216 / 194, 415 / 419
+// so the lines are at 2^13 prims for closest hit and 2^15 for occlusion.
 constexpr uint32_t TAIL_LANES = 16;
 constexpr size_t TAIL_CAP = 1u << 17;  // the waves of 8 blocks of 256 threads a CU
-constexpr uint32_t TAIL_PRIMS = 1u << 12;
+constexpr uint32_t CLOSEST_TAIL_PRIMS = 1u << 13, OCCLUDE_TAIL_PRIMS = 1u << 15;
 static size_t tail_cap(size_t threads) { return std::min<size_t>(threads / 64 * TAIL_LANES, TAIL_CAP); }
 static size_t tail_bytes(size_t cap) { return cap * (sizeof(TailRec) + TAIL_STK * sizeof(int2)); }
 // The tail of a launch of `grid` blocks whose spill stacks take `used` bytes of
@@ -2020,7 +2030,7 @@ static size_t tail_bytes(size_t cap) { return cap * (sizeof(TailRec) + TAIL_STK 
 static TailView make_tail(bool any, const SceneView& s, TraceScratch* scr, size_t used, int grid, int block) {
     TailView t;
     const uint32_t depth = any ? s.odepth : s.qdepth;
-    if (!s.cnodes || !s.prims64 || s.n_prims < TAIL_PRIMS || 3u * (uint64_t)depth + 8u > (uint64_t)(any ? gstk_occlude(8) : gstk_closest(8)))
+    if (!s.cnodes || !s.prims64 || s.n_prims < (any ? OCCLUDE_TAIL_PRIMS : CLOSEST_TAIL_PRIMS) || 3u * (uint64_t)depth + 8u > (uint64_t)(any ? gstk_occlude(8) : gstk_closest(8)))
         return t;
     const size_t waves = (size_t)grid * block / 64, cap = tail_cap((size_t)grid * block);
     uint8_t* at = (uint8_t*)scr->tail;
@@ -2060,7 +2070,7 @@ size_t trace_spill_bytes(const SceneView& s, int path, const TraceTuning& tun) {
 }
 
 bool trace_wants_tail(const SceneView& s, int path, uint64_t rays) {
-    return path == PATH_BATCHED && rays > CLOSEST_GROUP_MAX && s.cnodes && s.n_prims >= TAIL_PRIMS;
+    return path == PATH_BATCHED && rays > CLOSEST_GROUP_MAX && s.cnodes && s.n_prims >= CLOSEST_TAIL_PRIMS;
 }
 size_t trace_tail_bytes() { return tail_bytes(TAIL_CAP); }
 

@@ -11,10 +11,10 @@ from gpu_util import F32, FMAX, mesh_pair, random_rays
 pytestmark = pytest.mark.gpu
 
 
-def nan_scene(n):
+def nan_scene(n, lo=0.1, hi=0.6):
     """A soup and two triangles of size 1e-20 with a corner at the origin: for a
     ray from there 1/div is infinite and t = 0 * inf."""
-    v, idx = scenes.random_triangles(n, 5, 0.1, 0.6)
+    v, idx = scenes.random_triangles(n, 5, lo, hi)
     e = 1e-20
     tiny = np.array([[e, 0, 0], [0, e, 0], [0, 0, 0], [0, e, 0], [0, 0, e], [0, 0, 0]], F32)
     return np.concatenate([v, tiny]), np.concatenate([idx, np.arange(6, dtype=np.uint32).reshape(2, 3) + len(v)])
@@ -49,8 +49,8 @@ def test_limits_end_at_a_nan_hit(lanes, maxt):
 
 @pytest.mark.parametrize("maxt", [1.0, 0.2])
 def test_limits_of_rays_handed_over(maxt):
-    # past 2^20 rays and 4096 triangles the last rays go to the several-lane kernel
-    bvh, _ = mesh_pair(*nan_scene(5000), "sah")
+    # past 3 * 2^17 rays and 2^13 triangles the last rays go to the several-lane kernel
+    bvh, _ = mesh_pair(*nan_scene(9000, 0.02, 0.1), "sah")
     n = (1 << 20) + 777
     _, d = random_rays(n, 7)
     o = np.zeros_like(d)

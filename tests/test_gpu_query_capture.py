@@ -84,7 +84,7 @@ def same_on_replays(st, graph, q, want, between=lambda: None):
 @pytest.mark.parametrize("kind", ["closest", "any"])
 @pytest.mark.parametrize("warm", [1000, N])
 def test_a_large_call_captured_after_a_small_one(kind, warm):
-    v, idx = scenes.random_triangles(20000, 3)
+    v, idx = scenes.random_triangles(40000, 3)
     bvh = px.BVHAccelerator([px.Primitive.simple(px.TriangleMesh(None, None, False, idx, v))], 2, "sah")
     st = Stream()
     w = Query(bvh, *random_rays(warm, 4), kind)
@@ -109,7 +109,7 @@ def test_captured_spills_outlive_larger_calls():
     n = 60
     xs = 2.0 ** np.arange(n)
     v = np.concatenate([np.array([[x, 0, 0], [x, 1, 0], [x, 0, 1]]) for x in xs]).astype(F32)
-    sv, _ = scenes.random_triangles(5000, 8)
+    sv, _ = scenes.random_triangles(9000, 8)
     v = np.concatenate([v, sv]).astype(F32)
     idx = np.arange(len(v), dtype=np.uint32).reshape(-1, 3)
     bvh = px.BVHAccelerator([px.Primitive.simple(px.TriangleMesh(None, None, False, idx, v))], 1, "middle")

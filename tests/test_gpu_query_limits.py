@@ -34,7 +34,7 @@ def query(bvh, kind, rec, path):
 
 
 @pytest.mark.parametrize("kind", ["closest", "any"])
-@pytest.mark.parametrize("tris", [40, 3000, 30000])
+@pytest.mark.parametrize("tris", [40, 8000, 9000, 30000, 40000])
 @pytest.mark.parametrize("past", [-1, 0, 1, 77])
 def test_answers_on_either_side(kind, tris, past):
     bvh = soup(tris)
@@ -69,7 +69,7 @@ def test_no_jump_in_time(kind):
 def test_served_launches_past_the_limits(lanes):
     # launches of up to 2^21 rays gathered from requests of odd sizes, whose
     # last rays are handed over (lanes 1: finished where they run)
-    bvhs = [soup(20000, 1), soup(100000, 2)]
+    bvhs = [soup(40000, 1), soup(100000, 2)]
     sizes = [700001, 33, 650077, 1, 131071, 400003, 64, 290001]
     px.lib().pbrtx_set_closest_lanes(lanes)
     px.lib().pbrtx_set_ray_lanes(lanes)
@@ -112,3 +112,50 @@ def test_frames_whose_queues_hand_over(whole):
             assert np.array_equal(img.view(np.uint32), plain.view(np.uint32))
             assert st["shadow_rays"] == sp["shadow_rays"] and st["extension_rays"] == sp["extension_rays"]
     r.close()
+
+
+@pytest.mark.parametrize("kind,tris", [("closest", 4200), ("any", 4200), ("any", 16384)])
+def test_small_scenes_are_not_slowed_by_the_hand_over(kind, tris):
+    # coherent rays through a small scene end soon by themselves: by the rule no
+    # slower than with one lane a ray and no hand-over (it took 1.1 to 1.4 of it)
+    bvh, n = soup(tris), 620000
+    w = int(np.ceil(np.sqrt(n)))
+    k = np.arange(n)
+    d = np.stack([(k % w + 0.5) / w - 0.5, (k // w + 0.5) / w - 0.5, np.full(n, 1.1)], 1).astype(F32)
+    o = np.tile(np.array([0, 0, -3], F32), (n, 1))
+    rec = px.DeviceBuffer.from_array(px.RayBatch(o, d, 0.0, F32(FMAX) if kind == "closest" else F32(3.0)).a)
+    work, out = px.DeviceBuffer(32 * n), px.DeviceBuffer(16 * n)
+    t = px._lib.ctypes.c_float()
+    ms = {0: [], 1: []}
+    try:
+        for lap in range(24):
+            lanes = lap % 2
+            (px.lib().pbrtx_set_closest_lanes if kind == "closest" else px.lib().pbrtx_set_ray_lanes)(lanes)
+            check(px.lib().pbrtx_device_copy(work.ptr, rec.ptr, 32 * n, None))
+            check(px.lib().pbrtx_timer_start(None))
+            (bvh.intersect_device if kind == "closest" else bvh.intersect_p_device)(work.ptr, n, out.ptr)
+            check(px.lib().pbrtx_timer_stop(None, px._lib.ctypes.byref(t)))
+            ms[lanes].append(t.value)
+    finally:
+        px.reset_tuning()
+    assert sorted(ms[0])[5] < 1.06 * sorted(ms[1])[5], (sorted(ms[0])[5], sorted(ms[1])[5])
+
+
+@pytest.mark.parametrize("kind", ["closest", "any"])
+def test_stacks_too_long_to_hand_over(kind):
+    # boxes that all overlap, and rays along z through every one of them: their
+    # stacks outgrow a record of the hand-over, so they end where they run
+    k, n = 33000, (1 << 20) + 1
+    rng = np.random.default_rng(77)
+    z = np.sort(rng.uniform(-1, 1, k))
+    v = np.stack([np.stack([np.full(k, -1), np.full(k, -1), z], 1), np.stack([np.ones(k), np.ones(k), z], 1),
+                  np.stack([np.full(k, -0.95), np.full(k, -1), z], 1)], 1).reshape(-1, 3).astype(F32)
+    idx = np.arange(3 * k, dtype=np.uint32).reshape(-1, 3)
+    bvh = px.BVHAccelerator([px.Primitive.simple(px.TriangleMesh(None, None, False, idx, v))], 2, "sah")
+    rec = records(kind, n, 81)
+    few = rec[::16384]
+    few["ox"], few["oy"], few["oz"] = 0.7, -0.7, -2.0
+    few["dx"], few["dy"], few["dz"] = 1e-4, 1e-4, 1.0
+    few["tmax"] = FMAX
+    for a, b in zip(query(bvh, kind, rec, "plain"), query(bvh, kind, rec, "batched")):
+        assert np.array_equal(a, b)
