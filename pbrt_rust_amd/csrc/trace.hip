@@ -1390,8 +1390,8 @@ __device__ __forceinline__ float4 cload4(const void* p, uint32_t k) {
 // one per wave at its end 0.19 ms of the 1.30 of a 480x270x16 one.  (Buffers
 // of 256: 1.120 ms there, of 512: 1.105.)
 //
-// What bounds it: VALU issue.  A packet of that frame visits 5.9 records and
-// 1.3 leaves; it took 1440 VALU instructions at first, 860 now, and the kernel
+// What bounds it: its VALU instructions.  A packet of that frame visits 5.9
+// records and 1.3 leaves; it took 1440 of them at first, 860 now, and the kernel
 // 4.19 ms, 3.13 now (1024x1024x16 direct lighting: 2870 -> 1770 and 1.38 ->
 // 1.24 ms; 512x512x1: 120 -> 98 us).  What went: plane selects (the loads'
 // addresses carry the signs instead), a branch and a ballot of a branch's
